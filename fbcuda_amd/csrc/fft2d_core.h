@@ -191,17 +191,23 @@ __device__ __forceinline__ void loadColumnsWindowPerLane(const float* src, int s
   });
 }
 
-// Column pass (forward): N/2-point FFTs of the two packed columns, real-input
-// fix-up, packed rows written to the plane buffer.
-template <int N, bool SPLIT = false>
-__device__ __forceinline__ void columnPassForward(c32 (&z0)[N / 2], c32 (&z1)[N / 2], c32* plane,
-                                                  int l) {
-  constexpr int H = N / 2, RS = PlaneCfg<N>::RS;
+// Column pass (forward): N/2-point FFTs of the two packed columns and the real-input
+// fix-up, in registers ...
+template <int N>
+__device__ __forceinline__ void columnTransformForward(c32 (&z0)[N / 2], c32 (&z1)[N / 2],
+                                                       c32 (&p0)[N / 2], c32 (&p1)[N / 2]) {
+  constexpr int H = N / 2;
   regFFT<H, true>(z0);
   regFFT<H, true>(z1);
-  c32 p0[H], p1[H];
   realFixupForward<H>(z0, p0);
   realFixupForward<H>(z1, p1);
+}
+
+// ... and packed rows written to the plane buffer.
+template <int N, bool SPLIT = false>
+__device__ __forceinline__ void storeColumns(const c32 (&p0)[N / 2], const c32 (&p1)[N / 2],
+                                             c32* plane, int l) {
+  constexpr int H = N / 2, RS = PlaneCfg<N>::RS;
   if constexpr (SPLIT) {  // columns l and l + N/2
     c32* dst = plane + l;
     staticFor<H>([&](auto rr) {
@@ -216,6 +222,14 @@ __device__ __forceinline__ void columnPassForward(c32 (&z0)[N / 2], c32 (&z1)[N 
       ldsStore4(dst + r * RS, p0[r], p1[r]);
     });
   }
+}
+
+template <int N, bool SPLIT = false>
+__device__ __forceinline__ void columnPassForward(c32 (&z0)[N / 2], c32 (&z1)[N / 2], c32* plane,
+                                                  int l) {
+  c32 p0[N / 2], p1[N / 2];
+  columnTransformForward<N>(z0, z1, p0, p1);
+  storeColumns<N, SPLIT>(p0, p1, plane, l);
 }
 
 // Row pass: lane l transforms packed row l in place (natural order in and out).

@@ -24,10 +24,19 @@
 // takes two reduction steps per iteration: its 1024/N plane slots hold the BN + FO
 // forward transforms of both steps, so every lane transforms in every iteration
 // and 2 (BN + FO) transforms feed 2 BN FO products (one transform per 4, 8, 16
-// products).  Spectra pass through LDS once, and each lane keeps 64 complex
-// accumulators for its own frequency bins in VGPRs across the whole reduction.
-// Spectral rows 0 and N/2 travel packed as one complex row through the transforms;
-// the accumulators hold them apart.
+// products).  A planes are the (image, tile) pairs of the call, whatever the batch: a
+// workgroup's A planes come from several tiles when the batch is small.
+//
+// The products run on the matrix cores: v_mfma_f32_4x4x1 multiplies sixteen independent
+// 4 x 4 blocks, one block per frequency bin, so a wave accumulates 4 A planes x 4 W planes
+// of sixteen neighbouring bins per instruction, four instructions per complex product,
+// and the bins cost no vector arithmetic (which the transforms need all of).  Spectra pass
+// through LDS once; the 64 complex accumulators of a lane stay in registers across the
+// whole reduction.  Spectral rows 0 and N/2 of a real plane are Hermitian along x: after
+// the row pass they become N "virtual bins" in the place of packed row 0 (x: row 0 at x,
+// N/2 + x: row N/2 at x, and at 0 and N/2 the pairs of real values of each row), which
+// multiply like any other bin except for the two pairs, whose lanes drop the cross terms
+// by a zero factor.
 #include "common.h"
 
 #include <algorithm>
@@ -38,6 +47,7 @@ namespace fbfft_amd {
 namespace {
 
 constexpr int kThreads = 512;
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 struct ConvArgs {
   const fbfft_tile* ins;
@@ -47,7 +57,8 @@ struct ConvArgs {
   int wn[4];  // weight sizes: Cout, Cin, kH, kW
   int batch;
   int numTiles;
-  int splits;  // accGradParameters: workgroups along x sharing one reduction
+  int splits;  // accGradParameters: workgroups sharing one reduction
+  int aGroups, wGroups;  // workgroups along A and W planes
   float scale;
 };
 
@@ -96,241 +107,475 @@ struct ConvCfg {
   static constexpr int BN = FO;                    // A planes per workgroup
   static constexpr int RA = SLOTS / FO;            // A planes per round of inverse transforms
   static constexpr int RS = PlaneCfg<N>::RS;
-  static constexpr int PSZ = H * RS;               // packed plane in LDS (complex)
-  static constexpr int PB = H * N;                 // packed bins per plane
-  static constexpr int GRP = (PB >= kThreads) ? 1 : kThreads / PB;   // lane groups sharing a bin set
-  static constexpr int NBT = (PB >= kThreads) ? PB / kThreads : 1;   // bins per lane
-  static constexpr int FQ = FO / GRP;              // W planes per lane
-  static_assert(BN * FQ * NBT == 64, "64 complex accumulators per lane");
+  // packed plane in LDS (complex), padded so that the product loop's reads - half a wave
+  // takes 8 bins (64 bytes) of four planes at once - meet 64 different banks
+  static constexpr int PSZ = (H * RS + 23) / 32 * 32 + 8;
+  static constexpr int PB = H * N;                 // bins per plane
+  static constexpr int BLOCKS = PB / 16;           // groups of 16 bins, one per MFMA block
+  static constexpr int WAVES = kThreads / 64;
+  static constexpr int NBW = BLOCKS >= WAVES ? BLOCKS / WAVES : 1;  // bin groups per wave
+  static constexpr int SHARE = BLOCKS >= WAVES ? 1 : WAVES / BLOCKS;  // waves sharing a bin group
+  static constexpr int AB = BN / 4 / SHARE;        // blocks of 4 A planes per wave
+  static constexpr int WB = FO / 4;                // blocks of 4 W planes per wave
+  static_assert(PSZ >= H * RS && PSZ % 32 == 8, "plane stride");
+  static_assert(NBW * AB * WB == 16, "64 complex accumulators per lane");
+  static_assert(SPI * BN * T == kThreads / 2, "one half of the waves transforms A planes");
+  static_assert(RA == 4, "a round of inverse transforms takes one block of A planes");
 };
 
-// acc += a (x) w for the pass: a * conj(w) or a * w.  Four chained multiply-adds: formed
-// as a product that is then added, it is six instructions (multiply, multiply-add and
-// add per component - the compiler may not reassociate the sum), and this kernel is
-// bound by the vector instructions it issues.
-template <bool CONJ>
-__device__ __forceinline__ void accumulate(c32& acc, c32 a, c32 w) {
-  acc.x = __builtin_fmaf(a.x, w.x, acc.x);
-  acc.x = __builtin_fmaf(CONJ ? a.y : -a.y, w.y, acc.x);
-  acc.y = __builtin_fmaf(a.y, w.x, acc.y);
-  acc.y = __builtin_fmaf(CONJ ? -a.x : a.x, w.y, acc.y);
+// Makes LDS writes of the whole workgroup visible to it.  Only LDS is fenced: global loads
+// in flight (the next iteration's planes) stay in flight.
+__device__ __forceinline__ void ldsBarrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// split a packed row-0 value into its two real-row spectra
-__device__ __forceinline__ void unpack0(c32 self, c32 other, c32* r0, c32* rN2) {
-  *r0 = c32{0.5f * (self.x + other.x), 0.5f * (self.y - other.y)};
-  *rN2 = c32{0.5f * (self.y + other.y), 0.5f * (other.x - self.x)};
+// The lanes of a plane sit in one wave, whose LDS instructions execute in order: only the
+// compiler has to keep them in program order.
+__device__ __forceinline__ void planeSync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+
+// How the planes of one wave are fetched.  Their windows usually lie in one tensor: then a
+// row's address is a scalar base (step and row) plus a lane's 32-bit offset that never
+// changes, and a load costs no vector arithmetic.
+template <int N>
+struct WaveLoader {
+  // Whole: every window covers the whole transform plane.  Pairs, Singles: the windows cover
+  // the same rows (scalar tests), a lane's two columns as one 8-byte word or as two loads.
+  // Ragged: rows differ from plane to plane.  Scattered: so do strides, or the planes lie
+  // too far apart.
+  enum Mode { Empty, Whole, Pairs, Singles, Ragged, Scattered };
+  const char* base;  // of the wave, lowered so that every lane's offset is positive
+  int rowBytes;
+  unsigned off;      // of the lane's first column in row 0 of its transform plane
+  int mode, first, last;  // the same for the whole wave; Pairs, Singles: rows [first, last)
+  // rows [lo, lo + rows) of the lane's two columns lie in the window; three bytes, because
+  // registers are what this kernel is shortest of
+  unsigned window;
+
+  __device__ __forceinline__ unsigned lo() const { return window & 255u; }
+  __device__ __forceinline__ unsigned rowsA() const { return window >> 8 & 255u; }
+  __device__ __forceinline__ unsigned rowsB() const { return window >> 16; }
+
+  // ref: the lane's plane, valid or not
+  __device__ __forceinline__ void plan(const PlaneRef& ref, int l) {
+    const int xa = 2 * l - ref.padL;
+    const bool va = ref.valid && (unsigned)xa < (unsigned)ref.w;
+    const bool vb = ref.valid && (unsigned)(xa + 1) < (unsigned)ref.w;
+    const unsigned rows = min(max(ref.h, 0), N);
+    window = min((unsigned)ref.padU, (unsigned)N) | (va ? rows << 8 : 0u) | (vb ? rows << 16 : 0u);
+    // the first lane with a plane sets the base
+    const unsigned long long have = __builtin_amdgcn_ballot_w64(ref.valid && ref.h > 0 && ref.w > 0);
+    mode = Empty;
+    if (have == 0) return;
+    const int lead = __builtin_ctzll(have);
+    const unsigned long long p = (unsigned long long)ref.p;
+    const unsigned long long p0 =
+        (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)p, lead) |
+        (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(p >> 32), lead) << 32;
+    const int sy = __builtin_amdgcn_readlane(ref.sy, lead);
+    rowBytes = sy * (int)sizeof(float);
+    // a window starts at most N rows and N columns inside its plane
+    const long lower = ((long)(sy < 0 ? 0 : sy) * N + N) * (long)sizeof(float);
+    const long rel = (long)(p - p0) + lower + ((long)xa - (long)ref.padU * sy) * (long)sizeof(float);
+    base = (const char*)p0 - lower;
+    off = (unsigned)rel;
+    const bool here = (va || vb) && ref.h > 0;
+    const bool near = ref.sx == 1 && ref.sy == sy && sy >= 0 && sy < (1 << 22) && rel >= 0 &&
+                      rel < (1L << 31) - 8 && ref.padU >= 0 && ref.padU <= N;
+    const unsigned lead1 = __builtin_amdgcn_readlane((int)(rows << 8 | lo()), lead);
+    first = lead1 & 255u;
+    last = min(first + (int)(lead1 >> 8), N);
+    // rows on 8-byte boundaries, even left edge and width: the lane's two columns are one
+    // 8-byte word per row, inside or outside the window together
+    const bool pairs = ((sy | ref.padL | ref.w) & 1) == 0 && (p & 7) == 0;
+    const bool whole = window == ((unsigned)N << 8 | (unsigned)N << 16);
+    mode = __builtin_amdgcn_ballot_w64(here && !near) != 0 ? Scattered
+           : __builtin_amdgcn_ballot_w64(here && (rows << 8 | lo()) != lead1) != 0 ? Ragged
+           : __builtin_amdgcn_ballot_w64(here && !pairs) != 0 ? Singles
+           : __builtin_amdgcn_ballot_w64(!whole) != 0 ? Pairs : Whole;
+  }
+
+  // the two columns as z0[j] = (X[2j][x], X[2j+1][x]), x = 2l, and z1 the same for x = 2l + 1.
+  // stepBytes: how far the wave's planes have moved since plan().
+  __device__ __forceinline__ void load(long stepBytes, c32 (&z0)[N / 2], c32 (&z1)[N / 2]) const {
+    typedef float Pair __attribute__((ext_vector_type(2)));
+    typedef const __attribute__((address_space(1))) Pair* GlobalPair;
+    typedef const __attribute__((address_space(1))) float* GlobalFloat;
+    // The empty statements keep scalar base and lane offset apart up to the load, and the
+    // base a running sum (left alone the compiler keeps a scalar offset per row alive across
+    // the whole reduction).
+    unsigned o = off;
+    const char* rowBase = base + stepBytes;
+    auto pin = [&]() __attribute__((always_inline)) {
+      asm volatile("" : "+s"(rowBase));
+      asm volatile("" : "+v"(o));
+    };
+    auto set = [](c32& z, int odd, float v) __attribute__((always_inline)) { (odd ? z.y : z.x) = v; };
+    if (mode == Whole) {
+      staticFor<N>([&](auto yy) {
+        constexpr int y = decltype(yy)::value;
+        pin();
+        const Pair v = *(GlobalPair)(rowBase + o);
+        rowBase += rowBytes;
+        set(z0[y / 2], y % 2, v.x);
+        set(z1[y / 2], y % 2, v.y);
+      });
+    } else {
+      staticFor<N / 2>([&](auto jj) {
+        z0[decltype(jj)::value] = z1[decltype(jj)::value] = c32{0.0f, 0.0f};
+      });
+      if (mode == Pairs) {
+        if (rowsA() != 0) {
+          staticFor<N>([&](auto yy) {
+            constexpr int y = decltype(yy)::value;
+            pin();
+            if (y >= first && y < last) {
+              const Pair v = *(GlobalPair)(rowBase + o);
+              set(z0[y / 2], y % 2, v.x);
+              set(z1[y / 2], y % 2, v.y);
+            }
+            rowBase += rowBytes;
+          });
+        }
+      } else if (mode == Singles) {
+        const char* const rowBase0 = rowBase;
+        if (rowsA() != 0) {
+          staticFor<N>([&](auto yy) {
+            constexpr int y = decltype(yy)::value;
+            pin();
+            if (y >= first && y < last) set(z0[y / 2], y % 2, *(GlobalFloat)(rowBase + o));
+            rowBase += rowBytes;
+          });
+        }
+        rowBase = rowBase0 + sizeof(float);
+        if (rowsB() != 0) {
+          staticFor<N>([&](auto yy) {
+            constexpr int y = decltype(yy)::value;
+            pin();
+            if (y >= first && y < last) set(z1[y / 2], y % 2, *(GlobalFloat)(rowBase + o));
+            rowBase += rowBytes;
+          });
+        }
+      } else if (mode == Ragged) {
+        const unsigned lo = this->lo(), rowsA = this->rowsA(), rowsB = this->rowsB();
+        staticFor<N>([&](auto yy) {
+          constexpr int y = decltype(yy)::value;
+          pin();
+          GlobalFloat p = (GlobalFloat)(rowBase + o);
+          if (y - lo < rowsA) set(z0[y / 2], y % 2, p[0]);
+          if (y - lo < rowsB) set(z1[y / 2], y % 2, p[1]);
+          rowBase += rowBytes;
+        });
+      }
+    }
+  }
+
+  // mode Scattered: every lane its own pointer and strides
+  __device__ __forceinline__ void loadScattered(const PlaneRef& ref, int l, c32 (&z0)[N / 2],
+                                                c32 (&z1)[N / 2]) const {
+    typedef const __attribute__((address_space(1))) float* GlobalFloat;
+    const int xa = 2 * l - ref.padL;
+    const bool va = ref.valid && (unsigned)xa < (unsigned)ref.w;
+    const bool vb = ref.valid && (unsigned)(xa + 1) < (unsigned)ref.w;
+    GlobalFloat p = (GlobalFloat)(ref.p + (long)xa * ref.sx - (long)ref.padU * ref.sy);
+    staticFor<N>([&](auto yy) {
+      constexpr int y = decltype(yy)::value;
+      const bool vy = (unsigned)(y - ref.padU) < (unsigned)ref.h;
+      float a = 0.0f, b = 0.0f;
+      if (vy && va) a = p[0];
+      if (vy && vb) b = p[ref.sx];
+      (y % 2 ? z0[y / 2].y : z0[y / 2].x) = a;
+      (y % 2 ? z1[y / 2].y : z1[y / 2].x) = b;
+      p += ref.sy;
+    });
+  }
+};
 
 template <int N, int PASS>
 __global__ __launch_bounds__(kThreads) void iteratedConvKernel(ConvArgs a) {
   using C = ConvCfg<N>;
   constexpr int H = C::H, T = C::T, SLOTS = C::SLOTS, FO = C::FO, BN = C::BN, RS = C::RS,
-                PSZ = C::PSZ, PB = C::PB, GRP = C::GRP, NBT = C::NBT, FQ = C::FQ, SPI = C::SPI,
-                RA = C::RA;
+                PSZ = C::PSZ, SPI = C::SPI, RA = C::RA, NBW = C::NBW, AB = C::AB, WB = C::WB;
   static_assert((BN + FO) * SPI == SLOTS && BN % RA == 0, "slot layout");
   constexpr bool CONJ = (PASS != 1);
   __shared__ __align__(16) c32 lds[SLOTS * PSZ];
 
   const int t = threadIdx.x;
   const int s = t / T, l = t % T;
-  const int gidx = (GRP > 1) ? t / PB : 0;
-  const int bin0 = (GRP > 1) ? t % PB : t;
+  const int wave = __builtin_amdgcn_readfirstlane(t / 64);
+  const int lane = t % 64;
 
-  const int tile = blockIdx.x;        // passes 0, 1
-  const int w0 = blockIdx.y * FO;     // first W plane (f for passes 0 and 2, c for pass 1)
-  const int a0 = blockIdx.z * BN;     // first A plane (n for passes 0 and 1, c for pass 2)
   const int Cout = a.wn[0], Cin = a.wn[1];
-  const int steps = PASS == 0 ? Cin : PASS == 1 ? Cout : a.numTiles * a.batch;
-  // accGradParameters reduces over every (tile, image) pair; that reduction is cut
-  // into a.splits ranges along blockIdx.x whose results meet in an atomic add
+  const int rows = a.numTiles * a.batch;  // (image, tile) pairs
+  const int steps = PASS == 0 ? Cin : PASS == 1 ? Cout : rows;
+  // Passes 0, 1: one workgroup per (A group, W group).  Pass 2: the reduction is also cut
+  // into a.splits ranges whose results meet in an atomic add.  Workgroups are dealt
+  // round-robin to the 8 XCDs; every XCD takes a contiguous range of logical ids, W groups
+  // fastest, so that the workgroups that transform the same A planes share an L2.
+  const int total = a.splits * a.aGroups * a.wGroups;
+  const int per = (total + 7) / 8;
+  const int logical = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if ((int)blockIdx.x / 8 >= per || logical >= total) return;
+  const int w0 = logical % a.wGroups * FO;                // first W plane
+  const int a0 = logical / a.wGroups % a.aGroups * BN;    // first A plane
   const int perSplit = PASS == 2 ? ((steps + a.splits - 1) / a.splits + SPI - 1) / SPI * SPI : steps;
-  const int stepBegin = PASS == 2 ? (int)blockIdx.x * perSplit : 0;
+  const int stepBegin = PASS == 2 ? logical / (a.wGroups * a.aGroups) * perSplit : 0;
   const int stepEnd = min(steps, stepBegin + perSplit);
 
-  c32 acc[BN][FQ][NBT];
+  // acc[bin group][block of A][block of W]: lane (b, j) of a wave holds, at bin b of the
+  // group, W plane j of the block and its four A planes
+  floatx4 accR[NBW][AB][WB], accI[NBW][AB][WB];
 #pragma unroll
-  for (int i = 0; i < BN; ++i)
+  for (int n = 0; n < NBW; ++n)
 #pragma unroll
-    for (int j = 0; j < FQ; ++j)
+    for (int i = 0; i < AB; ++i)
 #pragma unroll
-      for (int k = 0; k < NBT; ++k) acc[i][j][k] = c32{0.f, 0.f};
+      for (int j = 0; j < WB; ++j) accR[n][i][j] = accI[n][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   c32* plane = lds + s * PSZ;
-  // slot s transforms plane sj of reduction step SPI * it + su
-  const int su = s / (BN + FO), sj = s % (BN + FO);
-  for (int it = stepBegin / SPI; it < (stepEnd + SPI - 1) / SPI; ++it) {
-    // ---- forward transforms of this iteration's A and W planes ----
-    {
-      const int step = SPI * it + su;
-      PlaneRef ref;
-      if (PASS == 0) {
-        ref = sj < BN ? tilePlane(a.ins[tile], a0 + sj, step, a.batch)
-                      : weightPlane(a, w0 + sj - BN, step);
-      } else if (PASS == 1) {
-        ref = sj < BN ? tilePlane(a.outs[tile], a0 + sj, step, a.batch)
-                      : weightPlane(a, step, w0 + sj - BN);
-      } else {
-        // past the last step the tile index is clamped; the plane is zeroed below
-        const int tl = min(step / a.batch, a.numTiles - 1), n = step % a.batch;
-        ref = sj < BN ? tilePlane(a.ins[tl], n, a0 + sj, a.batch)
-                      : tilePlane(a.outs[tl], n, w0 + sj - BN, a.batch);
-      }
-      c32 z0[H], z1[H];
-      if (ref.valid && step < stepEnd) {
-        loadColumnsWindowPerLane<N>(ref.p, ref.sy, ref.sx, ref.h, ref.w, ref.padL, ref.padU, l, z0,
-                                    z1);
-      } else {
-#pragma unroll
-        for (int j = 0; j < H; ++j) z0[j] = z1[j] = c32{0.f, 0.f};
-      }
-      columnPassForward<N>(z0, z1, plane, l);
+  // Slots: A planes of every step first, then W planes, so that each SIMD's two waves are
+  // one of either kind.  Slot s transforms plane sj of reduction step SPI * it + su.
+  const bool isA = s < SPI * BN;
+  const int su = isA ? s / BN : (s - SPI * BN) / FO, sj = isA ? s % BN : (s - SPI * BN) % FO;
+  // (su is the same for the planes of a wave)
+  const int suw = __builtin_amdgcn_readfirstlane(su);
+  // Passes 0 and 1: the wave's planes move by one stride from step to step, and how they are
+  // fetched is planned once.  (Planes whose strides differ - tiles of several tensors - are
+  // planned again at every step, like the tiles of pass 2.)
+  WaveLoader<N> loader;
+  auto planeAt = [&](int step, bool isA, int sj) __attribute__((always_inline)) {
+    if (PASS == 2) {
+      // past the last step the tile index is clamped; the plane is marked absent
+      const int tl = __builtin_amdgcn_readfirstlane(min(step / a.batch, a.numTiles - 1)), n = step % a.batch;
+      return isA ? tilePlane(a.ins[tl], n, a0 + sj, a.batch) : tilePlane(a.outs[tl], n, w0 + sj, a.batch);
     }
-    __syncthreads();
-    rowPassInPlace<N, true>(plane, l);
-    __syncthreads();
+    if (isA) {
+      const int row = a0 + sj;
+      const fbfft_tile& d = (PASS == 0 ? a.ins : a.outs)[row % a.numTiles];
+      return tilePlane(d, row / a.numTiles, step, a.batch);
+    }
+    return PASS == 0 ? weightPlane(a, w0 + sj, step) : weightPlane(a, step, w0 + sj);
+  };
+  long stride = 0;       // floats from step to step
+  int planned = 0;       // steps [0, planned) of the wave's planes follow the plan
+  if (PASS != 2) {
+    int mine = PASS == 0 ? a.ws[1] : a.ws[0], held = steps;
+    if (isA) {
+      const fbfft_tile& d = (PASS == 0 ? a.ins : a.outs)[(a0 + sj) % a.numTiles];
+      mine = d.stride[1];
+      held = d.size[1];
+    }
+    const int stride0 = __builtin_amdgcn_readfirstlane(mine);
+    const bool same = __builtin_amdgcn_ballot_w64(mine != stride0 || held < steps) == 0;
+    loader.plan(planeAt(0, isA, sj), l);
+    stride = stride0;
+    // (an odd stride moves the planes off their 8-byte boundaries)
+    if (same && loader.mode != WaveLoader<N>::Scattered &&
+        (loader.mode == WaveLoader<N>::Singles || loader.mode == WaveLoader<N>::Ragged || stride0 % 2 == 0))
+      planned = steps;
+  }
+  c32 z0[H], z1[H];
+  auto load = [&](int it) __attribute__((always_inline)) {
+    const int step = SPI * it + suw;
+    long stepBytes = (long)step * stride * (long)sizeof(float);
+    // the lane's plane where the plan does not cover the step; past the last step nothing is
+    // there.  (The lane's place is worked out afresh: nothing of this stays in registers.)
+    auto unplanned = [&](int& column) __attribute__((always_inline)) {
+      int tt = t;
+      asm volatile("" : "+v"(tt));
+      const int s2 = tt / T;
+      const bool isA2 = s2 < SPI * BN;
+      column = tt % T;
+      PlaneRef ref = planeAt(step, isA2, (isA2 ? s2 : s2 - SPI * BN) % BN);
+      ref.valid = ref.valid && step < stepEnd;
+      return ref;
+    };
+    int column;
+    if (step >= planned) {
+      const PlaneRef ref = unplanned(column);
+      loader.plan(ref, column);
+      stepBytes = 0;
+    }
+    // (one chain of branches with no early exit: every path sets all of z0 and z1, and the
+    // compiler sees that they need no registers before)
+    if (loader.mode == WaveLoader<N>::Scattered) {
+      const PlaneRef ref = unplanned(column);
+      loader.loadScattered(ref, column, z0, z1);
+    } else {
+      loader.load(stepBytes, z0, z1);
+    }
+  };
 
-    // ---- acc[a][w] += A_a (x) W_w on this lane's bins ----
-    // Packed row 0 holds P[x] = F0[x] + i*FH[x], the Hermitian spectra of the two
-    // real rows 0 and N/2.  Its lanes do not multiply packed values (that takes both
-    // products in every lane, fbfft/FFTIteratedConvolution.cuh:161-186): lane x < N/2
-    // accumulates the row-0 product at x and lane N/2 + x the row-N/2 product at x,
-    // one complex product each like every other bin.  x = 0 carries the real values
-    // at 0 and N/2 of its row as (re, im) and multiplies them separately.
-#pragma unroll 1
-    for (int u = 0; u < SPI; ++u) {
-      const c32* ldsu = lds + u * (BN + FO) * PSZ;
+  // product loop: lane (b, j) supplies plane j of a block of four at bin b of a group
+  const int b16 = lane / 4, j4 = lane % 4;
+  const int group0 = C::SHARE == 1 ? wave * NBW : wave % C::BLOCKS;  // first bin group
+  const int aBlock0 = C::SHARE == 1 ? 0 : wave / C::BLOCKS * AB;     // first block of A planes
+  const int bin0 = 16 * group0 + b16;
+  const int laneBin = bin0 / N * RS + bin0 % N;   // where the lane's bin sits in a plane
+  // ... and bin group n of the wave relative to it (more than one group only at N = 32)
+  auto groupOff = [](int n) { return n / 2 * RS + n % 2 * 16; };
+  static_assert(NBW == 1 || N == 32, "bin groups of a wave");
+  // the bins of real pairs: 0 and N/2 (at N = 32: the first bin of groups 0 and 1)
+  const bool pair = bin0 == 0 || (N < 32 && bin0 == H);
+  const float keep = pair ? 0.f : 1.f;
+
+  const int itBegin = stepBegin / SPI, itEnd = (stepEnd + SPI - 1) / SPI;
+  // (one more turn ahead of the first iteration, which only fetches)
+  for (int it = itBegin - 1; it < itEnd; ++it) {
+    if (it >= itBegin) {
+      // ---- forward transforms of this iteration's A and W planes ----
+      __builtin_amdgcn_s_setprio(0);
+      {
+        c32 p0[H], p1[H];
+        columnTransformForward<N>(z0, z1, p0, p1);
+        ldsBarrier();  // the spectra of the previous iteration are consumed by everybody
+        storeColumns<N>(p0, p1, plane, l);
+      }
+      planeSync();
+      rowPassInPlace<N, true>(plane, l);
+      planeSync();
+      {  // packed row 0, P[x] = F0[x] + i FH[x], to its virtual bins
+        const c32 p = plane[l], m = plane[l == 0 ? H : N - l];
+        planeSync();
+        plane[l] = l == 0 ? c32{p.x, m.x} : c32{0.5f * (p.x + m.x), 0.5f * (p.y - m.y)};
+        plane[H + l] = l == 0 ? c32{p.y, m.y} : c32{0.5f * (p.y + m.y), 0.5f * (m.x - p.x)};
+      }
+      ldsBarrier();
+    }
+    // On every SIMD the W wave takes its products first and goes on to its next transforms
+    // while the A wave multiplies: vector and matrix instructions of the two overlap instead
+    // of taking turns (16 x 32 x 256 x 256 image, 32 filters of 9 x 9: 555 -> 480 us; the
+    // A wave first 510 us, the W wave first throughout 475 us forward but 520 us for the
+    // weight gradient).
+    if (wave >= C::WAVES / 2) __builtin_amdgcn_s_setprio(3);
+    // the next iteration's planes travel under this iteration's products
+    load(it + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (it < itBegin) continue;
+
+    // ---- acc[a][w] += A_a (x) W_w ----
+    // a * conj(w) or a * w as re += ar wr +- ai wi, im += ai wr -+ ar wi; the bins of real
+    // pairs take (ar wr, ai wi): the cross terms' A is zeroed, the second product takes wi
+    // Operands are read one bin group ahead of the instructions that take them; the barriers
+    // keep the compiler from reading all of them first, which spills.
+    struct Operands {
+      c32 a[AB], w[WB];
+    };
+    // (two base addresses and constant offsets: the compiler's own choice is an address per
+    // read, kept alive across the reduction)
+    typedef const __attribute__((address_space(3))) vfloat2* LdsPair;
+    LdsPair baseA = (LdsPair)(lds + (4 * aBlock0 + j4) * PSZ + laneBin);
+    LdsPair baseW = (LdsPair)(lds + (SPI * BN + j4) * PSZ + laneBin);
+    asm volatile("" : "+v"(baseA), "+v"(baseW));
+    auto read = [&](auto gg) __attribute__((always_inline)) {
+      constexpr int u = decltype(gg)::value / NBW, n = decltype(gg)::value % NBW;
+      Operands o;
 #pragma unroll
-      for (int nb = 0; nb < NBT; ++nb) {
-        const int bin = bin0 + kThreads * nb;
-        const int r = bin / N, x = bin % N;
-        c32 wv[FQ];
-        if (r != 0) {
-          const int o = r * RS + x;
+      for (int i = 0; i < AB; ++i) {
+        const vfloat2 v = baseA[(u * BN + 4 * i) * PSZ + groupOff(n)];
+        o.a[i] = c32{v.x, v.y};
+      }
 #pragma unroll
-          for (int q = 0; q < FQ; ++q) wv[q] = ldsu[(BN + gidx + GRP * q) * PSZ + o];
+      for (int j = 0; j < WB; ++j) {
+        const vfloat2 v = baseW[(u * FO + 4 * j) * PSZ + groupOff(n)];
+        o.w[j] = c32{v.x, v.y};
+      }
+      return o;
+    };
+    Operands ops[2];
+    ops[0] = read(std::integral_constant<int, 0>{});
+    staticFor<SPI * NBW>([&](auto gg) {
+      constexpr int g = decltype(gg)::value, n = g % NBW;
+      if constexpr (g + 1 < SPI * NBW) ops[(g + 1) % 2] = read(std::integral_constant<int, g + 1>{});
+      __builtin_amdgcn_sched_barrier(0);
+      const Operands& o = ops[g % 2];
+      constexpr bool mayPair = n < 2;
+      const float cross = mayPair ? keep : 1.f;
+      // (first products of every accumulator, then second ones: no instruction waits for the
+      // one before it)
 #pragma unroll
-          for (int i = 0; i < BN; ++i) {
-            const c32 av = ldsu[i * PSZ + o];
+      for (int i = 0; i < AB; ++i)
 #pragma unroll
-            for (int q = 0; q < FQ; ++q) accumulate<CONJ>(acc[i][q][nb], av, wv[q]);
-          }
-        } else {
-          // Row 0.  v = this lane's real-row spectrum value of a plane: the row-0 or
-          // row-N/2 half of the packed pair (x, N - x), or for x = 0 the two real
-          // values at 0 and N/2 as (re, im).  The real pair must be multiplied
-          // component by component; written as the same four multiply-adds as a
-          // complex product, with the first factor split in (re, 0) and (0, im) and
-          // the second factor's components routed accordingly, so that all lanes of
-          // the row run one instruction stream.
-          const int xx = x & (H - 1);
-          const bool second = x >= H, pair = xx == 0;
-          const int i1 = xx, i2 = pair ? H : N - xx;
-          auto value = [&](const c32* p) __attribute__((always_inline)) {
-            const c32 self = p[i1], other = p[i2];
-            c32 r0, rH;
-            unpack0(self, other, &r0, &rH);
-            const c32 ends = second ? c32{self.y, other.y} : c32{self.x, other.x};
-            const c32 half = second ? rH : r0;
-            return pair ? ends : half;
-          };
-          float w2x[FQ];
+        for (int j = 0; j < WB; ++j) {
+          accR[n][i][j] = __builtin_amdgcn_mfma_f32_4x4x1f32(o.a[i].x, o.w[j].x, accR[n][i][j], 0, 0, 0);
+          accI[n][i][j] = __builtin_amdgcn_mfma_f32_4x4x1f32(o.a[i].y, mayPair && pair ? o.w[j].y : o.w[j].x, accI[n][i][j], 0, 0, 0);
+        }
 #pragma unroll
-          for (int q = 0; q < FQ; ++q) {
-            wv[q] = value(ldsu + (BN + gidx + GRP * q) * PSZ);
-            w2x[q] = pair ? wv[q].y : wv[q].x;
-          }
+      for (int i = 0; i < AB; ++i) {
+        const float ai = (CONJ ? cross : -cross) * o.a[i].y, ar = (CONJ ? -cross : cross) * o.a[i].x;
 #pragma unroll
-          for (int i = 0; i < BN; ++i) {
-            const c32 av = value(ldsu + i * PSZ);
-            const float a1y = pair ? 0.0f : av.y, a2x = pair ? 0.0f : av.x;
-#pragma unroll
-            for (int q = 0; q < FQ; ++q) {
-              c32& to = acc[i][q][nb];
-              to.x = __builtin_fmaf(av.x, wv[q].x, to.x);
-              to.x = __builtin_fmaf(CONJ ? a1y : -a1y, wv[q].y, to.x);
-              to.y = __builtin_fmaf(av.y, w2x[q], to.y);
-              to.y = __builtin_fmaf(CONJ ? -a2x : a2x, wv[q].y, to.y);
-            }
-          }
+        for (int j = 0; j < WB; ++j) {
+          accR[n][i][j] = __builtin_amdgcn_mfma_f32_4x4x1f32(ai, o.w[j].y, accR[n][i][j], 0, 0, 0);
+          accI[n][i][j] = __builtin_amdgcn_mfma_f32_4x4x1f32(ar, o.w[j].y, accI[n][i][j], 0, 0, 0);
         }
       }
-    }
-    __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
+    });
   }
 
-  // ---- inverse transforms, RA A planes x FO W planes per round ----
+  // ---- inverse transforms, RA = 4 A planes (one block) x FO W planes per round ----
   const float norm = (PASS == 2 ? a.scale : 1.0f) / (float)(N * N);
+  // (the lane's place is worked out afresh, so that nothing of it occupies registers above)
+  int te = t;
+  asm volatile("" : "+v"(te));
+  const int se = te / T, le = te % T, je = te % 4, be = te % 64 / 4;
+  c32* planeE = lds + se * PSZ;
+  const int binE = 16 * group0 + be, laneBinE = binE / N * RS + binE % N;
 #pragma unroll
   for (int rd = 0; rd < BN / RA; ++rd) {
-    // Row-0 lanes park their value in the plane's padding (columns N, N+1 of row
-    // x/2: N spare cells per plane) where the partner lane finds it.
+    ldsBarrier();
+    if (C::SHARE == 1 || aBlock0 / AB == rd / AB) {
 #pragma unroll
-    for (int ii = 0; ii < RA; ++ii)
+      for (int n = 0; n < NBW; ++n)
 #pragma unroll
-      for (int q = 0; q < FQ; ++q)
+        for (int j = 0; j < WB; ++j)
 #pragma unroll
-        for (int nb = 0; nb < NBT; ++nb) {
-          const int bin = bin0 + kThreads * nb;
-          const int x = bin % N;
-          const int o = bin < N ? (x / 2) * RS + N + x % 2 : (bin / N) * RS + x;
-          lds[(ii * FO + gidx + GRP * q) * PSZ + o] = acc[RA * rd + ii][q][nb];
-        }
-    __syncthreads();
-    // Row 0 back to its packed form Q[x] = S0[x] + i*SH[x], Q[N-x] = conj(S0[x]) +
-    // i*conj(SH[x]): the lane holding S0[x] fetches SH[x] and writes Q[x], the lane
-    // holding SH[x] fetches S0[x] and writes Q[N-x]; the two real pairs swap halves.
-#pragma unroll
-    for (int nb = 0; nb < NBT; ++nb) {
-      const int bin = bin0 + kThreads * nb;
-      if (bin < N) {
-        const int x = bin, xx = x & (H - 1);
-        const bool second = x >= H;
-        const int px = second ? xx : H + xx;  // partner's x
-        const int src = (px / 2) * RS + N + px % 2;
-        const int dst = xx == 0 ? x : second ? N - xx : x;
-#pragma unroll
-        for (int ii = 0; ii < RA; ++ii)
-#pragma unroll
-          for (int q = 0; q < FQ; ++q) {
-            c32* pl = lds + (ii * FO + gidx + GRP * q) * PSZ;
-            const c32 mine = acc[RA * rd + ii][q][nb];
-            const c32 other = pl[src];
-            c32 v;
-            if (xx == 0)
-              v = second ? c32{other.y, mine.y} : c32{mine.x, other.x};
-            else
-              v = second ? c32{other.x + mine.y, mine.x - other.y}
-                         : c32{mine.x - other.y, mine.y + other.x};
-            pl[dst] = v;
-          }
-      }
+          for (int i = 0; i < 4; ++i)
+            lds[(i * FO + 4 * j + je) * PSZ + laneBinE + groupOff(n)] =
+                c32{accR[n][rd % AB][j][i], accI[n][rd % AB][j][i]};
     }
-    __syncthreads();
-    rowPassInPlace<N, false>(plane, l);
-    __syncthreads();
+    ldsBarrier();
+    {  // virtual bins back to the packed row: Q[x] = S0[x] + i SH[x], Q[N-x] = conj(S0[x]) +
+       // i conj(SH[x]); lane 0 sorts the four real values into Q[0] and Q[N/2]
+      const c32 c0 = planeE[le], cH = planeE[H + le];
+      c32 q = c32{c0.x - cH.y, c0.y + cH.x}, qm = c32{c0.x + cH.y, cH.x - c0.y};
+      if (le == 0) {
+        q = c32{c0.x, cH.x};
+        qm = c32{c0.y, cH.y};
+      }
+      planeSync();
+      planeE[le] = q;
+      planeE[le == 0 ? H : N - le] = qm;
+    }
+    planeSync();
+    rowPassInPlace<N, false>(planeE, le);
+    planeSync();
     {
-      c32 z0[H], z1[H];
-      columnPassInverse<N>(plane, l, z0, z1);
-      const int ai = a0 + RA * rd + s / FO;
-      const int wi = w0 + s % FO;
+      columnPassInverse<N>(planeE, le, z0, z1);
+      const int ai = a0 + RA * rd + se / FO;
+      const int wi = w0 + se % FO;
       PlaneRef ref;
-      if (PASS == 0)
-        ref = tilePlane(a.outs[tile], ai, wi, a.batch);
-      else if (PASS == 1)
-        ref = tilePlane(a.ins[tile], ai, wi, a.batch);
-      else
+      if (PASS == 2) {
         ref = weightPlane(a, wi, ai);
+      } else {
+        const fbfft_tile& d = PASS == 0 ? a.outs[ai % a.numTiles] : a.ins[ai % a.numTiles];
+        ref = tilePlane(d, ai / a.numTiles, wi, a.batch);
+        ref.valid = ref.valid && wi < (PASS == 0 ? Cout : Cin);
+      }
       if (ref.valid) {
         if (PASS == 2 && a.splits > 1)
           storeColumnsWindow<N, true, true>(ref.p, ref.sy, ref.sx, ref.h, ref.w, ref.padL, ref.padU,
-                                            l, z0, z1, norm);
+                                            le, z0, z1, norm);
         else
-          storeColumnsWindow<N>(ref.p, ref.sy, ref.sx, ref.h, ref.w, ref.padL, ref.padU, l, z0, z1,
+          storeColumnsWindow<N>(ref.p, ref.sy, ref.sx, ref.h, ref.w, ref.padL, ref.padU, le, z0, z1,
                                 norm);
       }
     }
-    __syncthreads();
   }
 }
 
@@ -351,37 +596,38 @@ __global__ void zeroWeight(ConvArgs a) {
 }
 
 template <int N>
-int launchPass(int pass, const ConvArgs& a, bool deterministic, hipStream_t s) {
+int launchPass(int pass, ConvArgs a, bool deterministic, hipStream_t s) {
   using C = ConvCfg<N>;
   const int Cout = a.wn[0], Cin = a.wn[1];
-  if (pass == FBFFT_UPDATE_OUTPUT) {
-    dim3 grid(a.numTiles, ceilDiv(Cout, C::FO), ceilDiv(a.batch, C::BN));
-    iteratedConvKernel<N, 0><<<grid, kThreads, 0, s>>>(a);
-  } else if (pass == FBFFT_UPDATE_GRAD_INPUT) {
-    dim3 grid(a.numTiles, ceilDiv(Cin, C::FO), ceilDiv(a.batch, C::BN));
-    iteratedConvKernel<N, 1><<<grid, kThreads, 0, s>>>(a);
-  } else {
+  const long rows = (long)a.numTiles * a.batch;
+  a.wGroups = ceilDiv(pass == FBFFT_UPDATE_GRAD_INPUT ? Cin : Cout, C::FO);
+  a.aGroups = pass == FBFFT_ACC_GRAD_PARAMETERS ? ceilDiv(Cin, C::BN) : (int)((rows + C::BN - 1) / C::BN);
+  if (pass == FBFFT_ACC_GRAD_PARAMETERS) {
     // The reference runs one block per group of planes over the whole reduction
     // (fbfft/FFTIteratedConvolution.cuh:600-613).  With 256 CUs that leaves most of the
-    // chip idle, so the reduction is also split along x until there are about two
+    // chip idle, so the reduction is also split until there are about two
     // workgroups per CU; the partial gradients are then added atomically into a
     // zeroed weight tensor (summation order, hence the last bits, vary from run to
     // run).  A single split stores directly.
-    ConvArgs b = a;
-    const int groups = ceilDiv(Cout, C::FO) * ceilDiv(Cin, C::BN);
-    const int steps = a.numTiles * a.batch;
     // deterministic: the reference's schedule, one workgroup per plane group over the
     // whole reduction in a fixed order, no atomics (and most of the chip idle)
-    b.splits = deterministic
+    const int groups = a.aGroups * a.wGroups;
+    a.splits = deterministic
                    ? 1
-                   : std::max(1, std::min(ceilDiv(512, groups), ceilDiv(steps, 2 * C::SPI)));
-    if (b.splits > 1) {
+                   : std::max(1, std::min(ceilDiv(512, groups), (int)((rows + 2 * C::SPI - 1) / (2 * C::SPI))));
+    if (a.splits > 1) {
       const long total = (long)a.wn[0] * a.wn[1] * a.wn[2] * a.wn[3];
-      zeroWeight<<<dim3((unsigned)std::min<long>((total + 255) / 256, 4096)), 256, 0, s>>>(b);
+      zeroWeight<<<dim3((unsigned)std::min<long>((total + 255) / 256, 4096)), 256, 0, s>>>(a);
     }
-    dim3 grid(b.splits, ceilDiv(Cout, C::FO), ceilDiv(Cin, C::BN));
-    iteratedConvKernel<N, 2><<<grid, kThreads, 0, s>>>(b);
   }
+  const long total = (long)a.splits * a.aGroups * a.wGroups;
+  const dim3 grid((unsigned)((total + 7) / 8 * 8));
+  if (pass == FBFFT_UPDATE_OUTPUT)
+    iteratedConvKernel<N, 0><<<grid, kThreads, 0, s>>>(a);
+  else if (pass == FBFFT_UPDATE_GRAD_INPUT)
+    iteratedConvKernel<N, 1><<<grid, kThreads, 0, s>>>(a);
+  else
+    iteratedConvKernel<N, 2><<<grid, kThreads, 0, s>>>(a);
   return launchStatus();
 }
 

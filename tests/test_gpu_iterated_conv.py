@@ -253,3 +253,41 @@ def test_layer_weight_gradient_is_reproducible():
         torch.cuda.synchronize()
         runs.append(gw.cpu().numpy())
     assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
+
+
+@pytest.mark.parametrize("N,k,Nb,Cin,Cout", [(8, 3, 3, 5, 9), (16, 5, 1, 3, 17), (32, 5, 2, 9, 7),
+                                             (32, 19, 1, 2, 3)])
+def test_plane_groups_span_tiles_and_tensors(oracle, N, k, Nb, Cin, Cout):
+    """A workgroup's planes come from several tiles, here of two tensors with different row
+    strides and alignments: one dense with even rows, one a view with odd rows and offsets."""
+    d = dev()
+    w = synth.normal((Cout, Cin, k, k), seed=60, std=0.05)
+    wd = w.to(d)
+    shapes = [(Nb, Cin, N + 4, 2 * N), (Nb, Cin, N - 1, N + 7)]
+    xs, outs, gs, gins = [], [], [], []
+    for i, (b, c, h, wid) in enumerate(shapes):
+        pad = i  # the second tensor sits inside a larger one, one row down and one column in
+        store = synth.uniform((b, c + pad, h + 2 * pad, wid + 3 * pad), seed=61 + i).to(d)
+        xs.append(store[:, pad:, pad:pad + h, pad:pad + wid])
+        gstore = synth.normal((b, Cout, h - k + 1 + pad, wid - k + 1 + 2 * pad), seed=63 + i).to(d)
+        gs.append(gstore[:, :, pad:, pad:pad + wid - k + 1])
+        outs.append(torch.full(gs[i].shape, float("nan"), device=d))
+        gins.append(torch.full_like(store, float("nan"))[:, pad:, pad:pad + h, pad:pad + wid])
+    both = lambda a, b, p: [torch.cat(z) if torch.is_tensor(z[0]) else sum(z)
+                            for z in zip(*(F.make_tile_grid(u, v, k, k, N, p) for u, v in zip(a, b)))]
+    ins, os_, n = both(xs, outs, F.FFT_UpdateOutput)
+    assert F.FFTIteratedConvolution(N, ins, os_, wd, F.FFT_UpdateOutput, 1.0, Nb, n)
+    ins, os_, n = both(gins, gs, F.FFT_UpdateGradInput)
+    assert F.FFTIteratedConvolution(N, ins, os_, wd, F.FFT_UpdateGradInput, 1.0, Nb, n)
+    want = 0.0
+    for x, o, g, gi in zip(xs, outs, gs, gins):
+        xh, gh = x.cpu().numpy(), g.cpu().numpy()
+        assert rel(o.cpu().numpy(), oracle.corr2d_valid(xh, w.numpy())) < TOL_CONV
+        assert rel(gi.cpu().numpy(), oracle.corr2d_grad_input(gh, w.numpy(), *xh.shape[2:])) < TOL_CONV
+        want = want + oracle.corr2d_grad_weight(xh, gh, k, k)
+    ins, os_, n = both(xs, gs, F.FFT_AccGradParameters)
+    for deterministic in (False, True):
+        gw = torch.full_like(wd, float("nan"))
+        assert F.FFTIteratedConvolution(N, ins, os_, gw, F.FFT_AccGradParameters, 1.0, Nb, n,
+                                        deterministic=deterministic)
+        assert rel(gw.cpu().numpy(), want) < TOL_CONV
