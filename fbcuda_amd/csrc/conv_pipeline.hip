@@ -935,7 +935,8 @@ struct GemmPlan {
   int splits, slicesPerSplit;
 };
 
-inline GemmPlan planGemm(int bins, int I, int Jp, int Kp) {
+// (maxSplits: more ranges than that have no room in the workspace)
+inline GemmPlan planGemm(int bins, int I, int Jp, int Kp, int maxSplits) {
   GemmPlan p;
   long waves, target;
   int minSlices;
@@ -963,27 +964,29 @@ inline GemmPlan planGemm(int bins, int I, int Jp, int Kp) {
     minSlices = 16;
   }
   const int slices = Kp / GK2;
-  const int want = (int)std::min<long>(16, ceilDiv(target, waves));
+  const int want = (int)std::min<long>(maxSplits, ceilDiv(target, waves));
   const int most = std::max(1, slices / minSlices);
   p.slicesPerSplit = ceilDiv(slices, std::min(want, most));
   p.splits = ceilDiv(slices, p.slicesPerSplit);  // no range is empty
   return p;
 }
 
+constexpr int kAnySplits = 16;  // what planGemm cuts a reduction into at most
+
 template <int N>
-size_t workspaceFloat2(int I, int J, int K, bool outTiled) {
+size_t workspaceFloat2(int I, int J, int K, bool outTiled, int maxSplits = kAnySplits) {
   if (swapRoles(I, J, outTiled)) std::swap(I, J);
   const int SL = BMCfg<N>::SLOTS, bins = BMCfg<N>::BINS;
   const int Ip = roundUp(I, SL), Jp = roundUp(J, SL), Kp = roundUp(K, 8);
   return (size_t)bins * ((size_t)Kp * Ip + (size_t)Kp * Jp +
-                         (size_t)planGemm(bins, I, Jp, Kp).splits * I * Jp);
+                         (size_t)planGemm(bins, I, Jp, Kp, maxSplits).splits * I * Jp);
 }
 
 // P[i][j] = scale * sum_k X[i][k] * op(Y[j][k]) for planes x(i,k), y(j,k) -> planes out(i,j);
 // each PlaneSet names its first index "row" and its second "k".
 template <int N>
 int runPipeline(PlaneSet x, PlaneSet y, PlaneSet out, bool conjY, float scale, bool accumulate,
-                float2* ws, hipStream_t s) {
+                int maxSplits, float2* ws, hipStream_t s) {
   using C = BMCfg<N>;
   const int SL = C::SLOTS, bins = C::BINS;
   float xSign = 1.0f, ySign = conjY ? 1.0f : -1.0f;
@@ -1061,7 +1064,7 @@ int runPipeline(PlaneSet x, PlaneSet y, PlaneSet out, bool conjY, float scale, b
   g.Ip = Ip;
   g.Jp = Jp;
   g.Kp = Kp;
-  const GemmPlan plan = planGemm(bins, I, Jp, Kp);
+  const GemmPlan plan = planGemm(bins, I, Jp, Kp, maxSplits);
   g.IT = plan.IT;
   g.JT = plan.JT;
   g.splits = plan.splits;
@@ -1144,8 +1147,8 @@ void tile(PlaneSet& p, bool imageIsRow, int tilesY, int tilesX, int stepY, int s
 
 template <int N>
 int runPass(int pass, const PlaneSet& x, const PlaneSet& y, const PlaneSet& out, float scale,
-            bool accumulate, float2* ws, hipStream_t s) {
-  return runPipeline<N>(x, y, out, /*conjY=*/pass != 1, scale, accumulate, ws, s);
+            bool accumulate, float2* ws, hipStream_t s, int maxSplits = kAnySplits) {
+  return runPipeline<N>(x, y, out, /*conjY=*/pass != 1, scale, accumulate, maxSplits, ws, s);
 }
 
 }  // namespace
@@ -1169,31 +1172,69 @@ static void passDims(int pass, int B, int Cin, int Cout, int* I, int* J, int* K)
   else { *I = Cin; *J = Cout; *K = B; }
 }
 
-size_t convWorkspaceBytes(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH,
-                          int kW) {
-  if (N > 32) return convSplitWorkspaceBytes(pass, N, B, Cin, Cout);
+// workspace of a pass on windows of N <= 32 points
+static size_t windowsBytes(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW,
+                           int maxSplits) {
   int ty, tx;
   tileGrid(pass, N, H, W, kH, kW, &ty, &tx);
   if ((long)B * ty * tx > (1L << 30)) return 0;
   int I, J, K;
   passDims(pass, B * ty * tx, Cin, Cout, &I, &J, &K);
   const bool outTiled = pass != 2 && ty * tx > 1;  // the weight gradient is never tiled
-  size_t n = N == 8 ? workspaceFloat2<8>(I, J, K, outTiled)
-                    : N == 16 ? workspaceFloat2<16>(I, J, K, outTiled)
-                              : workspaceFloat2<32>(I, J, K, outTiled);
+  size_t n = N == 8 ? workspaceFloat2<8>(I, J, K, outTiled, maxSplits)
+                    : N == 16 ? workspaceFloat2<16>(I, J, K, outTiled, maxSplits)
+                              : workspaceFloat2<32>(I, J, K, outTiled, maxSplits);
   return n * sizeof(float2);
+}
+
+size_t convWorkspaceBytes(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH,
+                          int kW) {
+  if (N > 32) return convSplitWorkspaceBytes(pass, N, B, Cin, Cout);
+  return windowsBytes(pass, N, B, Cin, Cout, H, W, kH, kW, kAnySplits);
+}
+
+// The transform size a pass runs on, and how many ranges its reduction may be cut into.  A
+// caller's 64 or 128 points stand for a transform of the whole image; the same convolution
+// cut into 8-, 16- or 32-point windows runs on the bin-major pipeline, which is the faster
+// path whenever its spectra are no larger than the plane-major ones: a filter plane then
+// costs a quarter to a sixty-fourth of its 64-point spectrum, and no spectrum takes the
+// plane-major shape.  Three passes, plane-major / windows: 32 x 32 x 60 x 60 images, 64
+// filters of 5 x 5 216 / 145 us; 24 x 48 x 40 x 40, 96 of 8 x 8 339 / 151 us; 8 x 200 x
+// 50 x 58, 300 of 1 x 1 2170 / 273 us; 128 points, 16 x 32 x 100 x 100, 64 of 8 x 8 490 /
+// 207 us.  "No larger" is also what keeps the windows within the workspace of the size the
+// caller named - with one range of the reduction where several have no room.  (With twice
+// that workspace 11 x 11 filters on 60 x 60 images would move to windows too: 217 -> 227
+// us.)  Filters larger than 32 or filling most of a window stay plane-major.
+struct PassSize {
+  int N, maxSplits;
+};
+static PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
+  if (N > 32) {
+    const size_t room = convSplitWorkspaceBytes(pass, N, B, Cin, Cout);
+    const int n = fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW);
+    for (int maxSplits : {kAnySplits, 1}) {
+      const size_t need = n == 0 ? 0 : windowsBytes(pass, n, B, Cin, Cout, H, W, kH, kW, maxSplits);
+      if (need != 0 && need <= room) return {n, maxSplits};
+    }
+  }
+  return {N, kAnySplits};
 }
 
 // pass 0: x = input [B][Cin][H][W], y = weight [Cout][Cin][kH][kW], out = output [B][Cout][oH][oW]
 // pass 1: x = gradOutput [B][Cout][oH][oW], y = weight, out = gradInput [B][Cin][H][W]
 // pass 2: x = input, y = gradOutput, out = gradWeight [Cout][Cin][kH][kW]
-// strides in floats.  Images larger than the transform (N <= 32 only) are cut into
-// overlapping windows that ride through the same three kernels as extra rows
+// strides in floats.  Images larger than the transform (N <= 32, by the caller's choice or by
+// passSize's) are cut into overlapping windows that ride through the same three kernels as extra rows
 // (passes 0 and 1) or extra reduction steps (pass 2).
 int launchConvPass(int pass, int N, float* x, const int* xStride, const int* xSize, float* y,
                    const int* yStride, const int* ySize, float* out, const int* outStride,
                    const int* outSize, float scale, bool accumulate, void* workspace,
                    hipStream_t s) {
+  const int* in = pass == 1 ? outSize : xSize;    // the layer's input / gradInput extents
+  const int* wt = pass == 2 ? outSize : ySize;    // the filter extents
+  const int H = in[2], W = in[3], kH = wt[2], kW = wt[3];
+  const PassSize size = passSize(pass, N, in[0], wt[1], wt[0], H, W, kH, kW);
+  N = size.N;
   if (N > 32)
     return launchConvSplit(pass, N, x, xStride, xSize, y, yStride, ySize, out, outStride, outSize,
                            scale, accumulate, workspace, s);
@@ -1211,9 +1252,6 @@ int launchConvPass(int pass, int N, float* x, const int* xStride, const int* xSi
     py = planes(y, yStride, ySize, 1, 0);
     po = planes(out, outStride, outSize, 1, 0);
   }
-  const int* in = pass == 1 ? outSize : xSize;    // the layer's input / gradInput extents
-  const int* wt = pass == 2 ? outSize : ySize;    // the filter extents
-  const int H = in[2], W = in[3], kH = wt[2], kW = wt[3];
   int ty, tx;
   tileGrid(pass, N, H, W, kH, kW, &ty, &tx);
   if (ty * tx > 1) {
@@ -1236,9 +1274,9 @@ int launchConvPass(int pass, int N, float* x, const int* xStride, const int* xSi
   }
   float2* ws = static_cast<float2*>(workspace);
   switch (N) {
-    case 8: return runPass<8>(pass, px, py, po, scale, accumulate, ws, s);
-    case 16: return runPass<16>(pass, px, py, po, scale, accumulate, ws, s);
-    case 32: return runPass<32>(pass, px, py, po, scale, accumulate, ws, s);
+    case 8: return runPass<8>(pass, px, py, po, scale, accumulate, ws, s, size.maxSplits);
+    case 16: return runPass<16>(pass, px, py, po, scale, accumulate, ws, s, size.maxSplits);
+    case 32: return runPass<32>(pass, px, py, po, scale, accumulate, ws, s, size.maxSplits);
   }
   return FBFFT_UNSUPPORTED_SIZE;
 }

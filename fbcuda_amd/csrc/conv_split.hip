@@ -1,4 +1,6 @@
-// Convolution-layer passes for 64- and 128-point transforms.
+// Convolution-layer passes for 64- and 128-point transforms of the whole image: what those
+// sizes run when windows of 32 points or fewer would hold more spectrum (passSize in
+// conv_pipeline.hip).
 //
 // Planes of that size do not fit the one-workgroup-per-plane-group forward and
 // inverse kernels of the bin-major pipeline, so these sizes run the composition the

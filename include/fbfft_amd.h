@@ -229,8 +229,10 @@ size_t fbfft_make_tiles_for_pass(int pass, const fbfft_tensor* input, const fbff
  * [Cout][Cin][kH][kW], output / gradOutput [B][Cout][H-kH+1][W-kW+1], fftSize in
  * {8,16,32,64,128}, kH, kW <= fftSize.  Valid cross-correlation, no kernel flip.
  * Sizes up to 32 hand bin-major spectra between three fused kernels; 64 and 128
- * run fbfft2D -> transposeMM -> fbifft2D on plane-major spectra in the workspace
- * and need H, W <= fftSize.  With fftSize <= 32 the image may be larger than the
+ * need H, W <= fftSize and run the same three kernels on 8-, 16- or 32-point windows
+ * of the image where their spectra are no larger than those of the named size, and
+ * fbfft2D -> transposeMM -> fbifft2D on plane-major spectra in the workspace
+ * otherwise (filters that fill most of a 32-point window or exceed it).  With fftSize <= 32 the image may be larger than the
  * transform: it is then cut into overlapping fftSize x fftSize windows whose
  * origins advance by fftSize-kH+1 rows / fftSize-kW+1 columns (the tiling of
  * FFTIteratedConvolution, fbfft/FFTIteratedConvolution.cuh:71-88), and the
@@ -249,9 +251,7 @@ size_t fbfft_make_tiles_for_pass(int pass, const fbfft_tensor* input, const fbff
  * 91 us against 102 us at 32; 32 for both gradients); every size computes the same
  * convolution.  The reference leaves the choice to its caller (the FFTSize template
  * parameter of fbfft/FFTIteratedConvolution.cuh:624); 64 and 128 are only taken when asked
- * for - on this hardware 32-point windows measure faster than a 64- or 128-point
- * transform of the whole image (60 x 60 images, 5 x 5 filters: 36 us against 74 us and
- * 229 us). */
+ * for. */
 int fbfft_conv_choose_fft_size(int pass, int batch, int cin, int cout, int H, int W, int kH,
                                int kW);
 

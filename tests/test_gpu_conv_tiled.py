@@ -152,3 +152,32 @@ def test_fft_size_zero_is_the_library_choice(oracle, H, W, k):
     assert F.conv_fprop_static(x, w, out, 0) == F.Success
     torch.cuda.synchronize()
     assert torch.equal(out, res[0][0])
+
+
+@pytest.mark.parametrize("N,H,W,k,Bn,Cin,Cout", [
+    (64, 60, 60, 5, 16, 16, 32),     # every pass in windows; the input gradient with one range
+    (64, 64, 33, 8, 17, 20, 40),
+    (128, 100, 97, 3, 4, 33, 20),
+    (64, 60, 57, 5, 1, 2, 3),        # windows padded to whole plane groups do not fit: plane-major
+    (64, 61, 64, 20, 6, 5, 7),       # little of a window is kept: plane-major
+    (64, 62, 64, 33, 6, 5, 7),       # filter larger than a window: plane-major
+])
+def test_named_sizes_above_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin, Cout):
+    """64 and 128 points run on windows or on plane-major spectra, whichever is faster, both
+    within the workspace of the named size (the bytes behind it stay as they were)."""
+    d = dev()
+    x = synth.uniform((Bn, Cin, H, W), seed=70, device=d)
+    w = synth.normal((Cout, Cin, k, k), seed=71, std=0.05, device=d)
+    g = synth.normal((Bn, Cout, H - k + 1, W - k + 1), seed=72, device=d)
+    out, gi, gw = (torch.full_like(t, float("nan")) for t in (g, x, w))
+    for pass_, call in ((0, lambda s: F.conv_fprop(x, w, out, N, s)),
+                        (1, lambda s: F.conv_bprop(g, w, gi, N, s)),
+                        (2, lambda s: F.conv_accgrad(x, g, gw, N, s))):
+        n = F.conv_workspace(pass_, Bn, Cin, Cout, N)
+        space = torch.full((n + 256,), 77, dtype=torch.uint8, device=d)
+        assert call(space[:n]) == F.Success
+        assert bool((space[n:] == 77).all())
+    xh, wh, gh = x.cpu().numpy(), w.cpu().numpy(), g.cpu().numpy()
+    assert rel(out.cpu().numpy(), oracle.corr2d_valid(xh, wh)) < TOL_CONV
+    assert rel(gi.cpu().numpy(), oracle.corr2d_grad_input(gh, wh, H, W)) < TOL_CONV
+    assert rel(gw.cpu().numpy(), oracle.corr2d_grad_weight(xh, gh, k, k)) < TOL_CONV
