@@ -239,6 +239,22 @@ def test_view_rejects_strides_beyond_32_bits():
     assert F.view(torch.empty(4).as_strided((1, 2), (2 ** 31 - 1, 1))).stride[0] == 2 ** 31 - 1
 
 
+@pytest.mark.parametrize("shape", [(), (3,), (5, 0), (7, 17, 2), (2, 3, 9, 5), (2, 3, 17, 32, 2)])
+def test_packed_descriptor_is_the_view(shape):
+    """The byte string that a call passes is the fbfft_tensor that view fills in, for every rank,
+    contiguous and strided, and operands that view refuses raise the same error."""
+    import torch
+    t = torch.zeros(shape)
+    for u in (t, t.transpose(0, -1) if t.dim() else t, t[1:] if t.dim() else t):
+        assert F._desc(u) == bytes(F.view(u))
+    for bad in (t.double(), torch.zeros((1,) * 6), torch.empty(4).as_strided((1, 2), (2 ** 31, 1)),
+                torch.empty(1).expand(2 ** 31)):
+        with pytest.raises((TypeError, ValueError)) as want:
+            F.view(bad)
+        with pytest.raises(want.type, match="^" + re.escape(str(want.value)) + "$"):
+            F._desc(bad)
+
+
 def test_iterated_conv_refuses_filters_larger_than_the_transform():
     """Validated on the host before anything is launched: returns 0 (not launched)."""
     import torch
