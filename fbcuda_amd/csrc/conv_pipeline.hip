@@ -1194,28 +1194,42 @@ size_t convWorkspaceBytes(int pass, int N, int B, int Cin, int Cout, int H, int 
 }
 
 // The transform size a pass runs on, and how many ranges its reduction may be cut into.  A
-// caller's 64 or 128 points stand for a transform of the whole image; the same convolution
-// cut into 8-, 16- or 32-point windows runs on the bin-major pipeline, which is the faster
-// path whenever its spectra are no larger than the plane-major ones: a filter plane then
-// costs a quarter to a sixty-fourth of its 64-point spectrum, and no spectrum takes the
-// plane-major shape.  Three passes, plane-major / windows: 32 x 32 x 60 x 60 images, 64
-// filters of 5 x 5 216 / 145 us; 24 x 48 x 40 x 40, 96 of 8 x 8 339 / 151 us; 8 x 200 x
-// 50 x 58, 300 of 1 x 1 2170 / 273 us; 128 points, 16 x 32 x 100 x 100, 64 of 8 x 8 490 /
-// 207 us.  "No larger" is also what keeps the windows within the workspace of the size the
-// caller named - with one range of the reduction where several have no room.  (With twice
-// that workspace 11 x 11 filters on 60 x 60 images would move to windows too: 217 -> 227
-// us.)  Filters larger than 32 or filling most of a window stay plane-major.
+// caller's size names the workspace; the same convolution cut into smaller windows - the
+// library's own choice for the layer - is faster wherever the windows' spectra are clearly
+// the smaller ones: a filter plane costs a quarter or less, and windows end nearer to the
+// edge of an image that leaves much of the named transform empty.  That is also what keeps
+// the windows within the workspace of the named size.
+//
+// 64 and 128 points (plane-major spectra of the whole image) give way to windows that hold
+// no more spectrum, with one range of the reduction where several have no room.  Three
+// passes, plane-major / windows: 32 x 32 x 60 x 60 images, 64 filters of 5 x 5 216 / 145 us;
+// 24 x 48 x 40 x 40, 96 of 8 x 8 339 / 151 us; 8 x 200 x 50 x 58, 300 of 1 x 1 2170 / 273 us;
+// 128 points, 16 x 32 x 100 x 100, 64 of 8 x 8 490 / 207 us.  (With twice that workspace 11 x
+// 11 filters on 60 x 60 images would move to windows too: 217 -> 227 us.)  Filters larger
+// than 32 or filling most of a window stay plane-major.
+//
+// 16 and 32 points are the same kernels on either side, where smaller transforms pay more
+// per value: windows are taken up to 85 % of the named size's workspace, 70 % for the weight
+// gradient (many windows make a long reduction over small tiles).  One pass, named 32 points
+// / windows of n, us at the windows' share of the workspace: forward 128 x 64 x 27 x 27, 192
+// of 5 x 5 99.6 / 91.0 (n = 16, 80 %), 128 x 48 x 18 x 26, 128 of 5 x 5 59.2 / 53.3 (16,
+// 84 %), 32 x 64 x 27 x 27, 192 of 5 x 5 56.6 / 32.1 (16, 42 %), 64 x 96 x 13 x 13, 256 of
+// 3 x 3 91.7 / 34.3 (8, 15 %); input gradient of 16 x 128 x 30 x 30, 128 of 3 x 3 55.4 / 33.0
+// (8, 36 %); weight gradient 128 x 192 x 27 x 27, 64 of 5 x 5 99.5 / 107.9 (16, 93 %: stays),
+// 16 x 32 x 100 x 100, 64 of 3 x 3 74.9 / 75.4 (16, 79 %: stays), 64 x 96 x 23 x 23, 256 of
+// 5 x 5 103.3 / 87.6 (16, 61 %), 32 x 64 x 27 x 27, 192 of 5 x 5 42.9 / 37.0 (16, 55 %).
 struct PassSize {
   int N, maxSplits;
 };
 static PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
-  if (N > 32) {
-    const size_t room = convSplitWorkspaceBytes(pass, N, B, Cin, Cout);
-    const int n = fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW);
-    for (int maxSplits : {kAnySplits, 1}) {
-      const size_t need = n == 0 ? 0 : windowsBytes(pass, n, B, Cin, Cout, H, W, kH, kW, maxSplits);
-      if (need != 0 && need <= room) return {n, maxSplits};
-    }
+  const int n = fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW);
+  if (n == 0 || n >= N) return {N, kAnySplits};
+  const size_t room = convWorkspaceBytes(pass, N, B, Cin, Cout, H, W, kH, kW);
+  const size_t percent = N > 32 ? 100 : pass == 2 ? 70 : 85;
+  for (int maxSplits : {kAnySplits, 1}) {
+    const size_t need = windowsBytes(pass, n, B, Cin, Cout, H, W, kH, kW, maxSplits);
+    if (need != 0 && need <= room - room / 100 * (100 - percent)) return {n, maxSplits};
+    if (N <= 32) break;  // fewer ranges than the product asks for cost more than windows give
   }
   return {N, kAnySplits};
 }

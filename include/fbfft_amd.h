@@ -228,11 +228,12 @@ size_t fbfft_make_tiles_for_pass(int pass, const fbfft_tensor* input, const fbff
  * Shapes throughout: input / gradInput [B][Cin][H][W], weight / gradWeight
  * [Cout][Cin][kH][kW], output / gradOutput [B][Cout][H-kH+1][W-kW+1], fftSize in
  * {8,16,32,64,128}, kH, kW <= fftSize.  Valid cross-correlation, no kernel flip.
- * Sizes up to 32 hand bin-major spectra between three fused kernels; 64 and 128
- * need H, W <= fftSize and run the same three kernels on 8-, 16- or 32-point windows
- * of the image where their spectra are no larger than those of the named size, and
- * fbfft2D -> transposeMM -> fbifft2D on plane-major spectra in the workspace
- * otherwise (filters that fill most of a 32-point window or exceed it).  With fftSize <= 32 the image may be larger than the
+ * Sizes up to 32 hand bin-major spectra between three fused kernels, on smaller windows
+ * than the named size where these hold clearly less spectrum; 64 and 128 need H, W <=
+ * fftSize and run the same three kernels on 8-, 16- or 32-point windows of the image where
+ * their spectra are no larger than those of the named size, and fbfft2D -> transposeMM ->
+ * fbifft2D on plane-major spectra in the workspace otherwise (filters that fill most of a
+ * 32-point window or exceed it).  With fftSize <= 32 the image may be larger than the
  * transform: it is then cut into overlapping fftSize x fftSize windows whose
  * origins advance by fftSize-kH+1 rows / fftSize-kW+1 columns (the tiling of
  * FFTIteratedConvolution, fbfft/FFTIteratedConvolution.cuh:71-88), and the
@@ -247,8 +248,9 @@ size_t fbfft_make_tiles_for_pass(int pass, const fbfft_tensor* input, const fbff
  * {8, 16, 32} (at least kH and kW) that is expected to run the pass fastest - the one
  * that moves the fewest spectrum values over its windows and filter planes, weighted by
  * the measured rate of each size; 0 if the filter is larger than the image or than 32.
- * The passes of one layer may get different sizes (configs[3]: 16 for the forward pass,
- * 91 us against 102 us at 32; 32 for both gradients); every size computes the same
+ * The passes of one layer may get different sizes (128 x 64 x 27 x 27 images, 192
+ * filters of 5 x 5: 16 for the forward pass and the weight gradient, 32 for the input
+ * gradient); every size computes the same
  * convolution.  The reference leaves the choice to its caller (the FFTSize template
  * parameter of fbfft/FFTIteratedConvolution.cuh:624); 64 and 128 are only taken when asked
  * for. */

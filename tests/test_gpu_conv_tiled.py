@@ -165,6 +165,26 @@ def test_fft_size_zero_is_the_library_choice(oracle, H, W, k):
 def test_named_sizes_above_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin, Cout):
     """64 and 128 points run on windows or on plane-major spectra, whichever is faster, both
     within the workspace of the named size (the bytes behind it stay as they were)."""
+    passes_on_named_workspace(oracle, N, H, W, k, Bn, Cin, Cout)
+
+
+@pytest.mark.parametrize("N,H,W,k,Bn,Cin,Cout", [
+    (32, 27, 27, 5, 9, 20, 40),      # 16-point windows in the forward pass
+    (32, 13, 13, 3, 17, 33, 50),     # 8- and 16-point windows, channels past a tile's edge
+    (32, 16, 9, 3, 5, 3, 20),        # an image that fits 16 points whole
+    (32, 100, 61, 3, 2, 20, 24),     # larger than the named transform
+    (32, 30, 32, 11, 6, 5, 7),       # little of a smaller window is kept: the named size
+    (16, 13, 14, 3, 8, 20, 24),      # 8-point windows
+    (16, 8, 8, 1, 3, 7, 9),
+    (8, 7, 8, 3, 3, 7, 9),           # nothing smaller
+])
+def test_named_sizes_up_to_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin, Cout):
+    """16 and 32 points run on smaller windows where those hold less spectrum, within the
+    workspace of the named size."""
+    passes_on_named_workspace(oracle, N, H, W, k, Bn, Cin, Cout)
+
+
+def passes_on_named_workspace(oracle, N, H, W, k, Bn, Cin, Cout):
     d = dev()
     x = synth.uniform((Bn, Cin, H, W), seed=70, device=d)
     w = synth.normal((Cout, Cin, k, k), seed=71, std=0.05, device=d)
@@ -173,7 +193,7 @@ def test_named_sizes_above_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin
     for pass_, call in ((0, lambda s: F.conv_fprop(x, w, out, N, s)),
                         (1, lambda s: F.conv_bprop(g, w, gi, N, s)),
                         (2, lambda s: F.conv_accgrad(x, g, gw, N, s))):
-        n = F.conv_workspace(pass_, Bn, Cin, Cout, N)
+        n = F.conv_workspace_image(pass_, Bn, Cin, Cout, H, W, k, k, N)
         space = torch.full((n + 256,), 77, dtype=torch.uint8, device=d)
         assert call(space[:n]) == F.Success
         assert bool((space[n:] == 77).all())
