@@ -354,7 +354,7 @@ def conv_extras(F, synth, torch, dev, extra):
     _, t = timed(mmp, 200, 200, torch)
     extra["transposeMM_packed_configs3_us"] = round(t * 1e6, 1)
     del Ap, Bp, Cp, x, w, out, ws
-    # a 64-point layer (plane-major spectra through transposeMM): 32x32x60x60 * 64x32x5x5
+    # a layer named 64 points, which run in windows of 32 or fewer: 32x32x60x60 * 64x32x5x5
     x6 = synth.normal((32, 32, 60, 60), seed=50, device=dev)
     w6 = synth.normal((64, 32, 5, 5), seed=51, std=0.02, device=dev)
     o6 = torch.empty((32, 64, 56, 56), device=dev)

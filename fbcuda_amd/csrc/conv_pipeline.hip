@@ -1208,16 +1208,16 @@ size_t convWorkspaceBytes(int pass, int N, int B, int Cin, int Cout, int H, int 
 // 11 filters on 60 x 60 images would move to windows too: 217 -> 227 us.)  Filters larger
 // than 32 or filling most of a window stay plane-major.
 //
-// 16 and 32 points are the same kernels on either side, where smaller transforms pay more
-// per value: windows are taken up to 85 % of the named size's workspace, 70 % for the weight
-// gradient (many windows make a long reduction over small tiles).  One pass, named 32 points
-// / windows of n, us at the windows' share of the workspace: forward 128 x 64 x 27 x 27, 192
-// of 5 x 5 99.6 / 91.0 (n = 16, 80 %), 128 x 48 x 18 x 26, 128 of 5 x 5 59.2 / 53.3 (16,
-// 84 %), 32 x 64 x 27 x 27, 192 of 5 x 5 56.6 / 32.1 (16, 42 %), 64 x 96 x 13 x 13, 256 of
-// 3 x 3 91.7 / 34.3 (8, 15 %); input gradient of 16 x 128 x 30 x 30, 128 of 3 x 3 55.4 / 33.0
-// (8, 36 %); weight gradient 128 x 192 x 27 x 27, 64 of 5 x 5 99.5 / 107.9 (16, 93 %: stays),
-// 16 x 32 x 100 x 100, 64 of 3 x 3 74.9 / 75.4 (16, 79 %: stays), 64 x 96 x 23 x 23, 256 of
-// 5 x 5 103.3 / 87.6 (16, 61 %), 32 x 64 x 27 x 27, 192 of 5 x 5 42.9 / 37.0 (16, 55 %).
+// 16 and 32 points are the same kernels on either side, and a caller who names them means
+// them: they give way only where most of the named transforms would be padding - windows
+// that need at most three fifths of the named size's workspace.  One pass, named 32 points /
+// windows of n, us at the windows' share of that workspace: 32 x 64 x 27 x 27 images, 192
+// filters of 5 x 5, forward 56.6 / 32.1 (n = 16, 42 %), weight gradient 42.9 / 37.0 (16, 55 %);
+// 64 x 96 x 13 x 13, 256 of 3 x 3, forward 91.7 / 34.3 (8, 15 %), input gradient 105.6 / 37.3
+// (16, 28 %); 16 x 128 x 30 x 30, 128 of 3 x 3, input gradient 55.4 / 33.0 (8, 36 %).  Above
+// the line less is left to win, and smaller transforms pay more per value: forward 128 x 64 x
+// 27 x 27, 192 of 5 x 5 99.6 / 91.0 (16, 80 %), weight gradient 16 x 32 x 100 x 100, 64 of
+// 3 x 3 74.9 / 75.4 (16, 79 %), 128 x 192 x 27 x 27, 64 of 5 x 5 99.5 / 107.9 (16, 93 %).
 struct PassSize {
   int N, maxSplits;
 };
@@ -1225,7 +1225,7 @@ static PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W
   const int n = fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW);
   if (n == 0 || n >= N) return {N, kAnySplits};
   const size_t room = convWorkspaceBytes(pass, N, B, Cin, Cout, H, W, kH, kW);
-  const size_t percent = N > 32 ? 100 : pass == 2 ? 70 : 85;
+  const size_t percent = N > 32 ? 100 : 60;
   for (int maxSplits : {kAnySplits, 1}) {
     const size_t need = windowsBytes(pass, n, B, Cin, Cout, H, W, kH, kW, maxSplits);
     if (need != 0 && need <= room - room / 100 * (100 - percent)) return {n, maxSplits};

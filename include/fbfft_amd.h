@@ -229,7 +229,7 @@ size_t fbfft_make_tiles_for_pass(int pass, const fbfft_tensor* input, const fbff
  * [Cout][Cin][kH][kW], output / gradOutput [B][Cout][H-kH+1][W-kW+1], fftSize in
  * {8,16,32,64,128}, kH, kW <= fftSize.  Valid cross-correlation, no kernel flip.
  * Sizes up to 32 hand bin-major spectra between three fused kernels, on smaller windows
- * than the named size where these hold clearly less spectrum; 64 and 128 need H, W <=
+ * than the named size where these need at most 60 % of its workspace; 64 and 128 need H, W <=
  * fftSize and run the same three kernels on 8-, 16- or 32-point windows of the image where
  * their spectra are no larger than those of the named size, and fbfft2D -> transposeMM ->
  * fbifft2D on plane-major spectra in the workspace otherwise (filters that fill most of a

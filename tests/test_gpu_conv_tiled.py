@@ -169,18 +169,18 @@ def test_named_sizes_above_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin
 
 
 @pytest.mark.parametrize("N,H,W,k,Bn,Cin,Cout", [
-    (32, 27, 27, 5, 9, 20, 40),      # 16-point windows in the forward pass
+    (32, 27, 27, 5, 9, 20, 40),      # 16-point windows in the weight gradient
     (32, 13, 13, 3, 17, 33, 50),     # 8- and 16-point windows, channels past a tile's edge
     (32, 16, 9, 3, 5, 3, 20),        # an image that fits 16 points whole
     (32, 100, 61, 3, 2, 20, 24),     # larger than the named transform
     (32, 30, 32, 11, 6, 5, 7),       # little of a smaller window is kept: the named size
-    (16, 13, 14, 3, 8, 20, 24),      # 8-point windows
-    (16, 8, 8, 1, 3, 7, 9),
+    (16, 13, 14, 3, 8, 20, 24),      # little to save: the named size
+    (16, 8, 8, 1, 3, 7, 9),          # 8-point windows
     (8, 7, 8, 3, 3, 7, 9),           # nothing smaller
 ])
 def test_named_sizes_up_to_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin, Cout):
-    """16 and 32 points run on smaller windows where those hold less spectrum, within the
-    workspace of the named size."""
+    """16 and 32 points run on smaller windows where those need at most three fifths of the
+    named size's workspace, and within it."""
     passes_on_named_workspace(oracle, N, H, W, k, Bn, Cin, Cout)
 
 
