@@ -58,9 +58,15 @@ struct ConvArgs {
   int batch;
   int numTiles;
   int splits;  // accGradParameters: workgroups sharing one reduction
-  int aGroups, wGroups;  // workgroups along A and W planes
+  int aGroups, wGroups;  // workgroups of this launch along A and W planes
+  int firstA, firstW;    // its first A and W plane; passes 0, 1: A planes count from ...
+  int image0;            // ... tile 0 of this image
   float scale;
 };
+
+// workgroups of one launch: a grid counts its lanes along x in 32 bits, and every XCD takes
+// the same number of workgroups
+constexpr long kMaxWorkgroups = 0xffffffffL / kThreads / 8 * 8;
 
 struct PlaneRef {
   float* p;
@@ -311,8 +317,7 @@ __global__ __launch_bounds__(kThreads) void iteratedConvKernel(ConvArgs a) {
   const int lane = t % 64;
 
   const int Cout = a.wn[0], Cin = a.wn[1];
-  const int rows = a.numTiles * a.batch;  // (image, tile) pairs
-  const int steps = PASS == 0 ? Cin : PASS == 1 ? Cout : rows;
+  const int steps = PASS == 0 ? Cin : PASS == 1 ? Cout : a.numTiles * a.batch;
   // Passes 0, 1: one workgroup per (A group, W group).  Pass 2: the reduction is also cut
   // into a.splits ranges whose results meet in an atomic add.  Workgroups are dealt
   // round-robin to the 8 XCDs; every XCD takes a contiguous range of logical ids, W groups
@@ -320,9 +325,9 @@ __global__ __launch_bounds__(kThreads) void iteratedConvKernel(ConvArgs a) {
   const int total = a.splits * a.aGroups * a.wGroups;
   const int per = (total + 7) / 8;
   const int logical = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  if ((int)blockIdx.x / 8 >= per || logical >= total) return;
-  const int w0 = logical % a.wGroups * FO;                // first W plane
-  const int a0 = logical / a.wGroups % a.aGroups * BN;    // first A plane
+  if (logical >= total) return;
+  const int w0 = a.firstW + logical % a.wGroups * FO;              // first W plane
+  const int a0 = a.firstA + logical / a.wGroups % a.aGroups * BN;  // first A plane
   const int perSplit = PASS == 2 ? ((steps + a.splits - 1) / a.splits + SPI - 1) / SPI * SPI : steps;
   const int stepBegin = PASS == 2 ? logical / (a.wGroups * a.aGroups) * perSplit : 0;
   const int stepEnd = min(steps, stepBegin + perSplit);
@@ -357,7 +362,7 @@ __global__ __launch_bounds__(kThreads) void iteratedConvKernel(ConvArgs a) {
     if (isA) {
       const int row = a0 + sj;
       const fbfft_tile& d = (PASS == 0 ? a.ins : a.outs)[row % a.numTiles];
-      return tilePlane(d, row / a.numTiles, step, a.batch);
+      return tilePlane(d, a.image0 + row / a.numTiles, step, a.batch);
     }
     return PASS == 0 ? weightPlane(a, w0 + sj, step) : weightPlane(a, step, w0 + sj);
   };
@@ -564,7 +569,7 @@ __global__ __launch_bounds__(kThreads) void iteratedConvKernel(ConvArgs a) {
         ref = weightPlane(a, wi, ai);
       } else {
         const fbfft_tile& d = PASS == 0 ? a.outs[ai % a.numTiles] : a.ins[ai % a.numTiles];
-        ref = tilePlane(d, ai / a.numTiles, wi, a.batch);
+        ref = tilePlane(d, a.image0 + ai / a.numTiles, wi, a.batch);
         ref.valid = ref.valid && wi < (PASS == 0 ? Cout : Cin);
       }
       if (ref.valid) {
@@ -599,9 +604,9 @@ template <int N>
 int launchPass(int pass, ConvArgs a, bool deterministic, hipStream_t s) {
   using C = ConvCfg<N>;
   const int Cout = a.wn[0], Cin = a.wn[1];
-  const long rows = (long)a.numTiles * a.batch;
-  a.wGroups = ceilDiv(pass == FBFFT_UPDATE_GRAD_INPUT ? Cin : Cout, C::FO);
-  a.aGroups = pass == FBFFT_ACC_GRAD_PARAMETERS ? ceilDiv(Cin, C::BN) : (int)((rows + C::BN - 1) / C::BN);
+  const long rows = (long)a.numTiles * a.batch;  // (image, tile) pairs
+  const long wGroups = ceilDiv(pass == FBFFT_UPDATE_GRAD_INPUT ? Cin : Cout, C::FO);
+  const long aGroups = pass == FBFFT_ACC_GRAD_PARAMETERS ? ceilDiv(Cin, C::BN) : (rows + C::BN - 1) / C::BN;
   if (pass == FBFFT_ACC_GRAD_PARAMETERS) {
     // The reference runs one block per group of planes over the whole reduction
     // (fbfft/FFTIteratedConvolution.cuh:600-613).  With 256 CUs that leaves most of the
@@ -611,24 +616,40 @@ int launchPass(int pass, ConvArgs a, bool deterministic, hipStream_t s) {
     // run).  A single split stores directly.
     // deterministic: the reference's schedule, one workgroup per plane group over the
     // whole reduction in a fixed order, no atomics (and most of the chip idle)
-    const int groups = a.aGroups * a.wGroups;
+    const long groups = aGroups * wGroups;
     a.splits = deterministic
                    ? 1
-                   : std::max(1, std::min(ceilDiv(512, groups), (int)((rows + 2 * C::SPI - 1) / (2 * C::SPI))));
+                   : (int)std::max(1L, std::min((512 + groups - 1) / groups, (rows + 2 * C::SPI - 1) / (2 * C::SPI)));
     if (a.splits > 1) {
       const long total = (long)a.wn[0] * a.wn[1] * a.wn[2] * a.wn[3];
       zeroWeight<<<dim3((unsigned)std::min<long>((total + 255) / 256, 4096)), 256, 0, s>>>(a);
     }
   }
-  const long total = (long)a.splits * a.aGroups * a.wGroups;
-  const dim3 grid((unsigned)((total + 7) / 8 * 8));
-  if (pass == FBFFT_UPDATE_OUTPUT)
-    iteratedConvKernel<N, 0><<<grid, kThreads, 0, s>>>(a);
-  else if (pass == FBFFT_UPDATE_GRAD_INPUT)
-    iteratedConvKernel<N, 1><<<grid, kThreads, 0, s>>>(a);
-  else
-    iteratedConvKernel<N, 2><<<grid, kThreads, 0, s>>>(a);
-  return launchStatus();
+  // one launch, unless its grid would be too large (more than one split has no such number
+  // of plane groups); then ranges of W groups and, below those, of A groups
+  const long wStep = std::min(wGroups, kMaxWorkgroups);
+  const long aStep = std::min(aGroups, kMaxWorkgroups / (wStep * a.splits));
+  for (long w = 0; w < wGroups; w += wStep) {
+    for (long g = 0; g < aGroups; g += aStep) {
+      a.wGroups = (int)std::min(wStep, wGroups - w);
+      a.aGroups = (int)std::min(aStep, aGroups - g);
+      a.firstW = (int)(w * C::FO);
+      const long firstA = g * C::BN;
+      a.firstA = (int)(pass == FBFFT_ACC_GRAD_PARAMETERS ? firstA : firstA % a.numTiles);
+      a.image0 = (int)(pass == FBFFT_ACC_GRAD_PARAMETERS ? 0 : firstA / a.numTiles);
+      const long total = (long)a.splits * a.aGroups * a.wGroups;
+      const dim3 grid((unsigned)((total + 7) / 8 * 8));
+      if (pass == FBFFT_UPDATE_OUTPUT)
+        iteratedConvKernel<N, 0><<<grid, kThreads, 0, s>>>(a);
+      else if (pass == FBFFT_UPDATE_GRAD_INPUT)
+        iteratedConvKernel<N, 1><<<grid, kThreads, 0, s>>>(a);
+      else
+        iteratedConvKernel<N, 2><<<grid, kThreads, 0, s>>>(a);
+      const int rc = launchStatus();
+      if (rc != FBFFT_SUCCESS) return rc;
+    }
+  }
+  return FBFFT_SUCCESS;
 }
 
 }  // namespace
@@ -652,6 +673,10 @@ int launchIteratedConv(int N, const fbfft_tile* ins, const fbfft_tile* outs, flo
   a.splits = 1;
   a.scale = scale;
   if (batch <= 0 || numTiles == 0 || wSize[0] <= 0 || wSize[1] <= 0) return 1;  // nothing to do
+  // The kernels count a reduction over (tile, image) pairs, and the tiles and the pairs of one
+  // launch (kMaxWorkgroups groups of up to 32), in 32 bits.  A weight gradient over more pairs
+  // than that came out as zeros.
+  if (numTiles > (pass == FBFFT_ACC_GRAD_PARAMETERS ? 0x7fff0000u / (unsigned)batch : 1u << 30)) return 0;
   int rc = N == 8    ? launchPass<8>(pass, a, deterministic, s)
            : N == 16 ? launchPass<16>(pass, a, deterministic, s)
                      : launchPass<32>(pass, a, deterministic, s);

@@ -266,6 +266,18 @@ def test_iterated_conv_refuses_filters_larger_than_the_transform():
     assert rc == 0
 
 
+def test_iterated_conv_refuses_more_pairs_than_32_bits_count():
+    """A weight gradient over 2^31 (tile, image) pairs is not launched (it came out as zeros):
+    decided on the host, descriptors are not read."""
+    import torch
+    w = torch.zeros((1, 1, 1, 1))
+    ins, outs = (F.Tile * 1)(), (F.Tile * 1)()
+    for batch, tiles in ((1 << 16, 1 << 15), (2 ** 31 - 1, 1), (1, 1 << 31), (3, (1 << 64) // 3 + 1)):
+        assert F.lib().fbfft_iterated_conv(8, ctypes.cast(ins, ctypes.c_void_p),
+                                           ctypes.cast(outs, ctypes.c_void_p), F.view(w), 2,
+                                           ctypes.c_float(1.0), batch, tiles, None) == 0
+
+
 def test_conv_choose_fft_size():
     """fftSize = 0 of the layer entry points: the choices recorded next to the measurements
     they came from (forward pass / input gradient / weight gradient, us per pass at

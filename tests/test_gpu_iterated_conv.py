@@ -291,3 +291,30 @@ def test_plane_groups_span_tiles_and_tensors(oracle, N, k, Nb, Cin, Cout):
         assert F.FFTIteratedConvolution(N, ins, os_, gw, F.FFT_AccGradParameters, 1.0, Nb, n,
                                         deterministic=deterministic)
         assert rel(gw.cpu().numpy(), want) < TOL_CONV
+
+
+@pytest.mark.parametrize("pass_", [0, 1, 2])
+def test_more_workgroups_than_one_grid_holds(pass_):
+    """A grid counts its lanes along x in 32 bits: 8388600 workgroups of 512.  Passes 0 and 1
+    over 8388608 groups of 32 (image, tile) pairs, the weight gradient over that many groups of
+    32 filter planes: 1 x 1 images and filters, so every value is one product."""
+    d = dev()
+    n = 32 * 8388608 - 1
+    tiles = 127                      # does not divide the pairs of the first grid
+    batch = -(-n // tiles)
+    one = torch.full((1, 1, 1, 1), 1.5, device=d)
+    if pass_ == 2:
+        small, big = one, torch.empty((1, n, 1, 1), device=d).uniform_(1, 2)
+        result = torch.full((n, 1, 1, 1), float("nan"), device=d)
+        ins, outs = F.make_tiles(small, [(0, 0, 1, 1, 0, 0)]), F.make_tiles(big, [(0, 0, 1, 1, 0, 0)])
+        assert F.FFTIteratedConvolution(8, ins[0], outs[0], result, pass_, 1.0, 1, 1)
+    else:
+        big = torch.empty((batch, 1, 1, tiles), device=d).uniform_(1, 2)
+        result = torch.full_like(big, float("nan"))
+        views = [(0, i, 1, 1, 0, 0) for i in range(tiles)]
+        src, dst = F.make_tiles(big, views), F.make_tiles(result, views)
+        ins, outs = (src, dst) if pass_ == 0 else (dst, src)
+        assert F.FFTIteratedConvolution(8, ins[0], outs[0], one, pass_, 1.0, batch, tiles)
+    result.sub_(big.view_as(result), alpha=1.5)
+    # a few roundings of values below 3; anything left out is NaN, anything misplaced differs by more
+    assert float(result.abs_().max()) < 1e-5
