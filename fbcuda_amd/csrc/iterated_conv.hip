@@ -620,6 +620,12 @@ int launchPass(int pass, ConvArgs a, bool deterministic, hipStream_t s) {
     a.splits = deterministic
                    ? 1
                    : (int)std::max(1L, std::min((512 + groups - 1) / groups, (rows + 2 * C::SPI - 1) / (2 * C::SPI)));
+    // Ranges hold whole iterations, so the last of them can be empty: those are not launched.
+    // (The ranges of an XCD are neighbours, and empty ones would all fall to the last XCD while
+    // the first takes a third round of workgroups: 34 x 29 x 35 x 35 images, 37 filters of 4 x 4,
+    // 26 ranges of which 23 hold something, 110.7 us with all of them launched, 77.4 us without.)
+    const long range = ((rows + a.splits - 1) / a.splits + C::SPI - 1) / C::SPI * C::SPI;
+    a.splits = (int)((rows + range - 1) / range);
     if (a.splits > 1) {
       const long total = (long)a.wn[0] * a.wn[1] * a.wn[2] * a.wn[3];
       zeroWeight<<<dim3((unsigned)std::min<long>((total + 255) / 256, 4096)), 256, 0, s>>>(a);

@@ -293,6 +293,20 @@ def test_plane_groups_span_tiles_and_tensors(oracle, N, k, Nb, Cin, Cout):
         assert rel(gw.cpu().numpy(), want) < TOL_CONV
 
 
+@pytest.mark.parametrize("N,Nb", [(32, 136), (32, 137), (16, 515), (8, 3), (8, 1539)])
+def test_weight_gradient_ranges_hold_every_pair_once(oracle, N, Nb):
+    """The reduction over images is cut into ranges of whole iterations; counts whose last
+    ranges would be empty (136 images in 26 ranges of 6), ragged ones and a single range."""
+    Cin, Cout, H, k = (29, 37, 10, 3) if N == 32 else (17, 3, 7, 3)
+    x = synth.uniform((Nb, Cin, H, H), seed=80)
+    g = synth.normal((Nb, Cout, H - k + 1, H - k + 1), seed=81)
+    gw = torch.full((Cout, Cin, k, k), float("nan"), device=dev())
+    xd, gd = x.to(dev()), g.to(dev())
+    ins, outs, n = F.make_tile_grid(xd, gd, k, k, N, F.FFT_AccGradParameters)
+    assert F.FFTIteratedConvolution(N, ins, outs, gw, F.FFT_AccGradParameters, 1.0, Nb, n)
+    assert rel(gw.cpu().numpy(), oracle.corr2d_grad_weight(x.numpy(), g.numpy(), k, k)) < TOL_CONV
+
+
 @pytest.mark.parametrize("pass_", [0, 1, 2])
 def test_more_workgroups_than_one_grid_holds(pass_):
     """A grid counts its lanes along x in 32 bits: 8388600 workgroups of 512.  Passes 0 and 1
