@@ -61,6 +61,7 @@ struct ConvArgs {
   int aGroups, wGroups;  // workgroups of this launch along A and W planes
   int firstA, firstW;    // its first A and W plane; passes 0, 1: A planes count from ...
   int image0;            // ... tile 0 of this image
+  int aPlanes;           // passes 0, 1: A planes per workgroup, at most BN
   float scale;
 };
 
@@ -327,7 +328,8 @@ __global__ __launch_bounds__(kThreads) void iteratedConvKernel(ConvArgs a) {
   const int logical = (blockIdx.x % 8) * per + blockIdx.x / 8;
   if (logical >= total) return;
   const int w0 = a.firstW + logical % a.wGroups * FO;              // first W plane
-  const int a0 = a.firstA + logical / a.wGroups % a.aGroups * BN;  // first A plane
+  const int aPlanes = PASS == 2 ? BN : a.aPlanes;
+  const int a0 = a.firstA + logical / a.wGroups % a.aGroups * aPlanes;  // first A plane
   const int perSplit = PASS == 2 ? ((steps + a.splits - 1) / a.splits + SPI - 1) / SPI * SPI : steps;
   const int stepBegin = PASS == 2 ? logical / (a.wGroups * a.aGroups) * perSplit : 0;
   const int stepEnd = min(steps, stepBegin + perSplit);
@@ -533,6 +535,7 @@ __global__ __launch_bounds__(kThreads) void iteratedConvKernel(ConvArgs a) {
   const int binE = 16 * group0 + be, laneBinE = binE / N * RS + binE % N;
 #pragma unroll
   for (int rd = 0; rd < BN / RA; ++rd) {
+    if (RA * rd >= aPlanes) break;
     ldsBarrier();
     if (C::SHARE == 1 || aBlock0 / AB == rd / AB) {
 #pragma unroll
@@ -570,7 +573,7 @@ __global__ __launch_bounds__(kThreads) void iteratedConvKernel(ConvArgs a) {
       } else {
         const fbfft_tile& d = PASS == 0 ? a.outs[ai % a.numTiles] : a.ins[ai % a.numTiles];
         ref = tilePlane(d, a.image0 + ai / a.numTiles, wi, a.batch);
-        ref.valid = ref.valid && wi < (PASS == 0 ? Cout : Cin);
+        ref.valid = ref.valid && wi < (PASS == 0 ? Cout : Cin) && RA * rd + se / FO < aPlanes;
       }
       if (ref.valid) {
         if (PASS == 2 && a.splits > 1)
@@ -606,7 +609,23 @@ int launchPass(int pass, ConvArgs a, bool deterministic, hipStream_t s) {
   const int Cout = a.wn[0], Cin = a.wn[1];
   const long rows = (long)a.numTiles * a.batch;  // (image, tile) pairs
   const long wGroups = ceilDiv(pass == FBFFT_UPDATE_GRAD_INPUT ? Cin : Cout, C::FO);
-  const long aGroups = pass == FBFFT_ACC_GRAD_PARAMETERS ? ceilDiv(Cin, C::BN) : (rows + C::BN - 1) / C::BN;
+  // Passes 0 and 1 over a few pairs leave most of the CUs idle when every workgroup takes BN of
+  // them; with a short reduction the first loads, the inverse transforms and the stores are most
+  // of a workgroup's time, and that is spread over the CUs instead (one workgroup per CU: 256
+  // VGPRs).  Slots beyond aPlanes transform the next workgroup's planes and drop the result.
+  // BN planes / spread, us: 3 x 1 x 24 x 32, 21 filters of 2 x 2, 8 points 23.9 / 8.8 (one
+  // workgroup per tile 21.8); 2 x 4 x 72 x 80, 17 of 7 x 7, 32 points, every other column 36.6 /
+  // 26.8 (31.4).  In a longer reduction the iterations are the time, and more workgroups only
+  // transform more: 10 x 81 x 113 x 110, 20 of 5 x 5, 32 points 263 / 306.  Around the line, 32
+  // points: 18 steps 94 / 85 (1 x 15 x 148 x 148, input gradient of 18 filters of 6 x 6), 20
+  // steps 78 / 83 (3 x 20 x 97 x 98, 53 of 11 x 11), 23 steps 89 / 97.
+  a.aPlanes = C::BN;
+  const int steps = pass == FBFFT_UPDATE_OUTPUT ? Cin : Cout;
+  if (pass != FBFFT_ACC_GRAD_PARAMETERS && steps <= 18) {
+    const long groups = std::max(1L, computeUnits() / wGroups);
+    a.aPlanes = (int)std::min<long>(C::BN, (rows + groups - 1) / groups);
+  }
+  const long aGroups = pass == FBFFT_ACC_GRAD_PARAMETERS ? ceilDiv(Cin, C::BN) : (rows + a.aPlanes - 1) / a.aPlanes;
   if (pass == FBFFT_ACC_GRAD_PARAMETERS) {
     // The reference runs one block per group of planes over the whole reduction
     // (fbfft/FFTIteratedConvolution.cuh:600-613).  With 256 CUs that leaves most of the
@@ -640,7 +659,7 @@ int launchPass(int pass, ConvArgs a, bool deterministic, hipStream_t s) {
       a.wGroups = (int)std::min(wStep, wGroups - w);
       a.aGroups = (int)std::min(aStep, aGroups - g);
       a.firstW = (int)(w * C::FO);
-      const long firstA = g * C::BN;
+      const long firstA = g * a.aPlanes;
       a.firstA = (int)(pass == FBFFT_ACC_GRAD_PARAMETERS ? firstA : firstA % a.numTiles);
       a.image0 = (int)(pass == FBFFT_ACC_GRAD_PARAMETERS ? 0 : firstA / a.numTiles);
       const long total = (long)a.splits * a.aGroups * a.wGroups;
