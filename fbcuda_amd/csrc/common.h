@@ -111,6 +111,12 @@ size_t describedWorkspaceBytes(int pass, int N, long rows, int Cin, int Cout);
 int launchDescribedConv(int pass, int N, const fbfft_tile* ins, const fbfft_tile* outs, float* weight,
                         const int* wStride, const int* wSize, float scale, int batch, int numTiles,
                         void* workspace, hipStream_t s);
+// what launchConvPass makes of a caller's transform size: the points of the windows it runs on
+// (N itself: as named), and how many ranges their reduction may be cut into
+struct PassSize {
+  int N, maxSplits;
+};
+PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW);
 int launchConvPass(int pass, int N, float* x, const int* xStride, const int* xSize, float* y,
                    const int* yStride, const int* ySize, float* out, const int* outStride,
                    const int* outSize, float scale, bool accumulate, void* workspace,

@@ -933,6 +933,7 @@ struct GemmPlan {
   enum Kind { RegsSplitK, RegsWide, Direct64, Direct128 } kind;
   int IT, JT;
   int splits, slicesPerSplit;
+  long waves;  // of one range
 };
 
 // (maxSplits: more ranges than that have no room in the workspace)
@@ -968,18 +969,41 @@ inline GemmPlan planGemm(int bins, int I, int Jp, int Kp, int maxSplits) {
   const int most = std::max(1, slices / minSlices);
   p.slicesPerSplit = ceilDiv(slices, std::min(want, most));
   p.splits = ceilDiv(slices, p.slicesPerSplit);  // no range is empty
+  p.waves = waves;
   return p;
 }
 
 constexpr int kAnySplits = 16;  // what planGemm cuts a reduction into at most
 
+// What a pass on windows takes: workspace and an estimate of its time.
+struct WindowsCost {
+  size_t bytes;
+  double us;
+};
+
+// The estimate: three launches, every spectrum value written and read once, and the
+// contraction's products over whole tiles - at the rate of one wave per SIMD where the waves
+// are fewer than that, and of whole rounds of two per SIMD in binGemmRegsWide.  Fitted to 6600
+// random layers of 64 and 128 points on one MI355X; it is within 20 % of nine in ten of them.
 template <int N>
-size_t workspaceFloat2(int I, int J, int K, bool outTiled, int maxSplits = kAnySplits) {
+WindowsCost windowsCost(int I, int J, int K, bool outTiled, int maxSplits) {
   if (swapRoles(I, J, outTiled)) std::swap(I, J);
   const int SL = BMCfg<N>::SLOTS, bins = BMCfg<N>::BINS;
   const int Ip = roundUp(I, SL), Jp = roundUp(J, SL), Kp = roundUp(K, 8);
-  return (size_t)bins * ((size_t)Kp * Ip + (size_t)Kp * Jp +
-                         (size_t)planGemm(bins, I, Jp, Kp, maxSplits).splits * I * Jp);
+  const GemmPlan plan = planGemm(bins, I, Jp, Kp, maxSplits);
+  WindowsCost c;
+  c.bytes = sizeof(float2) * bins * ((size_t)Kp * Ip + (size_t)Kp * Jp + (size_t)plan.splits * I * Jp);
+  const double products = (double)bins * roundUp(I, I <= 32 ? 32 : 64) * roundUp(Jp, 64) * Kp;
+  const bool wide = plan.kind == GemmPlan::RegsWide;
+  const long waves = plan.waves * plan.splits;
+  const double idle = waves < 1024 ? 1024.0 / waves : wide ? (waves + 2047) / 2048 * 2048.0 / waves : 1.0;
+  c.us = 15 + 0.14e-6 * 2 * c.bytes + (wide ? 0.055e-6 : 0.04e-6) * products * idle;
+  return c;
+}
+
+template <int N>
+size_t workspaceFloat2(int I, int J, int K, bool outTiled) {
+  return windowsCost<N>(I, J, K, outTiled, kAnySplits).bytes / sizeof(float2);
 }
 
 // P[i][j] = scale * sum_k X[i][k] * op(Y[j][k]) for planes x(i,k), y(j,k) -> planes out(i,j);
@@ -1172,25 +1196,34 @@ static void passDims(int pass, int B, int Cin, int Cout, int* I, int* J, int* K)
   else { *I = Cin; *J = Cout; *K = B; }
 }
 
-// workspace of a pass on windows of N <= 32 points
-static size_t windowsBytes(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW,
-                           int maxSplits) {
+// a pass on windows of N <= 32 points; no bytes: too many windows
+static WindowsCost windowsPass(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW,
+                               int maxSplits) {
   int ty, tx;
   tileGrid(pass, N, H, W, kH, kW, &ty, &tx);
-  if ((long)B * ty * tx > (1L << 30)) return 0;
+  if ((long)B * ty * tx > (1L << 30)) return {0, 0};
   int I, J, K;
   passDims(pass, B * ty * tx, Cin, Cout, &I, &J, &K);
   const bool outTiled = pass != 2 && ty * tx > 1;  // the weight gradient is never tiled
-  size_t n = N == 8 ? workspaceFloat2<8>(I, J, K, outTiled, maxSplits)
-                    : N == 16 ? workspaceFloat2<16>(I, J, K, outTiled, maxSplits)
-                              : workspaceFloat2<32>(I, J, K, outTiled, maxSplits);
-  return n * sizeof(float2);
+  return N == 8    ? windowsCost<8>(I, J, K, outTiled, maxSplits)
+         : N == 16 ? windowsCost<16>(I, J, K, outTiled, maxSplits)
+                   : windowsCost<32>(I, J, K, outTiled, maxSplits);
 }
 
 size_t convWorkspaceBytes(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH,
                           int kW) {
   if (N > 32) return convSplitWorkspaceBytes(pass, N, B, Cin, Cout);
-  return windowsBytes(pass, N, B, Cin, Cout, H, W, kH, kW, kAnySplits);
+  return windowsPass(pass, N, B, Cin, Cout, H, W, kH, kW, kAnySplits).bytes;
+}
+
+// The same estimate for plane-major spectra of N = 64 or 128 points (conv_split.hip), where
+// transposeMM takes 4 k at a time.
+static double planeMajorMicroseconds(int pass, int N, int B, int Cin, int Cout) {
+  int I, J, K;
+  passDims(pass, B, Cin, Cout, &I, &J, &K);
+  const double planes = (double)I * K + (double)J * K + (double)I * J, XY = (N / 2 + 1) * (double)N;
+  return 33 + 0.22e-6 * 2 * sizeof(float2) * planes * XY +
+         0.033e-6 * XY * roundUp(I, 32) * (double)roundUp(J, 32) * roundUp(K, 4);
 }
 
 // The transform size a pass runs on, and how many ranges its reduction may be cut into.  A
@@ -1201,12 +1234,20 @@ size_t convWorkspaceBytes(int pass, int N, int B, int Cin, int Cout, int H, int 
 // the windows within the workspace of the named size.
 //
 // 64 and 128 points (plane-major spectra of the whole image) give way to windows that hold
-// no more spectrum, with one range of the reduction where several have no room.  Three
-// passes, plane-major / windows: 32 x 32 x 60 x 60 images, 64 filters of 5 x 5 216 / 145 us;
-// 24 x 48 x 40 x 40, 96 of 8 x 8 339 / 151 us; 8 x 200 x 50 x 58, 300 of 1 x 1 2170 / 273 us;
-// 128 points, 16 x 32 x 100 x 100, 64 of 8 x 8 490 / 207 us.  (With twice that workspace 11 x
-// 11 filters on 60 x 60 images would move to windows too: 217 -> 227 us.)  Filters larger
-// than 32 or filling most of a window stay plane-major.
+// no more spectrum and are not expected to take longer, with as many ranges of the reduction
+// as there is room for.  Three passes, plane-major / windows: 32 x 32 x 60 x 60 images, 64
+// filters of 5 x 5 216 / 145 us; 24 x 48 x 40 x 40, 96 of 8 x 8 339 / 151 us; 8 x 200 x 50 x
+// 58, 300 of 1 x 1 2170 / 273 us; 128 points, 16 x 32 x 100 x 100, 64 of 8 x 8 490 / 207 us.
+// Less spectrum alone does not make a weight gradient faster: its windows are longer
+// reductions over tiles that many channels or few filters leave partly empty (64 points, 173 x
+// 80 x 63 x 64, 362 of 3 x 3 1375 / 2000 us; 162 x 299 x 60 x 60, 115 of 6 x 6 1346 / 1796 us;
+// 128 points, 93 x 193 x 122 x 119, 41 of 8 x 8 1360 / 1772 us), and where the planned ranges
+// lack a little room (128 points, 153 x 3 x 73 x 70, 33 of 2 x 2: plane-major 308, 1 range 528,
+// the 15 that fit 212 us; 64 points, 85 x 32 x 33 x 61, 66 of 7 x 7: 124, 1 range 241, the 3
+// that fit 173 us, so plane-major).  Of 6570 random layers whose windows fit, 12 take over 3 %
+// longer than plane-major by this rule (at most 18 %), 7 over 10 % longer than on windows; by
+// the spectrum alone 59 take over 3 % longer, at most 45 %.  Filters larger than 32 or filling
+// most of a window stay plane-major.
 //
 // 16 and 32 points are the same kernels on either side, and a caller who names them means
 // them: they give way only where most of the named transforms would be padding - windows
@@ -1218,20 +1259,21 @@ size_t convWorkspaceBytes(int pass, int N, int B, int Cin, int Cout, int H, int 
 // the line less is left to win, and smaller transforms pay more per value: forward 128 x 64 x
 // 27 x 27, 192 of 5 x 5 99.6 / 91.0 (16, 80 %), weight gradient 16 x 32 x 100 x 100, 64 of
 // 3 x 3 74.9 / 75.4 (16, 79 %), 128 x 192 x 27 x 27, 64 of 5 x 5 99.5 / 107.9 (16, 93 %).
-struct PassSize {
-  int N, maxSplits;
-};
-static PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
+PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
+  const PassSize named{N, kAnySplits};
   const int n = fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW);
-  if (n == 0 || n >= N) return {N, kAnySplits};
+  if (n == 0 || n >= N) return named;
   const size_t room = convWorkspaceBytes(pass, N, B, Cin, Cout, H, W, kH, kW);
-  const size_t percent = N > 32 ? 100 : 60;
-  for (int maxSplits : {kAnySplits, 1}) {
-    const size_t need = windowsBytes(pass, n, B, Cin, Cout, H, W, kH, kW, maxSplits);
-    if (need != 0 && need <= room - room / 100 * (100 - percent)) return {n, maxSplits};
-    if (N <= 32) break;  // fewer ranges than the product asks for cost more than windows give
+  if (N <= 32) {
+    const WindowsCost c = windowsPass(pass, n, B, Cin, Cout, H, W, kH, kW, kAnySplits);
+    return c.bytes != 0 && c.bytes <= room - room / 100 * 40 ? PassSize{n, kAnySplits} : named;
   }
-  return {N, kAnySplits};
+  for (int maxSplits = kAnySplits; maxSplits > 0; --maxSplits) {
+    const WindowsCost c = windowsPass(pass, n, B, Cin, Cout, H, W, kH, kW, maxSplits);
+    if (c.bytes != 0 && c.bytes <= room)
+      return c.us <= planeMajorMicroseconds(pass, N, B, Cin, Cout) ? PassSize{n, maxSplits} : named;
+  }
+  return named;
 }
 
 // pass 0: x = input [B][Cin][H][W], y = weight [Cout][Cin][kH][kW], out = output [B][Cout][oH][oW]

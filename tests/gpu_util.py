@@ -1,5 +1,7 @@
 """Shared helpers of the GPU parity tests: they call the product through its C ABI
 (fbcuda_amd -> libfbfft_amd.so) and check it against the CPU oracle."""
+import ctypes
+
 import numpy as np
 import torch
 
@@ -7,6 +9,19 @@ import fbcuda_amd as F
 
 TOL_FFT = 1e-5    # rel-L2 per transform (vs the fp32 transcription and vs the fp64 DFT)
 TOL_CONV = 1e-4   # rel-L2 per full convolution
+
+
+class PassSize(ctypes.Structure):
+    _fields_ = [("N", ctypes.c_int), ("maxSplits", ctypes.c_int)]
+
+
+def pass_size(pass_, N, B, cin, cout, H, W, k):
+    """(points, ranges at most) that a layer pass named N points runs on: the library's own
+    host function, which is no part of the C ABI (common.h)."""
+    fn = F.lib()._ZN9fbfft_amd8passSizeEiiiiiiiii
+    fn.argtypes, fn.restype = [ctypes.c_int] * 9, PassSize
+    r = fn(pass_, N, B, cin, cout, H, W, k, k)
+    return r.N, r.maxSplits
 
 
 def dev():

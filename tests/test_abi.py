@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import fbcuda_amd as F
+from gpu_util import pass_size
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -276,6 +277,34 @@ def test_iterated_conv_refuses_more_pairs_than_32_bits_count():
         assert F.lib().fbfft_iterated_conv(8, ctypes.cast(ins, ctypes.c_void_p),
                                            ctypes.cast(outs, ctypes.c_void_p), F.view(w), 2,
                                            ctypes.c_float(1.0), batch, tiles, None) == 0
+
+
+@pytest.mark.parametrize("pass_,N,B,cin,cout,H,W,k,want", [
+    # ranges: the largest number that the named workspace has room for (16: as many as planned)
+    (2, 128, 153, 3, 33, 73, 70, 2, (16, 15)),
+    (2, 64, 95, 13, 34, 43, 43, 2, (16, 7)),
+    (2, 128, 8, 5, 52, 125, 125, 3, (16, 3)),
+    (2, 64, 85, 32, 66, 33, 61, 7, (64, 16)),      # 3 ranges of 6: plane-major 124 us, windows 173
+    (2, 64, 36, 18, 107, 56, 62, 8, (64, 16)),     # 1 range of 2: 85, 92
+    # windows that fit with all ranges and are slower all the same
+    (2, 64, 173, 80, 362, 63, 64, 3, (64, 16)),    # 1375, 1992
+    (2, 64, 162, 299, 115, 60, 60, 6, (64, 16)),   # 1346, 1796
+    (2, 128, 93, 193, 41, 122, 119, 8, (128, 16)),  # 1360, 1772
+    (0, 64, 57, 247, 190, 63, 64, 8, (64, 16)),    # 799, 954
+    # and faster ones
+    (0, 64, 32, 32, 64, 60, 60, 5, (32, 16)),
+    (1, 64, 32, 32, 64, 60, 60, 5, (16, 1)),       # 1 range of 2
+    (2, 64, 32, 32, 64, 60, 60, 5, (32, 16)),
+    (2, 128, 16, 32, 64, 100, 100, 8, (32, 16)),
+    # 32 points: three fifths of the named workspace
+    (0, 32, 32, 64, 192, 27, 27, 5, (16, 16)),     # 42 %
+    (2, 32, 32, 64, 192, 27, 27, 5, (16, 16)),     # 55 %
+    (0, 32, 128, 64, 192, 27, 27, 5, (32, 16)),    # 80 %
+])
+def test_transform_size_of_a_named_layer(pass_, N, B, cin, cout, H, W, k, want):
+    """The size and the ranges that a layer pass runs on, decided on the host from the layer
+    alone, on both sides of each line of the rule."""
+    assert pass_size(pass_, N, B, cin, cout, H, W, k) == want
 
 
 def test_conv_choose_fft_size():

@@ -9,7 +9,7 @@ import torch
 
 import fbcuda_amd as F
 from fbcuda_amd import synth
-from gpu_util import check, TOL_CONV, dev, rel
+from gpu_util import check, TOL_CONV, dev, pass_size, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -154,49 +154,63 @@ def test_fft_size_zero_is_the_library_choice(oracle, H, W, k):
     assert torch.equal(out, res[0][0])
 
 
-@pytest.mark.parametrize("N,H,W,k,Bn,Cin,Cout", [
-    (64, 60, 60, 5, 16, 16, 32),     # every pass in windows; the input gradient with one range
-    (64, 64, 33, 8, 17, 20, 40),
-    (128, 100, 97, 3, 4, 33, 20),
-    (64, 60, 57, 5, 1, 2, 3),        # windows padded to whole plane groups do not fit: plane-major
-    (64, 61, 64, 20, 6, 5, 7),       # little of a window is kept: plane-major
-    (64, 62, 64, 33, 6, 5, 7),       # filter larger than a window: plane-major
+@pytest.mark.parametrize("N,H,W,k,Bn,Cin,Cout,sizes", [
+    (64, 60, 60, 5, 16, 16, 32, (32, 16, 32)),
+    (64, 64, 33, 8, 17, 20, 40, (16, 64, 32)),     # planned ranges do not fit: fewer, or plane-major
+    (64, 43, 41, 4, 21, 3, 54, (16, 64, 16)),      # weight gradient: 2 of the planned 8 ranges fit
+    (128, 100, 97, 3, 4, 33, 20, (16, 16, 16)),
+    (64, 60, 57, 5, 1, 2, 3, (64, 64, 64)),        # windows padded to whole plane groups do not fit
+    (64, 61, 64, 20, 6, 5, 7, (64, 64, 64)),       # little of a window is kept
+    (64, 62, 64, 33, 6, 5, 7, (64, 64, 64)),       # filter larger than a window
 ])
-def test_named_sizes_above_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin, Cout):
+def test_named_sizes_above_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin, Cout, sizes):
     """64 and 128 points run on windows or on plane-major spectra, whichever is faster, both
     within the workspace of the named size (the bytes behind it stay as they were)."""
-    passes_on_named_workspace(oracle, N, H, W, k, Bn, Cin, Cout)
+    passes_on_named_workspace(oracle, N, H, W, k, Bn, Cin, Cout, sizes)
 
 
-@pytest.mark.parametrize("N,H,W,k,Bn,Cin,Cout", [
-    (32, 27, 27, 5, 9, 20, 40),      # 16-point windows in the weight gradient
-    (32, 13, 13, 3, 17, 33, 50),     # 8- and 16-point windows, channels past a tile's edge
-    (32, 16, 9, 3, 5, 3, 20),        # an image that fits 16 points whole
-    (32, 100, 61, 3, 2, 20, 24),     # larger than the named transform
-    (32, 30, 32, 11, 6, 5, 7),       # little of a smaller window is kept: the named size
-    (16, 13, 14, 3, 8, 20, 24),      # little to save: the named size
-    (16, 8, 8, 1, 3, 7, 9),          # 8-point windows
-    (8, 7, 8, 3, 3, 7, 9),           # nothing smaller
+@pytest.mark.parametrize("N,H,W,k,Bn,Cin,Cout,sizes", [
+    (32, 27, 27, 5, 9, 20, 40, (32, 32, 16)),
+    (32, 13, 13, 3, 17, 33, 50, (8, 16, 8)),       # channels past a tile's edge
+    (32, 16, 9, 3, 5, 3, 20, (16, 16, 16)),        # an image that fits 16 points whole
+    (32, 100, 61, 3, 2, 20, 24, (32, 16, 32)),     # larger than the named transform
+    (32, 30, 32, 11, 6, 5, 7, (32, 32, 32)),       # little of a smaller window is kept
+    (16, 13, 14, 3, 8, 20, 24, (16, 16, 16)),      # little to save
+    (16, 8, 8, 1, 3, 7, 9, (8, 8, 8)),
+    (8, 7, 8, 3, 3, 7, 9, (8, 8, 8)),              # nothing smaller
 ])
-def test_named_sizes_up_to_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin, Cout):
+def test_named_sizes_up_to_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin, Cout, sizes):
     """16 and 32 points run on smaller windows where those need at most three fifths of the
     named size's workspace, and within it."""
-    passes_on_named_workspace(oracle, N, H, W, k, Bn, Cin, Cout)
+    passes_on_named_workspace(oracle, N, H, W, k, Bn, Cin, Cout, sizes)
 
 
-def passes_on_named_workspace(oracle, N, H, W, k, Bn, Cin, Cout):
+def passes_on_named_workspace(oracle, N, H, W, k, Bn, Cin, Cout, sizes):
+    """sizes: the transform each pass runs on.  Results are reproducible bit for bit, so a call
+    on windows of n points is one that names n, and no call that names another size."""
     d = dev()
     x = synth.uniform((Bn, Cin, H, W), seed=70, device=d)
     w = synth.normal((Cout, Cin, k, k), seed=71, std=0.05, device=d)
     g = synth.normal((Bn, Cout, H - k + 1, W - k + 1), seed=72, device=d)
     out, gi, gw = (torch.full_like(t, float("nan")) for t in (g, x, w))
-    for pass_, call in ((0, lambda s: F.conv_fprop(x, w, out, N, s)),
-                        (1, lambda s: F.conv_bprop(g, w, gi, N, s)),
-                        (2, lambda s: F.conv_accgrad(x, g, gw, N, s))):
-        n = F.conv_workspace_image(pass_, Bn, Cin, Cout, H, W, k, k, N)
-        space = torch.full((n + 256,), 77, dtype=torch.uint8, device=d)
-        assert call(space[:n]) == F.Success
-        assert bool((space[n:] == 77).all())
+    calls = ((out, lambda n, s: F.conv_fprop(x, w, out, n, s)),
+             (gi, lambda n, s: F.conv_bprop(g, w, gi, n, s)),
+             (gw, lambda n, s: F.conv_accgrad(x, g, gw, n, s)))
+    for pass_, (result, call) in enumerate(calls):
+        def run(points):
+            n = F.conv_workspace_image(pass_, Bn, Cin, Cout, H, W, k, k, points)
+            space = torch.full((n + 256,), 77, dtype=torch.uint8, device=d)
+            result.fill_(float("nan"))
+            assert call(points, space[:n]) == F.Success
+            assert bool((space[n:] == 77).all())
+            return result.clone()
+        named = run(N)
+        assert pass_size(pass_, N, Bn, Cin, Cout, H, W, k)[0] == sizes[pass_]
+        all_ranges = pass_size(pass_, N, Bn, Cin, Cout, H, W, k)[1] == 16
+        for n in (8, 16, 32):
+            if k <= n < N and pass_size(pass_, n, Bn, Cin, Cout, H, W, k)[0] == n and all_ranges:
+                assert torch.equal(named, run(n)) == (n == sizes[pass_]), (pass_, n)
+        result.copy_(named)
     xh, wh, gh = x.cpu().numpy(), w.cpu().numpy(), g.cpu().numpy()
     assert rel(out.cpu().numpy(), oracle.corr2d_valid(xh, wh)) < TOL_CONV
     assert rel(gi.cpu().numpy(), oracle.corr2d_grad_input(gh, wh, H, W)) < TOL_CONV
