@@ -296,6 +296,41 @@ def test_plane_groups_span_tiles_and_tensors(oracle, N, k, Nb, Cin, Cout):
         assert rel(gw.cpu().numpy(), want) < TOL_CONV
 
 
+def strided(t, form):
+    """t's values on the device in another layout: odd plane strides (8-byte words that are
+    aligned in every other plane only), or every other column."""
+    b, c, h, w = t.shape
+    if form == "odd planes":
+        s = h * (w + w % 2) + 1
+        u = torch.full((b * c * s + 1,), float("nan"), device=dev())[:-1]
+        u = u.as_strided((b, c, h, w), (c * s, s, w + w % 2, 1))
+    else:
+        u = torch.full((b, c, h, 2 * w), float("nan"), device=dev())[..., ::2]
+    return u.copy_(t)
+
+
+@pytest.mark.parametrize("form", ["odd planes", "every other column"])
+@pytest.mark.parametrize("N,k,Nb,Cin,Cout,H,W", [(8, 2, 3, 5, 7, 12, 10), (16, 4, 2, 19, 5, 20, 30),
+                                                 (32, 6, 2, 3, 21, 32, 44), (32, 2, 9, 5, 3, 38, 32)])
+def test_fused_kernel_on_planes_that_change_alignment_or_stride(oracle, N, k, Nb, Cin, Cout, H, W, form):
+    """Even widths and row strides, so that a lane's two columns may move as one word - in the
+    planes that start on one; and planes that no word load serves.  Images and filters, every pass."""
+    x = synth.uniform((Nb, Cin, H, W), seed=90)
+    w = synth.normal((Cout, Cin, k, k), seed=91, std=0.05)
+    g = synth.normal((Nb, Cout, H - k + 1, W - k + 1), seed=92)
+    xd, wd, gd = (strided(t, form) for t in (x, w, g))
+    for pass_ in (0, 1, 2):
+        ops = [xd, wd, gd]
+        slot = {0: 2, 1: 0, 2: 1}[pass_]
+        ops[slot] = strided(torch.full_like((x, w, g)[slot], float("nan")), form)
+        ins, outs, n = F.make_tile_grid(ops[0], ops[2], k, k, N, pass_)
+        assert F.FFTIteratedConvolution(N, ins, outs, ops[1], pass_, 1.0, Nb, n)
+        want = (oracle.corr2d_valid(x.numpy(), w.numpy()) if pass_ == 0 else
+                oracle.corr2d_grad_input(g.numpy(), w.numpy(), H, W) if pass_ == 1 else
+                oracle.corr2d_grad_weight(x.numpy(), g.numpy(), k, k))
+        assert rel(ops[slot].cpu().numpy(), want) < TOL_CONV
+
+
 @pytest.mark.parametrize("N,Nb", [(32, 136), (32, 137), (16, 515), (8, 3), (8, 1539)])
 def test_weight_gradient_ranges_hold_every_pair_once(oracle, N, Nb):
     """The reduction over images is cut into ranges of whole iterations; counts whose last
