@@ -1249,16 +1249,25 @@ static double planeMajorMicroseconds(int pass, int N, int B, int Cin, int Cout) 
 // the spectrum alone 59 take over 3 % longer, at most 45 %.  Filters larger than 32 or filling
 // most of a window stay plane-major.
 //
-// 16 and 32 points are the same kernels on either side, and a caller who names them means
-// them: they give way only where most of the named transforms would be padding - windows
-// that need at most three fifths of the named size's workspace.  One pass, named 32 points /
-// windows of n, us at the windows' share of that workspace: 32 x 64 x 27 x 27 images, 192
-// filters of 5 x 5, forward 56.6 / 32.1 (n = 16, 42 %), weight gradient 42.9 / 37.0 (16, 55 %);
-// 64 x 96 x 13 x 13, 256 of 3 x 3, forward 91.7 / 34.3 (8, 15 %), input gradient 105.6 / 37.3
-// (16, 28 %); 16 x 128 x 30 x 30, 128 of 3 x 3, input gradient 55.4 / 33.0 (8, 36 %).  Above
-// the line less is left to win, and smaller transforms pay more per value: forward 128 x 64 x
-// 27 x 27, 192 of 5 x 5 99.6 / 91.0 (16, 80 %), weight gradient 16 x 32 x 100 x 100, 64 of
-// 3 x 3 74.9 / 75.4 (16, 79 %), 128 x 192 x 27 x 27, 64 of 5 x 5 99.5 / 107.9 (16, 93 %).
+// 16 and 32 points are the same kernels on either side, and a caller who names them may mean
+// them (size 0 is there for the fastest): they give way only where most of the named transforms
+// would be padding, windows that need at most three fifths of the named size's workspace.  The
+// line is drawn for that, not where the gain ends.  One pass, named 32 points / windows of n,
+// us at the windows' share of that workspace: 32 x 64 x 27 x 27 images, 192 filters of 5 x 5,
+// forward 56.6 / 32.1 (n = 16, 42 %), weight gradient 42.9 / 37.0 (16, 55 %); 64 x 96 x 13 x
+// 13, 256 of 3 x 3, forward 91.7 / 34.3 (8, 15 %), input gradient 105.6 / 37.3 (16, 28 %);
+// 2030 random layers below it 4 to 88 % faster.  Above it, given up: weight gradient 103.3 /
+// 87.6 (61 %), forward 59.2 / 53.3 (84 %), 128 x 64 x 27 x 27, 192 of 5 x 5 99.6 / 91.0 (16, 80
+// %); and no gain: weight gradient 16 x 32 x 100 x 100, 64 of 3 x 3 74.9 / 75.4 (16, 79 %),
+// 128 x 192 x 27 x 27, 64 of 5 x 5 99.5 / 107.9 (16, 93 %).
+//
+// From 16 to 8 points the contraction has a quarter of the bins, 32, and small products leave
+// most of the chip idle with one chain of slices each, whatever the spectra save (forward 28 x
+// 45 x 8 x 9, 15 of 3 x 3, 16 / 8 points 14.8 / 16.6 us; input gradient 2 x 4 x 12 x 12, 50 of
+// 1 x 1 14.8 / 16.4; weight gradient 4 x 310 x 25 x 25, 175 of 6 x 6 38.9 / 49.3): there the
+// estimates must not differ by more than 5 % to the windows' disadvantage, either.  Of 5790
+// random layers below the line 223 took over 3 % longer on 8 points and 66 over 10 %; by both
+// tests 92 and 17 (30 x 243 x 14 x 11, 245 of 4 x 4, input gradient 47.2 / 59.0 the most).
 PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
   const PassSize named{N, kAnySplits};
   const int n = fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW);
@@ -1266,7 +1275,9 @@ PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int k
   const size_t room = convWorkspaceBytes(pass, N, B, Cin, Cout, H, W, kH, kW);
   if (N <= 32) {
     const WindowsCost c = windowsPass(pass, n, B, Cin, Cout, H, W, kH, kW, kAnySplits);
-    return c.bytes != 0 && c.bytes <= room - room / 100 * 40 ? PassSize{n, kAnySplits} : named;
+    if (c.bytes == 0 || c.bytes > room - room / 100 * 40) return named;
+    if (N == 16 && c.us > 1.05 * windowsPass(pass, N, B, Cin, Cout, H, W, kH, kW, kAnySplits).us) return named;
+    return {n, kAnySplits};
   }
   for (int maxSplits = kAnySplits; maxSplits > 0; --maxSplits) {
     const WindowsCost c = windowsPass(pass, n, B, Cin, Cout, H, W, kH, kW, maxSplits);

@@ -300,6 +300,13 @@ def test_iterated_conv_refuses_more_pairs_than_32_bits_count():
     (0, 32, 32, 64, 192, 27, 27, 5, (16, 16)),     # 42 %
     (2, 32, 32, 64, 192, 27, 27, 5, (16, 16)),     # 55 %
     (0, 32, 128, 64, 192, 27, 27, 5, (32, 16)),    # 80 %
+    # 16 points: the same, and no smaller product left to less of the chip
+    (0, 16, 9, 20, 40, 8, 8, 1, (8, 16)),
+    (1, 16, 64, 96, 128, 14, 14, 3, (16, 16)),     # 137 %
+    (0, 16, 28, 45, 15, 8, 9, 3, (16, 16)),        # 50 %, 14.8 us, on 8 points 16.6
+    (1, 16, 2, 4, 50, 12, 12, 1, (16, 16)),        # 51 %, 14.8, 16.4
+    (2, 16, 4, 310, 175, 25, 25, 6, (16, 16)),     # 60 %, 38.9, 49.3
+    (2, 16, 2, 64, 300, 10, 10, 3, (8, 16)),
 ])
 def test_transform_size_of_a_named_layer(pass_, N, B, cin, cout, H, W, k, want):
     """The size and the ranges that a layer pass runs on, decided on the host from the layer

@@ -176,7 +176,8 @@ def test_named_sizes_above_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin
     (32, 100, 61, 3, 2, 20, 24, (32, 16, 32)),     # larger than the named transform
     (32, 30, 32, 11, 6, 5, 7, (32, 32, 32)),       # little of a smaller window is kept
     (16, 13, 14, 3, 8, 20, 24, (16, 16, 16)),      # little to save
-    (16, 8, 8, 1, 3, 7, 9, (8, 8, 8)),
+    (16, 8, 8, 1, 3, 7, 9, (8, 16, 8)),            # a small product would leave the chip idle
+    (16, 8, 8, 1, 40, 30, 60, (8, 8, 8)),
     (8, 7, 8, 3, 3, 7, 9, (8, 8, 8)),              # nothing smaller
 ])
 def test_named_sizes_up_to_32_on_their_own_workspace(oracle, N, H, W, k, Bn, Cin, Cout, sizes):
