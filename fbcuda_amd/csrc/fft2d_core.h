@@ -120,77 +120,6 @@ __device__ __forceinline__ void loadColumnsWindow(const float* src, int sy, int 
   }
 }
 
-// The same two columns for callers whose window geometry differs from lane to
-// lane of a wave (tile descriptors of different planes): the per-row terms are
-// then vector arithmetic, and skipping the loads outside the window (tiles with
-// 9 x 9 filters load 81 of 1024 samples) costs less than clamping every address.
-template <int N>
-__device__ __forceinline__ void loadColumnsWindowPerLane(const float* src, int sy, int sx, int h,
-                                                         int w, int padL, int padU, int l,
-                                                         c32 (&z0)[N / 2], c32 (&z1)[N / 2]) {
-  const int xa = 2 * l - padL, xb = xa + 1;
-  const bool va = (unsigned)xa < (unsigned)w, vb = (unsigned)xb < (unsigned)w;
-  // element (y, xa) of the plane is pa[y * sy]; pa itself may point outside the
-  // window and is only dereferenced under the tests
-  // (global address space stated explicitly: the plane pointer comes out of a
-  // descriptor in memory, and a generic pointer would make these flat loads)
-  typedef const __attribute__((address_space(1))) float* GlobalPtr;
-  // When every lane of the wave sees rows that start on 8-byte boundaries and a
-  // window whose left edge and width are even, its two columns are one 8-byte word
-  // per row, inside or outside the window together.
-  const bool pairs = sx == 1 && ((sy | padL | w) & 1) == 0 &&
-                     (reinterpret_cast<uintptr_t>(src) & 7) == 0;
-  if (__builtin_amdgcn_ballot_w64(!pairs) == 0) {
-    typedef float Pair __attribute__((ext_vector_type(2)));
-    typedef const __attribute__((address_space(1))) Pair* GlobalPtr2;
-    GlobalPtr2 pp = (GlobalPtr2)(src + xa - (long)padU * sy);
-    const int sy2 = sy / 2;
-    Pair r[N];
-    // ... and when every lane's window covers the whole transform (the inner tiles of a
-    // larger image), nothing is zeroed and nothing is tested row by row
-    const bool whole = padU == 0 && padL == 0 && h >= N && w >= N;
-    if (__builtin_amdgcn_ballot_w64(!whole) == 0) {
-      staticFor<N>([&](auto yy) {
-        constexpr int y = decltype(yy)::value;
-        r[y] = pp[(long)y * sy2];
-      });
-      staticFor<N / 2>([&](auto jj) {
-        constexpr int j = decltype(jj)::value;
-        z0[j] = c32{r[2 * j].x, r[2 * j + 1].x};
-        z1[j] = c32{r[2 * j].y, r[2 * j + 1].y};
-      });
-      return;
-    }
-    staticFor<N>([&](auto yy) {
-      constexpr int y = decltype(yy)::value;
-      r[y] = Pair{0.0f, 0.0f};
-      if ((unsigned)(y - padU) < (unsigned)h && va) r[y] = pp[(long)y * sy2];
-    });
-    staticFor<N / 2>([&](auto jj) {
-      constexpr int j = decltype(jj)::value;
-      z0[j] = c32{r[2 * j].x, r[2 * j + 1].x};
-      z1[j] = c32{r[2 * j].y, r[2 * j + 1].y};
-    });
-    return;
-  }
-  GlobalPtr pa = (GlobalPtr)(src + (long)xa * sx - (long)padU * sy);
-  GlobalPtr pb = pa + sx;
-  float ra[N], rb[N];
-  staticFor<N>([&](auto yy) {
-    constexpr int y = decltype(yy)::value;
-    const bool vy = (unsigned)(y - padU) < (unsigned)h;
-    ra[y] = 0.0f;
-    rb[y] = 0.0f;
-    if (vy && va) ra[y] = pa[(long)y * sy];
-    if (vy && vb) rb[y] = pb[(long)y * sy];
-  });
-  staticFor<N / 2>([&](auto jj) {
-    constexpr int j = decltype(jj)::value;
-    z0[j] = c32{ra[2 * j], ra[2 * j + 1]};
-    z1[j] = c32{rb[2 * j], rb[2 * j + 1]};
-  });
-}
-
 // Column pass (forward): N/2-point FFTs of the two packed columns and the real-input
 // fix-up, in registers ...
 template <int N>
