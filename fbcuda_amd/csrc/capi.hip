@@ -298,9 +298,9 @@ extern "C" int fbfft_conv_choose_fft_size(int pass, int batch, int cin, int cout
   // INPUT.  Smaller transforms run a little below the rate of 32-point ones (measured
   // over nine layer shapes: 1.15 x per value at 16 points, 1.5 x at 8), and their weight
   // gradients further below (1.25 x and 2 x: many windows make a long reduction over small
-  // tiles).  The larger transform on a tie.  64 and 128 are never chosen: their layers run
-  // plane-major spectra through transposeMM and measure slower than 32-point windows on
-  // every shape tried.
+  // tiles).  The larger transform on a tie.  64 and 128 are never chosen: windows are faster on
+  // most layers, and a caller who names 64 or 128 has the plane-major spectra where they are
+  // (passSize in conv_pipeline.hip).
   int best = 0;
   double bestCost = 0;
   for (int N = 8; N <= 32; N *= 2) {

@@ -44,6 +44,9 @@
 // identity; weight gradient (input plane, output plane, image), op = conj.  The
 // kernels always compute sum_k A * conj(B); the forward transforms store a
 // spectrum conjugated where the pass needs it.
+//
+// Figures below name two layers: the 27 x 27 layer, 128 x 64 x 27 x 27 images and 192 filters
+// of 5 x 5, and the 256 x 256 layer, 16 x 32 x 256 x 256 images and 32 filters of 9 x 9.
 #include "common.h"
 #include "fft2d_core.h"
 #include "fft_regs.h"
@@ -55,8 +58,8 @@ namespace {
 
 constexpr int kT = 256;
 // lanes of a transform workgroup: 16 planes of 32 x 32, so that a bin leaves or arrives as
-// a 128-byte run (measured at configs[3] / configs[4]: 128 lanes, 64-byte runs, +10 % /
-// +12 % per pass; 512 lanes, one workgroup per CU, +8 % / +6 %)
+// a 128-byte run (measured at the 27 x 27 / the 256 x 256 layer: 128 lanes, 64-byte runs,
+// +10 % / +12 % per pass; 512 lanes, one workgroup per CU, +8 % / +6 %)
 constexpr int kTF = 256;
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
@@ -116,14 +119,14 @@ struct PlaneWindow {
 };
 
 // DESCRIBED is a compile-time fact (the kernels' PAIRS == 2 instantiations): carried as a
-// run-time test it cost the tiled sets 2 % (configs[4]: 290 against 284 us).
+// run-time test it cost the tiled sets 2 % (the 256 x 256 layer: 290 against 284 us).
 template <bool DESCRIBED>
 __device__ __forceinline__ PlaneWindow planeWindow(const PlaneSet& ps, int row, int k) {
   if constexpr (DESCRIBED) {
     const int comp = ps.described == 1 ? row : k, other = ps.described == 1 ? k : row;
     // image-major: consecutive composites are consecutive tiles of one image - in a
     // row-major tiling neighbours in memory, which is what 16 planes of a workgroup should
-    // be (tile-major, 16 images of one tile: 345 instead of 296 us at configs[4])
+    // be (tile-major, 16 images of one tile: 345 instead of 296 us at the 256 x 256 layer)
     const fbfft_tile& d = ps.tiles[comp % ps.numTiles];
     const int n = comp / ps.numTiles;
     PlaneWindow win;
@@ -213,7 +216,7 @@ __device__ __forceinline__ void forwardBinMajorBody(const ForwardJob& job, int w
     const PlaneWindow win = planeWindow<PAIRS == 2>(ps, min(row, ps.R - 1), min(k, ps.K - 1));
     const bool present = row < ps.R && k < ps.K && win.valid;
     // 4-byte loads (odd widths or strides): the lane takes columns l and l + N/2, so that
-    // a load instruction reads neighbouring floats (configs[3]: input gradient 108.0 ->
+    // a load instruction reads neighbouring floats (the 27 x 27 layer: input gradient 108.0 ->
     // 101.6 us, weight gradient 108.0 -> 104.1 us; forward pass unchanged).  PAIRS = 2
     // (described sets: the windows are only known on the device) decides per plane
     // between 8-byte and 4-byte loads of columns 2l and 2l + 1.
@@ -366,17 +369,17 @@ __global__ __launch_bounds__(kTF) void inverseBinMajor(const float2* Cs, int I, 
     planeSync();
     c32 z0[H], z1[H];
     // PAIRS = 0, no 8-byte stores: a lane takes columns l and l + N/2, so that each store
-    // instruction writes a contiguous run per plane (configs[3]: 102.4 -> 101.5 us).
+    // instruction writes a contiguous run per plane (the 27 x 27 layer: 102.4 -> 101.5 us).
     // PAIRS = 2 (described sets): columns 2l and 2l + 1, 8-byte or 4-byte stores decided
     // per plane.
     columnPassInverse<N, PAIRS == 0>(plane, l, z0, z1);
     // (Parking the cropped planes in LDS and writing them out as 16-byte runs - one
     // contiguous stream for dense outputs, row quads for windows of a tiled image - was
-    // measured and is slower, 35.9 -> 36.6 us at configs[3] and 112 -> 131 us at
-    // the kernel waits on its own chain of phases, not on store requests.
+    // measured and is slower, 35.9 -> 36.6 us at the 27 x 27 layer and 112 -> 131 us at
+    // the 256 x 256 layer: the kernel waits on its own chain of phases, not on store requests.
     // The dense case again with each wave parking its own four planes - one aligned run
     // of memory, no workgroup barrier - and nontemporal 16-byte stores: 106.8-108.3 us
-    // per forward pass at configs[3] against 106.7-108.2, no change.)
+    // per forward pass at the 27 x 27 layer against 106.7-108.2, no change.)
     if (j < out.K) {  // out.K: number of valid output planes along j
       if (win.valid) {
         if constexpr (PAIRS == 2) {
@@ -874,7 +877,7 @@ __global__ __launch_bounds__(kT, 3) void binGemmRegsWide(GemmArgs g) {
   };
   const int first = blockIdx.y * g.slicesPerSplit;
   // two register sets instead of three: 153 registers, three waves per SIMD instead of two
-  // (configs[4]: 294.6 -> 290.1 us per forward pass)
+  // (the 256 x 256 layer: 294.6 -> 290.1 us per forward pass)
   ringOfTwo<GemmSliceWide>(first, 1, min(first + g.slicesPerSplit, g.Kp / GK2) - first, fetch,
                            multiply);
 
@@ -904,7 +907,7 @@ inline int roundUp(int a, int b) { return (a + b - 1) / b * b; }
 // always put the window index on j: the inverse kernel transforms 16 consecutive j per
 // workgroup, and 16 neighbouring windows of one output plane store whole stretches of
 // image rows where 16 output planes of one window store 24-float pieces 248 floats apart
-// (configs[4]: 337 -> 308 us per forward pass).  Otherwise: the assignment with fewer
+// (the 256 x 256 layer: 337 -> 308 us per forward pass).  Otherwise: the assignment with fewer
 // padded tile elements.
 inline bool swapRoles(int I, int J, bool outTiled) {
   if (outTiled) return true;
@@ -923,10 +926,10 @@ inline bool swapRoles(int I, int J, bool outTiled) {
 // idle and the reduction is long - 8- and 16-point transforms have 32 and 128 bins, and a
 // weight gradient reduces over every image and window - up to 16 of them, enough for
 // about two waves per SIMD in the register kernels and one round of workgroups in the LDS
-// kernels, each keeping at least `minSlices` k-slices (weight gradient of configs[3] on
+// kernels, each keeping at least `minSlices` k-slices (weight gradient of the 27 x 27 layer on
 // 8-point windows: 423 -> 238 us; 64 x 64 x 512 per bin on 16-point windows: 73 -> 63 us;
 // ranges of 8 slices cost 6 % where 16 slices are all there are).  32-point transforms on short sides
-// have 512 bins and never split (measured on the weight gradient of configs[4], 32 x 32
+// have 512 bins and never split (measured on the weight gradient of the 256 x 256 layer, 32 x 32
 // per bin over 1936 windows, 2048 waves: two ranges 337 -> 345 us, four 362: that
 // contraction is not short of waves).
 struct GemmPlan {
@@ -1102,8 +1105,8 @@ int runPipeline(PlaneSet x, PlaneSet y, PlaneSet out, bool conjY, float scale, b
     case GemmPlan::Direct128: binGemmDirect<GI><<<ggrid, dim3(kT), 0, s>>>(g); break;
   }
   // Two runs per workgroup pay when the paired launch still fills the chip for three
-  // rounds or more (two workgroups are resident per CU): 112 -> 108 us at configs[4],
-  // 1936 paired workgroups; at configs[3] pairing would leave 768 workgroups, one and a
+  // rounds or more (two workgroups are resident per CU): 112 -> 108 us at the 256 x 256 layer,
+  // 1936 paired workgroups; at the 27 x 27 layer pairing would leave 768 workgroups, one and a
   // half rounds, and costs 35.5 -> 37.1 us.
   const bool pairedRuns = Jp / SL >= 2 && (long)ceilDiv(Jp / SL, 2) * I >= 3L * 2 * computeUnits();
   const int runGroups = pairedRuns ? ceilDiv(Jp / SL, 2) : Jp / SL;

@@ -13,7 +13,7 @@
 //   updateGradInput  cout       outs[t](n_a, f)   weight(f, c_w)    a * w       -> ins[t](n_a, c_w)  / N^2
 //   accGradParams    tile, n    ins[t](n, c_a)    outs[t](n, f_w)   a * conj(w) -> weight(f_w, c_a) * scale / N^2
 //
-// updateOutput and updateGradInput run one workgroup per (tile, A group, W group).
+// updateOutput and updateGradInput run one workgroup per (A group, W group).
 // accGradParameters reduces over all tiles and images; its reduction is also cut
 // into ranges that separate workgroups accumulate and add atomically into the
 // zeroed weight gradient, so that the chip is filled.
@@ -24,8 +24,8 @@
 // takes two reduction steps per iteration: its 1024/N plane slots hold the BN + FO
 // forward transforms of both steps, so every lane transforms in every iteration
 // and 2 (BN + FO) transforms feed 2 BN FO products (one transform per 4, 8, 16
-// products).  A planes are the (image, tile) pairs of the call, whatever the batch: a
-// workgroup's A planes come from several tiles when the batch is small.
+// products).  A planes of passes 0 and 1 are the (image, tile) pairs of the call, whatever
+// the batch: a workgroup's A planes come from several tiles when the batch is small.
 //
 // The products run on the matrix cores: v_mfma_f32_4x4x1 multiplies sixteen independent
 // 4 x 4 blocks, one block per frequency bin, so a wave accumulates 4 A planes x 4 W planes

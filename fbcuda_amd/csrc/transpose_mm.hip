@@ -835,7 +835,7 @@ int launchTransposeMM(const float* A, long a0, long a1, const float* B, long b0,
     // Equal work items are dealt to the CUs in whole numbers: the launch lasts as
     // long as the fullest CU.  32-row tiles re-read B twice as often and pay more per
     // matrix instruction, so they are taken only where they even the load out
-    // (configs[3]: 816 items of 64 rows are 3.19 per CU, four on the fullest - 72 us;
+    // (128 x 64 x 192 over 544 bins: 816 items of 64 rows are 3.19 per CU, four on the fullest - 72 us;
     // 1632 of 32 rows are 6.4, seven on the fullest - 68 us; at 2, 4 or 8 items of 64
     // rows per CU the larger tile wins by 3-9 %).
     const int cus = computeUnits();

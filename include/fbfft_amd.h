@@ -158,8 +158,8 @@ int fbfft_iterated_conv(int fftSize, const fbfft_tile* ins, const fbfft_tile* ou
  * reference's schedule - one workgroup per group of weight planes walks the whole
  * (tile, image) reduction in a fixed order (fbfft/FFTIteratedConvolution.cuh:
  * 600-613), no atomic adds - so the result is bit-for-bit reproducible from run to
- * run, at the price of leaving most of the chip idle (configs[4]: 10.5 ms instead of
- * 0.63 ms).  fbfft_conv_accgrad on the whole image is both reproducible and fast; it
+ * run, at the price of leaving most of the chip idle (16 x 32 x 256 x 256 images, 32
+ * filters of 9 x 9: 6.2 ms instead of 0.5 ms).  fbfft_conv_accgrad on the whole image is both reproducible and fast; it
  * needs a workspace.  The other passes are reproducible either way.  Unknown flag
  * bits return 0. */
 #define FBFFT_DETERMINISTIC 1u
@@ -174,8 +174,8 @@ int fbfft_iterated_conv_ex(int fftSize, const fbfft_tile* ins, const fbfft_tile*
  * outs[t] (*) weight, weight = scale * sum_(t, n) ins[t] (*) outs[t]), computed by the
  * three kernels of the convolution layer entry points instead of the fused kernel: each
  * filter plane is transformed once per call rather than once per tile and image group,
- * and the per-frequency products run on the matrix cores (configs[4]: 0.29 ms against
- * 0.62 ms).  The weight gradient is reproducible bit for bit from run to run.
+ * and the per-frequency products run on tiles of many planes (16 x 32 x 256 x 256 images,
+ * 32 filters of 9 x 9: 0.28 ms against 0.5 ms).  The weight gradient is reproducible bit for bit from run to run.
  * workspace: device memory of fbfft_iterated_conv_workspace(fftSize, pass, batchSize,
  * numTiles, cin, cout) bytes, 256-byte aligned; contents need not survive.  Returns as
  * fbfft_iterated_conv: 1 launched, 0 nothing matched (pass, fftSize in {8, 16, 32},
@@ -231,9 +231,10 @@ size_t fbfft_make_tiles_for_pass(int pass, const fbfft_tensor* input, const fbff
  * Sizes up to 32 hand bin-major spectra between three fused kernels, on smaller windows
  * than the named size where these need at most 60 % of its workspace; 64 and 128 need H, W <=
  * fftSize and run the same three kernels on 8-, 16- or 32-point windows of the image where
- * their spectra are no larger than those of the named size, and fbfft2D -> transposeMM ->
- * fbifft2D on plane-major spectra in the workspace otherwise (filters that fill most of a
- * 32-point window or exceed it).  With fftSize <= 32 the image may be larger than the
+ * their spectra are no larger than those of the named size and the pass is expected to take
+ * no longer, and fbfft2D -> transposeMM -> fbifft2D on plane-major spectra in the workspace
+ * otherwise (filters that fill most of a 32-point window or exceed it, long weight-gradient
+ * reductions).  With fftSize <= 32 the image may be larger than the
  * transform: it is then cut into overlapping fftSize x fftSize windows whose
  * origins advance by fftSize-kH+1 rows / fftSize-kW+1 columns (the tiling of
  * FFTIteratedConvolution, fbfft/FFTIteratedConvolution.cuh:71-88), and the
