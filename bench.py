@@ -354,7 +354,7 @@ def conv_extras(F, synth, torch, dev, extra):
     _, t = timed(mmp, 200, 200, torch)
     extra["transposeMM_packed_configs3_us"] = round(t * 1e6, 1)
     del Ap, Bp, Cp, x, w, out, ws
-    # a layer named 64 points, which run in windows of 32 or fewer: 32x32x60x60 * 64x32x5x5
+    # a layer named 64 points, which runs in 32-point windows: 32x32x60x60 * 64x32x5x5
     x6 = synth.normal((32, 32, 60, 60), seed=50, device=dev)
     w6 = synth.normal((64, 32, 5, 5), seed=51, std=0.02, device=dev)
     o6 = torch.empty((32, 64, 56, 56), device=dev)
@@ -367,8 +367,8 @@ def conv_extras(F, synth, torch, dev, extra):
             raise RuntimeError("fbfft_conv_fprop (64) failed")
     _, t = timed(conv64, 200, 200, torch)
     flop64 = 2.0 * 32 * 64 * 56 * 56 * 32 * 25
-    extra["fft_conv_64pt_32x32x60x60_k5_f64_ms_per_iter"] = round(t * 1e3, 4)
-    extra["fft_conv_64pt_direct_equiv_TFLOPs"] = round(flop64 / t / 1e12, 1)
+    extra["fft_conv_named_64_32x32x60x60_k5_ms_per_iter"] = round(t * 1e3, 4)
+    extra["fft_conv_named_64_direct_equiv_TFLOPs"] = round(flop64 / t / 1e12, 1)
     del x6, w6, o6, ws6
     # configs[4]
     x4 = synth.uniform((16, 32, 256, 256), seed=40, device=dev)
