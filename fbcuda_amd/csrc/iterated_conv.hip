@@ -624,6 +624,9 @@ int launchPass(int pass, ConvArgs a, bool deterministic, hipStream_t s) {
   if (pass != FBFFT_ACC_GRAD_PARAMETERS && steps <= 18) {
     const long groups = std::max(1L, computeUnits() / wGroups);
     a.aPlanes = (int)std::min<long>(C::BN, (rows + groups - 1) / groups);
+    // ... where that leaves out a round of inverse transforms (5 of 8 planes and both rounds,
+    // 79 x 8 x 111 x 108, input gradient of 8 filters of 5 x 5: 44.6 / 48.7)
+    if (ceilDiv(a.aPlanes, C::RA) * C::RA == C::BN) a.aPlanes = C::BN;
   }
   const long aGroups = pass == FBFFT_ACC_GRAD_PARAMETERS ? ceilDiv(Cin, C::BN) : (rows + a.aPlanes - 1) / a.aPlanes;
   if (pass == FBFFT_ACC_GRAD_PARAMETERS) {

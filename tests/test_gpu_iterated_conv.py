@@ -259,7 +259,7 @@ def test_layer_weight_gradient_is_reproducible():
 # more than 18 steps, or every CU with a workgroup: all slots)
 @pytest.mark.parametrize("N,k,Nb,Cin,Cout", [(8, 3, 3, 5, 9), (16, 5, 1, 3, 17), (32, 5, 2, 9, 7),
                                              (32, 19, 1, 2, 3), (32, 5, 2, 19, 18), (16, 5, 9, 18, 19),
-                                             (8, 2, 77, 3, 2), (32, 3, 61, 2, 20)])
+                                             (8, 2, 77, 3, 2), (32, 3, 61, 2, 20), (32, 3, 61, 2, 9)])
 def test_plane_groups_span_tiles_and_tensors(oracle, N, k, Nb, Cin, Cout):
     """A workgroup's planes come from several tiles, here of two tensors with different row
     strides and alignments: one dense with even rows, one a view with odd rows and offsets."""
