@@ -145,9 +145,11 @@ int fbfft_transpose_mm_packed(const fbfft_tensor* A, const fbfft_tensor* B, cons
 /* detail::FFTIteratedConvolution<FFTSize> (fbfft/FFTIteratedConvolution.cuh:624-755).
  * ins / outs are DEVICE pointers to numTiles descriptors each.  weight is
  * [Cout][Cin][kH][kW].  Returns 1 if a kernel was launched, 0 if the pass code or
- * FFT size matched nothing (the reference's bool) or the filter is larger than
- * the transform (kH or kW > fftSize), and a negative fbfft_error
- * (-FBFFT_HIP_ERROR ...) on launch failure.  FBFFT_ACC_GRAD_PARAMETERS overwrites
+ * FFT size matched nothing (the reference's bool), the filter is larger than
+ * the transform (kH or kW > fftSize) or the counts are beyond what the kernels index
+ * (FBFFT_ACC_GRAD_PARAMETERS: numTiles * batchSize above 0x7fff0000; other passes:
+ * numTiles above 2^30), and a negative fbfft_error (-FBFFT_HIP_ERROR ...) on launch
+ * failure.  FBFFT_ACC_GRAD_PARAMETERS overwrites
  * weight with scale * gradient; partial sums of several workgroups meet in atomic
  * adds, so its last bits can differ from run to run. */
 int fbfft_iterated_conv(int fftSize, const fbfft_tile* ins, const fbfft_tile* outs,
