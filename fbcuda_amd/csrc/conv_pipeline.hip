@@ -19,6 +19,8 @@
 //      counters show A + B fetched
 //      from HBM exactly once (the tiles of a bin share an L2: workgroup ids are
 //      remapped per XCD) and C written once with coalesced stores.
+//      binGemmSplit: the same product on the bf16 matrix instructions, fp32 operands
+//      split into three bf16 values each.
 //      binGemmRegsWide / binGemmRegsSplitK: the same product without LDS for
 //      products with a side of up to 32 (planGemm picks kernel, tiles and the
 //      ranges a long reduction is cut into).
@@ -900,6 +902,186 @@ __global__ __launch_bounds__(kT, 3) void binGemmRegsWide(GemmArgs g) {
   }
 }
 
+// The same product on the bf16 matrix instructions, for products that outweigh their operands
+// (planGemm).  fp32 matrix instructions are what bounds
+// binGemmDirect there (155 TFLOP/s); the bf16 ones run at 1600 to 1750 on random operands (the power
+// limit; 2400 on zeros).  An fp32 value is the sum of three bf16 values without remainder,
+// a = a0 + a1 + a2: the upper half of its bits, the remainder rounded to 8 bits, and what is
+// left, which has at most 8.  Of the nine products of pieces the six largest are formed; the
+// three dropped ones are below 2^-23 |a b| each and of either sign, products of pieces
+// are exact in fp32, and a sum is rounded once per 16 k and product of pieces where the
+// fp32 instructions round every 2 k.  Against 64 bits over random operands: K = 64 1.1e-7, K =
+// 1024 4.9e-7 (relative 2-norm); fp32 instructions 1.4e-7 and 5.8e-7.
+//
+// One workgroup = one bin x a (64 x 64) tile, 4 waves of 32 x 32.  A slice of 16 k passes
+// through registers, where each value is split once, into LDS as bf16, [piece][re, im][k
+// half][row] of 8 k: what a lane of v_mfma_f32_32x32x16_bf16 supplies is one 16-byte read.
+// The next slice's loads fly under this one's products.  114 registers and 24.6 KB of LDS leave
+// room for four workgroups per CU.  Four real products per complex one: three (as above) would need a
+// third split operand on each side, and LDS reads then take longer than the products saved.
+// 128 x 64, 64 x 128 and 128 x 128 tiles and a second LDS buffer measured 1 to 40 % slower
+// (fewer workgroups per CU); each wave splitting what it reads, from the stages that
+// global_load_lds fills, 25 % slower.
+// us per launch, binGemmDirect / this: 128 x 192 x 64 over 512 bins 53.6 / 47.2; 264 x 307 x 273
+// over 128 193 / 161; without its matrix instructions the latter takes 104, without its
+// stores 156, without the splits 146.
+typedef __bf16 Bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned Quad __attribute__((ext_vector_type(4)));
+typedef unsigned Duo __attribute__((ext_vector_type(2)));
+constexpr int GK3 = 16;
+
+// the bf16 pieces of two floats, two to a word.  The first piece is cut off, not rounded: the
+// largest finite floats would round to infinity.
+__device__ __forceinline__ void split2(float x, float y, unsigned& p0, unsigned& p1, unsigned& p2) {
+  typedef float Float2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 Bf16x2 __attribute__((ext_vector_type(2)));
+  auto bits = [](float f) { return __builtin_bit_cast(unsigned, f); };
+  auto real = [](unsigned u) { return __builtin_bit_cast(float, u); };
+  auto upper = [&](float a, float b) { return __builtin_amdgcn_perm(bits(b), bits(a), 0x07060302u); };
+  p0 = upper(x, y);
+  const float rx = x - real(bits(x) & 0xffff0000u), ry = y - real(bits(y) & 0xffff0000u);
+  p1 = __builtin_bit_cast(unsigned, __builtin_convertvector(Float2{rx, ry}, Bf16x2));
+  p2 = upper(rx - real(p1 << 16), ry - real(p1 & 0xffff0000u));
+}
+
+struct SplitOperand {
+  Quad v[3][2][2][64];
+};
+
+// four k of one row, quarter q of the slice
+__device__ __forceinline__ void parkSplit(SplitOperand& s, int row, int q, const PlainPair (&v)[4]) {
+  Duo p[3][2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      unsigned p0, p1, p2;
+      split2(v[2 * e][c], v[2 * e + 1][c], p0, p1, p2);
+      p[0][c][e] = p0;
+      p[1][c][e] = p1;
+      p[2][c][e] = p2;
+    }
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) reinterpret_cast<Duo*>(&s.v[i][c][q / 2][row])[q % 2] = p[i][c];
+}
+
+// Makes LDS writes of the whole workgroup visible to it; global loads stay in flight.
+__device__ __forceinline__ void ldsBarrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+__global__ __launch_bounds__(kT, 4) void binGemmSplit(GemmArgs g) {
+  __shared__ __align__(16) SplitOperand opA, opB;
+  const int t = threadIdx.x;
+  const int lane = t % 64;
+  const int w = __builtin_amdgcn_readfirstlane(t / 64);
+  const int r = lane % 32, h = lane / 32;
+  const int total = g.bins * g.IT * g.JT;
+  const int per = (total + 7) / 8;
+  const int logical = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (logical >= total) return;
+  const int bin = logical / (g.IT * g.JT);
+  const int rem = logical % (g.IT * g.JT);
+  const int i0 = (rem / g.JT) * 64, j0 = (rem % g.JT) * 64;
+  const int rb = w % 2, cb = w / 2;  // this wave's 32-row and 32-column block
+  const bool pairs = bin == 0 || 2 * bin == g.N;  // bins of real pairs: (ar br, ai bi)
+
+  // this workgroup's range of the reduction: rows k-rows, a multiple of 8
+  const int first = blockIdx.y * g.slicesPerSplit * GK2;
+  const int rows = min(g.slicesPerSplit * GK2, g.Kp - first);
+  const int slices = (rows + GK3 - 1) / GK3;
+  // lane l of wave w loads k-rows 4w .. 4w+3 of row l of each operand, clamped into the padded
+  // arrays (what is beyond them feeds accumulators that are never stored)
+  const unsigned laneA = (unsigned)min(i0 + lane, g.Ip - 1) * (unsigned)sizeof(float2);
+  const unsigned laneB = (unsigned)min(j0 + lane, g.Jp - 1) * (unsigned)sizeof(float2);
+  const long rowA = (long)g.Ip * sizeof(float2), rowB = (long)g.Jp * sizeof(float2);
+  const char* const baseA = (const char*)(g.A + ((long)bin * g.Kp + first) * g.Ip);
+  const char* const baseB = (const char*)(g.B + ((long)bin * g.Kp + first) * g.Jp);
+  PlainPair va[4], vb[4];
+  auto request = [&](int sl) __attribute__((always_inline)) {
+    const int k = min(sl * GK3 + 4 * w, rows - 4);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      va[u] = *(const GlobalPair*)(scalarBase(baseA + (k + u) * rowA) + laneOffset(laneA));
+      vb[u] = *(const GlobalPair*)(scalarBase(baseB + (k + u) * rowB) + laneOffset(laneB));
+    }
+  };
+
+  floatx16 re, im;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) re[v] = im[v] = 0.f;
+
+  auto loop = [&](auto realPairs) __attribute__((always_inline)) {
+    constexpr bool PAIRS = decltype(realPairs)::value;
+    for (int sl = 0; sl < slices; ++sl) {
+      if (sl * GK3 + 4 * w >= rows) {  // the last slice may be half a slice
+#pragma unroll
+        for (int u = 0; u < 4; ++u) va[u] = vb[u] = PlainPair{0.f, 0.f};
+      }
+      parkSplit(opA, lane, w, va);
+      parkSplit(opB, lane, w, vb);
+      request(min(sl + 1, slices - 1));
+      ldsBarrier();
+      // products of pieces, the smallest first
+      constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+      const Quad sign = Quad{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
+      Quad a[3][2], b[3][2];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          b[i][c] = opB.v[i][c][h][32 * cb + r];
+          a[i][c] = opA.v[i][c][h][32 * rb + r];
+        }
+      auto multiply = [&](Quad x, Quad y, floatx16& c) __attribute__((always_inline)) {
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(Bf16x8, x),
+                                                    __builtin_bit_cast(Bf16x8, y), c, 0, 0, 0);
+      };
+#pragma unroll
+      for (int p = 0; p < 6; ++p) {
+        const Quad ar = a[PA[p]][0], ai = a[PA[p]][1], br = b[PB[p]][0], bi = b[PB[p]][1];
+        multiply(ar, br, re);
+        if constexpr (PAIRS) {
+          multiply(ai, bi, im);
+        } else {
+          multiply(ai, br, im);
+          multiply(ai, bi, re);
+          multiply(ar, bi ^ sign, im);
+        }
+      }
+      ldsBarrier();
+    }
+  };
+  request(0);
+  if (pairs)
+    loop(std::true_type{});
+  else
+    loop(std::false_type{});
+
+  float2* Cb = g.C + blockIdx.y * g.splitStride + (long)bin * g.I * g.Jp;
+  if (i0 + 32 * rb + 32 <= g.I && j0 + 32 * cb + 32 <= g.Jp) {
+    const unsigned laneC = (unsigned)(4 * h * g.Jp + r) * (unsigned)sizeof(float2);
+    char* const waveC = (char*)(Cb + (long)(i0 + 32 * rb) * g.Jp + j0 + 32 * cb);
+    const long rowC = (long)g.Jp * sizeof(float2);
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      *(GlobalPair*)(scalarBase(waveC + (8 * (v / 4) + v % 4) * rowC) + laneOffset(laneC)) =
+          PlainPair{re[v], im[v]};
+    return;
+  }
+  const int j = j0 + 32 * cb + r;
+  if (j >= g.Jp) return;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int i = i0 + 32 * rb + 8 * (v / 4) + 4 * h + v % 4;
+    if (i < g.I) Cb[(long)i * g.Jp + j] = float2{re[v], im[v]};
+  }
+}
+
 inline int roundUp(int a, int b) { return (a + b - 1) / b * b; }
 
 // Which operand takes the 128-wide side of the GEMM tile (and with it the role of i, the
@@ -933,7 +1115,7 @@ inline bool swapRoles(int I, int J, bool outTiled) {
 // per bin over 1936 windows, 2048 waves: two ranges 337 -> 345 us, four 362: that
 // contraction is not short of waves).
 struct GemmPlan {
-  enum Kind { RegsSplitK, RegsWide, Direct64, Direct128 } kind;
+  enum Kind { RegsSplitK, RegsWide, Direct64, Direct128, Split } kind;
   int IT, JT;
   int splits, slicesPerSplit;
   long waves;  // of one range
@@ -973,6 +1155,21 @@ inline GemmPlan planGemm(int bins, int I, int Jp, int Kp, int maxSplits) {
   p.slicesPerSplit = ceilDiv(slices, std::min(want, most));
   p.splits = ceilDiv(slices, p.slicesPerSplit);  // no range is empty
   p.waves = waves;
+  // binGemmSplit where the products outweigh the operands by enough: each spectrum value enters
+  // I J K / (I J + I K + J K) complex products.  Whole layers on a loaded chip, three passes
+  // back to back, binGemmDirect / this by that quotient: 93 (66 x 273 x 25 x 26, 307 of 2 x 2)
+  // 761 / 708 us; 43 (128 x 128 x 28 x 28, 128 of 5 x 5) 367 / 354; 38 (180 x 65 x 12 x 20, 195 of
+  // 10 x 10) 394 / 369; below, the launch waits for memory, splitting has few products to
+  // pay for it and the bf16 instructions' power slows the transforms around them: 37 (128 x 64
+  // x 28 x 28, 256 of 5 x 5) 416 / 423, 35 (the 27 x 27 layer) 324 / 332, 28 (64 x 64 x 30 x 30, 64 of 4
+  // x 4) 151 / 160.  And not with fewer workgroups than two per CU (2 x 178 x 38 x 46, 33 of 5
+  // x 5, 128 workgroups: 13.9 / 16.5) or ranges of fewer than 48 k.
+  if ((p.kind == GemmPlan::Direct64 || p.kind == GemmPlan::Direct128) && p.slicesPerSplit >= 6 &&
+      1.0 / I + 1.0 / Jp + 1.0 / Kp <= 1.0 / 38 &&
+      (long)bins * ceilDiv(I, 64) * p.JT * p.splits >= 2 * 256) {
+    p.kind = GemmPlan::Split;
+    p.IT = ceilDiv(I, 64);
+  }
   return p;
 }
 
@@ -1103,6 +1300,7 @@ int runPipeline(PlaneSet x, PlaneSet y, PlaneSet out, bool conjY, float scale, b
     case GemmPlan::RegsWide: binGemmRegsWide<<<ggrid, dim3(kT), 0, s>>>(g); break;
     case GemmPlan::Direct64: binGemmDirect<64><<<ggrid, dim3(kT), 0, s>>>(g); break;
     case GemmPlan::Direct128: binGemmDirect<GI><<<ggrid, dim3(kT), 0, s>>>(g); break;
+    case GemmPlan::Split: binGemmSplit<<<ggrid, dim3(kT), 0, s>>>(g); break;
   }
   // Two runs per workgroup pay when the paired launch still fills the chip for three
   // rounds or more (two workgroups are resident per CU): 112 -> 108 us at the 256 x 256 layer,
