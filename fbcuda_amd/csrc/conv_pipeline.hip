@@ -716,7 +716,8 @@ __device__ __forceinline__ void ringOfTwo(int first, int step, int n, Fetch fetc
 }
 
 // Both sides short (up to 32 rows and 32 columns per bin, any K - the weight gradient
-// of a layer with few planes reduces over every image and window): one workgroup per
+// of a layer with few planes reduces over every image and window), and products too small to
+// fill the chip with larger tiles (planGemm): one workgroup per 32 x 32 tile of a
 // bin and range of the reduction; its four waves take every fourth k-slice each and
 // wave 0 adds the four 32 x 32 partial tiles in wave order (through LDS) before it
 // stores, so the result does not depend on timing.
@@ -730,17 +731,21 @@ __global__ __launch_bounds__(kT, 4) void binGemmRegsSplitK(GemmArgs g) {
   // (the wave's number in a scalar register: its slices and their addresses are scalar)
   const int lane = t % 64, w = __builtin_amdgcn_readfirstlane(t / 64);
   const int r = lane % 32, h = lane / 32;
-  const int per = (g.bins + 7) / 8;
-  const int bin = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  if (bin >= g.bins) return;
+  const int total = g.bins * g.IT * g.JT;
+  const int per = (total + 7) / 8;
+  const int logical = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (logical >= total) return;
+  const int bin = logical / (g.IT * g.JT);
+  const int rem = logical % (g.IT * g.JT);
+  const int i0 = rem / g.JT * 32, j0 = rem % g.JT * 32;
   const bool pairs = bin == 0 || 2 * bin == g.N;  // bins of real pairs: (ar br, ai bi)
   const float cross = pairs ? 0.f : 1.f;
 
   // operand columns beyond the padded arrays are clamped (they feed accumulators that
   // are never stored).  An address is a scalar base (bin, k-rows) plus the lane's fixed
   // 32-bit offset: no vector arithmetic per load.
-  const unsigned laneA = (unsigned)(h * g.Ip + min(r, g.Ip - 1)) * (unsigned)sizeof(float2);
-  const unsigned laneB = (unsigned)(h * g.Jp + min(r, g.Jp - 1)) * (unsigned)sizeof(float2);
+  const unsigned laneA = (unsigned)(h * g.Ip + min(i0 + r, g.Ip - 1)) * (unsigned)sizeof(float2);
+  const unsigned laneB = (unsigned)(h * g.Jp + min(j0 + r, g.Jp - 1)) * (unsigned)sizeof(float2);
   const char* const binA = (const char*)(g.A + (long)bin * g.Kp * g.Ip);
   const char* const binB = (const char*)(g.B + (long)bin * g.Kp * g.Jp);
   const long sa = 2L * g.Ip * sizeof(float2), sb = 2L * g.Jp * sizeof(float2);  // two k-rows
@@ -797,12 +802,13 @@ __global__ __launch_bounds__(kT, 4) void binGemmRegsSplitK(GemmArgs g) {
       k3[v] += red[u][32 + v][lane];
     }
   float2* Cb = g.C + blockIdx.y * g.splitStride + (long)bin * g.I * g.Jp;
-  if (r < g.Jp) {
+  const int j = j0 + r;
+  if (j < g.Jp) {
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const int i = 8 * (v / 4) + 4 * h + v % 4;
+      const int i = i0 + 8 * (v / 4) + 4 * h + v % 4;
       if (i < g.I)
-        Cb[(long)i * g.Jp + r] =
+        Cb[(long)i * g.Jp + j] =
             pairs ? float2{k1[v], -k3[v]} : float2{k1[v] - k3[v], k1[v] + k2[v]};
     }
   }
@@ -1155,6 +1161,19 @@ inline GemmPlan planGemm(int bins, int I, int Jp, int Kp, int maxSplits) {
   p.slicesPerSplit = ceilDiv(slices, std::min(want, most));
   p.splits = ceilDiv(slices, p.slicesPerSplit);  // no range is empty
   p.waves = waves;
+  // A small product on few workgroups is one chain of slices each, on an idle chip:
+  // binGemmRegsSplitK's 32 x 32 tiles are two to eight times as many workgroups, and each cuts
+  // its chain in four.  us, binGemmRegsWide / 32 x 32 tiles: 192 workgroups 8.4 / 4.8, 384 7.9
+  // / 5.7, 768 8.8 / 6.8 (4.7 slices), but 1152 4.8 / 6.9 (1 slice; 6 slices, 1536: 13.2 / 11.1);
+  // binGemmDirect<64> / 32 x 32 tiles: 384 (one image, 64 x 27 x 27, 192 of 5 x 5, 8 slices)
+  // 7.9 / 7.6, 192 (10) 7.9 / 6.1, 128 (24) 14.6 / 8.0, 768 (21) 13.6 / 12.2, but 512 (5) 6.6 / 7.1.
+  const long tiles = (long)bins * ceilDiv(I, 32) * ceilDiv(Jp, 32) * p.splits;
+  if ((p.kind == GemmPlan::RegsWide && (tiles <= 768 || (p.slicesPerSplit >= 6 && tiles <= 1536))) ||
+      (p.kind == GemmPlan::Direct64 && p.slicesPerSplit >= 8 && tiles <= 768)) {
+    p.kind = GemmPlan::RegsSplitK;
+    p.IT = ceilDiv(I, 32);
+    p.JT = ceilDiv(Jp, 32);
+  }
   // binGemmSplit where the products outweigh the operands by enough: each spectrum value enters
   // I J K / (I J + I K + J K) complex products.  Whole layers on a loaded chip, three passes
   // back to back, binGemmDirect / this by that quotient: 93 (66 x 273 x 25 x 26, 307 of 2 x 2)
@@ -1194,7 +1213,7 @@ WindowsCost windowsCost(int I, int J, int K, bool outTiled, int maxSplits) {
   WindowsCost c;
   c.bytes = sizeof(float2) * bins * ((size_t)Kp * Ip + (size_t)Kp * Jp + (size_t)plan.splits * I * Jp);
   const double products = (double)bins * roundUp(I, I <= 32 ? 32 : 64) * roundUp(Jp, 64) * Kp;
-  const bool wide = plan.kind == GemmPlan::RegsWide;
+  const bool wide = I <= 32 && Jp > 32;  // what binGemmRegsWide runs, its small products apart
   const long waves = plan.waves * plan.splits;
   const double idle = waves < 1024 ? 1024.0 / waves : wide ? (waves + 2047) / 2048 * 2048.0 / waves : 1.0;
   c.us = 15 + 0.14e-6 * 2 * c.bytes + (wide ? 0.055e-6 : 0.04e-6) * products * idle;

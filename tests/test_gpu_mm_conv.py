@@ -491,3 +491,17 @@ def test_conv_fprop_batch_beyond_a_16_bit_grid_index(oracle):
     want = oracle.corr2d_valid_at(x.cpu().numpy(), w.cpu().numpy(), coords)
     oh = out.cpu().numpy()
     assert rel(oh[coords[:, 0], coords[:, 1], coords[:, 2], coords[:, 3]], want) < TOL_CONV
+
+
+# the contraction of small products, a 32 x 32 tile per workgroup: either side on the rows, ends of
+# the tiles, a long reduction on two rows of tiles (binGemmDirect's shape) and on one
+# (binGemmRegsWide's), with and without a reduction cut into ranges
+@pytest.mark.parametrize("N,H,k,Bn,Cin,Cout", [
+    (8, 8, 3, 33, 80, 34), (8, 7, 2, 65, 88, 48), (8, 8, 3, 5, 9, 40), (8, 8, 3, 32, 81, 33),
+    (16, 14, 5, 3, 200, 65), (16, 16, 7, 40, 12, 9), (8, 8, 4, 2, 300, 70)])
+def test_conv_fprop_small_products(oracle, N, H, k, Bn, Cin, Cout):
+    x = synth.normal((Bn, Cin, H, H), seed=30).numpy()
+    w = synth.normal((Cout, Cin, k, k), seed=31, std=0.02).numpy()
+    rc, got = conv(x, w, N)
+    assert rc == F.Success
+    assert rel(got, oracle.corr2d_valid(x, w)) < 1e-6
