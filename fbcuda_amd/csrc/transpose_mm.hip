@@ -16,7 +16,7 @@
 // so that stores cover whole runs.  Only this contraction uses MFMA; it is the one
 // dense product of the convolution path.
 //
-// Two kernels:
+// Three kernels:
 //  * the fast path (transposeMMDirectKernel, further down) for operands whose runs of
 //    bin pairs are 16-byte aligned: 64 x 32 tiles, four waves of one bin pair each,
 //    slices of k copied from HBM into LDS without passing through registers, two
@@ -25,7 +25,9 @@
 //    a workgroup of 8 waves owns a 64 x 64 tile, wave w owning bin w.  Per 4-deep
 //    slice of k it parks opA and opB in LDS split into real and imaginary planes
 //    [bin][k][row] (conjugation folded into the sign of the imaginary plane, edges
-//    zeroed), two buffers deep, while the slice after next is in flight in registers.
+//    zeroed), two buffers deep, while the slice after next is in flight in registers;
+//  * transposeMMLanesKernel for products too small to fill the matrix kernels' tiles
+//    (launchSmall).
 //
 // Packed spectra (fbfft_transpose_mm_packed): operands [..][..][N/2][N] whose row 0
 // holds P[x] = F0[x] + i FH[x], the spectra of the two real rows 0 and N/2 of an
@@ -38,6 +40,7 @@
 // P[N-x] when a slice is parked; the epilogue combines C0[x] and CH[x] into P[x] and
 // P[N-x].  x = 0 pairs with x = N/2: both hold two real values, which multiply
 // component by component (no cross terms).
+#include <algorithm>
 #include <utility>
 
 #include "common.h"
@@ -796,6 +799,142 @@ bool storesAsFloat4(const float* C, long c0, long c1) {
 }
 
 
+// Small products, where the matrix kernels' tiles are mostly empty or the few of them are each
+// one long chain of slices: a lane owns a bin and TI x TJ elements of C there, with ordinary
+// multiply-adds; a load brings 64 consecutive bins of one element.  The KW waves of a workgroup
+// take every KW-th k each, the next one's values in flight under this one's products, and add
+// up in LDS in wave order.  What bounds it is what one CU can ask for at a time, about 45 GB/s.
+// us, matrix kernel / this: 1 x 30 x 323 (N = 16) 77.5 / 34.4 with tiles of 1 x 8, 2 x 193 x 29
+// (32) 22 / 8.3, 15 x 18 x 318 82 / 29, 9 x 16 x 5 8.3 / 4.0.  (Sixteen waves: the same.)
+template <int TI, int TJ, int KW>
+__global__ __launch_bounds__(64 * KW) void transposeMMLanesKernel(MMArgs a, int iTiles, int jTiles, int total) {
+  constexpr int E = TI * TJ;
+  __shared__ float2 red[KW * E * 64];
+  const int lane = threadIdx.x % 64;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int logical = logicalWorkItem(total);
+  if (logical >= total) return;
+  const int rem = logical % (iTiles * jTiles);
+  const int i0 = rem / jTiles * TI, j0 = rem % jTiles * TJ;
+  const int x = logical / (iTiles * jTiles) * 64 + lane;
+  const unsigned bin = (unsigned)min(x, a.XY - 1) * (unsigned)sizeof(float2);
+
+  float2 acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = float2{0.f, 0.f};
+  struct Values {
+    float2 a[TI], b[TJ];
+  };
+  // (rows and columns beyond C take the last one's values; they are not stored)
+  auto fetch = [&](Values& v, int k) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+      v.a[i] = *reinterpret_cast<const float2*>(
+          reinterpret_cast<const char*>(a.A + min(i0 + i, a.I - 1) * a.aRow + k * a.aK) + bin);
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+      v.b[j] = *reinterpret_cast<const float2*>(
+          reinterpret_cast<const char*>(a.B + min(j0 + j, a.J - 1) * a.bCol + k * a.bK) + bin);
+  };
+  auto multiply = [&](const Values& v) __attribute__((always_inline)) {
+    float bi[TJ];
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) bi[j] = a.bSign * v.b[j].y;
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+      const float ar = v.a[i].x, ai = a.aSign * v.a[i].y;
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) {
+        acc[i][j].x = __builtin_fmaf(ar, v.b[j].x, __builtin_fmaf(-ai, bi[j], acc[i][j].x));
+        acc[i][j].y = __builtin_fmaf(ar, bi[j], __builtin_fmaf(ai, v.b[j].x, acc[i][j].y));
+      }
+    }
+  };
+  if (w < a.K) {
+    Values v0, v1;
+    fetch(v0, w);
+    for (int k = w; k < a.K; k += 2 * KW) {
+      if (k + KW < a.K) fetch(v1, k + KW);
+      multiply(v0);
+      if (k + KW >= a.K) break;
+      if (k + 2 * KW < a.K) fetch(v0, k + 2 * KW);
+      multiply(v1);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) red[(w * E + i * TJ + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < (E + KW - 1) / KW; ++u) {
+    const int e = w + u * KW;
+    if (e >= E) break;
+    float2 v = red[e * 64 + lane];
+#pragma unroll
+    for (int k = 1; k < KW; ++k) {
+      const float2 o = red[(k * E + e) * 64 + lane];
+      v.x += o.x;
+      v.y += o.y;
+    }
+    const int i = i0 + e / TJ, j = j0 + e % TJ;
+    if (i >= a.I || j >= a.J || x >= a.XY) continue;
+    float2* dst = reinterpret_cast<float2*>(a.C + (long)i * a.cRow + (long)j * a.cCol + 2L * x);
+    if (a.accumulate) {
+      v.x += dst->x;
+      v.y += dst->y;
+    }
+    *dst = float2{v.x * a.invNorm, v.y * a.invNorm};
+  }
+}
+
+// workgroups of transposeMMLanesKernel
+inline double laneItems(const MMArgs& m, int ti, int tj) {
+  return (double)ceilDiv(m.XY, 64) * ceilDiv(m.I, ti) * ceilDiv(m.J, tj);
+}
+
+template <int TI, int TJ, int KW>
+int launchLanes(const MMArgs& m, hipStream_t s) {
+  const int total = (int)laneItems(m, TI, TJ);
+  transposeMMLanesKernel<TI, TJ, KW><<<dim3((total + 7) / 8 * 8), dim3(64 * KW), 0, s>>>(
+      m, ceilDiv(m.I, TI), ceilDiv(m.J, TJ), total);
+  return launchStatus();
+}
+
+// Small products to transposeMMLanesKernel; -1: not one.  Both times are estimated, in us, from
+// the chain of slices of the fullest CU: 45 GB/s of operands a CU there, 0.62 us (up to 32 rows:
+// 0.87) per four k here, fitted to 90 random products of 24 to 1632 work items; C takes the same
+// on either side.  Around the line, matrix kernel / lanes: 27 x 54 x 24 (N = 32) 15.7 / 13.8, 18 x
+// 100 x 17 20.2 / 13.8, but 81 x 28 x 55 16.9 / 27.9, 252 x 10 x 76 (N = 16) 17.8 / 20.8.
+int launchSmall(MMArgs m, hipStream_t s) {
+  const double cus = computeUnits();
+  const double items = (double)m.chunks * ceilDiv(m.I, 64) * ceilDiv(m.J, 32);
+  const double matrix = 6 + std::max(1.0, items / cus) * (m.I <= 32 ? 0.87 : 0.62) * ((m.K + 3) / 4);
+  if (m.J < m.I) {  // C^T = opB^T opA^T: the short side on the rows
+    std::swap(m.I, m.J);
+    std::swap(m.A, m.B);
+    std::swap(m.aRow, m.bCol);
+    std::swap(m.aK, m.bK);
+    std::swap(m.cRow, m.cCol);
+    std::swap(m.aSign, m.bSign);
+  }
+  int ti = m.I == 1 ? 1 : m.I == 2 ? 2 : 4, tj = ti == 4 ? 4 : 8;
+  if (laneItems(m, ti, tj) < cus / 2) {  // few workgroups: smaller tiles
+    ti = std::min(ti, 2);
+    tj = 2;
+  }
+  const double groups = laneItems(m, ti, tj);
+  const double lanes = 3 + std::max(1.0, groups / cus) * m.K * (ti + tj) * 512 / 45e3;
+  if (groups > 1 << 20 || lanes >= matrix) return -1;
+  if (tj == 2) return ti == 1 ? launchLanes<1, 2, 8>(m, s) : launchLanes<2, 2, 8>(m, s);
+  if (ti == 1) return launchLanes<1, 8, 8>(m, s);
+  if (ti == 2) return launchLanes<2, 8, 8>(m, s);
+  // (up to 16 k: 26 M products, 15 x 292 x 11, 21.0 us on eight waves, 16.6 on four)
+  return m.K <= 16 ? launchLanes<4, 4, 4>(m, s) : launchLanes<4, 4, 8>(m, s);
+}
+
 template <typename G>
 int launchPlain(const MMArgs& m, bool vec4, hipStream_t s) {
   const int total = workItems<G>(m);
@@ -829,6 +968,7 @@ int launchTransposeMM(const float* A, long a0, long a1, const float* B, long b0,
   const MMArgs m = makeArgs(A, a0, a1, B, b0, b1, C, c0, c1, I, J, K, XY, conjA, conjB, accumulate,
                             invNorm, ceilDiv(XY, XB));
   const bool vec4 = movesAsFloat4(A, a0, a1, B, b0, b1, XY);
+  if (const int rc = launchSmall(m, s); rc >= 0) return rc;
   // (the fast path keeps a lane's offset within its tile, up to 63 rows, in 32 bits)
   const bool rowsNear = m.aRow >= 0 && m.aRow < (1L << 24) && m.bCol >= 0 && m.bCol < (1L << 24);
   if (vec4 && rowsNear && storesAsFloat4(C, c0, c1)) {

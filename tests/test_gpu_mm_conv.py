@@ -505,3 +505,35 @@ def test_conv_fprop_small_products(oracle, N, H, k, Bn, Cin, Cout):
     rc, got = conv(x, w, N)
     assert rc == F.Success
     assert rel(got, oracle.corr2d_valid(x, w)) < 1e-6
+
+
+def mm_vs_fp64(oracle, conjA, conjB, I, J, K, shape, tol):
+    xy = shape[0] * shape[1]
+    A = synth.normal(((K, I) if conjA else (I, K)) + shape + (2,), seed=1).numpy()
+    B = synth.normal(((J, K) if conjB else (K, J)) + shape + (2,), seed=2).numpy()
+    rc, got = mm(A, B, conjA, conjB, 0.125)
+    assert rc == F.Success
+    want = oracle.transpose_mm64(A.reshape(A.shape[0], A.shape[1], xy, 2),
+                                 B.reshape(B.shape[0], B.shape[1], xy, 2), conjA, conjB, 0.125)
+    assert rel(got.reshape(I, J, xy, 2), want) < tol
+
+
+# transposeMMLanesKernel, every tile it has: 1 x 2 and 2 x 2 (few workgroups), 1 x 8, 2 x 8, 4 x 4 on
+# four waves (up to 16 k) and on eight; ends of the tiles, of the 64 bins and of the waves' k
+@pytest.mark.parametrize("conjA,conjB", ROLES)
+@pytest.mark.parametrize("I,J,K,shape", [
+    (1, 7, 9, (9, 16)), (6, 5, 70, (5, 8)), (3, 2, 17, (1, 65)), (1, 201, 20, (17, 32)),
+    (150, 2, 7, (17, 32)), (49, 5, 10, (17, 32)), (5, 51, 30, (17, 32)), (7, 50, 17, (1, 543))])
+def test_mm_lanes(oracle, conjA, conjB, I, J, K, shape):
+    # one multiply-add per k in each wave and a short sum: at most sqrt(2 K) roundings of 2^-24
+    # of a sum that grows like the square root of K
+    mm_vs_fp64(oracle, conjA, conjB, I, J, K, shape, np.sqrt(2 * K + 8) * 2.0 ** -24)
+
+
+# products too large for it: the matrix kernels' ragged tiles and k tails
+@pytest.mark.parametrize("I,J,K,shape,role", [
+    (260, 170, 1, (17, 32), 0), (130, 140, 2, (17, 32), 1), (131, 141, 3, (17, 32), 2),
+    (129, 143, 6, (17, 32), 0), (66, 193, 13, (17, 32), 1), (130, 140, 5, (1, 543), 2),
+    (129, 131, 6, (1, 545), 0), (193, 66, 9, (1, 543), 1)])
+def test_mm_matrix_kernels_ragged(oracle, I, J, K, shape, role):
+    mm_vs_fp64(oracle, *ROLES[role], I, J, K, shape, TOL_FFT / 10)
