@@ -122,6 +122,13 @@ int launchConvPass(int pass, int N, float* x, const int* xStride, const int* xSi
                    const int* outSize, float scale, bool accumulate, void* workspace,
                    hipStream_t s);
 
+// small forward passes and input gradients, without transforms (conv_small.hip): whether a pass
+// that would run on N points is one, and its launch
+bool runsSmall(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW);
+int launchConvSmall(int pass, const float* x, const int* xStride, const int* xSize, const float* y,
+                    const int* yStride, const int* ySize, float* out, const int* outStride, const int* outSize,
+                    hipStream_t s);
+
 // the same passes for 64- and 128-point transforms (conv_split.hip)
 size_t convSplitWorkspaceBytes(int pass, int N, int B, int Cin, int Cout);
 int launchConvSplit(int pass, int N, float* x, const int* xStride, const int* xSize, float* y,

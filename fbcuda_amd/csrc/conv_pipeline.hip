@@ -53,6 +53,8 @@
 #include "fft2d_core.h"
 #include "fft_regs.h"
 
+#include <algorithm>
+#include <cmath>
 #include <utility>
 
 namespace fbfft_amd {
@@ -1507,6 +1509,48 @@ PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int k
   return named;
 }
 
+// Small layers need no transforms: convSmall (conv_small.hip) sums over the taps in one launch.
+// They take the place of the transforms of the library's own choice of size, however a call comes
+// to that (size 0, by its name, or in place of a larger named size), so that equal sizes still
+// give equal bits; any other size that a call runs on is a transform of that size.
+// Both times are estimated: its chain of filter rows on the fullest CU (fitted to 190 random passes
+// of 2 to 5000 workgroups, within 25 % of all of them that take less than 30 us), and the three
+// launches as above, less the 3 us by which that estimate is high where they are shortest; it
+// has to be 15 % ahead.  us, transforms / sums: forward 9 x 5 x 8 x 7, 9 filters of 3 x 3 11.1 /
+// 3.8; 7 x 4 x 55 x 55, 10 of 2 x 2 28.9 / 5.9; 2 x 24 x 8 x 8, 338 of 2 x 2 11.9 / 4.6; 23 x 80 x 9 x 9, 25 of
+// 3 x 3 14.3 / 11.2; input gradient 47 x 11 x 10 x 11, 143 of 1 x 1 24.9 / 6.2; 2 x 45 x 12 x 12, 21 of 5
+// x 5 11.5 / 9.5.  Not there: 5 x 17 x 9 x 9, 15 of 7 x 7 11.9 / 15; 1 x 64 x 27 x 27, 192 of 5 x 5 16.3 / 23.
+bool runsSmall(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
+  const int C = pass == 0 ? Cin : Cout, M = pass == 0 ? Cout : Cin;
+  if (pass == 2 || kW > 11 || (long)C * kH * kW > 2048) return false;
+  const double pixels = (double)B * (pass == 0 ? (double)(H - kH + 1) * (W - kW + 1) : (double)H * W);
+  const double full = std::max(1.0, std::ceil(pixels / 64) * ceilDiv(M, 8) / 256);
+  if (full > 64) return false;
+  const double chain = ceilDiv(C * kH, 8) * kW;
+  const double sums = pass == 0 ? 3.1 + 0.88 * full + chain * (0.037 + 0.049 * full)
+                                : 3.5 + 0.51 * full + chain * (0.033 + (0.072 + 0.025 / kW) * full);
+  if (N != fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW)) return false;
+  const double transforms = windowsPass(pass, N, B, Cin, Cout, H, W, kH, kW, kAnySplits).us;
+  return sums < 0.85 * (transforms - 3);
+}
+
+// Whether a pass may take that way: it reads its operands while it writes its result, where the
+// pipeline has read all of them before, so the result must not overlap them; a lane's offset
+// within the images of its workgroup is counted in 31 bits of bytes.
+static bool smallMayRun(const float* x, const int* xStride, const int* xSize, const float* y, const int* yStride,
+                        const int* ySize, const float* out, const int* outStride, const int* outSize) {
+  const auto last = [](const float* p, const int* stride, const int* size) {
+    for (int d = 0; d < 4; ++d) p += (long)stride[d] * (size[d] - 1);
+    return p;
+  };
+  for (int d = 0; d < 4; ++d)
+    if (xStride[d] < 0 || yStride[d] < 0 || outStride[d] < 0) return false;
+  const float* const end = last(out, outStride, outSize);
+  if ((out <= last(x, xStride, xSize) && x <= end) || (out <= last(y, yStride, ySize) && y <= end)) return false;
+  const double images = 64.0 / ((double)outSize[2] * outSize[3]) + 2;
+  return images * xStride[0] + (double)xSize[2] * xStride[2] + (double)xSize[3] * xStride[3] < (1 << 29);
+}
+
 // pass 0: x = input [B][Cin][H][W], y = weight [Cout][Cin][kH][kW], out = output [B][Cout][oH][oW]
 // pass 1: x = gradOutput [B][Cout][oH][oW], y = weight, out = gradInput [B][Cin][H][W]
 // pass 2: x = input, y = gradOutput, out = gradWeight [Cout][Cin][kH][kW]
@@ -1522,6 +1566,9 @@ int launchConvPass(int pass, int N, float* x, const int* xStride, const int* xSi
   const int H = in[2], W = in[3], kH = wt[2], kW = wt[3];
   const PassSize size = passSize(pass, N, in[0], wt[1], wt[0], H, W, kH, kW);
   N = size.N;
+  if (runsSmall(pass, N, in[0], wt[1], wt[0], H, W, kH, kW) &&
+      smallMayRun(x, xStride, xSize, y, yStride, ySize, out, outStride, outSize))
+    return launchConvSmall(pass, x, xStride, xSize, y, yStride, ySize, out, outStride, outSize, s);
   if (N > 32)
     return launchConvSplit(pass, N, x, xStride, xSize, y, yStride, ySize, out, outStride, outSize,
                            scale, accumulate, workspace, s);

@@ -256,7 +256,10 @@ size_t fbfft_make_tiles_for_pass(int pass, const fbfft_tensor* input, const fbff
  * gradient); every size computes the same
  * convolution.  The reference leaves the choice to its caller (the FFTSize template
  * parameter of fbfft/FFTIteratedConvolution.cuh:624); 64 and 128 are only taken when asked
- * for. */
+ * for.  Where a small forward pass or input gradient would run on this size - by size 0, by its
+ * name or in place of a larger named size - and three launches would take longer than the sums
+ * over the filter taps themselves, it is summed directly, in one launch (the same bits for each
+ * of those calls; a result that overlaps an operand keeps the transforms). */
 int fbfft_conv_choose_fft_size(int pass, int batch, int cin, int cout, int H, int W, int kH,
                                int kW);
 
