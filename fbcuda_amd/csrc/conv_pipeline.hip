@@ -21,7 +21,7 @@
 //      remapped per XCD) and C written once with coalesced stores.
 //      binGemmSplit: the same product on the bf16 matrix instructions, fp32 operands
 //      split into three bf16 values each.
-//      binGemmRegsWide / binGemmRegsSplitK: the same product without LDS for
+//      binGemmRegsWide / binGemmRegsNarrow / binGemmRegsSplitK: the same product without LDS for
 //      products with a side of up to 32 (planGemm picks kernel, tiles and the
 //      ranges a long reduction is cut into).
 //   3. inverseBinMajor:  C[bin][i][j] -> planes, gathering runs of SLOTS
@@ -910,6 +910,97 @@ __global__ __launch_bounds__(kT, 3) void binGemmRegsWide(GemmArgs g) {
   }
 }
 
+// ... and for up to 16 rows: the same on v_mfma_f32_16x16x4_f32.  A wave owns 16 rows x 64
+// columns; lane (c, q) loads 16 bytes of B per four k - columns j0 + 2c and j0 + 2c + 1 at k = q - of
+// either half of the columns, and 8 bytes of A.  The matrix work of 16 rows that are not there
+// is what bounded the 32-row form: us, 201 x 74 x 17 x 14 images, 9 filters of 8 x 8, input gradient
+// 34.6 -> 16.0; 27 x 4 x 100 x 100, 152 of 9 x 9, input gradient 103.5 -> 58.0; 15 x 7 x 111 x 111, 372
+// of 9 x 9, forward 168.7 -> 139.5.
+struct GemmSliceNarrow {
+  float2 a[2];
+  float4 b[2][2];
+};
+
+__global__ __launch_bounds__(kT, 4) void binGemmRegsNarrow(GemmArgs g) {
+  const int t = threadIdx.x;
+  const int lane = t % 64, w = __builtin_amdgcn_readfirstlane(t / 64);
+  const int c = lane % 16, q = lane / 16;
+  const int total = g.bins * g.JT;
+  const int per = (total + 7) / 8;
+  const int logical = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (logical >= total) return;
+  const int bin = logical / g.JT;
+  const int j0 = (logical % g.JT * 4 + w) * 64;
+  if (j0 >= g.Jp) return;
+  const bool pairs = bin == 0 || 2 * bin == g.N;  // bins of real pairs: (ar br, ai bi)
+  const float cross = pairs ? 0.f : 1.f;
+
+  // operand columns beyond the padded arrays are clamped, as above
+  const unsigned laneA = (unsigned)(q * g.Ip + min(c, g.Ip - 1)) * (unsigned)sizeof(float2);
+  unsigned laneB[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+    laneB[u] = (unsigned)(q * g.Jp + min(32 * u + 2 * c, g.Jp - 2 - j0)) * (unsigned)sizeof(float2);
+  const char* const binA = (const char*)(g.A + (long)bin * g.Kp * g.Ip);
+  const char* const binB = (const char*)(g.B + (long)bin * g.Kp * g.Jp + j0);
+  const long sa = 4L * g.Ip * sizeof(float2), sb = 4L * g.Jp * sizeof(float2);  // four k-rows
+
+  typedef float floatx4 __attribute__((ext_vector_type(4)));
+  floatx4 k1[4], k2[4], k3[4];  // of columns 2c, 2c + 1, 32 + 2c, 33 + 2c
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) k1[n][v] = k2[n][v] = k3[n][v] = 0.f;
+
+  auto fetch = [&](GemmSliceNarrow& s, int sl) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const long k4 = (long)sl * 2 + h;
+      const PlainPair va = *(const GlobalPair*)(scalarBase(binA + k4 * sa) + laneOffset(laneA));
+      s.a[h] = float2{va.x, va.y};
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const PlainQuad vb = *(const GlobalQuad*)(scalarBase(binB + k4 * sb) + laneOffset(laneB[u]));
+        s.b[h][u] = float4{vb.x, vb.y, vb.z, vb.w};
+      }
+    }
+  };
+  auto multiply = [&](const GemmSliceNarrow& s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float2 a = s.a[h];
+      const float as = __builtin_fmaf(cross, a.y, a.x);
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const float4 b = s.b[h][n / 2];
+        const float br = n % 2 ? b.z : b.x, bi = n % 2 ? b.w : b.y;
+        k1[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(as, br, k1[n], 0, 0, 0);
+        k2[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, -br - bi, k2[n], 0, 0, 0);
+        k3[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, __builtin_fmaf(cross, br, -bi), k3[n], 0, 0, 0);
+      }
+    }
+  };
+  const int first = blockIdx.y * g.slicesPerSplit;
+  ringOfThree<GemmSliceNarrow>(first, 1, min(first + g.slicesPerSplit, g.Kp / GK2) - first, fetch, multiply);
+
+  float2* Cb = g.C + blockIdx.y * g.splitStride + (long)bin * g.I * g.Jp;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int j = j0 + 32 * u + 2 * c;
+    if (j >= g.Jp) continue;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = 4 * q + v;
+      if (i >= g.I) continue;
+      auto value = [&](int n) {
+        return pairs ? float2{k1[n][v], -k3[n][v]} : float2{k1[n][v] - k3[n][v], k1[n][v] + k2[n][v]};
+      };
+      const float2 lo = value(2 * u), hi = value(2 * u + 1);
+      *reinterpret_cast<float4*>(Cb + (long)i * g.Jp + j) = float4{lo.x, lo.y, hi.x, hi.y};
+    }
+  }
+}
+
 // The same product on the bf16 matrix instructions, for products that outweigh their operands
 // (planGemm).  fp32 matrix instructions are what bounds
 // binGemmDirect there (155 TFLOP/s); the bf16 ones run at 1600 to 1750 on random operands (the power
@@ -1123,7 +1214,7 @@ inline bool swapRoles(int I, int J, bool outTiled) {
 // per bin over 1936 windows, 2048 waves: two ranges 337 -> 345 us, four 362: that
 // contraction is not short of waves).
 struct GemmPlan {
-  enum Kind { RegsSplitK, RegsWide, Direct64, Direct128, Split } kind;
+  enum Kind { RegsSplitK, RegsWide, RegsNarrow, Direct64, Direct128, Split } kind;
   int IT, JT;
   int splits, slicesPerSplit;
   long waves;  // of one range
@@ -1176,6 +1267,8 @@ inline GemmPlan planGemm(int bins, int I, int Jp, int Kp, int maxSplits) {
     p.IT = ceilDiv(I, 32);
     p.JT = ceilDiv(Jp, 32);
   }
+  // up to 16 rows: 91 random products 0.97 to 2.2 times as fast as on 32-row tiles
+  if (p.kind == GemmPlan::RegsWide && I <= 16) p.kind = GemmPlan::RegsNarrow;
   // binGemmSplit where the products outweigh the operands by enough: each spectrum value enters
   // I J K / (I J + I K + J K) complex products.  Whole layers on a loaded chip, three passes
   // back to back, binGemmDirect / this by that quotient: 93 (66 x 273 x 25 x 26, 307 of 2 x 2)
@@ -1319,6 +1412,7 @@ int runPipeline(PlaneSet x, PlaneSet y, PlaneSet out, bool conjY, float scale, b
   switch (plan.kind) {
     case GemmPlan::RegsSplitK: binGemmRegsSplitK<<<ggrid, dim3(kT), 0, s>>>(g); break;
     case GemmPlan::RegsWide: binGemmRegsWide<<<ggrid, dim3(kT), 0, s>>>(g); break;
+    case GemmPlan::RegsNarrow: binGemmRegsNarrow<<<ggrid, dim3(kT), 0, s>>>(g); break;
     case GemmPlan::Direct64: binGemmDirect<64><<<ggrid, dim3(kT), 0, s>>>(g); break;
     case GemmPlan::Direct128: binGemmDirect<GI><<<ggrid, dim3(kT), 0, s>>>(g); break;
     case GemmPlan::Split: binGemmSplit<<<ggrid, dim3(kT), 0, s>>>(g); break;

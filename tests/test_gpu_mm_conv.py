@@ -537,3 +537,15 @@ def test_mm_lanes(oracle, conjA, conjB, I, J, K, shape):
     (129, 131, 6, (1, 545), 0), (193, 66, 9, (1, 543), 1)])
 def test_mm_matrix_kernels_ragged(oracle, I, J, K, shape, role):
     mm_vs_fp64(oracle, *ROLES[role], I, J, K, shape, TOL_FFT / 10)
+
+
+# binGemmRegsNarrow: 1 to 16 rows (either operand on them), columns beside the end of a wave's 64
+# and of its two halves, one slice of k and an odd number
+@pytest.mark.parametrize("Bn,Cin,Cout", [
+    (70, 9, 1), (65, 17, 5), (129, 40, 16), (97, 3, 15), (2, 24, 64), (16, 25, 127), (1, 8, 96)])
+def test_conv_fprop_up_to_16_rows(oracle, Bn, Cin, Cout):
+    x = synth.normal((Bn, Cin, 30, 31), seed=30).numpy()
+    w = synth.normal((Cout, Cin, 11, 12), seed=31, std=0.02).numpy()
+    rc, got = conv(x, w, 32)
+    assert rc == F.Success
+    assert rel(got, oracle.corr2d_valid(x, w)) < 1e-6
