@@ -84,6 +84,7 @@ PyObject* guarded(Py_ssize_t given, Py_ssize_t wanted, F body) {
   try {
     return body();
   } catch (...) {
+    PyErr_Clear();
     Py_RETURN_NOTIMPLEMENTED;
   }
 }
