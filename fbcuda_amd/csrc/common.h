@@ -92,6 +92,15 @@ int launchTransposeMM(const float* A, long a0, long a1, const float* B, long b0,
                       long c0, long c1, int I, int J, int K, int XY, bool conjA, bool conjB,
                       bool accumulate, float invNorm, hipStream_t s);
 
+// the kernel that launchTransposeMM runs a product on, the tile of C that a workgroup of it takes
+// (lanes: the short side of C on the rows) and its waves
+struct ProductRoute {
+  enum Kind { Registers, Direct, Lanes };
+  int kind, rows, cols, waves;
+};
+ProductRoute productRoute(const float* A, long a0, long a1, const float* B, long b0, long b1, const float* C,
+                          long c0, long c1, int I, int J, int K, int XY, bool conjA, bool conjB);
+
 int launchTransposeMMPacked(const float* A, long a0, long a1, const float* B, long b0, long b1,
                             float* C, long c0, long c1, int I, int J, int K, int N, bool conjA,
                             bool conjB, bool accumulate, float invNorm, hipStream_t s);

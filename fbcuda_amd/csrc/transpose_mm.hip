@@ -27,7 +27,7 @@
 //    [bin][k][row] (conjugation folded into the sign of the imaginary plane, edges
 //    zeroed), two buffers deep, while the slice after next is in flight in registers;
 //  * transposeMMLanesKernel for products too small to fill the matrix kernels' tiles
-//    (launchSmall).
+//    (lanesRoute).
 //
 // Packed spectra (fbfft_transpose_mm_packed): operands [..][..][N/2][N] whose row 0
 // holds P[x] = F0[x] + i FH[x], the spectra of the two real rows 0 and N/2 of an
@@ -903,16 +903,9 @@ int launchLanes(const MMArgs& m, hipStream_t s) {
   return launchStatus();
 }
 
-// Small products to transposeMMLanesKernel; -1: not one.  Both times are estimated, in us, from
-// the chain of slices of the fullest CU: 45 GB/s of operands a CU there, 0.62 us (up to 32 rows:
-// 0.87) per four k here, fitted to 90 random products of 24 to 1632 work items; C takes the same
-// on either side.  Around the line, matrix kernel / lanes: 27 x 54 x 24 (N = 32) 15.7 / 13.8, 18 x
-// 100 x 17 20.2 / 13.8, but 81 x 28 x 55 16.9 / 27.9, 252 x 10 x 76 (N = 16) 17.8 / 20.8.
-int launchSmall(MMArgs m, hipStream_t s) {
-  const double cus = computeUnits();
-  const double items = (double)m.chunks * ceilDiv(m.I, 64) * ceilDiv(m.J, 32);
-  const double matrix = 6 + std::max(1.0, items / cus) * (m.I <= 32 ? 0.87 : 0.62) * ((m.K + 3) / 4);
-  if (m.J < m.I) {  // C^T = opB^T opA^T: the short side on the rows
+// C^T = opB^T opA^T where that puts the short side on the rows
+MMArgs shortSideOnRows(MMArgs m) {
+  if (m.J < m.I) {
     std::swap(m.I, m.J);
     std::swap(m.A, m.B);
     std::swap(m.aRow, m.bCol);
@@ -920,19 +913,76 @@ int launchSmall(MMArgs m, hipStream_t s) {
     std::swap(m.cRow, m.cCol);
     std::swap(m.aSign, m.bSign);
   }
-  int ti = m.I == 1 ? 1 : m.I == 2 ? 2 : 4, tj = ti == 4 ? 4 : 8;
-  if (laneItems(m, ti, tj) < cus / 2) {  // few workgroups: smaller tiles
+  return m;
+}
+
+// Whether C lies apart from both operands.  transposeMMLanesKernel needs that: its tiles are
+// separate workgroups, and one would store what another has yet to read.  A workgroup of the matrix
+// kernels reads whole rows of A and whole columns of B before it stores, so C in the place of A (or
+// B) comes out right there as long as one tile spans its columns (or rows).
+bool resultApart(const MMArgs& m) {
+  struct Bytes {
+    intptr_t first, end;
+  };
+  const auto bytes = [&](const float* p, long s0, int n0, long s1, int n1) {
+    const long d0 = s0 * (n0 - 1), d1 = s1 * (n1 - 1);
+    const intptr_t at = reinterpret_cast<intptr_t>(p);
+    return Bytes{at + (std::min(d0, 0L) + std::min(d1, 0L)) * (long)sizeof(float),
+                 at + (std::max(d0, 0L) + std::max(d1, 0L) + 2L * m.XY) * (long)sizeof(float)};
+  };
+  if (m.K <= 0) return true;  // nothing is read
+  const Bytes a = bytes(m.A, m.aRow, m.I, m.aK, m.K), b = bytes(m.B, m.bCol, m.J, m.bK, m.K),
+              c = bytes(m.C, m.cRow, m.I, m.cCol, m.J);
+  return (c.end <= a.first || a.end <= c.first) && (c.end <= b.first || b.end <= c.first);
+}
+
+// Small products to transposeMMLanesKernel.  Both times are estimated, in us, from
+// the chain of slices of the fullest CU: 45 GB/s of operands a CU there, 0.62 us (up to 32 rows:
+// 0.87) per four k here, fitted to 90 random products of 24 to 1632 work items; C takes the same
+// on either side.  Around the line, matrix kernel / lanes: 27 x 54 x 24 (N = 32) 15.7 / 13.8, 18 x
+// 100 x 17 20.2 / 13.8, but 81 x 28 x 55 16.9 / 27.9, 252 x 10 x 76 (N = 16) 17.8 / 20.8.
+bool lanesRoute(const MMArgs& m, ProductRoute* r) {
+  const double cus = computeUnits();
+  const double items = (double)m.chunks * ceilDiv(m.I, 64) * ceilDiv(m.J, 32);
+  const double matrix = 6 + std::max(1.0, items / cus) * (m.I <= 32 ? 0.87 : 0.62) * ((m.K + 3) / 4);
+  const MMArgs t = shortSideOnRows(m);
+  int ti = t.I == 1 ? 1 : t.I == 2 ? 2 : 4, tj = ti == 4 ? 4 : 8;
+  if (laneItems(t, ti, tj) < cus / 2) {  // few workgroups: smaller tiles
     ti = std::min(ti, 2);
     tj = 2;
   }
-  const double groups = laneItems(m, ti, tj);
+  const double groups = laneItems(t, ti, tj);
   const double lanes = 3 + std::max(1.0, groups / cus) * m.K * (ti + tj) * 512 / 45e3;
-  if (groups > 1 << 20 || lanes >= matrix) return -1;
-  if (tj == 2) return ti == 1 ? launchLanes<1, 2, 8>(m, s) : launchLanes<2, 2, 8>(m, s);
-  if (ti == 1) return launchLanes<1, 8, 8>(m, s);
-  if (ti == 2) return launchLanes<2, 8, 8>(m, s);
-  // (up to 16 k: 26 M products, 15 x 292 x 11, 21.0 us on eight waves, 16.6 on four)
-  return m.K <= 16 ? launchLanes<4, 4, 4>(m, s) : launchLanes<4, 4, 8>(m, s);
+  if (groups > 1 << 20 || lanes >= matrix || !resultApart(m)) return false;
+  // (4 x 4 up to 16 k: 26 M products, 15 x 292 x 11, 21.0 us on eight waves, 16.6 on four)
+  *r = ProductRoute{ProductRoute::Lanes, ti, tj, ti == 4 && m.K <= 16 ? 4 : 8};
+  return true;
+}
+
+int launchLanesRoute(const ProductRoute& r, const MMArgs& m, hipStream_t s) {
+  const MMArgs t = shortSideOnRows(m);
+  if (r.cols == 2) return r.rows == 1 ? launchLanes<1, 2, 8>(t, s) : launchLanes<2, 2, 8>(t, s);
+  if (r.rows == 1) return launchLanes<1, 8, 8>(t, s);
+  if (r.rows == 2) return launchLanes<2, 8, 8>(t, s);
+  return r.waves == 4 ? launchLanes<4, 4, 4>(t, s) : launchLanes<4, 4, 8>(t, s);
+}
+
+ProductRoute routeOf(const MMArgs& m, bool vec4, bool vec4C) {
+  ProductRoute r;
+  if (lanesRoute(m, &r)) return r;
+  // (the fast path keeps a lane's offset within its tile, up to 63 rows, in 32 bits)
+  const bool rowsNear = m.aRow >= 0 && m.aRow < (1L << 24) && m.bCol >= 0 && m.bCol < (1L << 24);
+  if (!vec4 || !rowsNear || !vec4C) return {ProductRoute::Registers, Wide::TI, Wide::TJ, Wide::WAVES};
+  // Equal work items are dealt to the CUs in whole numbers: the launch lasts as
+  // long as the fullest CU.  32-row tiles re-read B twice as often and pay more per
+  // matrix instruction, so they are taken only where they even the load out
+  // (128 x 64 x 192 over 544 bins: 816 items of 64 rows are 3.19 per CU, four on the fullest - 72 us;
+  // 1632 of 32 rows are 6.4, seven on the fullest - 68 us; at 2, 4 or 8 items of 64
+  // rows per CU the larger tile wins by 3-9 %).
+  const int cus = computeUnits();
+  auto evenness = [&](int items) { return (double)items / cus / ceilDiv(items, cus); };
+  const bool halves = evenness(directWorkItems<32>(m)) > evenness(directWorkItems<64>(m)) + 0.05;
+  return {ProductRoute::Direct, halves ? 32 : 64, DTJ, DTHREADS / 64};
 }
 
 template <typename G>
@@ -961,6 +1011,13 @@ int launchPacked(const MMArgs& mainRows, const MMArgs& row0, bool vec4, hipStrea
 
 // A, B, C: complex-as-float views collapsed to [d0][d1][xy][2] with unit xy
 // stride; s0/s1 are the float strides of the first two dimensions.
+ProductRoute productRoute(const float* A, long a0, long a1, const float* B, long b0, long b1, const float* C,
+                          long c0, long c1, int I, int J, int K, int XY, bool conjA, bool conjB) {
+  const MMArgs m = makeArgs(A, a0, a1, B, b0, b1, const_cast<float*>(C), c0, c1, I, J, K, XY, conjA, conjB,
+                            false, 1.f, ceilDiv(XY, XB));
+  return routeOf(m, movesAsFloat4(A, a0, a1, B, b0, b1, XY), storesAsFloat4(C, c0, c1));
+}
+
 int launchTransposeMM(const float* A, long a0, long a1, const float* B, long b0, long b1, float* C,
                       long c0, long c1, int I, int J, int K, int XY, bool conjA, bool conjB,
                       bool accumulate, float invNorm, hipStream_t s) {
@@ -968,27 +1025,15 @@ int launchTransposeMM(const float* A, long a0, long a1, const float* B, long b0,
   const MMArgs m = makeArgs(A, a0, a1, B, b0, b1, C, c0, c1, I, J, K, XY, conjA, conjB, accumulate,
                             invNorm, ceilDiv(XY, XB));
   const bool vec4 = movesAsFloat4(A, a0, a1, B, b0, b1, XY);
-  if (const int rc = launchSmall(m, s); rc >= 0) return rc;
-  // (the fast path keeps a lane's offset within its tile, up to 63 rows, in 32 bits)
-  const bool rowsNear = m.aRow >= 0 && m.aRow < (1L << 24) && m.bCol >= 0 && m.bCol < (1L << 24);
-  if (vec4 && rowsNear && storesAsFloat4(C, c0, c1)) {
-    // Equal work items are dealt to the CUs in whole numbers: the launch lasts as
-    // long as the fullest CU.  32-row tiles re-read B twice as often and pay more per
-    // matrix instruction, so they are taken only where they even the load out
-    // (128 x 64 x 192 over 544 bins: 816 items of 64 rows are 3.19 per CU, four on the fullest - 72 us;
-    // 1632 of 32 rows are 6.4, seven on the fullest - 68 us; at 2, 4 or 8 items of 64
-    // rows per CU the larger tile wins by 3-9 %).
-    const int cus = computeUnits();
-    auto evenness = [&](int items) { return (double)items / cus / ceilDiv(items, cus); };
-    const int items64 = directWorkItems<64>(m), items32 = directWorkItems<32>(m);
-    if (evenness(items32) > evenness(items64) + 0.05) {
-      transposeMMDirectKernel<32><<<dim3((items32 + 7) / 8 * 8), dim3(DTHREADS), 0, s>>>(m, items32);
-    } else {
-      transposeMMDirectKernel<64><<<dim3((items64 + 7) / 8 * 8), dim3(DTHREADS), 0, s>>>(m, items64);
-    }
-    return launchStatus();
-  }
-  return launchPlain<Wide>(m, vec4, s);
+  const ProductRoute r = routeOf(m, vec4, storesAsFloat4(C, c0, c1));
+  if (r.kind == ProductRoute::Lanes) return launchLanesRoute(r, m, s);
+  if (r.kind == ProductRoute::Registers) return launchPlain<Wide>(m, vec4, s);
+  const int items64 = directWorkItems<64>(m), items32 = directWorkItems<32>(m);
+  if (r.rows == 32)
+    transposeMMDirectKernel<32><<<dim3((items32 + 7) / 8 * 8), dim3(DTHREADS), 0, s>>>(m, items32);
+  else
+    transposeMMDirectKernel<64><<<dim3((items64 + 7) / 8 * 8), dim3(DTHREADS), 0, s>>>(m, items64);
+  return launchStatus();
 }
 
 // The same contraction on packed spectra [d0][d1][N/2][N][2]: rows 1 .. N/2-1 as

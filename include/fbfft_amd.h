@@ -121,8 +121,10 @@ int fbfft_c2c_2d_inverse_pass1(const fbfft_tensor* src, const fbfft_tensor* dst,
  * first two and the last are contiguous and collapse to xy:
  *   A [I][K][xy][2] (conjA: [K][I][xy][2]),  B [K][J][xy][2] (conjB: [J][K][xy][2])
  *   C[i][j][xy] = invNorm * ((accumulate ? C[i][j][xy] : 0) + sum_k opA * opB)
- * where opX conjugates when conjX is set.  Returns an fbfft_error (the
- * reference returns void and aborts on bad shapes). */
+ * where opX conjugates when conjX is set.  C may be A itself (conjA = 0, the same address, sizes
+ * and strides) where J <= 32, or B itself (conjB = 0) where I <= 32; any other overlap of C with an
+ * operand is not defined.  Returns an fbfft_error (the reference returns void and aborts on bad
+ * shapes). */
 int fbfft_transpose_mm(const fbfft_tensor* A, const fbfft_tensor* B, const fbfft_tensor* C,
                        int conjA, int conjB, int accumulate, float invNorm,
                        fbfft_stream_t stream);

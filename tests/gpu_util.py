@@ -24,6 +24,27 @@ def pass_size(pass_, N, B, cin, cout, H, W, k):
     return r.N, r.maxSplits
 
 
+class ProductRoute(ctypes.Structure):
+    _fields_ = [(f, ctypes.c_int) for f in ("kind", "rows", "cols", "waves")]
+
+
+REGISTERS, DIRECT, LANES = range(3)
+
+
+def product_route(A, B, C, conjA, conjB):
+    """The kernel (REGISTERS, DIRECT or LANES), rows and columns of its tile and waves that
+    transposeMM runs on A, B, C [d0][d1]...[2]: the library's own host function (common.h), which
+    looks at addresses, strides and sizes only."""
+    fn = F.lib()._ZN9fbfft_amd12productRouteEPKfllS1_llS1_lliiiibb
+    l, i, b = ctypes.c_long, ctypes.c_int, ctypes.c_bool
+    fn.argtypes, fn.restype = [ctypes.c_void_p, l, l] * 3 + [i] * 4 + [b] * 2, ProductRoute
+    I, K = (A.shape[1], A.shape[0]) if conjA else A.shape[:2]
+    xy = int(np.prod(C.shape[2:-1]))
+    r = fn(*(v for t in (A, B, C) for v in (t.data_ptr(), t.stride(0), t.stride(1))), I, C.shape[1], K, xy,
+           conjA, conjB)
+    return r.kind, r.rows, r.cols, r.waves
+
+
 def dev():
     return torch.device("cuda:0")
 

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 import fbcuda_amd as F
-from gpu_util import pass_size
+from gpu_util import DIRECT, LANES, REGISTERS, pass_size, product_route
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -349,3 +349,25 @@ def test_conv_choose_fft_size():
     assert L.fbfft_conv_choose_fft_size(3, 4, 3, 5, 27, 27, 5, 5) == 0
     assert L.fbfft_conv_choose_fft_size(0, 0, 3, 5, 27, 27, 5, 5) == 0
     assert L.fbfft_conv_workspace_image(0, 4, 3, 5, 64, 64, 33, 3, 0) == 0
+
+
+@pytest.mark.parametrize("I,J,K", [(16, 8, 8), (8, 16, 16), (32, 32, 32), (5, 3, 3), (150, 8, 8)])
+def test_mm_small_products_in_place_keep_the_kernels_that_read_first(I, J, K):
+    """A small product goes to the kernel whose tiles are separate workgroups only where C lies
+    apart from A and B: in place of one of them, or with one element in common, it keeps the matrix
+    kernels, and just beside them it does not."""
+    import torch
+    xy = 544
+    space = torch.empty((3, 160, 160 * xy * 2 + 2))  # no element is read or written
+
+    def operand(n, d0, d1, shift=0):
+        return space[n].view(-1).as_strided((d0, d1, xy, 2), (d1 * xy * 2, xy * 2, 2, 1),
+                                            space[n].storage_offset() + shift)
+    A, B, C = operand(0, I, K), operand(1, K, J), operand(2, I, J)
+    assert product_route(A, B, C, False, False)[0] == LANES
+    for other, into in ((A, 0), (B, 1)):
+        assert product_route(A, B, operand(into, I, J), False, False)[0] == DIRECT
+        last = other.numel()
+        assert product_route(A, B, operand(into, I, J, last - 4), False, False)[0] == DIRECT
+        assert product_route(A, B, operand(into, I, J, last - 2), False, False)[0] == REGISTERS  # 8-byte aligned
+        assert product_route(A, B, operand(into, I, J, last), False, False)[0] == LANES

@@ -6,7 +6,7 @@ import torch
 
 import fbcuda_amd as F
 from fbcuda_amd import synth
-from gpu_util import check, TOL_CONV, TOL_FFT, dev, rel
+from gpu_util import LANES, check, TOL_CONV, TOL_FFT, dev, product_route, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -528,6 +528,25 @@ def test_mm_lanes(oracle, conjA, conjB, I, J, K, shape):
     # one multiply-add per k in each wave and a short sum: at most sqrt(2 K) roundings of 2^-24
     # of a sum that grows like the square root of K
     mm_vs_fp64(oracle, conjA, conjB, I, J, K, shape, np.sqrt(2 * K + 8) * 2.0 ** -24)
+
+
+# C in the place of A (J <= 32) or of B (I <= 32), on sizes that run on transposeMMLanesKernel elsewhere:
+# 16-byte and 8-byte aligned, several tiles of the side that may be long
+@pytest.mark.parametrize("odd", [0, 1])
+@pytest.mark.parametrize("I,J", [(16, 8), (8, 16), (32, 32), (3, 5), (150, 8), (8, 150)])
+def test_mm_in_place(oracle, I, J, odd):
+    xy = 544 - odd
+    inA = J <= 32
+    K = J if inA else I
+    A, B = synth.normal((I, K, xy, 2), seed=1), synth.normal((K, J, xy, 2), seed=2)
+    Ad, Bd = A.to(dev()), B.to(dev())
+    Cd = Ad if inA else Bd
+    assert product_route(Ad, Bd, torch.empty((I, J, xy, 2), device=dev()), False, False)[0] == LANES
+    assert product_route(Ad, Bd, Cd, False, False)[0] != LANES
+    assert F.transposeMM(Ad, Bd, Cd, 0.125) == F.Success
+    torch.cuda.synchronize()
+    want = oracle.transpose_mm64(A.numpy(), B.numpy(), False, False, 0.125)
+    assert rel(Cd.cpu().numpy(), want) < TOL_FFT / 10
 
 
 # products too large for it: the matrix kernels' ragged tiles and k tails
