@@ -936,40 +936,21 @@ bool resultApart(const MMArgs& m) {
   return (c.end <= a.first || a.end <= c.first) && (c.end <= b.first || b.end <= c.first);
 }
 
-// Small products to transposeMMLanesKernel.  Both times are estimated, in us, from
-// the chain of slices of the fullest CU: 45 GB/s of operands a CU there, 0.62 us (up to 32 rows:
-// 0.87) per four k here, fitted to 90 random products of 24 to 1632 work items; C takes the same
-// on either side.  Around the line, matrix kernel / lanes: 27 x 54 x 24 (N = 32) 15.7 / 13.8, 18 x
-// 100 x 17 20.2 / 13.8, but 81 x 28 x 55 16.9 / 27.9, 252 x 10 x 76 (N = 16) 17.8 / 20.8.
-bool lanesRoute(const MMArgs& m, ProductRoute* r) {
-  const double cus = computeUnits();
-  const double items = (double)m.chunks * ceilDiv(m.I, 64) * ceilDiv(m.J, 32);
-  const double matrix = 6 + std::max(1.0, items / cus) * (m.I <= 32 ? 0.87 : 0.62) * ((m.K + 3) / 4);
+// the tile of transposeMMLanesKernel for a product
+ProductRoute lanesTile(const MMArgs& m) {
   const MMArgs t = shortSideOnRows(m);
   int ti = t.I == 1 ? 1 : t.I == 2 ? 2 : 4, tj = ti == 4 ? 4 : 8;
-  if (laneItems(t, ti, tj) < cus / 2) {  // few workgroups: smaller tiles
+  if (laneItems(t, ti, tj) < computeUnits() / 2) {  // few workgroups: smaller tiles
     ti = std::min(ti, 2);
     tj = 2;
   }
-  const double groups = laneItems(t, ti, tj);
-  const double lanes = 3 + std::max(1.0, groups / cus) * m.K * (ti + tj) * 512 / 45e3;
-  if (groups > 1 << 20 || lanes >= matrix || !resultApart(m)) return false;
-  // (4 x 4 up to 16 k: 26 M products, 15 x 292 x 11, 21.0 us on eight waves, 16.6 on four)
-  *r = ProductRoute{ProductRoute::Lanes, ti, tj, ti == 4 && m.K <= 16 ? 4 : 8};
-  return true;
+  // (4 x 4 up to 16 k: 263 random products 3 to 25 % faster on four waves than on eight in nine of ten, 114
+  // of 21 k and more 3 % slower in the middle)
+  return {ProductRoute::Lanes, ti, tj, ti == 4 && m.K <= 16 ? 4 : 8};
 }
 
-int launchLanesRoute(const ProductRoute& r, const MMArgs& m, hipStream_t s) {
-  const MMArgs t = shortSideOnRows(m);
-  if (r.cols == 2) return r.rows == 1 ? launchLanes<1, 2, 8>(t, s) : launchLanes<2, 2, 8>(t, s);
-  if (r.rows == 1) return launchLanes<1, 8, 8>(t, s);
-  if (r.rows == 2) return launchLanes<2, 8, 8>(t, s);
-  return r.waves == 4 ? launchLanes<4, 4, 4>(t, s) : launchLanes<4, 4, 8>(t, s);
-}
-
-ProductRoute routeOf(const MMArgs& m, bool vec4, bool vec4C) {
-  ProductRoute r;
-  if (lanesRoute(m, &r)) return r;
+// the matrix kernel for a product and its tile
+ProductRoute matrixTile(const MMArgs& m, bool vec4, bool vec4C) {
   // (the fast path keeps a lane's offset within its tile, up to 63 rows, in 32 bits)
   const bool rowsNear = m.aRow >= 0 && m.aRow < (1L << 24) && m.bCol >= 0 && m.bCol < (1L << 24);
   if (!vec4 || !rowsNear || !vec4C) return {ProductRoute::Registers, Wide::TI, Wide::TJ, Wide::WAVES};
@@ -983,6 +964,46 @@ ProductRoute routeOf(const MMArgs& m, bool vec4, bool vec4C) {
   auto evenness = [&](int items) { return (double)items / cus / ceilDiv(items, cus); };
   const bool halves = evenness(directWorkItems<32>(m)) > evenness(directWorkItems<64>(m)) + 0.05;
   return {ProductRoute::Direct, halves ? 32 : 64, DTJ, DTHREADS / 64};
+}
+
+// Small products run on transposeMMLanesKernel.  Both times are estimated, in us, from
+// the chain of slices of the fullest CU: 45 GB/s of operands a CU there, 0.62 us (up to 32 rows:
+// 0.87) per four k on the matrix kernels, fitted to 90 random products of 24 to 1632 work items.
+// Around the line, matrix kernel / lanes: 27 x 54 x 24 (N = 32) 15.7 / 13.8, 18 x
+// 100 x 17 20.2 / 13.8, but 81 x 28 x 55 16.9 / 27.9, 252 x 10 x 76 (N = 16) 17.8 / 20.8.
+// Those leave out what a workgroup does besides its k - it starts, and stores its part of C - which is most
+// of a product of few k in many small tiles: 253 x 100 x 2 (N = 16) 11.5 / 17.1, 369 x 460 x 1 (N = 8) 13.9 /
+// 26.8, 80 x 32 x 3 (N = 32) 6.8 / 7.9.  So a second pair of estimates, with that in them, must not see the
+// lanes behind, either.  Of 1844 random products that the first pair sends there, 90 of them over 3 %
+// slower than on the matrix kernels, the second leaves 13 (two over 10 %) and takes back 9 that
+// were over 3 % faster.
+bool lanesRoute(const MMArgs& m, const ProductRoute& lanes, const ProductRoute& matrix) {
+  const int icus = computeUnits(), k4 = ceilDiv(m.K, 4);
+  const double cus = icus, groups = laneItems(shortSideOnRows(m), lanes.rows, lanes.cols);
+  if (groups > 1 << 20) return false;
+  const double full = std::max(1.0, groups / cus), asked = (double)m.K * (lanes.rows + lanes.cols);
+  const double items = (double)m.chunks * ceilDiv(m.I, 64) * ceilDiv(m.J, 32);
+  if (3 + full * asked * 512 / 45e3 >= 6 + std::max(1.0, items / cus) * (m.I <= 32 ? 0.87 : 0.62) * k4) return false;
+  const double lanesUs =
+      2.5 + full * (0.0094 * asked + 0.01 * lanes.rows * lanes.cols + 0.41) + 0.1 * ceilDiv(m.K, lanes.waves);
+  const double matrixUs =
+      matrix.kind == ProductRoute::Registers ? 4.8 + ceilDiv(workItems<Wide>(m), icus) * (1.87 * k4 + 6.8)
+      : matrix.rows == 32 ? 3.6 + 0.16 * k4 + ceilDiv(directWorkItems<32>(m), icus) * (0.39 * k4 + 2.1)
+                          : 3.6 + 0.16 * k4 + ceilDiv(directWorkItems<64>(m), icus) * (0.78 * k4 + 3.1);
+  return lanesUs < 1.05 * matrixUs;
+}
+
+int launchLanesRoute(const ProductRoute& r, const MMArgs& m, hipStream_t s) {
+  const MMArgs t = shortSideOnRows(m);
+  if (r.cols == 2) return r.rows == 1 ? launchLanes<1, 2, 8>(t, s) : launchLanes<2, 2, 8>(t, s);
+  if (r.rows == 1) return launchLanes<1, 8, 8>(t, s);
+  if (r.rows == 2) return launchLanes<2, 8, 8>(t, s);
+  return r.waves == 4 ? launchLanes<4, 4, 4>(t, s) : launchLanes<4, 4, 8>(t, s);
+}
+
+ProductRoute routeOf(const MMArgs& m, bool vec4, bool vec4C) {
+  const ProductRoute lanes = lanesTile(m), matrix = matrixTile(m, vec4, vec4C);
+  return lanesRoute(m, lanes, matrix) && resultApart(m) ? lanes : matrix;
 }
 
 template <typename G>

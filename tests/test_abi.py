@@ -351,6 +351,20 @@ def test_conv_choose_fft_size():
     assert L.fbfft_conv_workspace_image(0, 4, 3, 5, 64, 64, 33, 3, 0) == 0
 
 
+# timed on both kernels (N points; matrix kernel / lanes): 11.5 / 17.1, 13.9 / 26.8, 19.9 / 26.1, 6.8 / 7.9, 16.9
+# / 27.9 us; 77.5 / 34.4, 15.7 / 13.8, 8.3 / 4.0, 20.2 / 13.8 us
+@pytest.mark.parametrize("I,J,K,N,kind", [
+    (253, 100, 2, 16, DIRECT), (369, 460, 1, 8, DIRECT), (198, 265, 1, 16, DIRECT), (80, 32, 3, 32, DIRECT),
+    (81, 28, 55, 32, DIRECT),
+    (1, 30, 323, 16, LANES), (27, 54, 24, 32, LANES), (9, 16, 5, 32, LANES), (18, 100, 17, 32, LANES)])
+def test_mm_route_is_the_faster_kernel(I, J, K, N, kind):
+    import torch
+    space = torch.empty(2 * (N // 2 + 1) * N * (I * K + K * J + I * J))
+    A, B, C = (t.view(d0, d1, N // 2 + 1, N, 2) for t, d0, d1 in zip(
+        space.split([2 * (N // 2 + 1) * N * n for n in (I * K, K * J, I * J)]), (I, K, I), (K, J, J)))
+    assert product_route(A, B, C, False, False)[0] == kind
+
+
 @pytest.mark.parametrize("I,J,K", [(16, 8, 8), (8, 16, 16), (32, 32, 32), (5, 3, 3), (150, 8, 8)])
 def test_mm_small_products_in_place_keep_the_kernels_that_read_first(I, J, K):
     """A small product goes to the kernel whose tiles are separate workgroups only where C lies
