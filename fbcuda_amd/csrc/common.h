@@ -132,8 +132,10 @@ int launchConvPass(int pass, int N, float* x, const int* xStride, const int* xSi
                    hipStream_t s);
 
 // small forward passes and input gradients, without transforms (conv_small.hip): whether a pass
-// that would run on N points is one, and its launch
+// that would run on N points is one, its estimated time (C planes in, M planes of OH x OW out), and its
+// launch
 bool runsSmall(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW);
+double convSmallMicroseconds(int pass, int B, int C, int M, int OH, int OW, int kH, int kW);
 int launchConvSmall(int pass, const float* x, const int* xStride, const int* xSize, const float* y,
                     const int* yStride, const int* ySize, float* out, const int* outStride, const int* outSize,
                     hipStream_t s);

@@ -1289,16 +1289,22 @@ inline GemmPlan planGemm(int bins, int I, int Jp, int Kp, int maxSplits) {
 
 constexpr int kAnySplits = 16;  // what planGemm cuts a reduction into at most
 
-// What a pass on windows takes: workspace and an estimate of its time.
+// What a pass on windows takes: workspace and two estimates of its time, the second for small passes.
 struct WindowsCost {
   size_t bytes;
-  double us;
+  double us, smallUs;
 };
 
 // The estimate: three launches, every spectrum value written and read once, and the
 // contraction's products over whole tiles - at the rate of one wave per SIMD where the waves
 // are fewer than that, and of whole rounds of two per SIMD in binGemmRegsWide.  Fitted to 6600
-// random layers of 64 and 128 points on one MI355X; it is within 20 % of nine in ten of them.
+// random layers of 64 and 128 points when only binGemmDirect, binGemmRegsWide and one tile of
+// binGemmRegsSplitK ran their contractions; of 4900 random passes of 8 us to 3 ms it is now within 20 % of
+// half, and 12 % high in the middle.  It is there to choose between sizes (passSize), whose
+// estimates share most of that.
+// The second estimate, for three launches of at most a few dozen us: a start each, spectra that
+// the caches hold, tiles and chains of slices of the kernel that runs.  Over 2600 random passes it is
+// within 9 % of nine in ten.
 template <int N>
 WindowsCost windowsCost(int I, int J, int K, bool outTiled, int maxSplits) {
   if (swapRoles(I, J, outTiled)) std::swap(I, J);
@@ -1312,6 +1318,11 @@ WindowsCost windowsCost(int I, int J, int K, bool outTiled, int maxSplits) {
   const long waves = plan.waves * plan.splits;
   const double idle = waves < 1024 ? 1024.0 / waves : wide ? (waves + 2047) / 2048 * 2048.0 / waves : 1.0;
   c.us = 15 + 0.14e-6 * 2 * c.bytes + (wide ? 0.055e-6 : 0.04e-6) * products * idle;
+  const bool tiles32 = plan.kind == GemmPlan::RegsSplitK;
+  const int rows = plan.kind == GemmPlan::RegsNarrow ? 16 : tiles32 || plan.kind == GemmPlan::RegsWide ? 32 : 64;
+  const int chain = tiles32 ? ceilDiv(plan.slicesPerSplit, 4) : plan.slicesPerSplit;
+  c.smallUs = (N == 8 ? 8.9 : N == 16 ? 10.7 : 15.3) + 0.46e-6 * c.bytes +
+              0.036e-6 * bins * roundUp(I, rows) * roundUp(Jp, tiles32 ? 32 : 64) * Kp + 0.3 * chain;
   return c;
 }
 
@@ -1517,7 +1528,7 @@ static WindowsCost windowsPass(int pass, int N, int B, int Cin, int Cout, int H,
                                int maxSplits) {
   int ty, tx;
   tileGrid(pass, N, H, W, kH, kW, &ty, &tx);
-  if ((long)B * ty * tx > (1L << 30)) return {0, 0};
+  if ((long)B * ty * tx > (1L << 30)) return {};
   int I, J, K;
   passDims(pass, B * ty * tx, Cin, Cout, &I, &J, &K);
   const bool outTiled = pass != 2 && ty * tx > 1;  // the weight gradient is never tiled
@@ -1607,25 +1618,31 @@ PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int k
 // They take the place of the transforms of the library's own choice of size, however a call comes
 // to that (size 0, by its name, or in place of a larger named size), so that equal sizes still
 // give equal bits; any other size that a call runs on is a transform of that size.
-// Both times are estimated: its chain of filter rows on the fullest CU (fitted to 190 random passes
-// of 2 to 5000 workgroups, within 25 % of all of them that take less than 30 us), and the three
+// Both times are estimated: its chain of filter rows on the fullest CU, and the three
 // launches as above, less the 3 us by which that estimate is high where they are shortest; it
 // has to be 15 % ahead.  us, transforms / sums: forward 9 x 5 x 8 x 7, 9 filters of 3 x 3 11.1 /
 // 3.8; 7 x 4 x 55 x 55, 10 of 2 x 2 28.9 / 5.9; 2 x 24 x 8 x 8, 338 of 2 x 2 11.9 / 4.6; 23 x 80 x 9 x 9, 25 of
 // 3 x 3 14.3 / 11.2; input gradient 47 x 11 x 10 x 11, 143 of 1 x 1 24.9 / 6.2; 2 x 45 x 12 x 12, 21 of 5
 // x 5 11.5 / 9.5.  Not there: 5 x 17 x 9 x 9, 15 of 7 x 7 11.9 / 15; 1 x 64 x 27 x 27, 192 of 5 x 5 16.3 / 23.
+// That leaves out a second round of workgroups on some CUs, loads whose lanes are in many images, and
+// loads of rows that a wave does not have: 81 x 12 x 6 x 6, 22 of 6 x 6 10.8 / 18.6; 25 x 59 x 5 x 5, 75 of 4 x 4
+// 14.4 / 23.8; input gradient 15 x 6 x 112 x 112, 2 of 2 x 9 28.7 / 41.5.
+// So a second pair of estimates (convSmallMicroseconds, smallUs) must not see them behind by more than
+// its error.  Of 4600 random passes of at most 400 images that the first pair sends there, 95 of them over 10
+// % slower than on transforms, 18 of those are left and 26 go back that were over 10 % faster.
 bool runsSmall(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
   const int C = pass == 0 ? Cin : Cout, M = pass == 0 ? Cout : Cin;
   if (pass == 2 || kW > 11 || (long)C * kH * kW > 2048) return false;
-  const double pixels = (double)B * (pass == 0 ? (double)(H - kH + 1) * (W - kW + 1) : (double)H * W);
-  const double full = std::max(1.0, std::ceil(pixels / 64) * ceilDiv(M, 8) / 256);
+  const int OH = pass == 0 ? H - kH + 1 : H, OW = pass == 0 ? W - kW + 1 : W;
+  const double full = std::max(1.0, std::ceil((double)B * OH * OW / 64) * ceilDiv(M, 8) / 256);
   if (full > 64) return false;
   const double chain = ceilDiv(C * kH, 8) * kW;
   const double sums = pass == 0 ? 3.1 + 0.88 * full + chain * (0.037 + 0.049 * full)
                                 : 3.5 + 0.51 * full + chain * (0.033 + (0.072 + 0.025 / kW) * full);
   if (N != fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW)) return false;
-  const double transforms = windowsPass(pass, N, B, Cin, Cout, H, W, kH, kW, kAnySplits).us;
-  return sums < 0.85 * (transforms - 3);
+  const WindowsCost transforms = windowsPass(pass, N, B, Cin, Cout, H, W, kH, kW, kAnySplits);
+  return sums < 0.85 * (transforms.us - 3) &&
+         convSmallMicroseconds(pass, B, C, M, OH, OW, kH, kW) < 1.07 * transforms.smallUs;
 }
 
 // Whether a pass may take that way: it reads its operands while it writes its result, where the

@@ -385,3 +385,16 @@ def test_mm_small_products_in_place_keep_the_kernels_that_read_first(I, J, K):
         assert product_route(A, B, operand(into, I, J, last - 4), False, False)[0] == DIRECT
         assert product_route(A, B, operand(into, I, J, last - 2), False, False)[0] == REGISTERS  # 8-byte aligned
         assert product_route(A, B, operand(into, I, J, last), False, False)[0] == LANES
+
+
+# timed both ways, transforms / sums: 10.8 / 18.6, 14.4 / 23.8, 13.5 / 18.9, 28.7 / 41.5 us; 11.1
+# / 3.8, 28.9 / 5.9, 24.9 / 6.2 us
+@pytest.mark.parametrize("pass_,B,cin,cout,H,W,kH,kW,small", [
+    (0, 81, 12, 22, 6, 6, 6, 6, False), (0, 25, 59, 75, 5, 5, 4, 4, False), (0, 71, 32, 15, 5, 5, 4, 4, False),
+    (1, 15, 6, 2, 112, 112, 2, 9, False),
+    (0, 9, 5, 9, 8, 7, 3, 3, True), (0, 7, 4, 10, 55, 55, 2, 2, True), (1, 47, 11, 143, 10, 11, 1, 1, True)])
+def test_small_layers_run_the_faster_way(pass_, B, cin, cout, H, W, kH, kW, small):
+    fn = F.lib()._ZN9fbfft_amd9runsSmallEiiiiiiiii
+    fn.argtypes, fn.restype = [ctypes.c_int] * 9, ctypes.c_bool
+    n = F.conv_choose_fft_size(pass_, B, cin, cout, H, W, kH, kW)
+    assert fn(pass_, n, B, cin, cout, H, W, kH, kW) == small
