@@ -140,6 +140,15 @@ int launchConvSmall(int pass, const float* x, const int* xStride, const int* xSi
                     const int* yStride, const int* ySize, float* out, const int* outStride, const int* outSize,
                     hipStream_t s);
 
+// what a pass of a caller's transform size runs on where its result overlaps no operand: convSmall,
+// plane-major spectra, or windows of N points with the contraction kernel Windows + GemmPlan::kind
+// (conv_pipeline.hip) and its reduction in so many ranges
+struct ConvRoute {
+  enum Kind { Small, PlaneMajor, Windows };
+  int kind, N, splits;
+};
+ConvRoute convRoute(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW);
+
 // the same passes for 64- and 128-point transforms (conv_split.hip)
 size_t convSplitWorkspaceBytes(int pass, int N, int B, int Cin, int Cout);
 int launchConvSplit(int pass, int N, float* x, const int* xStride, const int* xSize, float* y,

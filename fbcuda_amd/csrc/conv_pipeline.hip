@@ -1260,8 +1260,12 @@ inline GemmPlan planGemm(int bins, int I, int Jp, int Kp, int maxSplits) {
   // / 5.7, 768 8.8 / 6.8 (4.7 slices), but 1152 4.8 / 6.9 (1 slice; 6 slices, 1536: 13.2 / 11.1);
   // binGemmDirect<64> / 32 x 32 tiles: 384 (one image, 64 x 27 x 27, 192 of 5 x 5, 8 slices)
   // 7.9 / 7.6, 192 (10) 7.9 / 6.1, 128 (24) 14.6 / 8.0, 768 (21) 13.6 / 12.2, but 512 (5) 6.6 / 7.1.
+  // Not for up to 16 rows and three slices, where binGemmRegsNarrow is faster (500 random passes, 32 x 32
+  // tiles / it: one slice 1.07 in the middle and always slower, two 1.07, three 1.02; four and five 0.97
+  // to 1.10, six to ten 0.94).
   const long tiles = (long)bins * ceilDiv(I, 32) * ceilDiv(Jp, 32) * p.splits;
-  if ((p.kind == GemmPlan::RegsWide && (tiles <= 768 || (p.slicesPerSplit >= 6 && tiles <= 1536))) ||
+  if ((p.kind == GemmPlan::RegsWide && (I > 16 || p.slicesPerSplit >= 4) &&
+       (tiles <= 768 || (p.slicesPerSplit >= 6 && tiles <= 1536))) ||
       (p.kind == GemmPlan::Direct64 && p.slicesPerSplit >= 8 && tiles <= 768)) {
     p.kind = GemmPlan::RegsSplitK;
     p.IT = ceilDiv(I, 32);
@@ -1289,10 +1293,12 @@ inline GemmPlan planGemm(int bins, int I, int Jp, int Kp, int maxSplits) {
 
 constexpr int kAnySplits = 16;  // what planGemm cuts a reduction into at most
 
-// What a pass on windows takes: workspace and two estimates of its time, the second for small passes.
+// What a pass on windows takes: workspace, two estimates of its time, the second for small passes, and
+// its contraction.
 struct WindowsCost {
   size_t bytes;
   double us, smallUs;
+  GemmPlan plan;
 };
 
 // The estimate: three launches, every spectrum value written and read once, and the
@@ -1304,7 +1310,7 @@ struct WindowsCost {
 // estimates share most of that.
 // The second estimate, for three launches of at most a few dozen us: a start each, spectra that
 // the caches hold, tiles and chains of slices of the kernel that runs.  Over 2600 random passes it is
-// within 9 % of nine in ten.
+// within 10 % of nine in ten.
 template <int N>
 WindowsCost windowsCost(int I, int J, int K, bool outTiled, int maxSplits) {
   if (swapRoles(I, J, outTiled)) std::swap(I, J);
@@ -1312,6 +1318,7 @@ WindowsCost windowsCost(int I, int J, int K, bool outTiled, int maxSplits) {
   const int Ip = roundUp(I, SL), Jp = roundUp(J, SL), Kp = roundUp(K, 8);
   const GemmPlan plan = planGemm(bins, I, Jp, Kp, maxSplits);
   WindowsCost c;
+  c.plan = plan;
   c.bytes = sizeof(float2) * bins * ((size_t)Kp * Ip + (size_t)Kp * Jp + (size_t)plan.splits * I * Jp);
   const double products = (double)bins * roundUp(I, I <= 32 ? 32 : 64) * roundUp(Jp, 64) * Kp;
   const bool wide = I <= 32 && Jp > 32;  // what binGemmRegsWide runs, its small products apart
@@ -1319,9 +1326,10 @@ WindowsCost windowsCost(int I, int J, int K, bool outTiled, int maxSplits) {
   const double idle = waves < 1024 ? 1024.0 / waves : wide ? (waves + 2047) / 2048 * 2048.0 / waves : 1.0;
   c.us = 15 + 0.14e-6 * 2 * c.bytes + (wide ? 0.055e-6 : 0.04e-6) * products * idle;
   const bool tiles32 = plan.kind == GemmPlan::RegsSplitK;
-  const int rows = plan.kind == GemmPlan::RegsNarrow ? 16 : tiles32 || plan.kind == GemmPlan::RegsWide ? 32 : 64;
+  const bool narrow = plan.kind == GemmPlan::RegsNarrow;
+  const int rows = narrow ? 16 : tiles32 || plan.kind == GemmPlan::RegsWide ? 32 : 64;
   const int chain = tiles32 ? ceilDiv(plan.slicesPerSplit, 4) : plan.slicesPerSplit;
-  c.smallUs = (N == 8 ? 8.9 : N == 16 ? 10.7 : 15.3) + 0.46e-6 * c.bytes +
+  c.smallUs = (N == 8 ? 8.9 : N == 16 ? 10.7 : 15.3) - (narrow ? 0.5 : 0) + 0.46e-6 * c.bytes +
               0.036e-6 * bins * roundUp(I, rows) * roundUp(Jp, tiles32 ? 32 : 64) * Kp + 0.3 * chain;
   return c;
 }
@@ -1628,8 +1636,8 @@ PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int k
 // loads of rows that a wave does not have: 81 x 12 x 6 x 6, 22 of 6 x 6 10.8 / 18.6; 25 x 59 x 5 x 5, 75 of 4 x 4
 // 14.4 / 23.8; input gradient 15 x 6 x 112 x 112, 2 of 2 x 9 28.7 / 41.5.
 // So a second pair of estimates (convSmallMicroseconds, smallUs) must not see them behind by more than
-// its error.  Of 4600 random passes of at most 400 images that the first pair sends there, 95 of them over 10
-// % slower than on transforms, 18 of those are left and 26 go back that were over 10 % faster.
+// its error.  Of 2240 random passes that the first pair sends there 58 are over 10 % slower than on
+// transforms; 14 of those are left, the most 38 %, and 8 go back that were over 10 % faster.
 bool runsSmall(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
   const int C = pass == 0 ? Cin : Cout, M = pass == 0 ? Cout : Cin;
   if (pass == 2 || kW > 11 || (long)C * kH * kW > 2048) return false;
@@ -1660,6 +1668,14 @@ static bool smallMayRun(const float* x, const int* xStride, const int* xSize, co
   if ((out <= last(x, xStride, xSize) && x <= end) || (out <= last(y, yStride, ySize) && y <= end)) return false;
   const double images = 64.0 / ((double)outSize[2] * outSize[3]) + 2;
   return images * xStride[0] + (double)xSize[2] * xStride[2] + (double)xSize[3] * xStride[3] < (1 << 29);
+}
+
+ConvRoute convRoute(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
+  const PassSize size = passSize(pass, N, B, Cin, Cout, H, W, kH, kW);
+  if (runsSmall(pass, size.N, B, Cin, Cout, H, W, kH, kW)) return {ConvRoute::Small, size.N, 1};
+  if (size.N > 32) return {ConvRoute::PlaneMajor, size.N, 1};
+  const GemmPlan plan = windowsPass(pass, size.N, B, Cin, Cout, H, W, kH, kW, size.maxSplits).plan;
+  return {ConvRoute::Windows + plan.kind, size.N, plan.splits};
 }
 
 // pass 0: x = input [B][Cin][H][W], y = weight [Cout][Cin][kH][kW], out = output [B][Cout][oH][oW]

@@ -45,6 +45,24 @@ def product_route(A, B, C, conjA, conjB):
     return r.kind, r.rows, r.cols, r.waves
 
 
+class ConvRoute(ctypes.Structure):
+    _fields_ = [("kind", ctypes.c_int), ("N", ctypes.c_int), ("splits", ctypes.c_int)]
+
+
+# what a layer pass runs on: convSmall, plane-major spectra, or windows with binGemm<name>
+SMALL, PLANE_MAJOR, REGS_SPLIT_K, REGS_WIDE, REGS_NARROW, DIRECT64, DIRECT128, SPLIT = range(8)
+
+
+def conv_route(pass_, N, B, cin, cout, H, W, kH, kW=None):
+    """(kind, points, ranges of the reduction) of a layer pass named N points (0: the library's
+    choice), from the library's own host function (common.h)."""
+    fn = F.lib()._ZN9fbfft_amd9convRouteEiiiiiiiii
+    fn.argtypes, fn.restype = [ctypes.c_int] * 9, ConvRoute
+    kW = kH if kW is None else kW
+    r = fn(pass_, N or F.conv_choose_fft_size(pass_, B, cin, cout, H, W, kH, kW), B, cin, cout, H, W, kH, kW)
+    return r.kind, r.N, r.splits
+
+
 def dev():
     return torch.device("cuda:0")
 
