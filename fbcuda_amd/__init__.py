@@ -11,6 +11,7 @@ without the built library raises.
 import ctypes
 import os
 import struct
+import warnings
 
 from .params import FBFFTParameters, numHermitian  # noqa: F401
 
@@ -137,10 +138,18 @@ def _entry():
 _native = None
 
 
+class _General:
+    """In the place of a module that is not there: every call is made through _entry()."""
+
+    def __getattr__(self, name):
+        return lambda *args: NotImplemented
+
+
 def _load_native():
     """The entry points that small calls go through (csrc/binding.cpp): they fill the descriptors
     from the tensors themselves and return NotImplemented for anything but a plain call, which
-    the wrappers then make through _entry().  fbfft1D and fbifft1D of 4096 rows of 32 points, one
+    the wrappers then make through _entry(), as all of them are where the module is not built or, with
+    a warning, does not load.  fbfft1D and fbifft1D of 4096 rows of 32 points, one
     pass after the other: 10.3 us through _entry(), 6.2 us this way; fbfft2D and fbifft2D of 274
     planes of 8 x 8: 10.2 / 6.0 us."""
     global _native
@@ -149,8 +158,11 @@ def _load_native():
     try:
         from . import _binding
     except ImportError as e:
-        raise RuntimeError("fbcuda_amd/_binding.so cannot be loaded (%s): build it with `make -C "
-                           "fbcuda_amd/csrc`" % e) from e
+        if os.path.exists(os.path.join(_HERE, "_binding.so")):
+            warnings.warn("fbcuda_amd/_binding.so does not load (%s), small calls take longer: `make -C "
+                          "fbcuda_amd/csrc -B binding` builds it" % e, RuntimeWarning, stacklevel=3)
+        _native = _General()
+        return _native
     raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
     device = getattr(torch._C, "_cuda_getDevice", None)
     if raw and device:  # without them every call takes the general way

@@ -4,6 +4,9 @@ and the host-side mirror behaves like the reference's parameter class."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
+import warnings
 
 import numpy as np
 import pytest
@@ -409,3 +412,36 @@ def test_small_layers_run_the_faster_way(pass_, B, cin, cout, H, W, kH, kW, smal
     (2, 32, 8, 171, 20, 30, 30, 8, REGS_WIDE)])
 def test_contraction_of_a_short_side(pass_, N, B, cin, cout, H, W, k, kind):
     assert conv_route(pass_, N, B, cin, cout, H, W, k)[0] == kind
+
+
+def test_the_library_builds_without_python():
+    """The C ABI's own target needs hipcc only; the Python package's module is a target apart."""
+    csrc = os.path.join(ROOT, "fbcuda_amd", "csrc")
+    plan = subprocess.run(["make", "-C", csrc, "-n", "-B", "PYTHON=/nonexistent"], capture_output=True, text=True)
+    assert plan.returncode == 0 and "libfbfft_amd.so" in plan.stdout and "/nonexistent" not in plan.stderr
+    assert "binding" not in plan.stdout
+    assert "binding.cpp" in subprocess.run(["make", "-C", csrc, "-n", "-B", "binding"], capture_output=True,
+                                           text=True).stdout
+
+
+@pytest.mark.parametrize("built", [False, True])
+def test_calls_without_the_native_module_go_the_general_way(monkeypatch, tmp_path, built):
+    """Not built: the general way's results and errors, without a word; built and not loading: the
+    same, with a warning."""
+    import torch
+    monkeypatch.setattr(F, "_native", None)
+    monkeypatch.setattr(F, "_HERE", str(tmp_path))
+    monkeypatch.delattr(F, "_binding", raising=False)
+    monkeypatch.setitem(sys.modules, "fbcuda_amd._binding", None)
+    if built:
+        (tmp_path / "_binding.so").write_bytes(b"")
+    calls = []
+    monkeypatch.setattr(F, "_on_gpu", lambda *ts: calls.append("on_gpu"))
+    monkeypatch.setattr(F, "_stream", lambda stream: 0)
+    x, y = torch.zeros((2, 300)), torch.zeros((2, 151, 2))  # refused on the host, nothing is launched
+    with warnings.catch_warnings(record=True) as seen:
+        warnings.simplefilter("always")
+        assert F.fbfft1D(x, y) == F.UnsupportedSize
+        assert F.fbfft1D(x, y) == F.UnsupportedSize
+    assert calls == ["on_gpu"] * 2
+    assert [w.category for w in seen] == ([RuntimeWarning] if built else [])
