@@ -6,7 +6,8 @@ import torch
 
 import fbcuda_amd as F
 from fbcuda_amd import synth
-from gpu_util import LANES, check, TOL_CONV, TOL_FFT, dev, product_route, rel
+from gpu_util import (DIRECT, DIRECT64, LANES, REGISTERS, REGS_NARROW, TOL_CONV, TOL_FFT, check, conv_route, dev,
+                      product_route, rel)
 
 pytestmark = pytest.mark.gpu
 
@@ -308,7 +309,8 @@ def test_conv_split_path_strided_operands(oracle):
 @pytest.mark.parametrize("seed", range(24))
 def test_mm_random_shapes_and_views(oracle, seed):
     """Seeded random draw over I, J, K, the bin count, the role and accumulation,
-    with operands that are views into larger buffers (padded leading strides)."""
+    with operands that are views into larger buffers (padded leading strides).  Most run on
+    transposeMMLanesKernel; test_mm_matrix_kernels_random has such products on the matrix kernels."""
     rng = np.random.default_rng(3000 + seed)
     I, J, K = (int(v) for v in rng.integers(1, 140, 3))
     shape = (int(rng.integers(1, 10)), int(rng.integers(1, 20)))
@@ -335,7 +337,9 @@ def test_mm_random_shapes_and_views(oracle, seed):
 @pytest.mark.parametrize("seed", range(24))
 def test_conv_layer_random_shapes(oracle, seed):
     """All three passes on a seeded random layer (FFT size, image and filter
-    extents, plane counts), the input being a channel slice of a larger tensor."""
+    extents, plane counts), the input being a channel slice of a larger tensor.  Up to 32 points most
+    forward passes and input gradients are small enough to be summed without transforms;
+    test_gpu_conv_routes.py names layers for every contraction kernel."""
     rng = np.random.default_rng(4000 + seed)
     N = int(rng.choice([8, 16, 32, 64, 128], p=[0.2, 0.25, 0.3, 0.15, 0.1]))
     H, W = int(rng.integers(max(2, N // 2), N + 1)), int(rng.integers(max(2, N // 2), N + 1))
@@ -367,8 +371,9 @@ def test_conv_layer_random_shapes(oracle, seed):
 def test_conv_layer_random_shapes_many_planes(oracle, seed):
     """All three passes on seeded random layers whose plane counts (33 .. 72 images and
     output planes, 3 .. 40 input planes) put more than 32 rows on both sides of the
-    per-bin contraction: 64-row and 128-row tiles that lie inside the product whole next
-    to tiles that hang over its edges, reductions with and without a partial last slice."""
+    per-bin contraction of the forward pass, reductions with and without a partial last slice.  Most
+    forward passes and input gradients are summed without transforms; the 64-row and 128-row
+    tiles are in test_gpu_conv_routes.py."""
     rng = np.random.default_rng(5000 + seed)
     N = int(rng.choice([8, 16]))
     H, W = int(rng.integers(N // 2, N + 1)), int(rng.integers(N // 2, N + 1))
@@ -410,9 +415,9 @@ def test_conv_fprop_many_full_tiles(oracle, Cin):
 @pytest.mark.parametrize("K", [1, 2, 3, 4, 6, 7, 13])
 @pytest.mark.parametrize("shape", [(1, 2), (1, 8), (5, 2), (3, 8), (2, 17)])
 def test_mm_aligned_operands_k_tails(oracle, conjA, conjB, K, shape):
-    """Even bin counts in contiguous tensors take the kernel that copies slices of four
-    k straight into LDS: every remainder of K modulo four, bin counts below, at and
-    between multiples of the eight bins of a work item, tiles with clamped rows."""
+    """Even bin counts in contiguous tensors: every remainder of K modulo four, bin counts below, at
+    and between multiples of eight, rows beside the tiles' ends.  Products this small run on
+    transposeMMLanesKernel; test_mm_matrix_kernels_k_tails has them on the matrix kernels."""
     I, J = 70, 37
     xy = shape[0] * shape[1]
     A = synth.normal(((K, I) if conjA else (I, K)) + shape + (2,), seed=11 + K).numpy()
@@ -432,7 +437,8 @@ def test_mm_aligned_operands_k_tails(oracle, conjA, conjB, K, shape):
 
 @pytest.mark.parametrize("I,J,K,shape", [
     (128, 128, 5, (16, 32)),   # 512 work items of 64 x 32: two per CU, the larger tile
-    (128, 96, 6, (17, 32)),    # 408 of them: uneven, the smaller tile
+    (128, 96, 6, (17, 32)),    # 408 of them: 816 of the smaller would be as uneven
+    (128, 192, 5, (17, 32)),   # 816, 3.2 per CU: 1632 of the smaller tile are 6.4
 ])
 def test_mm_both_tile_shapes_of_the_aligned_path(oracle, I, J, K, shape):
     """The aligned path picks 64- or 32-row tiles by how evenly the work items spread
@@ -441,6 +447,7 @@ def test_mm_both_tile_shapes_of_the_aligned_path(oracle, I, J, K, shape):
     for conjA, conjB in ROLES[:2]:
         A = synth.normal(((K, I) if conjA else (I, K)) + shape + (2,), seed=21).numpy()
         B = synth.normal(((J, K) if conjB else (K, J)) + shape + (2,), seed=22).numpy()
+        assert route(A, B, I, J, conjA, conjB)[:2] == (DIRECT, 32 if J == 192 else 64)
         rc, got = mm(A, B, conjA, conjB, 0.5)
         assert rc == F.Success
         want = oracle.transpose_mm(A.reshape(A.shape[0], A.shape[1], xy, 2),
@@ -450,10 +457,9 @@ def test_mm_both_tile_shapes_of_the_aligned_path(oracle, I, J, K, shape):
 
 @pytest.mark.parametrize("seed", range(10))
 def test_mm_random_aligned_shapes(oracle, seed):
-    """Seeded random draw over contiguous operands with an even bin count (the kernel that
-    copies slices straight into LDS): I and J from below one tile to several, so that tiles
-    inside C whole - stored from a scalar base without tests - meet tiles that hang over its
-    last rows, columns or bins; every role, with and without accumulation."""
+    """Seeded random draw over contiguous operands with an even bin count: I and J from below one
+    tile to several; every role, with and without accumulation.  Most run on transposeMMLanesKernel;
+    test_mm_matrix_kernels_random has such products on the matrix kernels."""
     rng = np.random.default_rng(6000 + seed)
     I, J, K = int(rng.integers(20, 200)), int(rng.integers(20, 200)), int(rng.integers(1, 80))
     shape = (int(rng.integers(1, 6)), 2 * int(rng.integers(1, 9)))
@@ -493,9 +499,8 @@ def test_conv_fprop_batch_beyond_a_16_bit_grid_index(oracle):
     assert rel(oh[coords[:, 0], coords[:, 1], coords[:, 2], coords[:, 3]], want) < TOL_CONV
 
 
-# the contraction of small products, a 32 x 32 tile per workgroup: either side on the rows, ends of
-# the tiles, a long reduction on two rows of tiles (binGemmDirect's shape) and on one
-# (binGemmRegsWide's), with and without a reduction cut into ranges
+# small layers: most of these are summed without transforms (the contraction of small products, a 32 x 32
+# tile per workgroup, is in test_gpu_conv_routes.py)
 @pytest.mark.parametrize("N,H,k,Bn,Cin,Cout", [
     (8, 8, 3, 33, 80, 34), (8, 7, 2, 65, 88, 48), (8, 8, 3, 5, 9, 40), (8, 8, 3, 32, 81, 33),
     (16, 14, 5, 3, 200, 65), (16, 16, 7, 40, 12, 9), (8, 8, 4, 2, 300, 70)])
@@ -507,10 +512,17 @@ def test_conv_fprop_small_products(oracle, N, H, k, Bn, Cin, Cout):
     assert rel(got, oracle.corr2d_valid(x, w)) < 1e-6
 
 
-def mm_vs_fp64(oracle, conjA, conjB, I, J, K, shape, tol):
+def route(A, B, I, J, conjA, conjB):
+    """(kernel, rows, columns, waves) of a product of contiguous operands."""
+    C = torch.empty((I, J) + A.shape[2:])
+    return product_route(torch.from_numpy(A), torch.from_numpy(B), C, conjA, conjB)
+
+
+def mm_vs_fp64(oracle, conjA, conjB, I, J, K, shape, tol, kinds):
     xy = shape[0] * shape[1]
     A = synth.normal(((K, I) if conjA else (I, K)) + shape + (2,), seed=1).numpy()
     B = synth.normal(((J, K) if conjB else (K, J)) + shape + (2,), seed=2).numpy()
+    assert route(A, B, I, J, conjA, conjB)[0] in kinds
     rc, got = mm(A, B, conjA, conjB, 0.125)
     assert rc == F.Success
     want = oracle.transpose_mm64(A.reshape(A.shape[0], A.shape[1], xy, 2),
@@ -527,7 +539,7 @@ def mm_vs_fp64(oracle, conjA, conjB, I, J, K, shape, tol):
 def test_mm_lanes(oracle, conjA, conjB, I, J, K, shape):
     # one multiply-add per k in each wave and a short sum: at most sqrt(2 K) roundings of 2^-24
     # of a sum that grows like the square root of K
-    mm_vs_fp64(oracle, conjA, conjB, I, J, K, shape, np.sqrt(2 * K + 8) * 2.0 ** -24)
+    mm_vs_fp64(oracle, conjA, conjB, I, J, K, shape, np.sqrt(2 * K + 8) * 2.0 ** -24, (LANES,))
 
 
 # C in the place of A (J <= 32) or of B (I <= 32), on sizes that run on transposeMMLanesKernel elsewhere:
@@ -555,14 +567,62 @@ def test_mm_in_place(oracle, I, J, odd):
     (129, 143, 6, (17, 32), 0), (66, 193, 13, (17, 32), 1), (130, 140, 5, (1, 543), 2),
     (129, 131, 6, (1, 545), 0), (193, 66, 9, (1, 543), 1)])
 def test_mm_matrix_kernels_ragged(oracle, I, J, K, shape, role):
-    mm_vs_fp64(oracle, *ROLES[role], I, J, K, shape, TOL_FFT / 10)
+    mm_vs_fp64(oracle, *ROLES[role], I, J, K, shape, TOL_FFT / 10, (DIRECT, REGISTERS))
+
+
+def on_matrix_kernels(oracle, conjA, conjB, I, J, K, shape, accumulate, kind):
+    """A product whose C lies between the rows of A in one buffer, which keeps it on the matrix
+    kernels however small it is; the buffer's other elements stay."""
+    xy = shape[0] * shape[1]
+    rows, cols = (K, I) if conjA else (I, K)
+    space = synth.normal((max(rows, I), J + cols) + shape + (2,), seed=61).to(dev())
+    B = synth.normal(((J, K) if conjB else (K, J)) + shape + (2,), seed=62).to(dev())
+    A, C = space[:rows, J:], space[:I, :J]
+    assert product_route(A, B, C, conjA, conjB)[0] == kind
+    before = space.cpu().numpy().copy()
+    assert F.transposeMM(A, B, C, 0.25, conjA, conjB, accumulate) == F.Success
+    torch.cuda.synchronize()
+    after = space.cpu().numpy()
+    want = oracle.transpose_mm64(before[:rows, J:].reshape(rows, cols, xy, 2),
+                                 B.cpu().numpy().reshape(B.shape[0], B.shape[1], xy, 2), conjA, conjB, 0.25)
+    if accumulate:
+        want = want + 0.25 * before[:I, :J].reshape(I, J, xy, 2).astype(np.float64)
+    # a rounding of at most 2^-24 per two k (and for C) of three sums of up to twice the result
+    assert rel(after[:I, :J].reshape(I, J, xy, 2), want) < (np.sqrt(K) + 2) * 2.0 ** -24
+    after[:I, :J] = before[:I, :J]
+    assert np.array_equal(after, before)
+
+
+# every remainder of K modulo the four of a slice, bin counts below, at and between multiples of the eight of
+# a work item, clamped rows and columns; odd bin counts on the register path
+@pytest.mark.parametrize("conjA,conjB", ROLES)
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 6, 7, 13])
+@pytest.mark.parametrize("shape,kind", [((1, 2), DIRECT), ((1, 8), DIRECT), ((5, 2), DIRECT), ((3, 8), DIRECT),
+                                        ((2, 17), DIRECT), ((1, 5), REGISTERS), ((3, 5), REGISTERS)])
+def test_mm_matrix_kernels_k_tails(oracle, conjA, conjB, K, shape, kind):
+    for accumulate in (False, True):
+        on_matrix_kernels(oracle, conjA, conjB, 70, 37, K, shape, accumulate, kind)
+
+
+@pytest.mark.parametrize("seed", range(24))
+def test_mm_matrix_kernels_random(oracle, seed):
+    """I and J from below one tile to several, so that tiles inside C whole - stored from a scalar base
+    without tests - meet tiles that hang over its last rows, columns or bins."""
+    rng = np.random.default_rng(7000 + seed)
+    I, J, K = int(rng.integers(2, 200)), int(rng.integers(2, 200)), int(rng.integers(1, 80))
+    shape = (int(rng.integers(1, 6)), int(rng.integers(1, 18)))
+    conjA, conjB = ROLES[int(rng.integers(0, 3))]
+    on_matrix_kernels(oracle, conjA, conjB, I, J, K, shape, bool(rng.integers(0, 2)),
+                      REGISTERS if shape[0] * shape[1] % 2 else DIRECT)
 
 
 # binGemmRegsNarrow: 1 to 16 rows (either operand on them), columns beside the end of a wave's 64
 # and of its two halves, one slice of k and an odd number
 @pytest.mark.parametrize("Bn,Cin,Cout", [
-    (70, 9, 1), (65, 17, 5), (129, 40, 16), (97, 3, 15), (2, 24, 64), (16, 25, 127), (1, 8, 96)])
+    (70, 9, 1), (65, 17, 5), (129, 40, 16), (97, 3, 15), (8, 24, 64), (16, 25, 127), (1, 8, 96),
+    (2, 24, 64)])  # (the last on 16-point windows and 64-row tiles)
 def test_conv_fprop_up_to_16_rows(oracle, Bn, Cin, Cout):
+    assert conv_route(0, 32, Bn, Cin, Cout, 30, 31, 11, 12)[0] == (DIRECT64 if Bn == 2 else REGS_NARROW)
     x = synth.normal((Bn, Cin, 30, 31), seed=30).numpy()
     w = synth.normal((Cout, Cin, 11, 12), seed=31, std=0.02).numpy()
     rc, got = conv(x, w, 32)
