@@ -9,7 +9,7 @@ import torch
 
 import fbcuda_amd as F
 from fbcuda_amd import synth
-from gpu_util import dev, pass_size, rel
+from gpu_util import SMALL, conv_route, dev, pass_size, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -32,7 +32,7 @@ def workspace(B, cin, cout, H, W, k):
                        dtype=torch.uint8, device=dev())
 
 
-# every filter width; pixels and planes that do not fill the last workgroup, several images to a
+# forward, every filter width, and the input gradient of those of them that it is summed for, too; pixels and planes that do not fill the last workgroup, several images to a
 # workgroup, fewer filter rows than waves, one plane on either side
 @pytest.mark.parametrize("B,cin,cout,H,W,k", [
     (3, 7, 9, 8, 9, 1), (5, 10, 8, 7, 8, 2), (9, 5, 9, 8, 7, 3), (2, 4, 17, 11, 23, 4),
@@ -55,6 +55,47 @@ def test_both_passes_vs_fp64(oracle, B, cin, cout, H, W, k):
         assert F.conv_bprop(g.to(d), w.to(d), gi, 0, ws) == F.Success
         torch.cuda.synchronize()
         assert rel(gi.cpu().numpy(), oracle.corr2d_grad_input(g.numpy(), w.numpy(), H, W)) < bar(cout * k * k)
+
+
+# input gradients of the filter widths that are left, sides that differ, and as many filter values as LDS holds
+@pytest.mark.parametrize("B,cin,cout,H,W,kH,kW", [
+    (11, 4, 2, 7, 7, 6, 6), (1, 61, 3, 28, 28, 9, 9), (4, 42, 3, 23, 23, 10, 10), (14, 3, 4, 33, 33, 11, 11),
+    (3, 7, 9, 14, 13, 1, 5), (2, 9, 17, 20, 16, 7, 2), (3, 7, 9, 14, 13, 3, 11), (2, 9, 17, 20, 16, 11, 1),
+    (2, 9, 17, 20, 16, 2, 9), (3, 7, 9, 14, 13, 5, 4), (1, 8, 2048, 6, 6, 1, 1)])
+def test_input_gradient_and_sides_that_differ_vs_fp64(oracle, B, cin, cout, H, W, kH, kW):
+    d = dev()
+    x, w = synth.normal((B, cin, H, W), seed=30), synth.normal((cout, cin, kH, kW), seed=31)
+    g = synth.normal((B, cout, H - kH + 1, W - kW + 1), seed=32)
+    ws = torch.empty(max(F.conv_workspace_image(p, B, cin, cout, H, W, kH, kW, 0) for p in (0, 1)),
+                     dtype=torch.uint8, device=d)
+    # (61 and 42 input planes: the forward pass has too many taps)
+    assert [conv_route(p, 0, B, cin, cout, H, W, kH, kW)[0] == SMALL for p in (0, 1)] == [cin < 42, True]
+    gi, out = torch.full(tuple(x.shape), float("nan"), device=d), torch.full(tuple(g.shape), float("nan"), device=d)
+    assert F.conv_bprop(g.to(d), w.to(d), gi, 0, ws) == F.Success
+    assert F.conv_fprop(x.to(d), w.to(d), out, 0, ws) == F.Success
+    torch.cuda.synchronize()
+    assert rel(gi.cpu().numpy(), oracle.corr2d_grad_input(g.numpy(), w.numpy(), H, W)) < bar(cout * kH * kW)
+    assert rel(out.cpu().numpy(), oracle.corr2d_valid(x.numpy(), w.numpy())) < bar(cin * kH * kW)
+
+
+def test_infinite_filter_value_in_an_input_gradient(oracle):
+    """What the padding around a gradient meets counts as zero times the filter, so an infinite filter
+    value makes every element of its input plane infinite or not a number, and nothing else."""
+    B, cin, cout, H, k = 3, 7, 5, 9, 3
+    d = dev()
+    w, g = synth.normal((cout, cin, k, k), seed=31).to(d), synth.normal((B, cout, H - 2, H - 2), seed=32).to(d)
+    ws = workspace(B, cin, cout, H, H, k)
+    assert runs_small(1, B, cin, cout, H, H, k)
+    results = []
+    for value in (0.5, float("inf")):
+        w[1, 4, 0, 2] = value
+        gi = torch.empty((B, cin, H, H), device=d)
+        assert F.conv_bprop(g, w, gi, 0, ws) == F.Success
+        results.append(gi)
+    torch.cuda.synchronize()
+    others = torch.arange(cin, device=d) != 4
+    assert torch.equal(results[0][:, others], results[1][:, others])
+    assert not bool(torch.isfinite(results[1][:, 4]).any())
 
 
 def test_strided_views(oracle):

@@ -6,21 +6,24 @@ import torch
 
 import fbcuda_amd as F
 from fbcuda_amd import synth
-from gpu_util import dev
+from gpu_util import DIRECT64, SMALL, conv_route, dev
 
 pytestmark = pytest.mark.gpu
 
 
-def test_graph_capture_of_the_convolution_layer_and_transforms():
+# a layer whose forward pass and input gradient need no workspace, and one that goes through it
+@pytest.mark.parametrize("B,cin,cout,kind", [(8, 6, 10, SMALL), (64, 40, 48, DIRECT64)])
+def test_graph_capture_of_the_convolution_layer_and_transforms(B, cin, cout, kind):
     d = dev()
-    x = synth.normal((8, 6, 27, 27), seed=30, device=d)
-    w = synth.normal((10, 6, 5, 5), seed=31, std=0.02, device=d)
-    g = synth.normal((8, 10, 23, 23), seed=32, device=d)
+    assert [conv_route(p, 32, B, cin, cout, 27, 27, 5)[0] for p in (0, 1)] == [kind] * 2
+    x = synth.normal((B, cin, 27, 27), seed=30, device=d)
+    w = synth.normal((cout, cin, 5, 5), seed=31, std=0.02, device=d)
+    g = synth.normal((B, cout, 23, 23), seed=32, device=d)
     planes = synth.normal((300, 32, 32), seed=1, device=d)
     out, gi, gw = torch.empty_like(g), torch.empty_like(x), torch.empty_like(w)
     spec = torch.empty((300, 17, 32, 2), device=d)
     back = torch.empty_like(planes)
-    ws = [torch.empty(F.conv_workspace(p, 8, 6, 10, 32), dtype=torch.uint8, device=d) for p in range(3)]
+    ws = [torch.empty(F.conv_workspace(p, B, cin, cout, 32), dtype=torch.uint8, device=d) for p in range(3)]
 
     def run():
         assert F.conv_fprop(x, w, out, 32, ws[0]) == F.Success

@@ -8,7 +8,7 @@ import torch
 
 import fbcuda_amd as F
 from fbcuda_amd import synth
-from gpu_util import TOL_CONV, dev, rel
+from gpu_util import REGS_NARROW, SMALL, TOL_CONV, conv_route, dev, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -53,12 +53,15 @@ def test_static_scratch_matches_workspace_form(oracle):
     assert rel(out.cpu().numpy(), want64) < TOL_CONV
 
 
-def test_static_scratch_under_graph_capture_and_without_allocation():
+# a layer summed without transforms, and one whose spectra fill the scratch
+@pytest.mark.parametrize("B,Cin,Cout,kind", [(6, 10, 12, SMALL), (16, 24, 40, REGS_NARROW)])
+def test_static_scratch_under_graph_capture_and_without_allocation(B, Cin, Cout, kind):
     """After one eager call (which looks the array up) the entry point can be captured into
     a HIP graph, every replay equals the workspace form on the inputs of that moment, and
     device memory in use is the same before and after the calls."""
     d = dev()
-    B, Cin, Cout, H, W, k, N = 6, 10, 12, 27, 25, 5, 32
+    H, W, k, N = 27, 25, 5, 32
+    assert conv_route(0, N, B, Cin, Cout, H, W, k)[0] == kind
     x, w = _layer(B, Cin, Cout, H, W, k, 60)
     out = torch.full((B, Cout, H - k + 1, W - k + 1), float("nan"), device=d)
     empty_x = torch.zeros((0, Cin, H, W), device=d)
