@@ -1004,9 +1004,10 @@ __global__ __launch_bounds__(kT, 4) void binGemmRegsNarrow(GemmArgs g) {
 // The same product on the bf16 matrix instructions, for products that outweigh their operands
 // (planGemm).  fp32 matrix instructions are what bounds
 // binGemmDirect there (155 TFLOP/s); the bf16 ones run at 1600 to 1750 on random operands (the power
-// limit; 2400 on zeros).  An fp32 value is the sum of three bf16 values without remainder,
-// a = a0 + a1 + a2: the upper half of its bits, the remainder rounded to 8 bits, and what is
-// left, which has at most 8.  Of the nine products of pieces the six largest are formed; the
+// limit; 2400 on zeros).  An fp32 value of 2^-110 or more is the sum of three bf16 values without
+// remainder, a = a0 + a1 + a2: the upper half of its bits, the remainder rounded to 8 bits, and what is
+// left, which has at most 8.  (Below, the last piece ends at bf16's smallest subnormal, 2^-133: images of
+// 2^-100 and 2^-108 2.1e-7 from 64 bits, 2^-116 4.1e-7.  An infinity comes out as NaN.)  Of the nine products of pieces the six largest are formed; the
 // three dropped ones are below 2^-23 |a b| each and of either sign, products of pieces
 // are exact in fp32, and a sum is rounded once per 16 k and product of pieces where the
 // fp32 instructions round every 2 k.  Against 64 bits over random operands: K = 64 1.1e-7, K =

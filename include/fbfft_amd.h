@@ -244,6 +244,13 @@ size_t fbfft_make_tiles_for_pass(int pass, const fbfft_tensor* input, const fbff
  * FFTIteratedConvolution, fbfft/FFTIteratedConvolution.cuh:71-88), and the
  * windows ride through the same three kernels as extra images (forward pass,
  * input gradient) or extra reduction steps (weight gradient).
+ * Range: where the contraction outweighs its operands they are multiplied as three bf16 pieces each,
+ * as exactly as fp32 products for spectra of 2^-110 and more; a spectrum value below that is off by up
+ * to 2^-133.  Values that are not finite: an image's reaches every output whose taps meet it and no other
+ * image's outputs, a filter's likewise no other output plane (input gradient: input plane).  Which other
+ * elements of its own image or plane it reaches, and whether as infinity or NaN, depends on the way the
+ * pass runs: all of a window's with transforms, with sums those whose taps meet it, the zeros around a
+ * gradient counting as taps.
  * workspace: device memory of at least fbfft_conv_workspace_image() bytes for
  * that pass and image size (fbfft_conv_workspace() when H, W <= fftSize),
  * 256-byte aligned; its contents need not survive between calls. */

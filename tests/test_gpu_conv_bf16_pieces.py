@@ -1,12 +1,13 @@
 """Layers whose contraction splits its fp32 operands into bf16 pieces (binGemmSplit: 48 k or
-more, at least 38 products per spectrum value, two 64 x 64 tiles per CU), against the fp64 direct convolution."""
+more, at least 38 products per spectrum value, two 64 x 64 tiles per CU), against the fp64 direct convolution.
+(Input gradients, weight gradients and reductions in ranges: test_gpu_conv_routes.py.)"""
 import numpy as np
 import pytest
 import torch
 
 import fbcuda_amd as F
 from fbcuda_amd import synth
-from gpu_util import check, dev
+from gpu_util import SPLIT, check, conv_route, dev
 
 pytestmark = pytest.mark.gpu
 
@@ -20,6 +21,7 @@ def bar(K):
 
 def layer(N, B, cin, cout, H, k, scale=1.0):
     d = dev()
+    assert conv_route(0, N, B, cin, cout, H, H, k)[0] == SPLIT
     x = synth.normal((B, cin, H, H), seed=30).to(d) * scale
     w = synth.normal((cout, cin, k, k), seed=31, std=0.05).to(d)
     ws = torch.empty(F.conv_workspace(0, B, cin, cout, N), dtype=torch.uint8, device=d)
@@ -55,3 +57,15 @@ def test_pieces_scale_exactly(exponent):
     a = layer(16, 128, 128, 128, 15, 2)[2]
     b = layer(16, 128, 128, 128, 15, 2, 2.0 ** exponent)[2]
     assert torch.equal(a * 2.0 ** exponent, b)
+
+
+@pytest.mark.parametrize("exponent", [-100, -108, -116])
+def test_pieces_of_small_values(oracle, exponent):
+    """A piece that falls below the smallest normal number may be cut to zero: a spectrum value is off by
+    at most 2^-126 then, nothing against 2^-100, a 2^-14 of a spectrum of 15 x 15 values of 2^-116."""
+    N, B, cin, cout, H, k = 16, 272, 64, 160, 15, 2
+    x, w, out = layer(N, B, cin, cout, H, k, 2.0 ** exponent)
+    n = [0, 100, B - 1]
+    want = oracle.corr2d_valid((x[n].double() * 2.0 ** -exponent).float().cpu().numpy(), w.cpu().numpy())
+    got = out[n].double().cpu().numpy() * 2.0 ** -exponent
+    check("values of 2^%d" % exponent, got, want, bar(cin) + 2.0 ** -126 / (15 * 2.0 ** exponent))
