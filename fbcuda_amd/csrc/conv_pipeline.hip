@@ -1260,7 +1260,9 @@ inline GemmPlan planGemm(int bins, int I, int Jp, int Kp, int maxSplits) {
   // its chain in four.  us, binGemmRegsWide / 32 x 32 tiles: 192 workgroups 8.4 / 4.8, 384 7.9
   // / 5.7, 768 8.8 / 6.8 (4.7 slices), but 1152 4.8 / 6.9 (1 slice; 6 slices, 1536: 13.2 / 11.1);
   // binGemmDirect<64> / 32 x 32 tiles: 384 (one image, 64 x 27 x 27, 192 of 5 x 5, 8 slices)
-  // 7.9 / 7.6, 192 (10) 7.9 / 6.1, 128 (24) 14.6 / 8.0, 768 (21) 13.6 / 12.2, but 512 (5) 6.6 / 7.1.
+  // 7.9 / 7.6, 192 (10) 7.9 / 6.1, 128 (24) 14.6 / 8.0, 768 (21) 13.6 / 12.2, but 512 (5) 6.6 / 7.1.  Whole
+  // passes, 300 random products that leave binGemmDirect<64> this way: 0.96 of the time in the middle up to ten
+  // slices, 0.90 above, two of 768 tiles 3 % longer.
   // Not for up to 16 rows and three slices, where binGemmRegsNarrow is faster (500 random passes, 32 x 32
   // tiles / it: one slice 1.07 in the middle and always slower, two 1.07, three 1.02; four and five 0.97
   // to 1.10, six to ten 0.94).
@@ -1275,13 +1277,16 @@ inline GemmPlan planGemm(int bins, int I, int Jp, int Kp, int maxSplits) {
   // up to 16 rows: 91 random products 0.97 to 2.2 times as fast as on 32-row tiles
   if (p.kind == GemmPlan::RegsWide && I <= 16) p.kind = GemmPlan::RegsNarrow;
   // binGemmSplit where the products outweigh the operands by enough: each spectrum value enters
-  // I J K / (I J + I K + J K) complex products.  Whole layers on a loaded chip, three passes
+  // I J K / (I J + I K + J K) complex products.  Whole layers, three passes
   // back to back, binGemmDirect / this by that quotient: 93 (66 x 273 x 25 x 26, 307 of 2 x 2)
   // 761 / 708 us; 43 (128 x 128 x 28 x 28, 128 of 5 x 5) 367 / 354; 38 (180 x 65 x 12 x 20, 195 of
   // 10 x 10) 394 / 369; below, the launch waits for memory, splitting has few products to
-  // pay for it and the bf16 instructions' power slows the transforms around them: 37 (128 x 64
-  // x 28 x 28, 256 of 5 x 5) 416 / 423, 35 (the 27 x 27 layer) 324 / 332, 28 (64 x 64 x 30 x 30, 64 of 4
-  // x 4) 151 / 160.  And not with fewer workgroups than two per CU (2 x 178 x 38 x 46, 33 of 5
+  // pay for it and the bf16 instructions' power slows the transforms around them on a chip that has
+  // been loaded for long: 37 (128 x 64 x 28 x 28, 256 of 5 x 5) 416 / 423, 35 (the 27 x 27 layer) 324 / 332, 28
+  // (64 x 64 x 30 x 30, 64 of 4 x 4) 151 / 160.  In runs of a few ms, which do not reach that limit, 230
+  // random layers take 0.98 of binGemmDirect's time in the middle at 18 to 24 (0.93 to 1.03), 0.96 at 28
+  // to 32, 0.94 at 36 to 40 and 0.89 from 55 up, none above 28 longer: the line lies where
+  // neither kind of run loses.  And not with fewer workgroups than two per CU (2 x 178 x 38 x 46, 33 of 5
   // x 5, 128 workgroups: 13.9 / 16.5) or ranges of fewer than 48 k.
   if ((p.kind == GemmPlan::Direct64 || p.kind == GemmPlan::Direct128) && p.slicesPerSplit >= 6 &&
       1.0 / I + 1.0 / Jp + 1.0 / Kp <= 1.0 / 38 &&
