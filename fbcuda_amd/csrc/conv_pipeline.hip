@@ -913,9 +913,9 @@ __global__ __launch_bounds__(kT, 3) void binGemmRegsWide(GemmArgs g) {
 // ... and for up to 16 rows: the same on v_mfma_f32_16x16x4_f32.  A wave owns 16 rows x 64
 // columns; lane (c, q) loads 16 bytes of B per four k - columns j0 + 2c and j0 + 2c + 1 at k = q - of
 // either half of the columns, and 8 bytes of A.  The matrix work of 16 rows that are not there
-// is what bounded the 32-row form: us, 201 x 74 x 17 x 14 images, 9 filters of 8 x 8, input gradient
-// 34.6 -> 16.0; 27 x 4 x 100 x 100, 152 of 9 x 9, input gradient 103.5 -> 58.0; 15 x 7 x 111 x 111, 372
-// of 9 x 9, forward 168.7 -> 139.5.
+// is what bounded the 32-row form: us, 201 x 74 x 17 x 14 images, 9 filters of 8 x 8, named 32 points, weight
+// gradient 35.4 -> 16.9; 27 x 4 x 100 x 100, 152 of 9 x 9, weight gradient 109.8 -> 57.6, input gradient
+// 105.8 -> 85.8.
 struct GemmSliceNarrow {
   float2 a[2];
   float4 b[2][2];
@@ -1023,8 +1023,8 @@ __global__ __launch_bounds__(kT, 4) void binGemmRegsNarrow(GemmArgs g) {
 // (fewer workgroups per CU); each wave splitting what it reads, from the stages that
 // global_load_lds fills, 25 % slower.
 // us per launch, binGemmDirect / this: 128 x 192 x 64 over 512 bins 53.6 / 47.2; 264 x 307 x 273
-// over 128 193 / 161; without its matrix instructions the latter takes 104, without its
-// stores 156, without the splits 146.
+// over 128 194 / 149 to 161; of 161, 104 are left without its matrix instructions, 156 without its stores,
+// 146 without the splits.
 typedef __bf16 Bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned Quad __attribute__((ext_vector_type(4)));
 typedef unsigned Duo __attribute__((ext_vector_type(2)));
@@ -1558,7 +1558,8 @@ size_t convWorkspaceBytes(int pass, int N, int B, int Cin, int Cout, int H, int 
 }
 
 // The same estimate for plane-major spectra of N = 64 or 128 points (conv_split.hip), where
-// transposeMM takes 4 k at a time.
+// transposeMM's matrix kernels take 4 k at a time (of 700 random layers it is within 20 % of 63 in 100, 10 % high
+// in the middle).
 static double planeMajorMicroseconds(int pass, int N, int B, int Cin, int Cout) {
   int I, J, K;
   passDims(pass, B, Cin, Cout, &I, &J, &K);
@@ -1585,9 +1586,12 @@ static double planeMajorMicroseconds(int pass, int N, int B, int Cin, int Cout) 
 // 128 points, 93 x 193 x 122 x 119, 41 of 8 x 8 1360 / 1772 us), and where the planned ranges
 // lack a little room (128 points, 153 x 3 x 73 x 70, 33 of 2 x 2: plane-major 308, 1 range 528,
 // the 15 that fit 212 us; 64 points, 85 x 32 x 33 x 61, 66 of 7 x 7: 124, 1 range 241, the 3
-// that fit 173 us, so plane-major).  Of 6570 random layers whose windows fit, 12 take over 3 %
+// that fit 173 us, so plane-major).  Of 6570 random layers whose windows fit, 12 took over 3 %
 // longer than plane-major by this rule (at most 18 %), 7 over 10 % longer than on windows; by
-// the spectrum alone 59 take over 3 % longer, at most 45 %.  Filters larger than 32 or filling
+// the spectrum alone 59 took over 3 % longer, at most 45 %.  (Times and counts are those of the kernels
+// that the estimates were fitted to.  On the present ones 699 of 700 random layers whose windows fit with
+// all ranges run on windows, none of them over 3 % longer than plane-major, and the other is 18 % faster
+// there; the 85 x 32 x 33 x 61 layer takes 128 / 126, 36 x 18 x 56 x 62, 107 of 8 x 8, 88 / 125.)  Filters larger than 32 or filling
 // most of a window stay plane-major.
 //
 // 16 and 32 points are the same kernels on either side, and a caller who names them may mean
@@ -1608,7 +1612,10 @@ static double planeMajorMicroseconds(int pass, int N, int B, int Cin, int Cout) 
 // 1 x 1 14.8 / 16.4; weight gradient 4 x 310 x 25 x 25, 175 of 6 x 6 38.9 / 49.3): there the
 // estimates must not differ by more than 5 % to the windows' disadvantage, either.  Of 5790
 // random layers below the line 223 took over 3 % longer on 8 points and 66 over 10 %; by both
-// tests 92 and 17 (30 x 243 x 14 x 11, 245 of 4 x 4, input gradient 47.2 / 59.0 the most).
+// tests 92 and 17 (30 x 243 x 14 x 11, 245 of 4 x 4, input gradient 47.2 / 59.0 the most).  With the
+// contractions as they are now the second test keeps back more than it should: of 900 random layers below
+// the line two take over 3 % longer on 8 points (11 % the most), and of the 127 that it keeps on 16 all would
+// be 10 to 40 % faster; but the last of the three passes above takes 39.4 / 50.0.
 PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
   const PassSize named{N, kAnySplits};
   const int n = fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW);
@@ -1634,10 +1641,9 @@ PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int k
 // give equal bits; any other size that a call runs on is a transform of that size.
 // Both times are estimated: its chain of filter rows on the fullest CU, and the three
 // launches as above, less the 3 us by which that estimate is high where they are shortest; it
-// has to be 15 % ahead.  us, transforms / sums: forward 9 x 5 x 8 x 7, 9 filters of 3 x 3 11.1 /
-// 3.8; 7 x 4 x 55 x 55, 10 of 2 x 2 28.9 / 5.9; 2 x 24 x 8 x 8, 338 of 2 x 2 11.9 / 4.6; 23 x 80 x 9 x 9, 25 of
-// 3 x 3 14.3 / 11.2; input gradient 47 x 11 x 10 x 11, 143 of 1 x 1 24.9 / 6.2; 2 x 45 x 12 x 12, 21 of 5
-// x 5 11.5 / 9.5.  Not there: 5 x 17 x 9 x 9, 15 of 7 x 7 11.9 / 15; 1 x 64 x 27 x 27, 192 of 5 x 5 16.3 / 23.
+// has to be 15 % ahead.  us, the three launches / sums: forward 9 x 5 x 8 x 7, 9 filters of 3 x 3 11.2 /
+// 3.9; 7 x 4 x 55 x 55, 10 of 2 x 2 19.2 / 6.1; 2 x 24 x 8 x 8, 338 of 2 x 2 13.7 / 4.8; 23 x 80 x 9 x 9, 25 of
+// 3 x 3 14.3 / 11.2; input gradient 47 x 11 x 10 x 11, 143 of 1 x 1 26.2 / 6.4.  Not there: 5 x 17 x 9 x 9, 15 of 7 x 7 11.9 / 15; 1 x 64 x 27 x 27, 192 of 5 x 5 16.3 / 23.
 // That leaves out a second round of workgroups on some CUs, loads whose lanes are in many images, and
 // loads of rows that a wave does not have: 81 x 12 x 6 x 6, 22 of 6 x 6 10.8 / 18.6; 25 x 59 x 5 x 5, 75 of 4 x 4
 // 14.4 / 23.8; input gradient 15 x 6 x 112 x 112, 2 of 2 x 9 28.7 / 41.5.

@@ -804,8 +804,8 @@ bool storesAsFloat4(const float* C, long c0, long c1) {
 // multiply-adds; a load brings 64 consecutive bins of one element.  The KW waves of a workgroup
 // take every KW-th k each, the next one's values in flight under this one's products, and add
 // up in LDS in wave order.  What bounds it is what one CU can ask for at a time, about 45 GB/s.
-// us, matrix kernel / this: 1 x 30 x 323 (N = 16) 77.5 / 34.4 with tiles of 1 x 8, 2 x 193 x 29
-// (32) 22 / 8.3, 15 x 18 x 318 82 / 29, 9 x 16 x 5 8.3 / 4.0.  (Sixteen waves: the same.)
+// us, matrix kernel / this: 1 x 30 x 323 (N = 16) 77.9 / 9.4 (34.4 with tiles of 1 x 8), 2 x 193 x 29
+// (32) 21.8 / 6.6, 15 x 18 x 318 79 / 24, 9 x 16 x 5 8.3 / 3.6.  (Sixteen waves: the same.)
 template <int TI, int TJ, int KW>
 __global__ __launch_bounds__(64 * KW) void transposeMMLanesKernel(MMArgs a, int iTiles, int jTiles, int total) {
   constexpr int E = TI * TJ;
@@ -969,8 +969,8 @@ ProductRoute matrixTile(const MMArgs& m, bool vec4, bool vec4C) {
 // Small products run on transposeMMLanesKernel.  Both times are estimated, in us, from
 // the chain of slices of the fullest CU: 45 GB/s of operands a CU there, 0.62 us (up to 32 rows:
 // 0.87) per four k on the matrix kernels, fitted to 90 random products of 24 to 1632 work items.
-// Around the line, matrix kernel / lanes: 27 x 54 x 24 (N = 32) 15.7 / 13.8, 18 x
-// 100 x 17 20.2 / 13.8, but 81 x 28 x 55 16.9 / 27.9, 252 x 10 x 76 (N = 16) 17.8 / 20.8.
+// Around the line, matrix kernel / lanes: 27 x 54 x 24 (N = 32) 13.3 / 11.6, 18 x
+// 100 x 17 17.3 / 12.2, but 81 x 28 x 55 16.9 / 27.9, 252 x 10 x 76 (N = 16) 17.8 / 20.8.
 // Those leave out what a workgroup does besides its k - it starts, and stores its part of C - which is most
 // of a product of few k in many small tiles: 253 x 100 x 2 (N = 16) 11.5 / 17.1, 369 x 460 x 1 (N = 8) 13.9 /
 // 26.8, 80 x 32 x 3 (N = 32) 6.8 / 7.9.  So a second pair of estimates, with that in them, must not see the

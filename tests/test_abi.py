@@ -356,7 +356,7 @@ def test_conv_choose_fft_size():
 
 
 # timed on both kernels (N points; matrix kernel / lanes): 11.5 / 17.1, 13.9 / 26.8, 19.9 / 26.1, 6.8 / 7.9, 16.9
-# / 27.9 us; 77.5 / 34.4, 15.7 / 13.8, 8.3 / 4.0, 20.2 / 13.8 us
+# / 27.9 us; 77.9 / 9.4, 13.3 / 11.6, 8.3 / 3.6, 17.3 / 12.2 us
 @pytest.mark.parametrize("I,J,K,N,kind", [
     (253, 100, 2, 16, DIRECT), (369, 460, 1, 8, DIRECT), (198, 265, 1, 16, DIRECT), (80, 32, 3, 32, DIRECT),
     (81, 28, 55, 32, DIRECT),
@@ -392,7 +392,7 @@ def test_mm_small_products_in_place_keep_the_kernels_that_read_first(I, J, K):
 
 
 # timed both ways, transforms / sums: 10.8 / 18.6, 14.4 / 23.8, 13.5 / 18.9, 28.7 / 41.5 us; 11.1
-# / 3.8, 28.9 / 5.9, 24.9 / 6.2 us
+# / 3.9, 19.2 / 6.1, 26.2 / 6.4 us
 @pytest.mark.parametrize("pass_,B,cin,cout,H,W,kH,kW,small", [
     (0, 81, 12, 22, 6, 6, 6, 6, False), (0, 25, 59, 75, 5, 5, 4, 4, False), (0, 71, 32, 15, 5, 5, 4, 4, False),
     (1, 15, 6, 2, 112, 112, 2, 9, False),
