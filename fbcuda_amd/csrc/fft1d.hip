@@ -6,7 +6,8 @@
 // 8-byte accesses.  Each row is transformed as an N/2-point complex FFT of the
 // even/odd packing z[j] = x[2j] + i x[2j+1]: one lane per row up to N = 64, two
 // lanes for N = 128 and four for N = 256 (radix-G split read straight from LDS,
-// 32 points per lane in VGPRs, G uniform per wave).  The real-input fix-up runs
+// 32 points per lane in VGPRs, G uniform per wave; contiguous rows of 256 have a kernel of their own,
+// below).  The real-input fix-up runs
 // on the way out (forward) or on the way in (inverse) with lanes mapped to
 // consecutive output elements, so HBM stores are contiguous.  The reference
 // instead pairs two rows into one N-point complex transform; results agree to
@@ -189,7 +190,7 @@ __global__ __launch_bounds__(k1dThreads) void fft1dInverse(Row1D a) {
   }
 }
 
-// ---- N = 8 ... 256 with contiguous, 16-byte aligned operands ----
+// ---- N = 8 ... 128 with contiguous, 16-byte aligned operands ----
 //
 // Same staging as above, but the real-input fix-up never makes a pass of its own
 // through LDS: with one lane per row (N <= 64) the whole half-length transform is in
@@ -197,15 +198,11 @@ __global__ __launch_bounds__(k1dThreads) void fft1dInverse(Row1D a) {
 // that the fix-up pairs (k, N/2 - k) stay inside one lane - the forward transform
 // splits its outputs by parity, the inverse its inputs (E = IFFT(z even),
 // O = IFFT(z odd), x[j] = E[j] + w^j O[j], x[j + N/4] = E[j] - w^j O[j], summed on
-// the way out of LDS).  With four lanes per row (N = 256) the classes k = 0 and
-// 2 mod 4 still pair inside their lane; lanes 1 and 3 hold each other's partners:
-// forward each parks half of its transform in the row and finishes the pairs of
-// its other half, inverse each derives its own inputs from the pairs (the
-// partner's half of a pair is computed and dropped).  Spectra and rows then move between LDS and
-// HBM as plain 16-byte streams.
+// the way out of LDS).  Spectra and rows then move between LDS and HBM as plain 16-byte
+// streams.
 template <int N>
 struct CfgMid {
-  static_assert(N >= 8 && N <= 256, "one lane per row up to 64 points, then two or four");
+  static_assert(N >= 8 && N <= 128, "one lane per row up to 64 points, then two");
   static constexpr int H = N / 2;
   static constexpr int G = N <= 64 ? 1 : N / 64;  // lanes per row
   static constexpr int Q = H / G;           // points per lane (32)
@@ -259,59 +256,6 @@ __global__ __launch_bounds__(k1dThreads, 2) void fft1dMidForward(const float* __
         zrow[k] = val;
       }
     });
-  } else if constexpr (G == 4) {
-    splitFFT<H, 4, true>(zrow, g, tw, v);   // lane g: Z[4k + g]; g is the wave index
-    // The results are consumed in per-wave branches below the barrier.  Without this
-    // the compiler sinks the whole transform into those branches and keeps the 128
-    // raw values it was computed from alive across the barrier instead of the 32 results.
-#pragma unroll
-    for (int j = 0; j < Q; ++j) asm volatile("" : "+v"(v[j].x), "+v"(v[j].y));
-    __syncthreads();                        // all four lanes of a row have read it
-    // F[k] and F[H-k] from a = Z[k], b = Z[H-k]
-    auto fixBoth = [&](auto kp, c32 a, c32 bq) __attribute__((always_inline)) {
-      constexpr int k = decltype(kp)::value;
-      c32 fk, fhk;
-      realPairForward<N, k>(a, bq, fk, fhk);
-      zrow[k] = fk;
-      zrow[H - k] = fhk;
-    };
-    if (g == 0) {
-      const c32 z0 = v[0];
-      zrow[0] = c32{z0.x + z0.y, 0.0f};
-      zrow[H] = c32{z0.x - z0.y, 0.0f};
-      staticFor<Q / 2 - 1>([&](auto kk) {
-        constexpr int k = decltype(kk)::value + 1;  // bins 4k and H-4k
-        fixBoth(std::integral_constant<int, 4 * k>{}, v[slot<Q>(k)], v[slot<Q>(Q - k)]);
-      });
-      const c32 m = v[slot<Q>(Q / 2)];  // bin H/2
-      zrow[H / 2] = c32{m.x, -m.y};
-    } else if (g == 2) {
-      staticFor<Q / 2>([&](auto kk) {
-        constexpr int k = decltype(kk)::value;  // bins 4k+2 and H-4k-2
-        fixBoth(std::integral_constant<int, 4 * k + 2>{}, v[slot<Q>(k)], v[slot<Q>(Q - 1 - k)]);
-      });
-    } else {
-      // lanes 1 and 3: bin 4k+g pairs with H-4k-g = 4(Q-1-k) + (4-g), the other lane's.
-      // Each parks the upper half of its transform (k >= Q/2) at its natural positions ...
-      staticFor<Q / 2>([&](auto kk) {
-        constexpr int k = decltype(kk)::value + Q / 2;
-        zrow[4 * k + g] = v[slot<Q>(k)];
-      });
-    }
-    __syncthreads();
-    // ... and finishes the pairs of its own lower half: it alone reads and then
-    // overwrites the partner's parked values, and nobody reads its lower positions.
-    if (g == 1) {
-      staticFor<Q / 2>([&](auto kk) {
-        constexpr int k = decltype(kk)::value;
-        fixBoth(std::integral_constant<int, 4 * k + 1>{}, v[slot<Q>(k)], zrow[H - (4 * k + 1)]);
-      });
-    } else if (g == 3) {
-      staticFor<Q / 2>([&](auto kk) {
-        constexpr int k = decltype(kk)::value;
-        fixBoth(std::integral_constant<int, 4 * k + 3>{}, v[slot<Q>(k)], zrow[H - (4 * k + 3)]);
-      });
-    }
   } else {
     splitFFT<H, 2, true>(zrow, g, tw, v);   // lane g: Z[2k + g]
     __syncthreads();                        // both lanes of a row have read it
@@ -405,68 +349,6 @@ __global__ __launch_bounds__(k1dThreads, 2) void fft1dMidInverse(const float* __
       constexpr int j = decltype(jj)::value;
       zrow[j] = zz[slot<Q>(j)];
     });
-  } else if constexpr (G == 4) {
-    // lane g takes z[4m + g]; E_g = IFFT(z[4m + g]), x[j + Q q] = sum_g i^(g q) w^(g j) E_g[j]
-    auto pairFix = [&](auto kk, c32& zk, c32& zhk) __attribute__((always_inline)) {
-      constexpr int k = decltype(kk)::value;
-      const c32 a = zrow[k], bb = zrow[H - k];
-      const c32 e = c32{a.x + bb.x, a.y - bb.y};
-      const c32 d = c32{a.x - bb.x, a.y + bb.y};
-      const c32 o = mulRoot<N, k, false>(d);
-      zk = c32{e.x - o.y, e.y + o.x};
-      zhk = c32{e.x + o.y, o.x - e.y};
-    };
-    if (g == 0) {
-      const float f0 = zrow[0].x, fh = zrow[H].x;
-      zz[0] = c32{f0 + fh, f0 - fh};
-      staticFor<Q / 2 - 1>([&](auto mm) {
-        constexpr int m = decltype(mm)::value + 1;  // z[4m] and z[H - 4m] = z[4(Q - m)]
-        pairFix(std::integral_constant<int, 4 * m>{}, zz[m], zz[Q - m]);
-      });
-      const c32 a = zrow[H / 2];
-      zz[Q / 2] = c32{2.0f * a.x, -2.0f * a.y};
-    } else if (g == 2) {
-      staticFor<Q / 2>([&](auto mm) {
-        constexpr int m = decltype(mm)::value;      // z[4m+2] and z[H-4m-2] = z[4(Q-1-m)+2]
-        pairFix(std::integral_constant<int, 4 * m + 2>{}, zz[m], zz[Q - 1 - m]);
-      });
-    } else if (g == 1) {
-      staticFor<Q>([&](auto mm) {
-        constexpr int m = decltype(mm)::value;      // own z[4m+1]; the pair's other half is lane 3's
-        c32 drop;
-        pairFix(std::integral_constant<int, 4 * m + 1>{}, zz[m], drop);
-      });
-    } else {
-      staticFor<Q>([&](auto mm) {
-        constexpr int m = decltype(mm)::value;      // own z[4m+3] = z[H - k], k = 4(Q-1-m)+1
-        c32 drop;
-        pairFix(std::integral_constant<int, 4 * (Q - 1 - m) + 1>{}, drop, zz[m]);
-      });
-    }
-    regFFT<Q, false>(zz);
-    // w^(g j), w = e^(2 pi i / H); exponents of H/2 and more are the negated lower half
-    auto twist = [&](auto gg) __attribute__((always_inline)) {
-      constexpr int GG = decltype(gg)::value;
-      staticFor<Q>([&](auto jj) {
-        constexpr int j = decltype(jj)::value;
-        constexpr int ex = GG * j;
-        const c32 val = zz[slot<Q>(j)];
-        if constexpr (ex < H / 2) {
-          zz[slot<Q>(j)] = mulRoot<H, ex, false>(val);
-        } else {
-          const c32 r = mulRoot<H, ex - H / 2, false>(val);
-          zz[slot<Q>(j)] = c32{-r.x, -r.y};
-        }
-      });
-    };
-    if (g == 1) twist(std::integral_constant<int, 1>{});
-    if (g == 2) twist(std::integral_constant<int, 2>{});
-    if (g == 3) twist(std::integral_constant<int, 3>{});
-    __syncthreads();  // all four lanes of a row have read it
-    staticFor<Q>([&](auto jj) {
-      constexpr int j = decltype(jj)::value;
-      zrow[Q * g + j] = zz[slot<Q>(j)];
-    });
   } else {
     auto pairFix = [&](auto kk, c32& zk, c32& zhk) __attribute__((always_inline)) {
       constexpr int k = decltype(kk)::value;
@@ -516,23 +398,6 @@ __global__ __launch_bounds__(k1dThreads, 2) void fft1dMidInverse(const float* __
     float4 o;
     if constexpr (G == 1) {
       o = float4{base[4 * c4], base[4 * c4 + 1], base[4 * c4 + 2], base[4 * c4 + 3]};
-    } else if constexpr (G == 4) {
-      // complex outputs jc, jc+1 with jc = 2 c4 = j + Q q: A = T0 + (-1)^q T2,
-      // Bv = T1 + (-1)^q T3, x = A + i^q Bv
-      const int jc = 2 * c4, q4 = jc / Q, f = 2 * (jc % Q);
-      const float s2 = (q4 & 1) ? -1.0f : 1.0f;
-      float av[4], bv[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        av[e] = base[f + e] + s2 * base[2 * (2 * Q) + f + e];
-        bv[e] = base[2 * Q + f + e] + s2 * base[3 * (2 * Q) + f + e];
-      }
-      // i^q (bx, by): q=0 (bx, by), 1 (-by, bx), 2 (-bx, -by), 3 (by, -bx)
-      const bool rot = q4 & 1;
-      const float sg = (q4 == 0 || q4 == 3) ? 1.0f : -1.0f;   // sign of the first component
-      const float sh = (q4 == 0 || q4 == 1) ? 1.0f : -1.0f;   // sign of the second component
-      o = float4{av[0] + sg * (rot ? bv[1] : bv[0]), av[1] + sh * (rot ? bv[0] : bv[1]),
-                 av[2] + sg * (rot ? bv[3] : bv[2]), av[3] + sh * (rot ? bv[2] : bv[3])};
     } else {
       const int f = (4 * c4) % H;
       const float sg = 4 * c4 < H ? 1.0f : -1.0f;
@@ -541,6 +406,217 @@ __global__ __launch_bounds__(k1dThreads, 2) void fft1dMidInverse(const float* __
     }
     streamStore(dst + q, o);
   }
+}
+
+// ---- N = 256 with contiguous, 16-byte aligned operands ----
+//
+// A wave transforms eight rows by itself, eight lanes each, as 128 = 16 x 8 points: lane l
+// loads z[l + 8 m] straight into registers and runs 16 points over m, the wave exchanges through
+// LDS, and lane p runs the two 8-point transforms of k mod 16 = p and 16 - p (lane 0: 0 and 8),
+// which hold both halves of every fix-up pair (k, 128 - k).  The inverse runs backwards.
+// What bounds it is HBM.  Four waves of a workgroup share a table of roots and nothing else, and
+// 35 KB of LDS leave room for 16 waves per CU that load, compute and store on their own.  Four
+// lanes per row with the rows in LDS, two workgroups of 66 KB per CU in three phases each, took (us,
+// forward / inverse, before -> this) 98.1 / 90.5 -> 83.6 / 86.7 on 262144 rows (6.5 and 6.2 TB/s),
+// 7.9 / 7.9 -> 4.9 / 5.3 on 8192 and 7.3 / 7.2 -> 4.2 / 4.4 on 687, one chain of instructions each.
+constexpr int kWaveRows = 8, kRowBins = 129;
+
+struct Rows256 {
+  int wave, lane, p, row;  // p: lane of the row
+  int second;              // the second k mod 16 of this lane; the first one is p
+  int rest;                // k of pair i < 4 is p + 16 i, of the others rest + 16 i
+};
+
+__device__ __forceinline__ Rows256 rows256(int t) {
+  Rows256 c;
+  c.wave = __builtin_amdgcn_readfirstlane(t / 64);
+  c.lane = t % 64;
+  c.p = c.lane % 8;
+  c.row = c.lane / 8;
+  c.second = c.p ? 16 - c.p : 8;
+  c.rest = c.p ? c.p : -56;
+  return c;
+}
+
+// value l of class k (mod 16) of a row, between the two steps: no two lanes of a bank
+__device__ __forceinline__ int exchangeAt(const Rows256& c, int k, int l) {
+  return k * 64 + c.row * 8 + (l ^ (k & 7));
+}
+
+// what the wave wrote to LDS is there for all of its lanes
+__device__ __forceinline__ void waveExchange() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ c32 choose(bool first, c32 a, c32 b) {
+  return c32{first ? a.x : b.x, first ? a.y : b.y};
+}
+
+__global__ __launch_bounds__(k1dThreads, 4) void fft1d256Forward(const float* __restrict__ real,
+                                                                 float* __restrict__ cplx, int B) {
+  __shared__ __align__(16) c32 lds[k1dThreads / 64][kWaveRows * kRowBins];
+  __shared__ __align__(8) c32 tw[256];
+  const Rows256 c = rows256(threadIdx.x);
+  const int first = (blockIdx.x * (k1dThreads / 64) + c.wave) * kWaveRows;
+  const int rows = min(kWaveRows, B - first);
+  const c32* const src = reinterpret_cast<const c32*>(real) + (size_t)min(first + c.row, B - 1) * 128 + c.p;
+  c32 v[16];
+  staticFor<16>([&](auto mm) {
+    constexpr int m = decltype(mm)::value;
+    v[m] = src[8 * m];
+  });
+  fillTwiddles<true>(tw, threadIdx.x, k1dThreads);
+  __syncthreads();
+  if (rows <= 0) return;
+
+  regFFT<16, true>(v);
+  c32* const buf = lds[c.wave];
+  staticFor<16>([&](auto kk) {
+    constexpr int k = decltype(kk)::value;
+    c32 a = v[slot<16>(k)];
+    if constexpr (k > 0) a = cmul(a, tw[2 * k * c.p]);
+    buf[exchangeAt(c, k, c.p)] = a;
+  });
+  waveExchange();
+  c32 u[8], w[8];
+  staticFor<8>([&](auto jj) {
+    constexpr int j = decltype(jj)::value;
+    u[j] = buf[exchangeAt(c, c.p, j)];
+    w[j] = buf[exchangeAt(c, c.second, j)];
+  });
+  waveExchange();
+  regFFT<8, true>(u);
+  regFFT<8, true>(w);
+
+  // F[k] and F[128 - k] from Z[k], Z[128 - k], the halvings on the root and the final multiply-adds
+  c32* const out = buf + c.row * kRowBins;
+  const bool lane0 = c.p == 0;
+  staticFor<8>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    c32 a = u[slot<8>(i)], b = w[slot<8>(7 - i)];
+    if constexpr (i < 4) {
+      b = choose(lane0, u[slot<8>((8 - i) % 8)], b);
+    } else {
+      a = choose(lane0, w[slot<8>(i - 4)], a);
+      b = choose(lane0, w[slot<8>(11 - i)], b);
+    }
+    const int k0 = i < 4 ? c.p : c.rest;
+    const c32 e2 = c32{a.x + b.x, a.y - b.y};
+    const c32 root = tw[(k0 + 16 * i) & 255];
+    const c32 t = cmul(c32{a.y + b.y, b.x - a.x}, c32{0.5f * root.x, 0.5f * root.y});
+    out[k0 + 16 * i] = c32{__builtin_fmaf(0.5f, e2.x, t.x), __builtin_fmaf(0.5f, e2.y, t.y)};
+    out[128 - k0 - 16 * i] = c32{__builtin_fmaf(0.5f, e2.x, -t.x), __builtin_fmaf(-0.5f, e2.y, t.y)};
+  });
+  if (lane0) out[64] = cconj(u[slot<8>(4)]);
+  waveExchange();
+
+  // the rows of the wave are one stream in LDS and in HBM
+  const int total = rows * kRowBins;
+  float4* const dst = reinterpret_cast<float4*>(cplx + (size_t)first * 2 * kRowBins);
+  const float4* const l4 = reinterpret_cast<const float4*>(buf);
+  for (int q = c.lane; q < total / 2; q += 64) streamStore(dst + q, l4[q]);
+  if ((total & 1) && c.lane == 0)
+    reinterpret_cast<float2*>(cplx + (size_t)first * 2 * kRowBins)[total - 1] = buf[total - 1];
+}
+
+__global__ __launch_bounds__(k1dThreads, 4) void fft1d256Inverse(const float* __restrict__ cplx,
+                                                                 float* __restrict__ real, int B) {
+  __shared__ __align__(16) c32 lds[k1dThreads / 64][kWaveRows * kRowBins];
+  __shared__ __align__(8) c32 tw[256];
+  const Rows256 c = rows256(threadIdx.x);
+  const int first = (blockIdx.x * (k1dThreads / 64) + c.wave) * kWaveRows;
+  const int rows = min(kWaveRows, B - first);
+  c32* const buf = lds[c.wave];
+  if (rows > 0) {
+    const int total = rows * kRowBins;
+    const float4* const src = reinterpret_cast<const float4*>(cplx + (size_t)first * 2 * kRowBins);
+    constexpr int LOADS = (kWaveRows * kRowBins / 2 + 63) / 64;
+    float in[4 * LOADS];  // plain floats: always promoted to registers
+    staticFor<LOADS>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      const float4 f = src[min(c.lane + 64 * i, total / 2 - 1)];
+      in[4 * i] = f.x;
+      in[4 * i + 1] = f.y;
+      in[4 * i + 2] = f.z;
+      in[4 * i + 3] = f.w;
+    });
+    float4* const l4 = reinterpret_cast<float4*>(buf);
+    staticFor<LOADS>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      const int q = c.lane + 64 * i;
+      if (q < total / 2) l4[q] = float4{in[4 * i], in[4 * i + 1], in[4 * i + 2], in[4 * i + 3]};
+    });
+    if ((total & 1) && c.lane == 0)
+      buf[total - 1] = reinterpret_cast<const float2*>(cplx + (size_t)first * 2 * kRowBins)[total - 1];
+  }
+  fillTwiddles<false>(tw, threadIdx.x, k1dThreads);
+  __syncthreads();
+  if (rows <= 0) return;
+
+  // Z[k] and Z[128 - k] from F[k], F[128 - k] (gain 2); rows behind the last one are what LDS held
+  const c32* const from = buf + c.row * kRowBins;
+  const bool lane0 = c.p == 0;
+  c32 zk[8], zh[8];
+  staticFor<8>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    const int k0 = i < 4 ? c.p : c.rest;
+    c32 a = from[k0 + 16 * i], b = from[128 - k0 - 16 * i];
+    if constexpr (i == 0) {  // only the real parts of F[0] and F[128] reach a real result
+      a.y = lane0 ? 0.0f : a.y;
+      b.y = lane0 ? 0.0f : b.y;
+    }
+    const c32 e = c32{a.x + b.x, a.y - b.y};
+    const c32 o = cmul(c32{a.x - b.x, a.y + b.y}, tw[(k0 + 16 * i) & 255]);
+    zk[i] = c32{e.x - o.y, e.y + o.x};
+    zh[i] = c32{e.x + o.y, o.x - e.y};
+  });
+  const c32 middle = from[64];
+  waveExchange();
+  c32 u[8], w[8];
+  staticFor<8>([&](auto jj) {
+    constexpr int j = decltype(jj)::value;
+    if constexpr (j < 4)
+      u[j] = zk[j];
+    else if constexpr (j == 4)
+      u[j] = choose(lane0, c32{2.0f * middle.x, -2.0f * middle.y}, zk[j]);
+    else
+      u[j] = choose(lane0, zh[8 - j], zk[j]);
+    w[j] = choose(lane0, j < 4 ? zk[(j + 4) % 8] : zh[(11 - j) % 8], zh[7 - j]);
+  });
+  regFFT<8, false>(u);
+  regFFT<8, false>(w);
+  staticFor<8>([&](auto ll) {
+    constexpr int l = decltype(ll)::value;
+    c32 a = u[slot<8>(l)], b = w[slot<8>(l)];
+    if constexpr (l > 0) {
+      a = cmul(a, tw[2 * l * c.p]);
+      b = cmul(b, tw[2 * l * c.second]);
+    }
+    buf[exchangeAt(c, c.p, l)] = a;
+    buf[exchangeAt(c, c.second, l)] = b;
+  });
+  waveExchange();
+  c32 z[16];
+  staticFor<16>([&](auto kk) {
+    constexpr int k = decltype(kk)::value;
+    z[k] = buf[exchangeAt(c, k, c.p)];
+  });
+  waveExchange();
+  regFFT<16, false>(z);
+  // z[p + 8 m]; the rows' 16-byte words are permuted so that no bank holds two rows' columns
+  staticFor<16>([&](auto mm) {
+    constexpr int m = decltype(mm)::value;
+    buf[c.row * 128 + 8 * (m ^ c.row) + c.p] = z[slot<16>(m)];
+  });
+  waveExchange();
+  float4* const dst = reinterpret_cast<float4*>(real + (size_t)first * 256);
+  const float4* const l4 = reinterpret_cast<const float4*>(buf);
+  staticFor<kWaveRows>([&](auto rr) {
+    constexpr int r = decltype(rr)::value;
+    if (r < rows) streamStore(dst + r * 64 + c.lane, l4[r * 64 + (c.lane ^ (4 * r))]);
+  });
 }
 
 template <int N>
@@ -569,7 +645,7 @@ int launchFft1d(bool forward, int N, float* real, int sb, int sx, float* cplx, i
   const bool fast = padL == 0 && sx == 1 && sb % 2 == 0 && aligned(real, 8);
   if (N >= 8 && padL == 0 && sx == 1 && sb == N && ck == 2 && cb == N + 2 && aligned(real, 16) &&
       aligned(cplx, 16)) {
-    const int rowsPerGroup = N <= 64 ? k1dThreads : k1dThreads / (N / 64);
+    const int rowsPerGroup = N <= 64 ? k1dThreads : N == 128 ? k1dThreads / 2 : kWaveRows * (k1dThreads / 64);
     dim3 grid(ceilDiv(B, rowsPerGroup)), block(k1dThreads);
     if (N == 8) {
       if (forward)
@@ -598,9 +674,9 @@ int launchFft1d(bool forward, int N, float* real, int sb, int sx, float* cplx, i
         fft1dMidInverse<128><<<grid, block, 0, s>>>(cplx, real, B);
     } else {
       if (forward)
-        fft1dMidForward<256><<<grid, block, 0, s>>>(real, cplx, B);
+        fft1d256Forward<<<grid, block, 0, s>>>(real, cplx, B);
       else
-        fft1dMidInverse<256><<<grid, block, 0, s>>>(cplx, real, B);
+        fft1d256Inverse<<<grid, block, 0, s>>>(cplx, real, B);
     }
     return launchStatus();
   }

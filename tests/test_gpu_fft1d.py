@@ -161,3 +161,31 @@ def test_random_batches_pads_and_views(oracle, seed):
     bh = back.cpu().numpy()
     assert np.array_equal(bh == 777.0, back32 == 777.0), (N, B, padL, kind)
     assert rel(bh, back32) < TOL_FFT, (N, B, padL, kind)
+
+
+# rows of 256 points: whole and partly filled waves (8 rows) and workgroups (32), odd counts, whose last
+# spectrum ends between two 16-byte words
+@pytest.mark.parametrize("B", [1, 7, 8, 9, 24, 31, 32, 33, 4099])
+def test_rows_of_256(oracle, B):
+    x = synth.normal((B, 256), seed=B).numpy()
+    d = dev()
+    spec = torch.full((B + 1, 129, 2), 7.0, device=d)
+    back = torch.full((B + 1, 256), 7.0, device=d)
+    assert F.fbfft1D(torch.from_numpy(x).to(d), spec[:B]) == F.Success
+    assert F.fbifft1D(back[:B], spec[:B]) == F.Success
+    torch.cuda.synchronize()
+    assert bool((spec[B] == 7.0).all()) and bool((back[B] == 7.0).all())
+    # 128 = 16 x 8 points, a root and the fix-up: ten roundings of at most 2^-24 of a value that grows with
+    # the square root of its terms, each the 2-norm of two parts
+    bar = np.sqrt(2 * 10) * 2.0 ** -24
+    assert rel(spec[:B].cpu().numpy(), oracle.dft1d_r2c(x)) < bar
+    assert rel(back[:B].cpu().numpy(), 256 * x.astype(np.float64)) < 2 * bar
+
+
+def test_inverse_of_256_ignores_imaginary_ends(oracle):
+    """The imaginary parts of the first and last bin reach no real result, whatever they hold."""
+    spec = oracle.dft1d_r2c(synth.normal((5, 256), seed=3).numpy()).astype(np.float32)
+    rc, clean = ifft1d(spec)
+    spec[:, [0, 128], 1] = np.nan
+    rc2, got = ifft1d(spec)
+    assert rc == rc2 == F.Success and np.array_equal(got, clean)
