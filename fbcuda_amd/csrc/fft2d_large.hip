@@ -5,22 +5,27 @@
 // the Hermitian-halved axis is the horizontal frequency and the plane is stored
 // transposed, as the reference's second pass leaves it.
 //
-// One workgroup owns one plane, which stays in LDS between the passes (one
-// buffer, reused by every stage):
-//   1. coalesced 16-byte loads of the real plane into LDS, rows padded by 4 floats;
-//   2. row pass: lane y turns row y (N reals) into N/2 packed complex values and
-//      runs an N/2-point complex FFT in VGPRs plus the real-input fix-up;
-//      columns kx = 0 and kx = N/2 (both real along y) travel packed as one;
-//   3. the result is written back transposed ([kx][y], odd row stride: no bank
-//      conflicts either way);
-//   4. column pass: each N-point column FFT is split over G lanes (G = 2 for 64,
-//      G = 4 for 128; for 128 G is the wave index): lane g forms the radix-G
-//      decimation-in-frequency sums for its residue straight from LDS, applies
-//      W_N^(g*j) from an LDS copy of the twiddle table and finishes with a
-//      32-point FFT in VGPRs;
-//   5. results return to LDS as [kx][ky] and leave as one contiguous stream of
-//      16-byte stores; the packed column is unpacked on the way out.
-// The inverse runs the same steps backwards and crops on store.
+// One workgroup owns one plane, which stays in LDS between the passes (one buffer, reused by every
+// stage), and every stage but one belongs to a wave alone:
+//   1. a wave loads rows of the plane straight into registers, several lanes per row;
+//   2. row pass: N reals as N/2 packed complex values, in two steps of 4 or 8 points with an
+//      exchange through LDS between them, left there transposed ([kx][y], before the real-input fix-up);
+//   3. workgroup barrier;
+//   4. column pass: the lanes of a pair of columns kx and N/2 - kx hold both halves of every
+//      fix-up pair (k, N/2 - k), fix them up as they read them and run both columns in two
+//      steps; columns kx = 0 and kx = N/2 (both real along y) travel packed as one;
+//   5. the wave's columns leave as 16-byte stores, whole columns side by side (stores of 64
+//      bytes per column straight from the registers: 87 -> 99 us at 128 points); the packed column is
+//      unpacked on the way out.
+// The inverse runs the same steps backwards and crops on store; it takes one more barrier, to leave its rows
+// one after the other.
+//
+// What bounds them is HBM: 6.2 and 5.9 TB/s (128 points), 6.5 and 6.3 (64).  us, forward / inverse, before
+// (fewer lanes with 32 points each, which formed the first butterflies from LDS, every stage between barriers)
+// -> this: 4096 planes of 128 x 128 101.5 / 96.5 -> 87.4 / 91.0, 19 planes 8.4 / 8.0 -> 6.2 / 6.2, 3773 windows of
+// 73 x 91 87.0 / 85.9 -> 64.7 / 75.2; 16384 of 64 x 64 94.9 / 84.6 -> 83.8 / 86.3, 53 6.6 / 5.7 -> 4.6 / 5.1, 3247 of 36
+// x 58 22.0 / 22.8 -> 19.1 / 21.9.  At 128 points LDS was the limit while its accesses collided
+// (places from column to column 136 apart: 22.4 of 38.3 million active cycles, 94 / 105 us; 130: 3.6 of 19.4).
 #include "common.h"
 #include "fft_lds.h"
 #include "fft_regs.h"
@@ -28,424 +33,795 @@
 namespace fbfft_amd {
 namespace {
 
-template <int N>
-struct LargeCfg {
-  static constexpr int H = N / 2;
-  static constexpr int G = (N == 64) ? 2 : 4;   // lanes per column FFT
-  static constexpr int L = N / G;               // points per lane in the column pass (32)
-  static constexpr int THREADS = H * G;         // 64 or 256
-  static constexpr int RSF = N + 4;             // real-plane row stride in floats (16-byte rows)
-  static constexpr int RSI = (N == 128) ? N + 2 : N + 4;  // forward input stage: for 128 the rows are
-                                                // read as complex pairs by 2 lanes each, odd
-                                                // complex stride = no bank conflicts
-  static constexpr int GR = (N == 128) ? 2 : 1; // lanes per row transform
-  static constexpr int CS = N + 1;              // [kx][y|ky] row stride in complex
-  static constexpr int YS = H + 1;              // [y][kx] row stride in complex (inverse)
-  static constexpr int BUF_FLOATS =
-      (N * RSF > 2 * H * CS ? (N * RSF > 2 * N * YS ? N * RSF : 2 * N * YS)
-                            : (2 * H * CS > 2 * N * YS ? 2 * H * CS : 2 * N * YS));
-  static constexpr int F4_REAL = N * N / 4;           // float4 per real plane
-  static constexpr int F4_CPLX = (H + 1) * N / 2;     // float4 per spectrum plane
+// ---- 128 x 128 ----
+//
+// 512 lanes per plane.  Rows: a wave takes eight at a time,
+// eight lanes each, as 64 = 8 x 8 packed values; lane l loads z[l + 8 m] straight into registers and the
+// lanes of a row exchange through the row's own places in LDS, which hold [kx][y] in the end.  Columns:
+// sixteen lanes take kx and 64 - kx (kx = 0, which carries kx = 64 packed, with 32), which hold both halves of
+// every fix-up pair, as 128 = 8 x 16 points: lane l makes the pairs y = l + 16 m, runs 8 points over m
+// for both columns, and after the exchange lane (column, ky mod 8) runs 16.  The wave then stores its
+// columns, 1 KB each.  The inverse runs backwards.
+constexpr int kLanes128 = 512;
+// Complex values from column to column.  LDS serves 16 lanes of 8 bytes at a time: the lanes of two rows
+// (8 columns) meet 16 different places modulo 16, and so do those of a column.
+constexpr int kStride128 = 130;
+
+struct Lane128 {
+  int wave, lane;
+  int l, r;      // row pass: lane of the row, row of the wave's eight
+  int h, pair;   // column pass: lane of the pair, pair
+  int k0, k1;    // its columns
+  int c, q;      // after the exchange: column (0 or 1) and ky mod 8
 };
 
-template <int N, bool FAST_REAL, bool FAST_CPLX>
-__global__ __launch_bounds__(LargeCfg<N>::THREADS) void fft2dLargeForward(RealView real,
-                                                                         CplxView cplx, int padL,
-                                                                         int padU) {
-  using C = LargeCfg<N>;
-  constexpr int H = C::H, G = C::G, L = C::L, THREADS = C::THREADS, CS = C::CS;
-  __shared__ __align__(16) float buf[C::BUF_FLOATS];
-  __shared__ __align__(8) c32 tw[256];
-  const int t = threadIdx.x;
-  const int b = blockIdx.x;
-  fillTwiddles<true>(tw, t, THREADS);
+__device__ __forceinline__ Lane128 lane128(int t) {
+  Lane128 a;
+  a.wave = __builtin_amdgcn_readfirstlane(t / 64);
+  a.lane = t % 64;
+  a.l = a.lane % 8;
+  a.r = a.lane / 8;
+  a.h = a.lane % 16;
+  a.pair = a.wave * 4 + a.lane / 16;
+  a.k0 = a.pair;
+  a.k1 = a.pair ? 64 - a.pair : 32;
+  a.c = a.h / 8;
+  a.q = a.h % 8;
+  return a;
+}
 
-  constexpr int RSI = C::RSI;
-  // ---- 1. real plane -> LDS [y][x] ----
+// what the wave wrote to LDS is there for all of its lanes
+__device__ __forceinline__ void waveExchange() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// where a row keeps value l of class k between its two steps, and column c of a pair value l of class k
+// (of either parity for the two columns): sixteen lanes meet different places on both sides
+__device__ __forceinline__ int rowPlace(int k, int l, int y) { return (k * 8 + (l ^ k)) * kStride128 + y; }
+__device__ __forceinline__ int columnPlace(int column, int c, int k, int l) {
+  return column * kStride128 + k * 16 + (l ^ (2 * k) ^ c);
+}
+// where the inverse leaves the packed value j of row y: two rows side by side
+__device__ __forceinline__ int sampleAt(int y, int j) { return y * 64 + (j ^ (8 * (y & 1))); }
+
+template <bool FAST_REAL, bool FAST_CPLX>
+__global__ __launch_bounds__(kLanes128, 4) void fft2d128Forward(RealView real, CplxView cplx, int padL, int padU) {
+  __shared__ __align__(16) c32 cb[64 * kStride128];
+  __shared__ __align__(8) c32 tw[256];
+  const Lane128 a = lane128(threadIdx.x);
+  const int b = blockIdx.x;
+  // whether a wave's rows 64 i + 8 wave ... + 7 hold a row of the window
+  auto any = [&](int i) __attribute__((always_inline)) {
+    const int y = 64 * i + 8 * a.wave;
+    return FAST_REAL || (real.w > 0 && real.h > 0 && y < padU + real.h && y + 8 > padU);
+  };
+  const float* const src = real.data + (size_t)b * real.sb;
+
+  c32 z[2][8];
   if constexpr (FAST_REAL) {
-    const float4* src = reinterpret_cast<const float4*>(real.data + (size_t)b * real.sb);
-    const int rs4 = real.sy / 4;
-    staticFor<C::F4_REAL / THREADS>([&](auto ii) {
+    staticFor<2>([&](auto ii) {
       constexpr int i = decltype(ii)::value;
-      const int q = t + THREADS * i;
-      const float4 v = src[(size_t)(q / (N / 4)) * rs4 + q % (N / 4)];
-      float* d = buf + (q / (N / 4)) * RSI + 4 * (q % (N / 4));
-      if constexpr (RSI % 4 == 0) {
-        *reinterpret_cast<float4*>(d) = v;
-      } else {
-        *reinterpret_cast<float2*>(d) = float2{v.x, v.y};
-        *reinterpret_cast<float2*>(d + 2) = float2{v.z, v.w};
-      }
+      const c32* row = reinterpret_cast<const c32*>(src + (size_t)(64 * i + 8 * a.wave + a.r) * real.sy) + a.l;
+      staticFor<8>([&](auto mm) { z[i][decltype(mm)::value] = row[8 * decltype(mm)::value]; });
     });
   } else {
-    // Windowed plane (implicit zero padding, any strides): a lane keeps its column
-    // and walks down the rows.  Loads go out in batches of 16 at addresses clamped
-    // into the window, with no branch between them, and samples outside the window
-    // are zeroed when they are parked in LDS; batches below the window's last row
-    // load nothing.
-    const float* src = real.data + (size_t)b * real.sb;
-    const int yEnd = min(N, padU + real.h);
-    // rows that start on 16-byte boundaries and a window whose left edge and width are
-    // multiples of 4 (contiguous 60 x 60 planes, say) move as float4 the same way
-    const bool vec = real.sx == 1 && ((real.sy | real.sb | padL | real.w) & 3) == 0 &&
-                     (reinterpret_cast<uintptr_t>(real.data) & 15) == 0;
-    if (vec) {
-      constexpr int GPR = N / 4;           // float4 per row
-      constexpr int RPI4 = THREADS / GPR;  // rows per step
-      constexpr int STEPS = N / RPI4;      // 16
-      constexpr int HALF = STEPS / 2;
-      const int xg = t % GPR, yb = t / GPR;
-      const int xs = 4 * xg - padL;
-      const bool xin = (unsigned)xs < (unsigned)real.w;
-      const float* colp = src + min(max(xs, 0), real.w - 4);
-#pragma unroll
-      for (int j0 = 0; j0 < STEPS; j0 += HALF) {
-        float4 v[HALF];
-        if (j0 * RPI4 < yEnd) {
-#pragma unroll
-          for (int j = 0; j < HALF; ++j) {
-            const int ys = min(max(yb + RPI4 * (j0 + j) - padU, 0), real.h - 1);
-            v[j] = *reinterpret_cast<const float4*>(colp + (size_t)ys * real.sy);
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < HALF; ++j) {
-          const int y = yb + RPI4 * (j0 + j);
-          const bool ok = j0 * RPI4 < yEnd && xin && (unsigned)(y - padU) < (unsigned)real.h;
-          const float4 o = ok ? v[j] : float4{0.f, 0.f, 0.f, 0.f};
-          float* d = buf + y * RSI + 4 * xg;
-          if constexpr (RSI % 4 == 0) {
-            *reinterpret_cast<float4*>(d) = o;
-          } else {
-            *reinterpret_cast<float2*>(d) = float2{o.x, o.y};
-            *reinterpret_cast<float2*>(d + 2) = float2{o.z, o.w};
-          }
-        }
+    // implicit zero padding, any strides: loads at places clamped into the window, no branch
+    // between them, and what lies outside counts as zero; whole pairs where the window has only such
+    const bool pairs = real.sx == 1 && ((real.sy | real.sb | padL | real.w) & 1) == 0 &&
+                       (reinterpret_cast<uintptr_t>(real.data) & 7) == 0;
+    staticFor<2>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      const int y = 64 * i + 8 * a.wave + a.r - padU;
+      const bool yIn = (unsigned)y < (unsigned)real.h;
+      const float* row = src + (size_t)min(max(y, 0), real.h - 1) * real.sy;
+      if (any(i) && pairs) {
+        staticFor<8>([&](auto mm) {
+          const int x = 2 * (a.l + 8 * decltype(mm)::value) - padL;
+          z[i][decltype(mm)::value] = *reinterpret_cast<const c32*>(row + min(max(x, 0), real.w - 2));
+        });
+      } else if (any(i)) {
+        staticFor<8>([&](auto mm) {
+          const int x = 2 * (a.l + 8 * decltype(mm)::value) - padL;
+          z[i][decltype(mm)::value].x = row[(size_t)min(max(x, 0), real.w - 1) * real.sx];
+          z[i][decltype(mm)::value].y = row[(size_t)min(max(x + 1, 0), real.w - 1) * real.sx];
+        });
       }
-    } else {
-    constexpr int RPI = THREADS / N;   // rows per step of the walk
-    constexpr int BATCH = 16;
-    const int x = t % N, yb = t / N;
-    const int xs = x - padL;
-    const bool xin = (unsigned)xs < (unsigned)real.w;
-    const float* colp = src + (size_t)min(max(xs, 0), real.w - 1) * real.sx;
-#pragma unroll
-    for (int i0 = 0; i0 < N / RPI; i0 += BATCH) {
-      if (i0 * RPI < yEnd) {
-        float v[BATCH];
-#pragma unroll
-        for (int j = 0; j < BATCH; ++j) {
-          const int ys = min(max(yb + RPI * (i0 + j) - padU, 0), real.h - 1);
-          v[j] = colp[(size_t)ys * real.sy];
-        }
-#pragma unroll
-        for (int j = 0; j < BATCH; ++j) {
-          const int y = yb + RPI * (i0 + j);
-          buf[y * RSI + x] = (xin && (unsigned)(y - padU) < (unsigned)real.h) ? v[j] : 0.0f;
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < BATCH; ++j) buf[(yb + RPI * (i0 + j)) * RSI + x] = 0.0f;
-      }
-    }
-    }
-  }
-  __syncthreads();
-
-  c32* cb = reinterpret_cast<c32*>(buf);
-  if constexpr (C::GR == 1) {
-    // ---- 2. row pass: lane y, N reals -> H packed complex ----
-    c32 z[H];
-    if (t < N) {
-      const float* row = buf + t * RSI;
-      staticFor<H / 2>([&](auto mm) {
+      staticFor<8>([&](auto mm) {
         constexpr int m = decltype(mm)::value;
-        float4 v = *reinterpret_cast<const float4*>(row + 4 * m);
-        z[2 * m] = c32{v.x, v.y};
-        z[2 * m + 1] = c32{v.z, v.w};
+        const int x = 2 * (a.l + 8 * m) - padL;
+        z[i][m].x = yIn && (unsigned)x < (unsigned)real.w ? z[i][m].x : 0.0f;
+        z[i][m].y = yIn && (unsigned)(x + 1) < (unsigned)real.w ? z[i][m].y : 0.0f;
       });
-    }
-    __syncthreads();  // every row is in registers: the buffer may be overwritten
-    if (t < N) {
-      regFFT<H, true>(z);
-      // ---- 3. fix-up fused with the transposed write: [kx][y] ----
-      realFixupForwardEmit<H>(z, [&](auto kk, c32 val) {
-        constexpr int k = decltype(kk)::value;
-        cb[k * CS + t] = val;
-      });
-    }
-  } else {
-    // ---- 2. row pass split over two lanes: lane (y, gr) gets Z[2k + gr] of the
-    // H-point transform of row y; gr is uniform per wave ----
-    const int y = t % N, gr = t / N;
-    constexpr int LR = H / 2;
-    c32 v[LR];
-    splitFFT<H, 2, true>(reinterpret_cast<const c32*>(buf + y * RSI), gr, tw, v);
-    __syncthreads();  // every row consumed: the buffer may be overwritten
-    // ---- 3. fix-up: bins k' and H-k' have the same parity, so each lane finishes
-    // its own half; twiddles are compile-time in both branches ----
-    auto pairOut = [&](auto kp, c32 a, c32 bq) {
-      constexpr int k = decltype(kp)::value;  // bin k pairs with H-k
-      c32 fk, fhk;
-      realPairForward<N, k>(a, bq, fk, fhk);
-      cb[k * CS + y] = fk;
-      cb[(H - k) * CS + y] = fhk;
-    };
-    if (gr == 0) {
-      c32 z0 = v[0];
-      cb[y] = c32{z0.x + z0.y, z0.x - z0.y};
-      staticFor<LR / 2 - 1>([&](auto kk) {
-        constexpr int k = decltype(kk)::value + 1;  // bins 2k and H-2k
-        pairOut(std::integral_constant<int, 2 * k>{}, v[slot<LR>(k)], v[slot<LR>(LR - k)]);
-      });
-      c32 m = v[slot<LR>(LR / 2)];  // bin H/2
-      cb[(H / 2) * CS + y] = c32{m.x, -m.y};
-    } else {
-      staticFor<LR / 2>([&](auto kk) {
-        constexpr int k = decltype(kk)::value;  // bins 2k+1 and H-2k-1
-        pairOut(std::integral_constant<int, 2 * k + 1>{}, v[slot<LR>(k)], v[slot<LR>(LR - 1 - k)]);
-      });
-    }
+    });
   }
+  fillTwiddles<true>(tw, threadIdx.x, kLanes128);
   __syncthreads();
 
-  // ---- 4. column pass ----
-  const int col = t % H, g = t / H;
-  c32 v[L];
-  splitFFT<N, G, true>(cb + col * CS, g, tw, v);
-  __syncthreads();  // all columns consumed
-  // ---- 5. [kx][ky] back to LDS ----
-  staticFor<L>([&](auto kk) {
-    constexpr int k = decltype(kk)::value;
-    cb[col * CS + G * k + g] = v[slot<L>(k)];
+  // ---- rows ----
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (!any(i)) return;
+    regFFT<8, true>(z[i]);
+    staticFor<8>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      c32 v = z[i][slot<8>(k)];
+      if constexpr (k > 0) v = cmul(v, tw[4 * k * a.l]);
+      cb[rowPlace(k, a.l, 64 * i + 8 * a.wave + a.r)] = v;
+    });
+  });
+  waveExchange();
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (!any(i)) return;
+    staticFor<8>([&](auto jj) {
+      constexpr int j = decltype(jj)::value;
+      z[i][j] = cb[rowPlace(a.l, j, 64 * i + 8 * a.wave + a.r)];
+    });
+  });
+  waveExchange();
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (any(i)) regFFT<8, true>(z[i]);  // (rows outside are zeros)
+    staticFor<8>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      cb[(a.l + 8 * k) * kStride128 + 64 * i + 8 * a.wave + a.r] = z[i][slot<8>(k)];
+    });
   });
   __syncthreads();
 
-  // ---- copy out (H+1) x N complex; rows 0 and H come from packed row 0 ----
-  constexpr int ITERS = (C::F4_CPLX + THREADS - 1) / THREADS;
-  staticFor<ITERS>([&](auto ii) {
+  // ---- columns ----
+  {
+    c32 u[8], v[8];
+    const c32 root = tw[2 * a.pair], half = c32{0.5f * root.x, 0.5f * root.y};
+    staticFor<8>([&](auto mm) {
+      constexpr int m = decltype(mm)::value;
+      u[m] = cb[a.k0 * kStride128 + a.h + 16 * m];
+      v[m] = cb[a.k1 * kStride128 + a.h + 16 * m];
+    });
+    waveExchange();
+    staticFor<8>([&](auto mm) {
+      constexpr int m = decltype(mm)::value;
+      const c32 p = u[m], q = v[m];
+      const c32 e2 = c32{p.x + q.x, p.y - q.y};
+      const c32 t = cmul(c32{p.y + q.y, q.x - p.x}, half);
+      u[m] = c32{__builtin_fmaf(0.5f, e2.x, t.x), __builtin_fmaf(0.5f, e2.y, t.y)};
+      v[m] = c32{__builtin_fmaf(0.5f, e2.x, -t.x), __builtin_fmaf(-0.5f, e2.y, t.y)};
+      if (a.wave == 0) {  // (the pair of columns 0 and 32 is in the first wave)
+        const bool ends = a.pair == 0;
+        u[m] = ends ? c32{p.x + p.y, p.x - p.y} : u[m];
+        v[m] = ends ? c32{q.x, -q.y} : v[m];
+      }
+    });
+    regFFT<8, true>(u);
+    regFFT<8, true>(v);
+    staticFor<8>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      c32 p = u[slot<8>(k)], q = v[slot<8>(k)];
+      if constexpr (k > 0) {
+        const c32 w = tw[2 * k * a.h];
+        p = cmul(p, w);
+        q = cmul(q, w);
+      }
+      cb[columnPlace(a.k0, 0, k, a.h)] = p;
+      cb[columnPlace(a.k1, 1, k, a.h)] = q;
+    });
+  }
+  waveExchange();
+  {
+    const int column = a.c ? a.k1 : a.k0;
+    c32 v[16];
+    staticFor<16>([&](auto jj) {
+      constexpr int j = decltype(jj)::value;
+      v[j] = cb[columnPlace(column, a.c, a.q, j)];
+    });
+    waveExchange();
+    regFFT<16, true>(v);
+    staticFor<16>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      cb[column * kStride128 + a.q + 8 * k] = v[slot<16>(k)];
+    });
+  }
+  waveExchange();
+
+  // ---- the wave's columns out; rows 0 and 64 of the result come from packed column 0 ----
+  const int ky = 2 * a.lane;
+  float* const dst = cplx.data + (size_t)b * cplx.sb;
+  auto store = [&](int r, float4 o) __attribute__((always_inline)) {
+    if constexpr (FAST_CPLX) {
+      streamStore(reinterpret_cast<float4*>(dst) + r * 64 + a.lane, o);
+    } else {
+      float* to = dst + (size_t)r * cplx.sr + (size_t)ky * cplx.sc;
+      *reinterpret_cast<float2*>(to) = float2{o.x, o.y};
+      *reinterpret_cast<float2*>(to + cplx.sc) = float2{o.z, o.w};
+    }
+  };
+  auto column = [&](int k) __attribute__((always_inline)) {
+    return *reinterpret_cast<const float4*>(cb + k * kStride128 + ky);
+  };
+  staticFor<4>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
-    const int q = t + THREADS * i;
-    if (q < C::F4_CPLX) {
-      const int r = q / (N / 2);
-      const int ky = 2 * (q % (N / 2));
-      float4 o;
-      if (r == 0 || r == H) {
-        c32 a0 = cb[ky], a1 = cb[ky + 1];
-        c32 m0 = cb[(N - ky) & (N - 1)], m1 = cb[N - ky - 1];
-        if (r == 0)
-          o = float4{0.5f * (a0.x + m0.x), 0.5f * (a0.y - m0.y), 0.5f * (a1.x + m1.x),
-                     0.5f * (a1.y - m1.y)};
-        else
-          o = float4{0.5f * (a0.y + m0.y), 0.5f * (m0.x - a0.x), 0.5f * (a1.y + m1.y),
-                     0.5f * (m1.x - a1.x)};
-      } else {
-        c32 a0 = cb[r * CS + ky], a1 = cb[r * CS + ky + 1];
-        o = float4{a0.x, a0.y, a1.x, a1.y};
-      }
-      if constexpr (FAST_CPLX) {
-        streamStore(reinterpret_cast<float4*>(cplx.data + (size_t)b * cplx.sb) + q, o);
-      } else {
-        float* dst = cplx.data + (size_t)b * cplx.sb + (size_t)r * cplx.sr + (size_t)ky * cplx.sc;
-        *reinterpret_cast<float2*>(dst) = float2{o.x, o.y};
-        *reinterpret_cast<float2*>(dst + cplx.sc) = float2{o.z, o.w};
-      }
+    const int k = a.wave * 4 + i;
+    if (i == 0 && a.wave == 0) {
+      const float4 p = column(0);
+      const c32 m0 = cb[(128 - ky) & 127], m1 = cb[127 - ky];
+      store(0, float4{0.5f * (p.x + m0.x), 0.5f * (p.y - m0.y), 0.5f * (p.z + m1.x), 0.5f * (p.w - m1.y)});
+      store(64, float4{0.5f * (p.y + m0.y), 0.5f * (m0.x - p.x), 0.5f * (p.w + m1.y), 0.5f * (m1.x - p.z)});
+      store(32, column(32));
+    } else {
+      store(k, column(k));
+      store(64 - k, column(64 - k));
     }
   });
 }
 
-template <int N, bool FAST_REAL, bool FAST_CPLX>
-__global__ __launch_bounds__(LargeCfg<N>::THREADS) void fft2dLargeInverse(CplxView cplx,
-                                                                         RealView real, int padL,
-                                                                         int padU) {
-  using C = LargeCfg<N>;
-  constexpr int H = C::H, G = C::G, L = C::L, THREADS = C::THREADS, RSF = C::RSF, CS = C::CS,
-                YS = C::YS;
-  __shared__ __align__(16) float buf[C::BUF_FLOATS];
+template <bool FAST_REAL, bool FAST_CPLX>
+__global__ __launch_bounds__(kLanes128, 4) void fft2d128Inverse(CplxView cplx, RealView real, int padL, int padU) {
+  __shared__ __align__(16) c32 cb[64 * kStride128];
   __shared__ __align__(8) c32 tw[256];
-  const int t = threadIdx.x;
+  const Lane128 a = lane128(threadIdx.x);
   const int b = blockIdx.x;
-  fillTwiddles<false>(tw, t, THREADS);
-  c32* cb = reinterpret_cast<c32*>(buf);
+  // whether a wave's rows 64 i + 8 wave ... + 7 hold a row of the window
+  auto any = [&](int i) __attribute__((always_inline)) {
+    const int y = 64 * i + 8 * a.wave;
+    return FAST_REAL || (real.w > 0 && real.h > 0 && y < padU + real.h && y + 8 > padU);
+  };
 
-  // ---- copy in [kx][ky].  All loads are issued before any is consumed (no load
-  // sits behind a branch or a barrier); the lanes that hold row 0 also fetch row H
-  // and store the fold Z = F0 + i*FH. ----
-  static_assert(H * (N / 2) % THREADS == 0, "rows 0..H-1 divide evenly over the lanes");
-  constexpr int ITERS = H * (N / 2) / THREADS;
-  auto fetch4 = [&](int r, int ky, int q) {
+  // ---- the wave's columns in; column 0 carries 64 as its imaginary part ----
+  const int ky = 2 * a.lane;
+  const float* const src = cplx.data + (size_t)b * cplx.sb;
+  auto load = [&](int r) __attribute__((always_inline)) {
     if constexpr (FAST_CPLX) {
-      return reinterpret_cast<const float4*>(cplx.data + (size_t)b * cplx.sb)[q];
+      return reinterpret_cast<const float4*>(src)[r * 64 + a.lane];
     } else {
-      const float* src = cplx.data + (size_t)b * cplx.sb + (size_t)r * cplx.sr + (size_t)ky * cplx.sc;
-      float2 a = *reinterpret_cast<const float2*>(src);
-      float2 c = *reinterpret_cast<const float2*>(src + cplx.sc);
-      return float4{a.x, a.y, c.x, c.y};
+      const float* from = src + (size_t)r * cplx.sr + (size_t)ky * cplx.sc;
+      const float2 p = *reinterpret_cast<const float2*>(from), q = *reinterpret_cast<const float2*>(from + cplx.sc);
+      return float4{p.x, p.y, q.x, q.y};
     }
   };
-  float4 in[ITERS];
-  staticFor<ITERS>([&](auto ii) {
-    constexpr int i = decltype(ii)::value;
-    const int q = t + THREADS * i;
-    in[i] = fetch4(q / (N / 2), 2 * (q % (N / 2)), q);
-  });
   {
-    const int tq = t % (N / 2);  // lanes beyond the first N/2 fetch a duplicate they ignore
-    const float4 u = fetch4(H, 2 * tq, H * (N / 2) + tq);
-    if (t < N / 2) in[0] = float4{in[0].x - u.y, in[0].y + u.x, in[0].z - u.w, in[0].w + u.z};
+    float4 in[4][2];
+    staticFor<4>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      const int k = a.wave * 4 + i;
+      in[i][0] = load(k);
+      in[i][1] = load(k ? 64 - k : 32);
+    });
+    if (a.wave == 0) {
+      const float4 last = load(64);
+      in[0][0] = float4{in[0][0].x - last.y, in[0][0].y + last.x, in[0][0].z - last.w, in[0][0].w + last.z};
+    }
+    staticFor<4>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      const int k = a.wave * 4 + i;
+      *reinterpret_cast<float4*>(cb + k * kStride128 + ky) = in[i][0];
+      *reinterpret_cast<float4*>(cb + (k ? 64 - k : 32) * kStride128 + ky) = in[i][1];
+    });
   }
-  staticFor<ITERS>([&](auto ii) {
+  fillTwiddles<false>(tw, threadIdx.x, kLanes128);
+  waveExchange();
+  {
+    const int column = a.c ? a.k1 : a.k0;
+    c32 v[16];
+    staticFor<16>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      v[k] = cb[column * kStride128 + a.q + 8 * k];
+    });
+    waveExchange();
+    regFFT<16, false>(v);
+    staticFor<16>([&](auto ll) {
+      constexpr int l = decltype(ll)::value;
+      cb[columnPlace(column, a.c, a.q, l)] = v[slot<16>(l)];
+    });
+  }
+  __syncthreads();  // the roots
+  {
+    c32 u[8], v[8];
+    staticFor<8>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      u[k] = cb[columnPlace(a.k0, 0, k, a.h)];
+      v[k] = cb[columnPlace(a.k1, 1, k, a.h)];
+      if constexpr (k > 0) {
+        const c32 w = tw[2 * k * a.h];
+        u[k] = cmul(u[k], w);
+        v[k] = cmul(v[k], w);
+      }
+    });
+    waveExchange();
+    regFFT<8, false>(u);
+    regFFT<8, false>(v);
+    const c32 root = tw[2 * a.pair];
+    staticFor<8>([&](auto mm) {
+      constexpr int m = decltype(mm)::value;
+      const c32 p = u[slot<8>(m)], q = v[slot<8>(m)];
+      const c32 e = c32{p.x + q.x, p.y - q.y};
+      const c32 o = cmul(c32{p.x - q.x, p.y + q.y}, root);
+      c32 zk = c32{e.x - o.y, e.y + o.x}, zh = c32{e.x + o.y, o.x - e.y};
+      if (a.wave == 0) {
+        const bool ends = a.pair == 0;
+        zk = ends ? c32{p.x + p.y, p.x - p.y} : zk;
+        zh = ends ? c32{2.0f * q.x, -2.0f * q.y} : zh;
+      }
+      cb[a.k0 * kStride128 + a.h + 16 * m] = zk;
+      cb[a.k1 * kStride128 + a.h + 16 * m] = zh;
+    });
+  }
+  __syncthreads();
+
+  // ---- rows ----
+  c32 z[2][8];
+  staticFor<2>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
-    const int q = t + THREADS * i;
-    const int r = q / (N / 2);
-    const int ky = 2 * (q % (N / 2));
-    cb[r * CS + ky] = c32{in[i].x, in[i].y};
-    cb[r * CS + ky + 1] = c32{in[i].z, in[i].w};
+    if (!any(i)) return;
+    staticFor<8>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      z[i][k] = cb[(a.l + 8 * k) * kStride128 + 64 * i + 8 * a.wave + a.r];
+    });
   });
-  __syncthreads();
-
-  // ---- column pass (inverse) ----
-  const int col = t % H, g = t / H;
-  c32 v[L];
-  splitFFT<N, G, false>(cb + col * CS, g, tw, v);
-  __syncthreads();
-  // [y][kx]
-  staticFor<L>([&](auto kk) {
-    constexpr int k = decltype(kk)::value;
-    cb[(G * k + g) * YS + col] = v[slot<L>(k)];
+  waveExchange();
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (!any(i)) return;
+    regFFT<8, false>(z[i]);
+    staticFor<8>([&](auto ll) {
+      constexpr int l = decltype(ll)::value;
+      c32 v = z[i][slot<8>(l)];
+      if constexpr (l > 0) v = cmul(v, tw[4 * l * a.l]);
+      cb[rowPlace(a.l, l, 64 * i + 8 * a.wave + a.r)] = v;
+    });
   });
-  __syncthreads();
+  waveExchange();
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (!any(i)) return;
+    staticFor<8>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      z[i][k] = cb[rowPlace(k, a.l, 64 * i + 8 * a.wave + a.r)];
+    });
+  });
+  __syncthreads();  // every place is free: rows [y][column pair] from here on
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (!any(i)) return;
+    regFFT<8, false>(z[i]);
+    staticFor<8>([&](auto mm) {
+      constexpr int m = decltype(mm)::value;
+      cb[sampleAt(64 * i + 8 * a.wave + a.r, a.l + 8 * m)] = z[i][slot<8>(m)];
+    });
+  });
+  waveExchange();
 
-  if constexpr (THREADS == N) {
-    // ---- row pass (inverse): lane y ----
-    c32 z[H];
-    {
-      const c32* row = cb + t * YS;
-      realFixupInverseFetch<H>([&](auto kk) { return row[decltype(kk)::value]; }, z);
-      regFFT<H, false>(z);
-    }
-    __syncthreads();
-    {
-      float* row = buf + t * RSF;
-      staticFor<H / 2>([&](auto mm) {
-        constexpr int m = decltype(mm)::value;
-        c32 a = z[slot<H>(2 * m)], c = z[slot<H>(2 * m + 1)];
-        *reinterpret_cast<float4*>(row + 4 * m) = float4{a.x, a.y, c.x, c.y};
-      });
-    }
-    __syncthreads();
-
-    // ---- copy out, cropped to the window real covers ----
+  // ---- the wave's rows out, cropped to the window real covers ----
+  float* const dst = real.data + (size_t)b * real.sb;
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
     if constexpr (FAST_REAL) {
-      float4* dst = reinterpret_cast<float4*>(real.data + (size_t)b * real.sb);
-      const int rs4 = real.sy / 4;
-      staticFor<C::F4_REAL / THREADS>([&](auto ii) {
-        constexpr int i = decltype(ii)::value;
-        const int q = t + THREADS * i;
-        const int y = q / (N / 4), x4 = q % (N / 4);
-        streamStore(dst + (size_t)y * rs4 + x4, *reinterpret_cast<const float4*>(buf + y * RSF + 4 * x4));
+      staticFor<4>([&](auto jj) {
+        const int y = 64 * i + 8 * a.wave + 2 * decltype(jj)::value + a.lane / 32, x4 = a.lane % 32;
+        streamStore(reinterpret_cast<float4*>(dst + (size_t)y * real.sy) + x4,
+                    *reinterpret_cast<const float4*>(cb + sampleAt(y, 2 * x4)));
       });
     } else {
-      // a lane keeps its column and walks down the rows of the window
-      constexpr int RPI = THREADS / N;
-      const int x = t % N, xs = x - padL;
-      if ((unsigned)xs < (unsigned)real.w) {
-        float* colp = real.data + (size_t)b * real.sb + (size_t)xs * real.sx;
-        const int yEnd = min(N, padU + real.h);
-#pragma unroll 8
-        for (int y = padU + t / N; y < yEnd; y += RPI)
-          colp[(size_t)(y - padU) * real.sy] = buf[y * RSF + x];
-      }
-    }
-  } else {
-    // ---- row pass (inverse) over two lanes per row y.  The H-point inverse
-    // transform of z splits by the parity of its input index: lane g takes
-    // z[2m + g], whose real-input fix-up pairs (k, H - k) have the same parity, so
-    // neither lane repeats the other's fix-up.  With E = IFFT(z even), O = IFFT(z odd)
-    // the result is x[j] = E[j] + w^j O[j], x[j + H/2] = E[j] - w^j O[j], w = e^{2 pi i/H}.
-    // Lane 1 scales its half by w^j; the sum and difference are formed on the way
-    // out of LDS.  g is the same for a whole wave. ----
-    static_assert(THREADS == 2 * N, "two lanes per row");
-    constexpr int Q = H / 2;  // points per lane
-    const int y = t % N, g = t / N;
-    c32 zz[Q];
-    {
-      const c32* row = cb + y * YS;
-      auto pairFix = [&](auto kk, c32& zk, c32& zhk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        const c32 a = row[k], bb = row[H - k];
-        const c32 e = c32{a.x + bb.x, a.y - bb.y};
-        const c32 d = c32{a.x - bb.x, a.y + bb.y};
-        const c32 o = mulRoot<N, k, false>(d);
-        zk = c32{e.x - o.y, e.y + o.x};
-        zhk = c32{e.x + o.y, o.x - e.y};
-      };
-      if (g == 0) {
-        const c32 p0 = row[0];
-        zz[0] = c32{p0.x + p0.y, p0.x - p0.y};
-        staticFor<Q / 2 - 1>([&](auto mm) {
-          constexpr int k = 2 * (decltype(mm)::value + 1);  // 2, 4, ..., H/2 - 2
-          pairFix(std::integral_constant<int, k>{}, zz[k / 2], zz[(H - k) / 2]);
+      if (!any(i)) return;
+      float v[8][2];
+      staticFor<8>([&](auto rr) {
+        staticFor<2>([&](auto jj) {
+          constexpr int r = decltype(rr)::value, j = decltype(jj)::value;
+          const int x = a.lane + 64 * j;
+          v[r][j] = reinterpret_cast<const float*>(cb + sampleAt(64 * i + 8 * a.wave + r, x / 2))[x % 2];
         });
-        const c32 a = row[H / 2];
-        zz[Q / 2] = c32{2.0f * a.x, -2.0f * a.y};
-      } else {
-        staticFor<Q / 2>([&](auto mm) {
-          constexpr int k = 2 * decltype(mm)::value + 1;    // 1, 3, ..., H/2 - 1
-          pairFix(std::integral_constant<int, k>{}, zz[(k - 1) / 2], zz[(H - k - 1) / 2]);
+      });
+      staticFor<8>([&](auto rr) {
+        constexpr int r = decltype(rr)::value;
+        const int y = 64 * i + 8 * a.wave + r - padU;
+        if ((unsigned)y >= (unsigned)real.h) return;
+        float* const row = dst + (size_t)y * real.sy;
+        staticFor<2>([&](auto jj) {
+          constexpr int j = decltype(jj)::value;
+          const int x = a.lane + 64 * j - padL;
+          if ((unsigned)x < (unsigned)real.w) row[(size_t)x * real.sx] = v[r][j];
         });
-      }
-    }
-    regFFT<Q, false>(zz);
-    if (g == 1) {
-      staticFor<Q>([&](auto jj) {
-        constexpr int j = decltype(jj)::value;
-        zz[slot<Q>(j)] = mulRoot<H, j, false>(zz[slot<Q>(j)]);
       });
     }
-    __syncthreads();
-    {
-      // row y of the staging buffer: E as floats [0, H), w^j O as floats [H, N)
-      float* row = buf + y * RSF + H * g;
-      staticFor<Q / 2>([&](auto mm) {
-        constexpr int m = decltype(mm)::value;
-        c32 a = zz[slot<Q>(2 * m)], c = zz[slot<Q>(2 * m + 1)];
-        *reinterpret_cast<float4*>(row + 4 * m) = float4{a.x, a.y, c.x, c.y};
-      });
-    }
-    __syncthreads();
+  });
+}
 
-    // ---- copy out, cropped to the window real covers: real samples 2j, 2j+1 are
-    // (re, im) of x[j] ----
-    if constexpr (FAST_REAL) {
-      float4* dst = reinterpret_cast<float4*>(real.data + (size_t)b * real.sb);
-      const int rs4 = real.sy / 4;
-      staticFor<C::F4_REAL / THREADS>([&](auto ii) {
-        constexpr int i = decltype(ii)::value;
-        const int q = t + THREADS * i;
-        const int yy = q / (N / 4), x4 = q % (N / 4);
-        const int f = (4 * x4) % H;  // float offset of E[j], j = 2*x4 mod H/2
-        const float4 e = *reinterpret_cast<const float4*>(buf + yy * RSF + f);
-        const float4 w = *reinterpret_cast<const float4*>(buf + yy * RSF + H + f);
-        const float sg = 4 * x4 < H ? 1.0f : -1.0f;
-        streamStore(dst + (size_t)yy * rs4 + x4,
-                    float4{e.x + sg * w.x, e.y + sg * w.y, e.z + sg * w.z, e.w + sg * w.w});
-      });
-    } else {
-      // a lane keeps its column and walks down the rows of the window
-      constexpr int RPI = THREADS / N;
-      const int x = t % N, xs = x - padL;
-      if ((unsigned)xs < (unsigned)real.w) {
-        float* colp = real.data + (size_t)b * real.sb + (size_t)xs * real.sx;
-        const int yEnd = min(N, padU + real.h);
-        const float sg = x < H ? 1.0f : -1.0f;
-        const float* e = buf + x % H;
-#pragma unroll 8
-        for (int yy = padU + t / N; yy < yEnd; yy += RPI)
-          colp[(size_t)(yy - padU) * real.sy] = e[yy * RSF] + sg * e[yy * RSF + H];
-      }
-    }
+// ---- 64 x 64 ----
+//
+// The same with 128 lanes per plane.  Rows: 16 of a wave at a time, four lanes each, as 32 = 4 x 8 packed values:
+// lane l loads j = 2 l, 2 l + 1 of every eight, runs 4 points over each, and lane k mod 4 runs 8.  Columns: eight
+// lanes take kx and 32 - kx (0 with 16), as 64 = 8 x 8 points.  LDS holds [kx][y] without padding; y is
+// permuted by kx so that sixteen lanes meet different places modulo 16 everywhere.
+constexpr int kLanes64 = 128;
+
+struct Lane64 {
+  int wave, lane;
+  int l, r;     // row pass: lane of the row, row of the wave's sixteen
+  int h, pair;  // column pass: lane of the pair, pair
+  int k0, k1;   // its columns
+};
+
+__device__ __forceinline__ Lane64 lane64(int t) {
+  Lane64 a;
+  a.wave = __builtin_amdgcn_readfirstlane(t / 64);
+  a.lane = t % 64;
+  a.l = a.lane % 4;
+  a.r = a.lane / 4;
+  a.h = a.lane % 8;
+  a.pair = a.wave * 8 + a.lane / 8;
+  a.k0 = a.pair;
+  a.k1 = a.pair ? 32 - a.pair : 16;
+  return a;
+}
+
+__device__ __forceinline__ int at64(int column, int y) {
+  return column * 64 + (y ^ (8 * (column & 1) + 2 * (column & 2)));
+}
+// value j of class k of a row between its two steps, and value l of class k of a column
+__device__ __forceinline__ int rowPlace64(int k, int j, int y) { return at64(8 * k + 4 * (j & 1) + ((j >> 1) ^ k), y); }
+__device__ __forceinline__ int columnPlace64(int column, int k, int l) { return at64(column, 8 * k + (l ^ k)); }
+// where the inverse leaves the packed value j of row y
+__device__ __forceinline__ int sampleAt64(int y, int j) { return y * 32 + (j ^ (8 * (y & 1))); }
+
+// e^{-/+ 2 pi i m / 64}
+template <bool FWD>
+__device__ __forceinline__ void fillRoots64(c32* tw, int t) {
+  if (t < 64) {
+    const int h = (4 * t) & 127;
+    const float sign = t < 32 ? 1.0f : -1.0f;
+    const float c = sign * __builtin_bit_cast(float, kTwiddleBits[2 * h]);
+    const float s = sign * __builtin_bit_cast(float, kTwiddleBits[2 * h + 1]);
+    tw[t] = c32{c, FWD ? -s : s};
   }
+}
+
+template <bool FAST_REAL, bool FAST_CPLX>
+__global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, CplxView cplx, int padL, int padU) {
+  __shared__ __align__(16) c32 cb[32 * 64];
+  __shared__ __align__(8) c32 tw[64];
+  const Lane64 a = lane64(threadIdx.x);
+  const int b = blockIdx.x;
+  // whether a wave's rows 32 i + 16 wave ... + 15 hold a row of the window
+  auto any = [&](int i) __attribute__((always_inline)) {
+    const int y = 32 * i + 16 * a.wave;
+    return FAST_REAL || (real.w > 0 && real.h > 0 && y < padU + real.h && y + 16 > padU);
+  };
+  const float* const src = real.data + (size_t)b * real.sb;
+
+  float4 z[2][4];  // packed values 2 l + 8 m and the next
+  if constexpr (FAST_REAL) {
+    staticFor<2>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      const float4* row = reinterpret_cast<const float4*>(src + (size_t)(32 * i + 16 * a.wave + a.r) * real.sy) + a.l;
+      staticFor<4>([&](auto mm) { z[i][decltype(mm)::value] = row[4 * decltype(mm)::value]; });
+    });
+  } else {
+    // implicit zero padding, any strides: loads at places clamped into the window, no branch
+    // between them, and what lies outside counts as zero; whole words where the window has only such
+    const bool words = real.sx == 1 && ((real.sy | real.sb | padL | real.w) & 3) == 0 &&
+                       (reinterpret_cast<uintptr_t>(real.data) & 15) == 0;
+    staticFor<2>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      const int y = 32 * i + 16 * a.wave + a.r - padU;
+      const bool yIn = (unsigned)y < (unsigned)real.h;
+      const float* row = src + (size_t)min(max(y, 0), real.h - 1) * real.sy;
+      if (any(i) && words) {
+        staticFor<4>([&](auto mm) {
+          constexpr int m = decltype(mm)::value;
+          z[i][m] = *reinterpret_cast<const float4*>(row + min(max(4 * a.l + 16 * m - padL, 0), real.w - 4));
+        });
+      } else if (any(i)) {
+        staticFor<4>([&](auto mm) {
+          constexpr int m = decltype(mm)::value;
+          const int x = 4 * a.l + 16 * m - padL;
+          z[i][m].x = row[(size_t)min(max(x, 0), real.w - 1) * real.sx];
+          z[i][m].y = row[(size_t)min(max(x + 1, 0), real.w - 1) * real.sx];
+          z[i][m].z = row[(size_t)min(max(x + 2, 0), real.w - 1) * real.sx];
+          z[i][m].w = row[(size_t)min(max(x + 3, 0), real.w - 1) * real.sx];
+        });
+      }
+      staticFor<4>([&](auto mm) {
+        constexpr int m = decltype(mm)::value;
+        const int x = 4 * a.l + 16 * m - padL;
+        z[i][m].x = yIn && (unsigned)x < (unsigned)real.w ? z[i][m].x : 0.0f;
+        z[i][m].y = yIn && (unsigned)(x + 1) < (unsigned)real.w ? z[i][m].y : 0.0f;
+        z[i][m].z = yIn && (unsigned)(x + 2) < (unsigned)real.w ? z[i][m].z : 0.0f;
+        z[i][m].w = yIn && (unsigned)(x + 3) < (unsigned)real.w ? z[i][m].w : 0.0f;
+      });
+    });
+  }
+  fillRoots64<true>(tw, threadIdx.x);
+  __syncthreads();
+
+  // ---- rows ----
+  c32 v[2][8];
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (!any(i)) return;
+    c32 p[4], q[4];
+    staticFor<4>([&](auto mm) {
+      constexpr int m = decltype(mm)::value;
+      p[m] = c32{z[i][m].x, z[i][m].y};
+      q[m] = c32{z[i][m].z, z[i][m].w};
+    });
+    regFFT<4, true>(p);
+    regFFT<4, true>(q);
+    staticFor<4>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      c32 f = p[slot<4>(k)], g = q[slot<4>(k)];
+      if constexpr (k > 0) {
+        f = cmul(f, tw[4 * k * a.l]);
+        g = cmul(g, tw[4 * k * a.l + 2 * k]);
+      }
+      const int y = 32 * i + 16 * a.wave + a.r;
+      cb[rowPlace64(k, 2 * a.l, y)] = f;
+      cb[rowPlace64(k, 2 * a.l + 1, y)] = g;
+    });
+  });
+  waveExchange();
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    staticFor<8>([&](auto jj) {
+      constexpr int j = decltype(jj)::value;
+      v[i][j] = c32{0.0f, 0.0f};
+      if (any(i)) v[i][j] = cb[rowPlace64(a.l, j, 32 * i + 16 * a.wave + a.r)];
+    });
+  });
+  waveExchange();
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (any(i)) regFFT<8, true>(v[i]);  // (rows outside are zeros)
+    staticFor<8>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      cb[at64(a.l + 4 * k, 32 * i + 16 * a.wave + a.r)] = v[i][slot<8>(k)];
+    });
+  });
+  __syncthreads();
+
+  // ---- columns ----
+  c32 p[8], q[8];
+  const c32 root = tw[a.pair], half = c32{0.5f * root.x, 0.5f * root.y};
+  staticFor<8>([&](auto mm) {
+    constexpr int m = decltype(mm)::value;
+    p[m] = cb[at64(a.k0, a.h + 8 * m)];
+    q[m] = cb[at64(a.k1, a.h + 8 * m)];
+  });
+  waveExchange();
+  staticFor<8>([&](auto mm) {
+    constexpr int m = decltype(mm)::value;
+    const c32 f = p[m], g = q[m];
+    const c32 e2 = c32{f.x + g.x, f.y - g.y};
+    const c32 t = cmul(c32{f.y + g.y, g.x - f.x}, half);
+    p[m] = c32{__builtin_fmaf(0.5f, e2.x, t.x), __builtin_fmaf(0.5f, e2.y, t.y)};
+    q[m] = c32{__builtin_fmaf(0.5f, e2.x, -t.x), __builtin_fmaf(-0.5f, e2.y, t.y)};
+    if (a.wave == 0) {  // (the pair of columns 0 and 16 is in the first wave)
+      const bool ends = a.pair == 0;
+      p[m] = ends ? c32{f.x + f.y, f.x - f.y} : p[m];
+      q[m] = ends ? c32{g.x, -g.y} : q[m];
+    }
+  });
+  regFFT<8, true>(p);
+  regFFT<8, true>(q);
+  staticFor<8>([&](auto kk) {
+    constexpr int k = decltype(kk)::value;
+    c32 f = p[slot<8>(k)], g = q[slot<8>(k)];
+    if constexpr (k > 0) {
+      const c32 w = tw[k * a.h];
+      f = cmul(f, w);
+      g = cmul(g, w);
+    }
+    cb[columnPlace64(a.k0, k, a.h)] = f;
+    cb[columnPlace64(a.k1, k, a.h)] = g;
+  });
+  waveExchange();
+  staticFor<8>([&](auto jj) {
+    constexpr int j = decltype(jj)::value;
+    p[j] = cb[columnPlace64(a.k0, a.h, j)];
+    q[j] = cb[columnPlace64(a.k1, a.h, j)];
+  });
+  waveExchange();
+  regFFT<8, true>(p);
+  regFFT<8, true>(q);
+  staticFor<8>([&](auto kk) {
+    constexpr int k = decltype(kk)::value;
+    cb[at64(a.k0, a.h + 8 * k)] = p[slot<8>(k)];
+    cb[at64(a.k1, a.h + 8 * k)] = q[slot<8>(k)];
+  });
+  waveExchange();
+
+  // ---- the wave's columns out, two at a time; rows 0 and 32 of the result come from packed column 0 ----
+  const int ky = 2 * (a.lane % 32);
+  float* const dst = cplx.data + (size_t)b * cplx.sb;
+  auto store = [&](int r, float4 o) __attribute__((always_inline)) {
+    if constexpr (FAST_CPLX) {
+      streamStore(reinterpret_cast<float4*>(dst) + r * 32 + a.lane % 32, o);
+    } else {
+      float* to = dst + (size_t)r * cplx.sr + (size_t)ky * cplx.sc;
+      *reinterpret_cast<float2*>(to) = float2{o.x, o.y};
+      *reinterpret_cast<float2*>(to + cplx.sc) = float2{o.z, o.w};
+    }
+  };
+  staticFor<8>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    const int k = a.wave * 8 + i, column = a.lane < 32 ? k : k ? 32 - k : 16;
+    float4 o = *reinterpret_cast<const float4*>(cb + at64(column, ky));
+    if (i == 0 && a.wave == 0) {
+      const c32 m0 = cb[(64 - ky) & 63], m1 = cb[63 - ky];
+      if (a.lane < 32) {
+        store(32, float4{0.5f * (o.y + m0.y), 0.5f * (m0.x - o.x), 0.5f * (o.w + m1.y), 0.5f * (m1.x - o.z)});
+        o = float4{0.5f * (o.x + m0.x), 0.5f * (o.y - m0.y), 0.5f * (o.z + m1.x), 0.5f * (o.w - m1.y)};
+      }
+    }
+    store(column, o);
+  });
+}
+
+template <bool FAST_REAL, bool FAST_CPLX>
+__global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, RealView real, int padL, int padU) {
+  __shared__ __align__(16) c32 cb[32 * 64];
+  __shared__ __align__(8) c32 tw[64];
+  const Lane64 a = lane64(threadIdx.x);
+  const int b = blockIdx.x;
+  auto any = [&](int i) __attribute__((always_inline)) {
+    const int y = 32 * i + 16 * a.wave;
+    return FAST_REAL || (real.w > 0 && real.h > 0 && y < padU + real.h && y + 16 > padU);
+  };
+
+  // ---- the wave's columns in, two at a time; column 0 carries 32 as its imaginary part ----
+  const int ky = 2 * (a.lane % 32);
+  const float* const src = cplx.data + (size_t)b * cplx.sb;
+  auto load = [&](int r) __attribute__((always_inline)) {
+    if constexpr (FAST_CPLX) {
+      return reinterpret_cast<const float4*>(src)[r * 32 + a.lane % 32];
+    } else {
+      const float* from = src + (size_t)r * cplx.sr + (size_t)ky * cplx.sc;
+      const float2 f = *reinterpret_cast<const float2*>(from), g = *reinterpret_cast<const float2*>(from + cplx.sc);
+      return float4{f.x, f.y, g.x, g.y};
+    }
+  };
+  {
+    auto column = [&](int i) __attribute__((always_inline)) {
+      const int k = a.wave * 8 + i;
+      return a.lane < 32 ? k : k ? 32 - k : 16;
+    };
+    float4 in[8];
+    staticFor<8>([&](auto ii) { in[decltype(ii)::value] = load(column(decltype(ii)::value)); });
+    if (a.wave == 0) {
+      const float4 last = load(32);
+      if (a.lane < 32) in[0] = float4{in[0].x - last.y, in[0].y + last.x, in[0].z - last.w, in[0].w + last.z};
+    }
+    staticFor<8>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      *reinterpret_cast<float4*>(cb + at64(column(i), ky)) = in[i];
+    });
+  }
+  fillRoots64<false>(tw, threadIdx.x);
+  waveExchange();
+
+  // ---- columns ----
+  c32 p[8], q[8];
+  staticFor<8>([&](auto kk) {
+    constexpr int k = decltype(kk)::value;
+    p[k] = cb[at64(a.k0, a.h + 8 * k)];
+    q[k] = cb[at64(a.k1, a.h + 8 * k)];
+  });
+  waveExchange();
+  regFFT<8, false>(p);
+  regFFT<8, false>(q);
+  staticFor<8>([&](auto ll) {
+    constexpr int l = decltype(ll)::value;
+    cb[columnPlace64(a.k0, a.h, l)] = p[slot<8>(l)];
+    cb[columnPlace64(a.k1, a.h, l)] = q[slot<8>(l)];
+  });
+  __syncthreads();  // the roots
+  staticFor<8>([&](auto kk) {
+    constexpr int k = decltype(kk)::value;
+    p[k] = cb[columnPlace64(a.k0, k, a.h)];
+    q[k] = cb[columnPlace64(a.k1, k, a.h)];
+    if constexpr (k > 0) {
+      const c32 w = tw[k * a.h];
+      p[k] = cmul(p[k], w);
+      q[k] = cmul(q[k], w);
+    }
+  });
+  waveExchange();
+  regFFT<8, false>(p);
+  regFFT<8, false>(q);
+  const c32 root = tw[a.pair];
+  staticFor<8>([&](auto mm) {
+    constexpr int m = decltype(mm)::value;
+    const c32 f = p[slot<8>(m)], g = q[slot<8>(m)];
+    const c32 e = c32{f.x + g.x, f.y - g.y};
+    const c32 o = cmul(c32{f.x - g.x, f.y + g.y}, root);
+    c32 zk = c32{e.x - o.y, e.y + o.x}, zh = c32{e.x + o.y, o.x - e.y};
+    if (a.wave == 0) {
+      const bool ends = a.pair == 0;
+      zk = ends ? c32{f.x + f.y, f.x - f.y} : zk;
+      zh = ends ? c32{2.0f * g.x, -2.0f * g.y} : zh;
+    }
+    cb[at64(a.k0, a.h + 8 * m)] = zk;
+    cb[at64(a.k1, a.h + 8 * m)] = zh;
+  });
+  __syncthreads();
+
+  // ---- rows ----
+  c32 v[2][8];
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (!any(i)) return;
+    staticFor<8>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      v[i][k] = cb[at64(a.l + 4 * k, 32 * i + 16 * a.wave + a.r)];
+    });
+  });
+  waveExchange();
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (!any(i)) return;
+    regFFT<8, false>(v[i]);
+    staticFor<8>([&](auto jj) {
+      constexpr int j = decltype(jj)::value;
+      c32 f = v[i][slot<8>(j)];
+      if constexpr (j > 0) f = cmul(f, tw[2 * j * a.l]);
+      cb[rowPlace64(a.l, j, 32 * i + 16 * a.wave + a.r)] = f;
+    });
+  });
+  waveExchange();
+  float4 z[2][4];
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (!any(i)) return;
+    c32 f[4], g[4];
+    staticFor<4>([&](auto kk) {
+      constexpr int k = decltype(kk)::value;
+      f[k] = cb[rowPlace64(k, 2 * a.l, 32 * i + 16 * a.wave + a.r)];
+      g[k] = cb[rowPlace64(k, 2 * a.l + 1, 32 * i + 16 * a.wave + a.r)];
+    });
+    regFFT<4, false>(f);
+    regFFT<4, false>(g);
+    staticFor<4>([&](auto mm) {
+      constexpr int m = decltype(mm)::value;
+      z[i][m] = float4{f[slot<4>(m)].x, f[slot<4>(m)].y, g[slot<4>(m)].x, g[slot<4>(m)].y};
+    });
+  });
+  __syncthreads();  // every place is free: rows [y][column pair] from here on
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if (!any(i)) return;
+    staticFor<4>([&](auto mm) {
+      constexpr int m = decltype(mm)::value;
+      *reinterpret_cast<float4*>(cb + sampleAt64(32 * i + 16 * a.wave + a.r, 2 * a.l + 8 * m)) = z[i][m];
+    });
+  });
+  waveExchange();
+
+  // ---- the wave's rows out, cropped to the window real covers ----
+  float* const dst = real.data + (size_t)b * real.sb;
+  staticFor<2>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    if constexpr (FAST_REAL) {
+      staticFor<4>([&](auto jj) {
+        const int y = 32 * i + 16 * a.wave + 4 * decltype(jj)::value + a.lane / 16, x4 = a.lane % 16;
+        streamStore(reinterpret_cast<float4*>(dst + (size_t)y * real.sy) + x4,
+                    *reinterpret_cast<const float4*>(cb + sampleAt64(y, 2 * x4)));
+      });
+    } else {
+      if (!any(i)) return;
+      float o[16];
+      staticFor<16>([&](auto rr) {
+        constexpr int r = decltype(rr)::value;
+        o[r] = reinterpret_cast<const float*>(cb + sampleAt64(32 * i + 16 * a.wave + r, a.lane / 2))[a.lane % 2];
+      });
+      const int x = a.lane - padL;
+      if ((unsigned)x >= (unsigned)real.w) return;
+      staticFor<16>([&](auto rr) {
+        constexpr int r = decltype(rr)::value;
+        const int y = 32 * i + 16 * a.wave + r - padU;
+        if ((unsigned)y < (unsigned)real.h) dst[(size_t)y * real.sy + (size_t)x * real.sx] = o[r];
+      });
+    }
+  });
 }
 
 bool fastReal(int N, const RealView& r, int padL, int padU) {
@@ -457,33 +833,59 @@ bool fastCplx(int N, const CplxView& c) {
   return c.sc == 2 && c.sr == 2 * N && c.sb % 4 == 0 && aligned(c.data, 16);
 }
 
-template <int N>
-int launchForward(const RealView& real, const CplxView& cplx, int padL, int padU, hipStream_t s) {
-  dim3 grid(real.B), block(LargeCfg<N>::THREADS);
-  const bool fr = fastReal(N, real, padL, padU), fc = fastCplx(N, cplx);
+int launchForward64(const RealView& real, const CplxView& cplx, int padL, int padU, hipStream_t s) {
+  dim3 grid(real.B), block(kLanes64);
+  const bool fr = fastReal(64, real, padL, padU), fc = fastCplx(64, cplx);
   if (fr && fc)
-    fft2dLargeForward<N, true, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+    fft2d64Forward<true, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
   else if (fc)
-    fft2dLargeForward<N, false, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+    fft2d64Forward<false, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
   else if (fr)
-    fft2dLargeForward<N, true, false><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+    fft2d64Forward<true, false><<<grid, block, 0, s>>>(real, cplx, padL, padU);
   else
-    fft2dLargeForward<N, false, false><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+    fft2d64Forward<false, false><<<grid, block, 0, s>>>(real, cplx, padL, padU);
   return launchStatus();
 }
 
-template <int N>
-int launchInverse(const CplxView& cplx, const RealView& real, int padL, int padU, hipStream_t s) {
-  dim3 grid(real.B), block(LargeCfg<N>::THREADS);
-  const bool fr = fastReal(N, real, padL, padU), fc = fastCplx(N, cplx);
+int launchInverse64(const CplxView& cplx, const RealView& real, int padL, int padU, hipStream_t s) {
+  dim3 grid(real.B), block(kLanes64);
+  const bool fr = fastReal(64, real, padL, padU), fc = fastCplx(64, cplx);
   if (fr && fc)
-    fft2dLargeInverse<N, true, true><<<grid, block, 0, s>>>(cplx, real, padL, padU);
+    fft2d64Inverse<true, true><<<grid, block, 0, s>>>(cplx, real, padL, padU);
   else if (fc)
-    fft2dLargeInverse<N, false, true><<<grid, block, 0, s>>>(cplx, real, padL, padU);
+    fft2d64Inverse<false, true><<<grid, block, 0, s>>>(cplx, real, padL, padU);
   else if (fr)
-    fft2dLargeInverse<N, true, false><<<grid, block, 0, s>>>(cplx, real, padL, padU);
+    fft2d64Inverse<true, false><<<grid, block, 0, s>>>(cplx, real, padL, padU);
   else
-    fft2dLargeInverse<N, false, false><<<grid, block, 0, s>>>(cplx, real, padL, padU);
+    fft2d64Inverse<false, false><<<grid, block, 0, s>>>(cplx, real, padL, padU);
+  return launchStatus();
+}
+
+int launchForward128(const RealView& real, const CplxView& cplx, int padL, int padU, hipStream_t s) {
+  dim3 grid(real.B), block(kLanes128);
+  const bool fr = fastReal(128, real, padL, padU), fc = fastCplx(128, cplx);
+  if (fr && fc)
+    fft2d128Forward<true, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+  else if (fc)
+    fft2d128Forward<false, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+  else if (fr)
+    fft2d128Forward<true, false><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+  else
+    fft2d128Forward<false, false><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+  return launchStatus();
+}
+
+int launchInverse128(const CplxView& cplx, const RealView& real, int padL, int padU, hipStream_t s) {
+  dim3 grid(real.B), block(kLanes128);
+  const bool fr = fastReal(128, real, padL, padU), fc = fastCplx(128, cplx);
+  if (fr && fc)
+    fft2d128Inverse<true, true><<<grid, block, 0, s>>>(cplx, real, padL, padU);
+  else if (fc)
+    fft2d128Inverse<false, true><<<grid, block, 0, s>>>(cplx, real, padL, padU);
+  else if (fr)
+    fft2d128Inverse<true, false><<<grid, block, 0, s>>>(cplx, real, padL, padU);
+  else
+    fft2d128Inverse<false, false><<<grid, block, 0, s>>>(cplx, real, padL, padU);
   return launchStatus();
 }
 
@@ -492,16 +894,16 @@ int launchInverse(const CplxView& cplx, const RealView& real, int padL, int padU
 int launchFft2dLargeForward(int N, const RealView& real, const CplxView& cplx, int padL, int padU,
                             hipStream_t s) {
   if (real.B <= 0) return FBFFT_SUCCESS;
-  if (N == 64) return launchForward<64>(real, cplx, padL, padU, s);
-  if (N == 128) return launchForward<128>(real, cplx, padL, padU, s);
+  if (N == 64) return launchForward64(real, cplx, padL, padU, s);
+  if (N == 128) return launchForward128(real, cplx, padL, padU, s);
   return FBFFT_UNSUPPORTED_SIZE;
 }
 
 int launchFft2dLargeInverse(int N, const CplxView& cplx, const RealView& real, int padL, int padU,
                             hipStream_t s) {
   if (real.B <= 0) return FBFFT_SUCCESS;
-  if (N == 64) return launchInverse<64>(cplx, real, padL, padU, s);
-  if (N == 128) return launchInverse<128>(cplx, real, padL, padU, s);
+  if (N == 64) return launchInverse64(cplx, real, padL, padU, s);
+  if (N == 128) return launchInverse128(cplx, real, padL, padU, s);
   return FBFFT_UNSUPPORTED_SIZE;
 }
 

@@ -329,3 +329,33 @@ def test_batches_either_side_of_the_two_groups_per_wave_switch(oracle, N, B):
     assert per_plane_rel(got, want) < TOL_FFT
     err = (back / (N * N) - x).double().norm() / x.double().norm()
     assert bool(torch.isfinite(back).all()) and float(err) < TOL_FFT
+
+
+# windows in planes of 64 and 128 points that begin and end beside the rows of a wave (16 and 8 at a time, 32 and
+# 64 rows apart), whose samples move as words, as pairs and one by one, and spectra that do not move as words
+@pytest.mark.parametrize("N,h,w,padL,padU", [
+    (64, 1, 4, 0, 63), (64, 15, 60, 4, 1), (64, 16, 7, 1, 16), (64, 17, 64, 0, 15), (64, 33, 62, 2, 31),
+    (64, 64, 1, 63, 0), (64, 48, 33, 8, 16), (128, 1, 128, 0, 127), (128, 7, 6, 122, 1), (128, 8, 126, 2, 8),
+    (128, 9, 5, 1, 7), (128, 65, 127, 0, 63), (128, 128, 1, 127, 0), (128, 120, 100, 28, 8)])
+def test_windows_beside_the_rows_of_a_wave(oracle, N, h, w, padL, padU):
+    B = 3
+    x = synth.normal((B, h, w), seed=h + w).numpy()
+    rc, got = fft2d(x, N, padL, padU)
+    want = oracle.dft2d_r2c(x, N, padL, padU)
+    # fourteen (twelve) steps of butterflies, three roots and a fix-up, each a rounding of at most 2^-24 in both
+    # parts of a value that grows like the square root of its terms
+    bar = np.sqrt(2 * (np.log2(N) * 2 + 4)) * 2.0 ** -24
+    assert rc == F.Success and rel(got, want) < bar
+    d = dev()
+    wide = torch.full((B, N // 2 + 1, N, 4), 7.0, device=d)
+    view = wide[..., :2]
+    assert F.fbfft2D(torch.from_numpy(x).to(d), view, padL, padU) == F.Success
+    torch.cuda.synchronize()
+    assert np.array_equal(view.cpu().numpy(), got) and bool((wide[..., 2:] == 7.0).all())
+    back = torch.full((B, h + 2, w + 2), 7.0, device=d)
+    assert F.fbifft2D(view, back[:, 1:-1, 1:-1], padL, padU) == F.Success
+    torch.cuda.synchronize()
+    inner = back[:, 1:-1, 1:-1].cpu().numpy()
+    assert rel(inner, N * N * x.astype(np.float64)) < 2 * bar * np.sqrt(N * N / (h * w))
+    back[:, 1:-1, 1:-1] = 7.0
+    assert bool((back == 7.0).all())
