@@ -2,8 +2,8 @@
 // (replaces decimateInFrequency1DKernel, fbfft/FBFFTCommon.cuh:710-833, and its
 // dispatch tables in fbfft/FBFFT-inl.cuh:19-150).
 //
-// A workgroup of 256 lanes stages ROWS = 256/G rows in LDS with coalesced
-// 8-byte accesses.  Each row is transformed as an N/2-point complex FFT of the
+// A workgroup (256 lanes; of contiguous rows up to 64 points one wave) stages a row per G lanes in LDS with
+// coalesced 8-byte accesses (contiguous rows: 16).  Each row is transformed as an N/2-point complex FFT of the
 // even/odd packing z[j] = x[2j] + i x[2j+1]: one lane per row up to N = 64, two
 // lanes for N = 128 and four for N = 256 (radix-G split read straight from LDS,
 // 32 points per lane in VGPRs, G uniform per wave; contiguous rows of 256 have a kernel of their own,
@@ -200,40 +200,40 @@ __global__ __launch_bounds__(k1dThreads) void fft1dInverse(Row1D a) {
 // O = IFFT(z odd), x[j] = E[j] + w^j O[j], x[j + N/4] = E[j] - w^j O[j], summed on
 // the way out of LDS).  Spectra and rows then move between LDS and HBM as plain 16-byte
 // streams.
-template <int N>
+template <int N, int THREADS>
 struct CfgMid {
   static_assert(N >= 8 && N <= 128, "one lane per row up to 64 points, then two");
   static constexpr int H = N / 2;
   static constexpr int G = N <= 64 ? 1 : N / 64;  // lanes per row
   static constexpr int Q = H / G;           // points per lane (32)
-  static constexpr int ROWS = k1dThreads / G;
+  static constexpr int ROWS = THREADS / G;
   static constexpr int RS = H + 1;          // LDS row stride (complex) = spectrum row length
 };
 
-template <int N>
-__global__ __launch_bounds__(k1dThreads, 2) void fft1dMidForward(const float* __restrict__ real,
+template <int N, int THREADS>
+__global__ __launch_bounds__(THREADS, 2) void fft1dMidForward(const float* __restrict__ real,
                                                               float* __restrict__ cplx, int B) {
-  using C = CfgMid<N>;
+  using C = CfgMid<N, THREADS>;
   constexpr int H = C::H, G = C::G, Q = C::Q, ROWS = C::ROWS, RS = C::RS;
   __shared__ __align__(16) c32 lds[ROWS * RS];
   __shared__ __align__(8) c32 tw[256];
   const int t = threadIdx.x;
   const int b0 = blockIdx.x * ROWS;
   const int rows = min(ROWS, B - b0);
-  if constexpr (G > 1) fillTwiddles<true>(tw, t, k1dThreads);
+  if constexpr (G > 1) fillTwiddles<true>(tw, t, THREADS);
 
   // ---- rows -> LDS as packed complex z[j] = (x[2j], x[2j+1]), 16 bytes per load ----
-  constexpr int LOADS = ROWS * H / 2 / k1dThreads;
+  constexpr int LOADS = ROWS * H / 2 / THREADS;
   const float4* src = reinterpret_cast<const float4*>(real + (size_t)b0 * N);
   float4 in[LOADS];
   staticFor<LOADS>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
-    const int idx = t + k1dThreads * i;               // float4 index: row = idx / (H/2)
+    const int idx = t + THREADS * i;               // float4 index: row = idx / (H/2)
     in[i] = src[min(idx, rows * (H / 2) - 1)];
   });
   staticFor<LOADS>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
-    const int idx = t + k1dThreads * i;
+    const int idx = t + THREADS * i;
     c32* d = lds + (idx / (H / 2)) * RS + 2 * (idx % (H / 2));
     d[0] = c32{in[i].x, in[i].y};
     d[1] = c32{in[i].z, in[i].w};
@@ -289,15 +289,15 @@ __global__ __launch_bounds__(k1dThreads, 2) void fft1dMidForward(const float* __
   const int total = rows * RS;  // complex values of this workgroup
   float4* dst = reinterpret_cast<float4*>(cplx + (size_t)b0 * 2 * RS);
   const float4* l4 = reinterpret_cast<const float4*>(lds);
-  for (int q = t; q < total / 2; q += k1dThreads) streamStore(dst + q, l4[q]);
+  for (int q = t; q < total / 2; q += THREADS) streamStore(dst + q, l4[q]);
   if ((total & 1) && t == 0)
     reinterpret_cast<float2*>(cplx + (size_t)b0 * 2 * RS)[total - 1] = lds[total - 1];
 }
 
-template <int N>
-__global__ __launch_bounds__(k1dThreads, 2) void fft1dMidInverse(const float* __restrict__ cplx,
+template <int N, int THREADS>
+__global__ __launch_bounds__(THREADS, 2) void fft1dMidInverse(const float* __restrict__ cplx,
                                                               float* __restrict__ real, int B) {
-  using C = CfgMid<N>;
+  using C = CfgMid<N, THREADS>;
   constexpr int H = C::H, G = C::G, Q = C::Q, ROWS = C::ROWS, RS = C::RS;
   __shared__ __align__(16) c32 lds[ROWS * RS];
   const int t = threadIdx.x;
@@ -306,12 +306,12 @@ __global__ __launch_bounds__(k1dThreads, 2) void fft1dMidInverse(const float* __
 
   // ---- spectra -> LDS, the same [row][H+1] stream in both places ----
   const int total = rows * RS;
-  constexpr int LOADS = (ROWS * RS / 2 + k1dThreads - 1) / k1dThreads;
+  constexpr int LOADS = (ROWS * RS / 2 + THREADS - 1) / THREADS;
   const float4* src = reinterpret_cast<const float4*>(cplx + (size_t)b0 * 2 * RS);
   float in[4 * LOADS];  // plain floats: always promoted to registers
   staticFor<LOADS>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
-    const float4 v = src[min(t + k1dThreads * i, max(total / 2 - 1, 0))];
+    const float4 v = src[min(t + THREADS * i, max(total / 2 - 1, 0))];
     in[4 * i] = v.x;
     in[4 * i + 1] = v.y;
     in[4 * i + 2] = v.z;
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(k1dThreads, 2) void fft1dMidInverse(const float* __
   float4* l4 = reinterpret_cast<float4*>(lds);
   staticFor<LOADS>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
-    const int q = t + k1dThreads * i;
+    const int q = t + THREADS * i;
     if (q < total / 2) l4[q] = float4{in[4 * i], in[4 * i + 1], in[4 * i + 2], in[4 * i + 3]};
   });
   if ((total & 1) && t == 0)
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(k1dThreads, 2) void fft1dMidInverse(const float* __
 
   // ---- rows out, 16 bytes per store ----
   float4* dst = reinterpret_cast<float4*>(real + (size_t)b0 * N);
-  for (int q = t; q < rows * (N / 4); q += k1dThreads) {
+  for (int q = t; q < rows * (N / 4); q += THREADS) {
     const int r = q / (N / 4), c4 = q % (N / 4);
     const float* base = reinterpret_cast<const float*>(lds + r * RS);
     float4 o;
@@ -645,38 +645,38 @@ int launchFft1d(bool forward, int N, float* real, int sb, int sx, float* cplx, i
   const bool fast = padL == 0 && sx == 1 && sb % 2 == 0 && aligned(real, 8);
   if (N >= 8 && padL == 0 && sx == 1 && sb == N && ck == 2 && cb == N + 2 && aligned(real, 16) &&
       aligned(cplx, 16)) {
-    const int rowsPerGroup = N <= 64 ? k1dThreads : N == 128 ? k1dThreads / 2 : kWaveRows * (k1dThreads / 64);
-    dim3 grid(ceilDiv(B, rowsPerGroup)), block(k1dThreads);
-    if (N == 8) {
+    auto mid = [&](auto n, auto threads) {
+      constexpr int NN = decltype(n)::value, TT = decltype(threads)::value;
+      const dim3 grid(ceilDiv(B, CfgMid<NN, TT>::ROWS)), block(TT);
       if (forward)
-        fft1dMidForward<8><<<grid, block, 0, s>>>(real, cplx, B);
+        fft1dMidForward<NN, TT><<<grid, block, 0, s>>>(real, cplx, B);
       else
-        fft1dMidInverse<8><<<grid, block, 0, s>>>(cplx, real, B);
-    } else if (N == 16) {
-      if (forward)
-        fft1dMidForward<16><<<grid, block, 0, s>>>(real, cplx, B);
-      else
-        fft1dMidInverse<16><<<grid, block, 0, s>>>(cplx, real, B);
-    } else if (N == 32) {
-      if (forward)
-        fft1dMidForward<32><<<grid, block, 0, s>>>(real, cplx, B);
-      else
-        fft1dMidInverse<32><<<grid, block, 0, s>>>(cplx, real, B);
-    } else if (N == 64) {
-      if (forward)
-        fft1dMidForward<64><<<grid, block, 0, s>>>(real, cplx, B);
-      else
-        fft1dMidInverse<64><<<grid, block, 0, s>>>(cplx, real, B);
-    } else if (N == 128) {
-      if (forward)
-        fft1dMidForward<128><<<grid, block, 0, s>>>(real, cplx, B);
-      else
-        fft1dMidInverse<128><<<grid, block, 0, s>>>(cplx, real, B);
-    } else {
-      if (forward)
-        fft1d256Forward<<<grid, block, 0, s>>>(real, cplx, B);
-      else
-        fft1d256Inverse<<<grid, block, 0, s>>>(cplx, real, B);
+        fft1dMidInverse<NN, TT><<<grid, block, 0, s>>>(cplx, real, B);
+    };
+    // Workgroups of one wave up to 64 points: rows of 64, both transforms, us with 256 lanes / 64: 600 rows
+    // 9.1 / 8.0, 32768 10.8 / 9.5, 131072 24.9 / 22.0, 1048576 197 / 187; of 32, 4096 6.0 / 5.4 (in a graph; 7.1
+    // launched one by one either way); 8 and 16 points 0.93 to 1.0.  At 128 points a wave takes one half of its
+    // rows' transforms, so two waves are the fewest, while 256 lanes leave CUs idle: 600 rows 10.9 / 10.0,
+    // 28000 15.9 / 13.1, 40000 18.6 / 18.3, but 50000 20.3 / 21.9, 65536 23.3 / 25.3.
+    const std::integral_constant<int, 64> oneWave;
+    switch (N) {
+      case 8: mid(std::integral_constant<int, 8>{}, oneWave); break;
+      case 16: mid(std::integral_constant<int, 16>{}, oneWave); break;
+      case 32: mid(std::integral_constant<int, 32>{}, oneWave); break;
+      case 64: mid(std::integral_constant<int, 64>{}, oneWave); break;
+      case 128:
+        if (ceilDiv(B, 128) <= computeUnits())
+          mid(std::integral_constant<int, 128>{}, std::integral_constant<int, 128>{});
+        else
+          mid(std::integral_constant<int, 128>{}, std::integral_constant<int, 256>{});
+        break;
+      case 256: {
+        const dim3 grid(ceilDiv(B, kWaveRows * (k1dThreads / 64))), block(k1dThreads);
+        if (forward)
+          fft1d256Forward<<<grid, block, 0, s>>>(real, cplx, B);
+        else
+          fft1d256Inverse<<<grid, block, 0, s>>>(cplx, real, B);
+      }
     }
     return launchStatus();
   }

@@ -189,3 +189,23 @@ def test_inverse_of_256_ignores_imaginary_ends(oracle):
     spec[:, [0, 128], 1] = np.nan
     rc2, got = ifft1d(spec)
     assert rc == rc2 == F.Success and np.array_equal(got, clean)
+
+
+# ends of the workgroups of 64 rows (up to 64 points) and of 64 and 128 (128 points, either side of the switch)
+@pytest.mark.parametrize("N,B", [(8, 63), (8, 65), (16, 64), (16, 129), (32, 127), (32, 4097), (64, 1), (64, 191),
+                                 (128, 63), (128, 65), (128, 32768), (128, 32769), (128, 32897)])
+def test_ends_of_workgroups(oracle, N, B):
+    x = synth.normal((B, N), seed=N + B)
+    d = dev()
+    spec = torch.full((B + 1, N // 2 + 1, 2), 7.0, device=d)
+    back = torch.full((B + 1, N), 7.0, device=d)
+    xd = x.to(d)
+    assert F.fbfft1D(xd, spec[:B]) == F.Success
+    assert F.fbifft1D(back[:B], spec[:B]) == F.Success
+    torch.cuda.synchronize()
+    assert bool((spec[B] == 7.0).all()) and bool((back[B] == 7.0).all())
+    at = np.unique(np.r_[0:min(B, 70), max(0, B - 200):B])
+    # log2(N) + 2 roundings of at most 2^-24 in both parts of values that grow like the root of their terms
+    bar = np.sqrt(2 * (np.log2(N) + 2)) * 2.0 ** -24
+    assert rel(spec[:B].cpu().numpy()[at], oracle.dft1d_r2c(x.numpy()[at])) < bar
+    assert rel(back[:B].cpu().numpy(), N * x.numpy().astype(np.float64)) < 2 * bar
