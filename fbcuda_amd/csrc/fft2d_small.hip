@@ -29,6 +29,8 @@
 namespace fbfft_amd {
 namespace {
 
+enum RealMode { Window, Whole, Dense };
+
 template <int N, bool PACKED = false>
 struct SmallCfg {
   static constexpr int H = N / 2;
@@ -43,14 +45,20 @@ struct SmallCfg {
   static_assert(RS % 2 == 0 && PS % 2 == 0, "rows must stay 16-byte aligned");
 };
 
-// FAST_REAL: real is [B][N][N] with unit x stride, even row/batch strides,
+// REAL:      Whole: real is [B][N][N] with unit x stride, even row/batch strides,
 //            8-byte aligned base and zero padding -> 8-byte vector accesses.
+//            Dense: windows one after the other in memory, 16-byte aligned base.  A group's P
+//            windows are a whole number of 16-byte words, which move as one stream; rows of any width are
+//            taken apart and put end to end in LDS.  In place of 4-byte accesses to every other column
+//            (us, before -> this): inverse of 8192 windows of 27 x 27 in 32 points 14.5 -> 11.9, 60000 of
+//            28 x 28 95 -> 70, 160000 of 15 x 15 in 16 87 -> 50, 100000 of 7 x 7 in 8 14.4 -> 7.4.
+//            Window: anything else.
 // FAST_CPLX: each spectrum plane is contiguous and 16-byte aligned.
 // GPW:       groups of P planes a wave processes (1 or 2).  With 2, the loads of
 //            the second group are issued as soon as the first group's columns
 //            have left the registers, so they fly under the first group's row
 //            pass and stores: the wave pays the HBM latency once instead of twice.
-template <int N, bool FAST_REAL, bool FAST_CPLX, int GPW, bool PACKED>
+template <int N, int REAL, bool FAST_CPLX, int GPW, bool PACKED>
 __global__ __launch_bounds__(64) void fft2dSmallForward(RealView real, CplxView cplx, int padL,
                                                         int padU) {
   using C = SmallCfg<N, PACKED>;
@@ -65,7 +73,7 @@ __global__ __launch_bounds__(64) void fft2dSmallForward(RealView real, CplxView 
 
   auto load = [&](int b0, c32 (&z0)[H], c32 (&z1)[H]) __attribute__((always_inline)) {
     const int b = min(b0 + pl, B - 1);  // tail lanes redo the last plane and skip the store
-    if constexpr (FAST_REAL) {
+    if constexpr (REAL == Whole) {
       const float2* src = reinterpret_cast<const float2*>(real.data + (size_t)b * real.sb) + l;
       const int rs2 = real.sy / 2;
       staticFor<H>([&](auto jj) {
@@ -151,7 +159,50 @@ __global__ __launch_bounds__(64) void fft2dSmallForward(RealView real, CplxView 
 
   const int g0 = blockIdx.x * GPW * P;
   c32 za0[H], za1[H];
-  load(g0, za0, za1);
+  if constexpr (REAL == Dense) {
+    static_assert(GPW == 1, "one group per wave");
+    const int size = real.h * real.w, valid = min(P, B - g0) * size;
+    const float* const src = real.data + (size_t)g0 * size;
+    constexpr int WORDS = P * N * N / 4 / 64;
+    float in[4 * WORDS];  // plain floats: always promoted to registers
+    staticFor<WORDS>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      if (64 * i < valid / 4) {
+        const float4 v = reinterpret_cast<const float4*>(src)[min(lane + 64 * i, valid / 4 - 1)];
+        in[4 * i] = v.x;
+        in[4 * i + 1] = v.y;
+        in[4 * i + 2] = v.z;
+        in[4 * i + 3] = v.w;
+      }
+    });
+    float* const stage = reinterpret_cast<float*>(lds);
+    if (lane < valid % 4) stage[valid / 4 * 4 + lane] = src[valid / 4 * 4 + lane];
+    staticFor<WORDS>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      if (lane + 64 * i < valid / 4)
+        reinterpret_cast<float4*>(stage)[lane + 64 * i] = float4{in[4 * i], in[4 * i + 1], in[4 * i + 2], in[4 * i + 3]};
+    });
+    __syncthreads();
+    const float* const mine = stage + min(pl, B - 1 - g0) * size - padU * real.w + 2 * l - padL;
+    const bool first = (unsigned)(2 * l - padL) < (unsigned)real.w, next = (unsigned)(2 * l + 1 - padL) < (unsigned)real.w;
+    float a[N], c[N];
+    staticFor<N>([&](auto yy) {
+      constexpr int y = decltype(yy)::value;
+      a[y] = c[y] = 0.0f;
+      if ((unsigned)(y - padU) < (unsigned)real.h) {
+        if (first) a[y] = mine[y * real.w];
+        if (next) c[y] = mine[y * real.w + 1];
+      }
+    });
+    staticFor<H>([&](auto jj) {
+      constexpr int j = decltype(jj)::value;
+      za0[j] = c32{a[2 * j], a[2 * j + 1]};
+      za1[j] = c32{c[2 * j], c[2 * j + 1]};
+    });
+    __syncthreads();  // the windows have been consumed
+  } else {
+    load(g0, za0, za1);
+  }
   // A wave in its transform phases is given issue priority over the wave that shares
   // its SIMD while that one copies out.  Measured where every wave takes two groups
   // of 32 x 32 planes in one round: 21.80 -> 21.62 us; with one group per wave over
@@ -179,7 +230,7 @@ __device__ __forceinline__ bool aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
 
-template <int N, bool FAST_REAL, bool FAST_CPLX, int GPW, bool PACKED>
+template <int N, int REAL, bool FAST_CPLX, int GPW, bool PACKED>
 __global__ __launch_bounds__(64) void fft2dSmallInverse(CplxView cplx, RealView real, int padL,
                                                         int padU) {
   using C = SmallCfg<N, PACKED>;
@@ -253,7 +304,7 @@ __global__ __launch_bounds__(64) void fft2dSmallInverse(CplxView cplx, RealView 
     c32 z0[H], z1[H];
     columnPassInverse<N>(plane, l, z0, z1);
     const int b = b0 + pl;
-    if constexpr (FAST_REAL && N <= 16) {
+    if constexpr (REAL == Whole && N <= 16) {
       // Rows of 32 or 64 bytes: stored from the column layout, a wave instruction
       // would touch 16 or 8 cache lines with a fraction of each.  When the planes
       // of the group are contiguous in memory they go back through LDS instead and
@@ -279,8 +330,30 @@ __global__ __launch_bounds__(64) void fft2dSmallInverse(CplxView cplx, RealView 
         return;
       }
     }
+    if constexpr (REAL == Dense) {
+      const int size = real.h * real.w;
+      __syncthreads();  // the spectra have been consumed
+      float* const stage = reinterpret_cast<float*>(lds);
+      float* const mine = stage + pl * size - padU * real.w + 2 * l - padL;
+      const bool first = (unsigned)(2 * l - padL) < (unsigned)real.w, next = (unsigned)(2 * l + 1 - padL) < (unsigned)real.w;
+      staticFor<N>([&](auto yy) {
+        constexpr int y = decltype(yy)::value;
+        if ((unsigned)(y - padU) < (unsigned)real.h) {
+          const c32 a = z0[slot<H>(y / 2)], c = z1[slot<H>(y / 2)];
+          if (first) mine[y * real.w] = y % 2 ? a.y : a.x;
+          if (next) mine[y * real.w + 1] = y % 2 ? c.y : c.x;
+        }
+      });
+      __syncthreads();
+      const int valid = min(P, B - b0) * size;  // (of the last group, may end between two words)
+      float* const dst = real.data + (size_t)b0 * size;
+      for (int q = lane; q < valid / 4; q += 64)
+        streamStore(reinterpret_cast<float4*>(dst) + q, reinterpret_cast<const float4*>(stage)[q]);
+      if (lane < valid % 4) dst[valid / 4 * 4 + lane] = stage[valid / 4 * 4 + lane];
+      return;
+    }
     if (b < B) {
-      if constexpr (FAST_REAL) {
+      if constexpr (REAL == Whole) {
         float2* dst = reinterpret_cast<float2*>(real.data + (size_t)b * real.sb) + l;
         const int rs2 = real.sy / 2;
         staticFor<H>([&](auto jj) {
@@ -324,10 +397,15 @@ __global__ __launch_bounds__(64) void fft2dSmallInverse(CplxView cplx, RealView 
 // (On operands that stay in the last-level cache pairing is also ahead at 16384
 // planes, 21.7 against 22.5 us.)
 template <int N>
-bool pairGroups(int groups) {
+long residentWaves() {
   constexpr int ldsBytes = SmallCfg<N>::P * SmallCfg<N>::PS * (int)sizeof(c32);
   constexpr int wavesPerCU = (160 * 1024 / ldsBytes) < 32 ? (160 * 1024 / ldsBytes) : 32;
-  const long slots = (long)computeUnits() * wavesPerCU;
+  return (long)computeUnits() * wavesPerCU;
+}
+
+template <int N>
+bool pairGroups(int groups) {
+  const long slots = residentWaves<N>();
   return groups > slots && 4L * groups <= 7 * slots;
 }
 
@@ -340,26 +418,54 @@ bool fastCplx(int N, const CplxView& c) {
   return c.sc == 2 && c.sr == 2 * N && c.sb % 4 == 0 && aligned(c.data, 16);
 }
 
-// runs f(std::bool_constant<a>{}, std::bool_constant<b>{}) for the run-time pair (a, b)
+// Windows that move as one stream, and groups enough for the extra turn through LDS not to count, 4 waves per CU.
+// us, inverse, Window -> Dense: 300 windows of 27 x 27 in 32 points (75 groups) 5.2 -> 5.7, 643 of 7 x 7 in 8 (41) 2.9
+// -> 3.2, 4401 (276) 3.0 -> 3.4; at 1025 groups of 8, 16 and 32 points 4.1 -> 3.3, 5.2 -> 4.8, 9.5 -> 8.2.
+bool dense(const RealView& r, int groups) {
+  return r.sx == 1 && r.sy == r.w && (long)r.sb == (long)r.h * r.w && r.h > 0 && r.w > 0 && aligned(r.data, 16) &&
+         groups >= 4 * computeUnits();
+}
+
+// Forward, the loads of every other column meet in the L1, and the turn through LDS pays where waves would
+// otherwise take two groups, or, at 16 points, rows do not move as pairs, up to there (us, Window -> Dense):
+// 100000 windows of 7 x 7 in 8 points 11.4 -> 8.2, of 5 x 6 11.1 -> 8.0, 36000 of 13 x 13 in 16 15.0 -> 13.0, 20000
+// 8.4 -> 7.2; but 400000 of 7 x 7 31.7 -> 33.1, 160000 of 15 x 15 50.4 -> 51.2, 40000 of 14 x 14 12.8 -> 14.9, 16400
+// of 6 x 6 3.9 -> 4.2, 24576 of 23 x 23 in 32 points 28.8 -> 33.4.
+template <int N>
+bool denseForward(const RealView& r, int padL, int groups) {
+  if (N == 8) return pairGroups<N>(groups);
+  const bool pairs = windowMovesAsPairs(r.data, r.sy, r.sx, r.w, padL) && r.sb % 2 == 0;
+  return !pairs && 4L * groups <= 7 * residentWaves<N>();
+}
+
+// runs f(mode of the real operand, std::bool_constant<fast>{})
 template <typename F>
-void withFlags(bool a, bool b, F&& f) {
-  if (a && b) f(std::true_type{}, std::true_type{});
-  else if (a) f(std::true_type{}, std::false_type{});
-  else if (b) f(std::false_type{}, std::true_type{});
-  else f(std::false_type{}, std::false_type{});
+void withModes(int mode, bool fast, F&& f) {
+  auto run = [&](auto m) { fast ? f(m, std::true_type{}) : f(m, std::false_type{}); };
+  if (mode == Whole) run(std::integral_constant<int, Whole>{});
+  else if (mode == Dense) run(std::integral_constant<int, Dense>{});
+  else run(std::integral_constant<int, Window>{});
 }
 
 template <int N, bool PACKED>
 int launchForward(const RealView& real, const CplxView& cplx, int padL, int padU, hipStream_t s) {
   using C = SmallCfg<N, PACKED>;
   const int groups = ceilDiv(real.B, C::P);
+  const int mode = fastReal(N, real, padL, padU)                                              ? Whole
+                   : N <= 16 && denseForward<N>(real, padL, groups) && dense(real, groups) ? Dense
+                                                                                              : Window;
   dim3 block(64);
-  withFlags(fastReal(N, real, padL, padU), fastCplx(N, cplx), [&](auto fr, auto fc) {
-    constexpr bool FR = decltype(fr)::value, FC = decltype(fc)::value;
-    if (pairGroups<N>(groups))
-      fft2dSmallForward<N, FR, FC, 2, PACKED><<<dim3(ceilDiv(groups, 2)), block, 0, s>>>(real, cplx, padL, padU);
-    else
-      fft2dSmallForward<N, FR, FC, 1, PACKED><<<dim3(groups), block, 0, s>>>(real, cplx, padL, padU);
+  withModes(mode, fastCplx(N, cplx), [&](auto m, auto fc) {
+    constexpr int M = decltype(m)::value;
+    constexpr bool FC = decltype(fc)::value;
+    if constexpr (M == Dense) {
+      if constexpr (N <= 16)
+        fft2dSmallForward<N, M, FC, 1, PACKED><<<dim3(groups), block, 0, s>>>(real, cplx, padL, padU);
+    } else if (pairGroups<N>(groups)) {
+      fft2dSmallForward<N, M, FC, 2, PACKED><<<dim3(ceilDiv(groups, 2)), block, 0, s>>>(real, cplx, padL, padU);
+    } else {
+      fft2dSmallForward<N, M, FC, 1, PACKED><<<dim3(groups), block, 0, s>>>(real, cplx, padL, padU);
+    }
   });
   return launchStatus();
 }
@@ -368,13 +474,15 @@ template <int N, bool PACKED>
 int launchInverse(const CplxView& cplx, const RealView& real, int padL, int padU, hipStream_t s) {
   using C = SmallCfg<N, PACKED>;
   const int groups = ceilDiv(real.B, C::P);
+  const int mode = fastReal(N, real, padL, padU) ? Whole : dense(real, groups) ? Dense : Window;
   dim3 block(64);
-  withFlags(fastReal(N, real, padL, padU), fastCplx(N, cplx), [&](auto fr, auto fc) {
-    constexpr bool FR = decltype(fr)::value, FC = decltype(fc)::value;
+  withModes(mode, fastCplx(N, cplx), [&](auto m, auto fc) {
+    constexpr int M = decltype(m)::value;
+    constexpr bool FC = decltype(fc)::value;
     if (pairGroups<N>(groups))
-      fft2dSmallInverse<N, FR, FC, 2, PACKED><<<dim3(ceilDiv(groups, 2)), block, 0, s>>>(cplx, real, padL, padU);
+      fft2dSmallInverse<N, M, FC, 2, PACKED><<<dim3(ceilDiv(groups, 2)), block, 0, s>>>(cplx, real, padL, padU);
     else
-      fft2dSmallInverse<N, FR, FC, 1, PACKED><<<dim3(groups), block, 0, s>>>(cplx, real, padL, padU);
+      fft2dSmallInverse<N, M, FC, 1, PACKED><<<dim3(groups), block, 0, s>>>(cplx, real, padL, padU);
   });
   return launchStatus();
 }

@@ -359,3 +359,34 @@ def test_windows_beside_the_rows_of_a_wave(oracle, N, h, w, padL, padU):
     assert rel(inner, N * N * x.astype(np.float64)) < 2 * bar * np.sqrt(N * N / (h * w))
     back[:, 1:-1, 1:-1] = 7.0
     assert bool((back == 7.0).all())
+
+
+# windows one after the other in memory that move as streams of 16-byte words, either side of the batches that
+# do (1024 groups of 128 / N planes; forward up to 16 points only), whole and partly filled last groups, whose
+# floats end between two words, and windows beside them in memory that do not move that way
+@pytest.mark.parametrize("N,B,h,w,padL,padU", [
+    (32, 4096, 27, 27, 0, 0), (32, 4093, 27, 27, 0, 0), (32, 4097, 27, 27, 0, 0), (32, 4095, 5, 31, 1, 2), (32, 4094, 1, 1, 31, 31),
+    (32, 9001, 28, 28, 2, 1), (16, 8185, 13, 13, 1, 2), (16, 8191, 16, 15, 0, 0), (16, 8186, 1, 3, 13, 15),
+    (16, 31003, 13, 13, 0, 0), (8, 16369, 7, 7, 0, 1), (8, 16371, 3, 5, 3, 4), (8, 100003, 7, 5, 1, 1), (8, 100001, 1, 1, 7, 0)])
+def test_windows_that_move_as_streams(oracle, N, B, h, w, padL, padU):
+    d = dev()
+    x = synth.normal((B, h, w), seed=B).to(d)
+    spec = torch.full((B + 1, N // 2 + 1, N, 2), 7.0, device=d)
+    assert F.fbfft2D(x, spec[:B], padL, padU) == F.Success
+    flat = torch.full((B * h * w + 8,), 7.0, device=d)
+    back = flat[:B * h * w].view(B, h, w)
+    assert F.fbifft2D(spec[:B], back, padL, padU) == F.Success
+    other = torch.full((B, h + 1, w + 1), 7.0, device=d)  # the same windows, not one after the other
+    wide = torch.zeros((B, h, w + 1), device=d)
+    wide[:, :, :w] = x
+    spec2 = torch.empty_like(spec[:B])
+    assert F.fbfft2D(wide[:, :, :w], spec2, padL, padU) == F.Success
+    assert F.fbifft2D(spec[:B], other[:, :h, :w], padL, padU) == F.Success
+    torch.cuda.synchronize()
+    assert bool((spec[B] == 7.0).all()) and bool((flat[B * h * w:] == 7.0).all())
+    # (the compiler need not contract the same products to multiply-adds in both: roundings of 2^-24 apart)
+    assert rel(spec[:B].cpu().numpy(), spec2.cpu().numpy()) < 3e-7
+    assert rel(other[:, :h, :w].cpu().numpy(), back.cpu().numpy()) < 3e-7 * np.sqrt(N * N / (h * w))
+    at = np.unique(np.r_[0:16, B // 2:B // 2 + 16, B - 40:B])
+    assert rel(spec[:B].cpu().numpy()[at], oracle.dft2d_r2c(x.cpu().numpy()[at], N, padL, padU)) < TOL_FFT
+    assert rel(back.cpu().numpy(), N * N * x.cpu().numpy().astype(np.float64)) < TOL_FFT * np.sqrt(N * N / (h * w))
