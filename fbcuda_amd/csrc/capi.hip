@@ -248,6 +248,7 @@ int checkConvShapes(int pass, const fbfft_tensor* input, const fbfft_tensor* wei
                     const fbfft_tensor* output, int N) {
   if (!okTensor(input, 4) || !okTensor(weight, 4) || !okTensor(output, 4))
     return FBFFT_UNSUPPORTED_DIMENSION;
+  const bool named = N != 0;
   N = resolveFftSize(N, pass, input, weight);
   if (!convSizeOk(N)) return FBFFT_UNSUPPORTED_SIZE;
   const int B = input->size[0], Cin = input->size[1], H = input->size[2], W = input->size[3];
@@ -268,6 +269,7 @@ int convPass(int pass, const fbfft_tensor* input, const fbfft_tensor* weight,
   const int rc = checkConvShapes(pass, input, weight, output, N);
   if (rc != FBFFT_SUCCESS) return rc;
   if (empty(input) || empty(weight) || empty(output)) return FBFFT_SUCCESS;
+  const bool named = N != 0;
   N = resolveFftSize(N, pass, input, weight);
   const size_t need = fbfft_conv_workspace_image(pass, input->size[0], input->size[1],
                                                  weight->size[0], input->size[2], input->size[3],
@@ -282,7 +284,7 @@ int convPass(int pass, const fbfft_tensor* input, const fbfft_tensor* weight,
   } else {
     x = input, y = output, out = weight;
   }
-  return launchConvPass(pass, N, x->data, x->stride, x->size, y->data, y->stride, y->size,
+  return launchConvPass(pass, N, named, x->data, x->stride, x->size, y->data, y->stride, y->size,
                         out->data, out->stride, out->size, scale, accumulate, workspace, stream);
 }
 

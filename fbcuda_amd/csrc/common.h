@@ -126,7 +126,8 @@ struct PassSize {
   int N, maxSplits;
 };
 PassSize passSize(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW);
-int launchConvPass(int pass, int N, float* x, const int* xStride, const int* xSize, float* y,
+// named: the caller named N points, which size 0 leaves to the library
+int launchConvPass(int pass, int N, bool named, float* x, const int* xStride, const int* xSize, float* y,
                    const int* yStride, const int* ySize, float* out, const int* outStride,
                    const int* outSize, float scale, bool accumulate, void* workspace,
                    hipStream_t s);
@@ -140,11 +141,18 @@ int launchConvSmall(int pass, const float* x, const int* xStride, const int* xSi
                     const int* yStride, const int* ySize, float* out, const int* outStride, const int* outSize,
                     hipStream_t s);
 
-// what a pass of a caller's transform size runs on where its result overlaps no operand: convSmall,
-// plane-major spectra, or windows of N points with the contraction kernel Windows + GemmPlan::kind
-// (conv_pipeline.hip) and its reduction in so many ranges
+// filters of 1 x 1, without transforms (conv_point.hip)
+bool pointMayRun(int pass, const float* x, const int* xStride, const int* xSize, const float* y, const int* yStride,
+                 const int* ySize, const float* out, const int* outStride, const int* outSize);
+int launchConvPoint(int pass, const float* x, const int* xStride, const int* xSize, const float* y, const int* yStride,
+                    const int* ySize, float* out, const int* outStride, const int* outSize, float scale, bool accumulate,
+                    void* workspace, size_t room, hipStream_t s);
+
+// what a pass of a caller's transform size (0: left to the library) runs on where its result overlaps no
+// operand and planes have no gaps: convSmall, plane-major spectra, windows of N points with the contraction
+// kernel Windows + GemmPlan::kind (conv_pipeline.hip) and its reduction in so many ranges, or products of 1 x 1 filters
 struct ConvRoute {
-  enum Kind { Small, PlaneMajor, Windows };
+  enum Kind { Small, PlaneMajor, Windows, Point = Windows + 6 };
   int kind, N, splits;
 };
 ConvRoute convRoute(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW);

@@ -1682,9 +1682,21 @@ static bool smallMayRun(const float* x, const int* xStride, const int* xSize, co
   return images * xStride[0] + (double)xSize[2] * xStride[2] + (double)xSize[3] * xStride[3] < (1 << 29);
 }
 
+// Filters of 1 x 1 need no transform where the caller leaves the size to the library, or names one that gives
+// way to it (64 and 128; 8 to 32 points name the transforms that they run on).  Each pass is one
+// product then (conv_point.hip).  us, transforms / product, forward, input gradient, weight gradient: 45 x 79 x 118 x 118,
+// 50 filters 283, 306, 326 / 93, 100, 124; 175 x 21 x 186 x 187, 21 723, 723, 852 / 210, 211, 218; 16 x 27 x 120 x 120, 100 91,
+// 85, 123 / 31, 27, 39; 11 x 13 x 37 x 37, 298 28, (sums 14), 33 / 9, -, 16.  Of 40 random layers none took longer.
+static bool runsPoint(int N, bool named, int H, int W, int kH, int kW) {
+  return kH == 1 && kW == 1 && H * W >= 4 && (!named || N > 32);
+}
+
 ConvRoute convRoute(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
+  const bool named = N != 0;
+  if (!named) N = fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW);
   const PassSize size = passSize(pass, N, B, Cin, Cout, H, W, kH, kW);
   if (runsSmall(pass, size.N, B, Cin, Cout, H, W, kH, kW)) return {ConvRoute::Small, size.N, 1};
+  if (runsPoint(N, named, H, W, kH, kW)) return {ConvRoute::Point, size.N, 1};
   if (size.N > 32) return {ConvRoute::PlaneMajor, size.N, 1};
   const GemmPlan plan = windowsPass(pass, size.N, B, Cin, Cout, H, W, kH, kW, size.maxSplits).plan;
   return {ConvRoute::Windows + plan.kind, size.N, plan.splits};
@@ -1696,7 +1708,7 @@ ConvRoute convRoute(int pass, int N, int B, int Cin, int Cout, int H, int W, int
 // strides in floats.  Images larger than the transform (N <= 32, by the caller's choice or by
 // passSize's) are cut into overlapping windows that ride through the same three kernels as extra rows
 // (passes 0 and 1) or extra reduction steps (pass 2).
-int launchConvPass(int pass, int N, float* x, const int* xStride, const int* xSize, float* y,
+int launchConvPass(int pass, int N, bool named, float* x, const int* xStride, const int* xSize, float* y,
                    const int* yStride, const int* ySize, float* out, const int* outStride,
                    const int* outSize, float scale, bool accumulate, void* workspace,
                    hipStream_t s) {
@@ -1704,10 +1716,15 @@ int launchConvPass(int pass, int N, float* x, const int* xStride, const int* xSi
   const int* wt = pass == 2 ? outSize : ySize;    // the filter extents
   const int H = in[2], W = in[3], kH = wt[2], kW = wt[3];
   const PassSize size = passSize(pass, N, in[0], wt[1], wt[0], H, W, kH, kW);
+  const int given = N;
   N = size.N;
   if (runsSmall(pass, N, in[0], wt[1], wt[0], H, W, kH, kW) &&
       smallMayRun(x, xStride, xSize, y, yStride, ySize, out, outStride, outSize))
     return launchConvSmall(pass, x, xStride, xSize, y, yStride, ySize, out, outStride, outSize, s);
+  if (runsPoint(given, named, H, W, kH, kW) &&
+      pointMayRun(pass, x, xStride, xSize, y, yStride, ySize, out, outStride, outSize))
+    return launchConvPoint(pass, x, xStride, xSize, y, yStride, ySize, out, outStride, outSize, scale, accumulate,
+                           workspace, pass == 2 ? convWorkspaceBytes(2, given, in[0], wt[1], wt[0], H, W, 1, 1) : 0, s);
   if (N > 32)
     return launchConvSplit(pass, N, x, xStride, xSize, y, yStride, ySize, out, outStride, outSize,
                            scale, accumulate, workspace, s);

@@ -268,7 +268,10 @@ size_t fbfft_make_tiles_for_pass(int pass, const fbfft_tensor* input, const fbff
  * for.  Where a small forward pass or input gradient would run on this size - by size 0, by its
  * name or in place of a larger named size - and three launches would take longer than the sums
  * over the filter taps themselves, it is summed directly, in one launch (the same bits for each
- * of those calls; a result that overlaps an operand keeps the transforms). */
+ * of those calls; a result that overlaps an operand keeps the transforms).  Filters of 1 x 1
+ * are one product of matrices per pass, without transforms, with size 0, 64 or 128 (8, 16 and 32 name the
+ * transforms that they run on) where the planes of both image-sized tensors have no gaps and at least four
+ * elements; the weight gradient is reproducible there, too. */
 int fbfft_conv_choose_fft_size(int pass, int batch, int cin, int cout, int H, int W, int kH,
                                int kW);
 
