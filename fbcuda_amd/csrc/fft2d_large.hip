@@ -17,14 +17,16 @@
 //   5. the wave's columns leave as 16-byte stores, whole columns side by side (stores of 64
 //      bytes per column straight from the registers: 87 -> 99 us at 128 points); the packed column is
 //      unpacked on the way out.
-// The inverse runs the same steps backwards and crops on store; it takes one more barrier, to leave its rows
-// one after the other.
+// The inverse runs the same steps backwards and crops on store; at 128 points it takes one more barrier, to leave
+// its rows one after the other.
 //
-// What bounds them is HBM: 6.2 and 5.9 TB/s (128 points), 6.5 and 6.3 (64).  us, forward / inverse, before
+// What bounds them is HBM: 6.2 and 5.9 TB/s (128 points), 6.5 and 6.4 (64).  us, forward / inverse, before
 // (fewer lanes with 32 points each, which formed the first butterflies from LDS, every stage between barriers)
 // -> this: 4096 planes of 128 x 128 101.5 / 96.5 -> 87.4 / 91.0, 19 planes 8.4 / 8.0 -> 6.2 / 6.2, 3773 windows of
-// 73 x 91 87.0 / 85.9 -> 64.7 / 75.2; 16384 of 64 x 64 94.9 / 84.6 -> 83.8 / 86.3, 53 6.6 / 5.7 -> 4.6 / 5.1, 3247 of 36
-// x 58 22.0 / 22.8 -> 19.1 / 21.9.  At 128 points LDS was the limit while its accesses collided
+// 73 x 91 87.0 / 85.9 -> 64.7 / 75.2; 16384 of 64 x 64 95.2 / 85.7 -> 84.4 / 84.1, 53 6.6 / 5.7 -> 4.2 / 4.6, 3247 of 36
+// x 58 22.0 / 22.8 -> 18.9 / 22.2; buffers from HBM, 5000 of 64 x 64 33.7 / 33.0 -> 29.9 / 31.5, 3000 of 60 x 60 23.8
+// / 25.5 -> 23.4 / 26.4, of 50 x 50 21.7 / 23.5 -> 17.8 / 25.6 (little over one round of workgroups, whose inverse
+// lost; fewer workgroups per CU or nontemporal loads make it worse).  At 128 points LDS was the limit while its accesses collided
 // (places from column to column 136 apart: 22.4 of 38.3 million active cycles, 94 / 105 us; 130: 3.6 of 19.4).
 #include "common.h"
 #include "fft_lds.h"
@@ -432,7 +434,10 @@ __global__ __launch_bounds__(kLanes128, 4) void fft2d128Inverse(CplxView cplx, R
 // The same with 128 lanes per plane.  Rows: 16 of a wave at a time, four lanes each, as 32 = 4 x 8 packed values:
 // lane l loads j = 2 l, 2 l + 1 of every eight, runs 4 points over each, and lane k mod 4 runs 8.  Columns: eight
 // lanes take kx and 32 - kx (0 with 16), as 64 = 8 x 8 points.  LDS holds [kx][y] without padding; y is
-// permuted by kx so that sixteen lanes meet different places modulo 16 everywhere.
+// permuted by kx so that sixteen lanes meet different places modulo 16 everywhere.  A wave has its own roots, and
+// the inverse its samples among the places of its own rows, which leaves one barrier between the passes; the
+// forward kernel takes another so that each wave stores half of the plane in sequence (5000 planes to HBM 31.4 ->
+// 30.2 us in the median, pairs of columns before).
 constexpr int kLanes64 = 128;
 
 struct Lane64 {
@@ -455,32 +460,46 @@ __device__ __forceinline__ Lane64 lane64(int t) {
   return a;
 }
 
-__device__ __forceinline__ int at64(int column, int y) {
+__device__ __forceinline__ constexpr int at64(int column, int y) {
   return column * 64 + (y ^ (8 * (column & 1) + 2 * (column & 2)));
 }
-// value j of class k of a row between its two steps, and value l of class k of a column
-__device__ __forceinline__ int rowPlace64(int k, int j, int y) { return at64(8 * k + 4 * (j & 1) + ((j >> 1) ^ k), y); }
-__device__ __forceinline__ int columnPlace64(int column, int k, int l) { return at64(column, 8 * k + (l ^ k)); }
-// where the inverse leaves the packed value j of row y
-__device__ __forceinline__ int sampleAt64(int y, int j) { return y * 32 + (j ^ (8 * (y & 1))); }
+// Every exclusive or of columns or of y is one of places, so a lane's places differ from one of them by constants: what
+// meets its bits by exclusive or, the rest as the offset of the access.  In bytes, which leaves one instruction or
+// none to an access: 998 / 1057 vector instructions, forward / inverse, -> 856 / 915.
+__device__ __forceinline__ c32& placed64(c32* cb, int bytes) {
+  return *reinterpret_cast<c32*>(reinterpret_cast<char*>(cb) + bytes);
+}
+// y = h + 8 m of a column, from base = 8 at64(column, h)
+__device__ __forceinline__ constexpr int spacedPlace64(int base, int m) { return (base ^ 64 * (m & 1)) + 64 * (m & 6); }
+// value j of class k of a row between its two steps is column 8 k + 4 (j & 1) + ((j >> 1) ^ k): from
+// base = 8 at64(9 k, y), and of j = 2 l + e from 8 at64(l, y)
+__device__ __forceinline__ constexpr int rowValue64(int base, int j) { return (base ^ 8 * at64(j >> 1, 0)) + 2048 * (j & 1); }
+__device__ __forceinline__ constexpr int rowClass64(int base, int k, int e) {
+  return (base ^ 8 * at64(k, 0)) + 4096 * k + 2048 * e;
+}
+// value l of class k of a column is y = 8 k + (l ^ k): from base = 8 at64(column, 9 k) base ^ 8 l, and from 8 at64(column, l)
+__device__ __forceinline__ constexpr int columnClass64(int base, int k) { return (base ^ 8 * (9 * k & 15)) + 8 * (9 * k & 48); }
+// where the inverse leaves the packed value j of row 32 i + 16 wave + r: among the places of the wave's rows
+__device__ __forceinline__ constexpr int samplePlace64(int wave, int i, int r, int j) {
+  return 8 * (1024 * i + 64 * r + 32 * (j >> 4) + 16 * wave + ((j & 15) ^ (8 * (r & 1))));
+}
 
 // e^{-/+ 2 pi i m / 64}
 template <bool FWD>
-__device__ __forceinline__ void fillRoots64(c32* tw, int t) {
-  if (t < 64) {
-    const int h = (4 * t) & 127;
-    const float sign = t < 32 ? 1.0f : -1.0f;
-    const float c = sign * __builtin_bit_cast(float, kTwiddleBits[2 * h]);
-    const float s = sign * __builtin_bit_cast(float, kTwiddleBits[2 * h + 1]);
-    tw[t] = c32{c, FWD ? -s : s};
-  }
+__device__ __forceinline__ void fillRoots64(c32* tw, int lane) {
+  const int h = (4 * lane) & 127;
+  const float sign = lane < 32 ? 1.0f : -1.0f;
+  const float c = sign * __builtin_bit_cast(float, kTwiddleBits[2 * h]);
+  const float s = sign * __builtin_bit_cast(float, kTwiddleBits[2 * h + 1]);
+  tw[lane] = c32{c, FWD ? -s : s};
 }
 
 template <bool FAST_REAL, bool FAST_CPLX>
 __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, CplxView cplx, int padL, int padU) {
   __shared__ __align__(16) c32 cb[32 * 64];
-  __shared__ __align__(8) c32 tw[64];
+  __shared__ __align__(8) c32 roots[kLanes64 / 64][64];  // a wave's own: no barrier
   const Lane64 a = lane64(threadIdx.x);
+  c32* const tw = roots[a.wave];
   const int b = blockIdx.x;
   // whether a wave's rows 32 i + 16 wave ... + 15 hold a row of the window
   auto any = [&](int i) __attribute__((always_inline)) {
@@ -531,10 +550,11 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
       });
     });
   }
-  fillRoots64<true>(tw, threadIdx.x);
-  __syncthreads();
+  fillRoots64<true>(tw, a.lane);
+  waveExchange();
 
   // ---- rows ----
+  const int values = 8 * at64(a.l, 16 * a.wave + a.r), classes = 8 * at64(9 * a.l, 16 * a.wave + a.r);
   c32 v[2][8];
   staticFor<2>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
@@ -554,9 +574,8 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
         f = cmul(f, tw[4 * k * a.l]);
         g = cmul(g, tw[4 * k * a.l + 2 * k]);
       }
-      const int y = 32 * i + 16 * a.wave + a.r;
-      cb[rowPlace64(k, 2 * a.l, y)] = f;
-      cb[rowPlace64(k, 2 * a.l + 1, y)] = g;
+      placed64(cb, rowClass64(values, k, 0) + 256 * i) = f;
+      placed64(cb, rowClass64(values, k, 1) + 256 * i) = g;
     });
   });
   waveExchange();
@@ -565,7 +584,7 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
     staticFor<8>([&](auto jj) {
       constexpr int j = decltype(jj)::value;
       v[i][j] = c32{0.0f, 0.0f};
-      if (any(i)) v[i][j] = cb[rowPlace64(a.l, j, 32 * i + 16 * a.wave + a.r)];
+      if (any(i)) v[i][j] = placed64(cb, rowValue64(classes, j) + 256 * i);
     });
   });
   waveExchange();
@@ -574,18 +593,19 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
     if (any(i)) regFFT<8, true>(v[i]);  // (rows outside are zeros)
     staticFor<8>([&](auto kk) {
       constexpr int k = decltype(kk)::value;
-      cb[at64(a.l + 4 * k, 32 * i + 16 * a.wave + a.r)] = v[i][slot<8>(k)];
+      placed64(cb, values + 2048 * k + 256 * i) = v[i][slot<8>(k)];
     });
   });
   __syncthreads();
 
   // ---- columns ----
+  const int c0 = 8 * at64(a.k0, a.h), c1 = 8 * at64(a.k1, a.h), d0 = 8 * at64(a.k0, 9 * a.h), d1 = 8 * at64(a.k1, 9 * a.h);
   c32 p[8], q[8];
   const c32 root = tw[a.pair], half = c32{0.5f * root.x, 0.5f * root.y};
   staticFor<8>([&](auto mm) {
     constexpr int m = decltype(mm)::value;
-    p[m] = cb[at64(a.k0, a.h + 8 * m)];
-    q[m] = cb[at64(a.k1, a.h + 8 * m)];
+    p[m] = placed64(cb, spacedPlace64(c0, m));
+    q[m] = placed64(cb, spacedPlace64(c1, m));
   });
   waveExchange();
   staticFor<8>([&](auto mm) {
@@ -611,26 +631,26 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
       f = cmul(f, w);
       g = cmul(g, w);
     }
-    cb[columnPlace64(a.k0, k, a.h)] = f;
-    cb[columnPlace64(a.k1, k, a.h)] = g;
+    placed64(cb, columnClass64(c0, k)) = f;
+    placed64(cb, columnClass64(c1, k)) = g;
   });
   waveExchange();
   staticFor<8>([&](auto jj) {
     constexpr int j = decltype(jj)::value;
-    p[j] = cb[columnPlace64(a.k0, a.h, j)];
-    q[j] = cb[columnPlace64(a.k1, a.h, j)];
+    p[j] = placed64(cb, d0 ^ 8 * j);
+    q[j] = placed64(cb, d1 ^ 8 * j);
   });
   waveExchange();
   regFFT<8, true>(p);
   regFFT<8, true>(q);
   staticFor<8>([&](auto kk) {
     constexpr int k = decltype(kk)::value;
-    cb[at64(a.k0, a.h + 8 * k)] = p[slot<8>(k)];
-    cb[at64(a.k1, a.h + 8 * k)] = q[slot<8>(k)];
+    placed64(cb, spacedPlace64(c0, k)) = p[slot<8>(k)];
+    placed64(cb, spacedPlace64(c1, k)) = q[slot<8>(k)];
   });
-  waveExchange();
+  __syncthreads();
 
-  // ---- the wave's columns out, two at a time; rows 0 and 32 of the result come from packed column 0 ----
+  // ---- columns out, a half of the plane per wave, 1 KB at a time; rows 0 and 32 of the result come from packed column 0 ----
   const int ky = 2 * (a.lane % 32);
   float* const dst = cplx.data + (size_t)b * cplx.sb;
   auto store = [&](int r, float4 o) __attribute__((always_inline)) {
@@ -644,7 +664,7 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
   };
   staticFor<8>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
-    const int k = a.wave * 8 + i, column = a.lane < 32 ? k : k ? 32 - k : 16;
+    const int column = 16 * a.wave + 2 * i + a.lane / 32;
     float4 o = *reinterpret_cast<const float4*>(cb + at64(column, ky));
     if (i == 0 && a.wave == 0) {
       const c32 m0 = cb[(64 - ky) & 63], m1 = cb[63 - ky];
@@ -660,8 +680,9 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
 template <bool FAST_REAL, bool FAST_CPLX>
 __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, RealView real, int padL, int padU) {
   __shared__ __align__(16) c32 cb[32 * 64];
-  __shared__ __align__(8) c32 tw[64];
+  __shared__ __align__(8) c32 roots[kLanes64 / 64][64];  // a wave's own: no barrier
   const Lane64 a = lane64(threadIdx.x);
+  c32* const tw = roots[a.wave];
   const int b = blockIdx.x;
   auto any = [&](int i) __attribute__((always_inline)) {
     const int y = 32 * i + 16 * a.wave;
@@ -696,29 +717,30 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
       *reinterpret_cast<float4*>(cb + at64(column(i), ky)) = in[i];
     });
   }
-  fillRoots64<false>(tw, threadIdx.x);
+  fillRoots64<false>(tw, a.lane);
   waveExchange();
 
   // ---- columns ----
+  const int c0 = 8 * at64(a.k0, a.h), c1 = 8 * at64(a.k1, a.h), d0 = 8 * at64(a.k0, 9 * a.h), d1 = 8 * at64(a.k1, 9 * a.h);
   c32 p[8], q[8];
   staticFor<8>([&](auto kk) {
     constexpr int k = decltype(kk)::value;
-    p[k] = cb[at64(a.k0, a.h + 8 * k)];
-    q[k] = cb[at64(a.k1, a.h + 8 * k)];
+    p[k] = placed64(cb, spacedPlace64(c0, k));
+    q[k] = placed64(cb, spacedPlace64(c1, k));
   });
   waveExchange();
   regFFT<8, false>(p);
   regFFT<8, false>(q);
   staticFor<8>([&](auto ll) {
     constexpr int l = decltype(ll)::value;
-    cb[columnPlace64(a.k0, a.h, l)] = p[slot<8>(l)];
-    cb[columnPlace64(a.k1, a.h, l)] = q[slot<8>(l)];
+    placed64(cb, d0 ^ 8 * l) = p[slot<8>(l)];
+    placed64(cb, d1 ^ 8 * l) = q[slot<8>(l)];
   });
-  __syncthreads();  // the roots
+  waveExchange();
   staticFor<8>([&](auto kk) {
     constexpr int k = decltype(kk)::value;
-    p[k] = cb[columnPlace64(a.k0, k, a.h)];
-    q[k] = cb[columnPlace64(a.k1, k, a.h)];
+    p[k] = placed64(cb, columnClass64(c0, k));
+    q[k] = placed64(cb, columnClass64(c1, k));
     if constexpr (k > 0) {
       const c32 w = tw[k * a.h];
       p[k] = cmul(p[k], w);
@@ -740,19 +762,20 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
       zk = ends ? c32{f.x + f.y, f.x - f.y} : zk;
       zh = ends ? c32{2.0f * g.x, -2.0f * g.y} : zh;
     }
-    cb[at64(a.k0, a.h + 8 * m)] = zk;
-    cb[at64(a.k1, a.h + 8 * m)] = zh;
+    placed64(cb, spacedPlace64(c0, m)) = zk;
+    placed64(cb, spacedPlace64(c1, m)) = zh;
   });
   __syncthreads();
 
   // ---- rows ----
+  const int values = 8 * at64(a.l, 16 * a.wave + a.r), classes = 8 * at64(9 * a.l, 16 * a.wave + a.r);
   c32 v[2][8];
   staticFor<2>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
     if (!any(i)) return;
     staticFor<8>([&](auto kk) {
       constexpr int k = decltype(kk)::value;
-      v[i][k] = cb[at64(a.l + 4 * k, 32 * i + 16 * a.wave + a.r)];
+      v[i][k] = placed64(cb, values + 2048 * k + 256 * i);
     });
   });
   waveExchange();
@@ -764,10 +787,11 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
       constexpr int j = decltype(jj)::value;
       c32 f = v[i][slot<8>(j)];
       if constexpr (j > 0) f = cmul(f, tw[2 * j * a.l]);
-      cb[rowPlace64(a.l, j, 32 * i + 16 * a.wave + a.r)] = f;
+      placed64(cb, rowValue64(classes, j) + 256 * i) = f;
     });
   });
   waveExchange();
+  const int samples = samplePlace64(a.wave, 0, a.r, 2 * a.l);
   float4 z[2][4];
   staticFor<2>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
@@ -775,8 +799,8 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
     c32 f[4], g[4];
     staticFor<4>([&](auto kk) {
       constexpr int k = decltype(kk)::value;
-      f[k] = cb[rowPlace64(k, 2 * a.l, 32 * i + 16 * a.wave + a.r)];
-      g[k] = cb[rowPlace64(k, 2 * a.l + 1, 32 * i + 16 * a.wave + a.r)];
+      f[k] = placed64(cb, rowClass64(values, k, 0) + 256 * i);
+      g[k] = placed64(cb, rowClass64(values, k, 1) + 256 * i);
     });
     regFFT<4, false>(f);
     regFFT<4, false>(g);
@@ -785,13 +809,13 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
       z[i][m] = float4{f[slot<4>(m)].x, f[slot<4>(m)].y, g[slot<4>(m)].x, g[slot<4>(m)].y};
     });
   });
-  __syncthreads();  // every place is free: rows [y][column pair] from here on
+  waveExchange();  // every place of the wave is free: its samples from here on
   staticFor<2>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
     if (!any(i)) return;
     staticFor<4>([&](auto mm) {
       constexpr int m = decltype(mm)::value;
-      *reinterpret_cast<float4*>(cb + sampleAt64(32 * i + 16 * a.wave + a.r, 2 * a.l + 8 * m)) = z[i][m];
+      *reinterpret_cast<float4*>(&placed64(cb, (samples ^ 64 * (m & 1)) + 128 * (m & 2) + 8192 * i)) = z[i][m];
     });
   });
   waveExchange();
@@ -802,16 +826,16 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
     constexpr int i = decltype(ii)::value;
     if constexpr (FAST_REAL) {
       staticFor<4>([&](auto jj) {
-        const int y = 32 * i + 16 * a.wave + 4 * decltype(jj)::value + a.lane / 16, x4 = a.lane % 16;
-        streamStore(reinterpret_cast<float4*>(dst + (size_t)y * real.sy) + x4,
-                    *reinterpret_cast<const float4*>(cb + sampleAt64(y, 2 * x4)));
+        const int r = 4 * decltype(jj)::value + a.lane / 16, x4 = a.lane % 16;
+        streamStore(reinterpret_cast<float4*>(dst + (size_t)(32 * i + 16 * a.wave + r) * real.sy) + x4,
+                    *reinterpret_cast<const float4*>(&placed64(cb, samplePlace64(a.wave, i, r, 2 * x4))));
       });
     } else {
       if (!any(i)) return;
       float o[16];
       staticFor<16>([&](auto rr) {
         constexpr int r = decltype(rr)::value;
-        o[r] = reinterpret_cast<const float*>(cb + sampleAt64(32 * i + 16 * a.wave + r, a.lane / 2))[a.lane % 2];
+        o[r] = reinterpret_cast<const float*>(&placed64(cb, samplePlace64(a.wave, i, r, a.lane / 2)))[a.lane % 2];
       });
       const int x = a.lane - padL;
       if ((unsigned)x >= (unsigned)real.w) return;
