@@ -7,7 +7,7 @@
 // reference's external callers run (MM-inl.cuh:188-196): fbfft2D of both operands
 // into plane-major half spectra [d0][d1][N/2+1][N], transposeMM with the role's
 // conjugation, fbifft2D with crop on store.  All three stages are this library's
-// own kernels (fft2dLargeForward, transposeMMKernel, fft2dLargeInverse); the
+// own kernels (fft2d64/128Forward, transposeMM's, fft2d64/128Inverse); the
 // spectra live in the caller's workspace and cross HBM once each way.
 #include "common.h"
 
