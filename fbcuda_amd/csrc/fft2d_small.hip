@@ -426,6 +426,12 @@ bool dense(const RealView& r, int groups) {
          groups >= 4 * computeUnits();
 }
 
+// Inverse, the stream writes every float of a window from LDS, so the transform has to cover the window whole: one that
+// hangs over its edge, or is larger, keeps what it held there (and P of them need not fit in LDS).
+bool covered(int N, const RealView& r, int padL, int padU) {
+  return (long)padL + r.w <= N && (long)padU + r.h <= N;
+}
+
 // Forward, the loads of every other column meet in the L1, and the turn through LDS pays where waves would
 // otherwise take two groups, or, at 16 points, rows do not move as pairs, up to there (us, Window -> Dense):
 // 100000 windows of 7 x 7 in 8 points 11.4 -> 8.2, of 5 x 6 11.1 -> 8.0, 36000 of 13 x 13 in 16 15.0 -> 13.0, 20000
@@ -474,7 +480,9 @@ template <int N, bool PACKED>
 int launchInverse(const CplxView& cplx, const RealView& real, int padL, int padU, hipStream_t s) {
   using C = SmallCfg<N, PACKED>;
   const int groups = ceilDiv(real.B, C::P);
-  const int mode = fastReal(N, real, padL, padU) ? Whole : dense(real, groups) ? Dense : Window;
+  const int mode = fastReal(N, real, padL, padU)                               ? Whole
+                   : covered(N, real, padL, padU) && dense(real, groups) ? Dense
+                                                                               : Window;
   dim3 block(64);
   withModes(mode, fastCplx(N, cplx), [&](auto m, auto fc) {
     constexpr int M = decltype(m)::value;

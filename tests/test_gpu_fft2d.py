@@ -390,3 +390,31 @@ def test_windows_that_move_as_streams(oracle, N, B, h, w, padL, padU):
     at = np.unique(np.r_[0:16, B // 2:B // 2 + 16, B - 40:B])
     assert rel(spec[:B].cpu().numpy()[at], oracle.dft2d_r2c(x.cpu().numpy()[at], N, padL, padU)) < TOL_FFT
     assert rel(back.cpu().numpy(), N * N * x.cpu().numpy().astype(np.float64)) < TOL_FFT * np.sqrt(N * N / (h * w))
+
+
+# windows one after the other in memory, in batches that move as streams, that reach past the transform's right edge,
+# its bottom edge or both, or are larger than it: what it does not cover keeps what it held
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("N", [8, 16, 32])
+@pytest.mark.parametrize("dh,dw,padL,padU", [(0, 0, 1, 0), (0, 0, 0, 1), (-1, -2, 5, 3), (0, 3, 0, 0), (2, 0, 0, 0),
+                                             (5, 7, 2, 3), (0, 0, 1 << 30, 0), (-3, 0, 0, 2147483647)])
+def test_inverse_windows_past_the_transform(oracle, N, packed, dh, dw, padL, padU):
+    B, h, w = 4096 * 32 // N + 3, N + dh, N + dw
+    d = dev()
+    x = synth.normal((B, N, N), seed=N).to(d)
+    spec = torch.empty((B, N // 2 + (not packed), N, 2), device=d)
+    assert F.fbfft2D(x, spec) == F.Success
+    flat = torch.full((B * h * w + 8,), 7.0, device=d)
+    back = flat[:B * h * w].view(B, h, w)
+    assert F.fbifft2D(spec, back, padL, padU) == F.Success
+    torch.cuda.synchronize()
+    ch, cw = max(0, min(h, N - padU)), max(0, min(w, N - padL))
+    assert bool((flat[B * h * w:] == 7.0).all())
+    assert bool((back[:, ch:] == 7.0).all()) and bool((back[:, :, cw:] == 7.0).all())
+    if ch and cw:
+        want = N * N * x[:, padU:padU + ch, padL:padL + cw].double()
+        got = back[:, :ch, :cw].double()
+        assert float((got - want).norm() / want.norm()) < TOL_FFT * np.sqrt(N * N / (ch * cw))
+        at = np.r_[0:8, B - 8:B]
+        rc, ref = oracle.fbifft2d(oracle.fbfft2d(x.cpu().numpy()[at], N)[1], N, N)
+        assert rc == 0 and rel(got.cpu().numpy()[at], ref[:, padU:padU + ch, padL:padL + cw]) < TOL_FFT
