@@ -506,8 +506,14 @@ __global__ __launch_bounds__(k1dThreads, 4) void fft1d256Forward(const float* __
     const c32 e2 = c32{a.x + b.x, a.y - b.y};
     const c32 root = tw[(k0 + 16 * i) & 255];
     const c32 t = cmul(c32{a.y + b.y, b.x - a.x}, c32{0.5f * root.x, 0.5f * root.y});
-    out[k0 + 16 * i] = c32{__builtin_fmaf(0.5f, e2.x, t.x), __builtin_fmaf(0.5f, e2.y, t.y)};
-    out[128 - k0 - 16 * i] = c32{__builtin_fmaf(0.5f, e2.x, -t.x), __builtin_fmaf(-0.5f, e2.y, t.y)};
+    c32 f = c32{__builtin_fmaf(0.5f, e2.x, t.x), __builtin_fmaf(0.5f, e2.y, t.y)};
+    c32 fh = c32{__builtin_fmaf(0.5f, e2.x, -t.x), __builtin_fmaf(-0.5f, e2.y, t.y)};
+    if constexpr (i == 0) {  // F[0] and F[128] are real, whatever Z[0] is, and overflow only with their own sums
+      f = choose(lane0, c32{a.x + a.y, 0.0f}, f);
+      fh = choose(lane0, c32{a.x - a.y, 0.0f}, fh);
+    }
+    out[k0 + 16 * i] = f;
+    out[128 - k0 - 16 * i] = fh;
   });
   if (lane0) out[64] = cconj(u[slot<8>(4)]);
   waveExchange();
@@ -571,6 +577,7 @@ __global__ __launch_bounds__(k1dThreads, 4) void fft1d256Inverse(const float* __
     const c32 o = cmul(c32{a.x - b.x, a.y + b.y}, tw[(k0 + 16 * i) & 255]);
     zk[i] = c32{e.x - o.y, e.y + o.x};
     zh[i] = c32{e.x + o.y, o.x - e.y};
+    if constexpr (i == 0) zk[0] = choose(lane0, c32{a.x + b.x, a.x - b.x}, zk[0]);  // (no products with zeros)
   });
   const c32 middle = from[64];
   waveExchange();
@@ -591,7 +598,7 @@ __global__ __launch_bounds__(k1dThreads, 4) void fft1d256Inverse(const float* __
     constexpr int l = decltype(ll)::value;
     c32 a = u[slot<8>(l)], b = w[slot<8>(l)];
     if constexpr (l > 0) {
-      a = cmul(a, tw[2 * l * c.p]);
+      a = choose(lane0, a, cmul(a, tw[2 * l * c.p]));  // an infinite F[0] or F[128] stays one in every sample
       b = cmul(b, tw[2 * l * c.second]);
     }
     buf[exchangeAt(c, c.p, l)] = a;

@@ -209,3 +209,34 @@ def test_ends_of_workgroups(oracle, N, B):
     bar = np.sqrt(2 * (np.log2(N) + 2)) * 2.0 ** -24
     assert rel(spec[:B].cpu().numpy()[at], oracle.dft1d_r2c(x.numpy()[at])) < bar
     assert rel(back[:B].cpu().numpy(), N * x.numpy().astype(np.float64)) < 2 * bar
+
+
+@pytest.mark.parametrize("N", [8, 32, 64, 128, 256])
+def test_ends_of_spectra_near_and_beyond_the_largest_float(N):
+    """F[0] and F[N/2] are real and overflow only where their own sum does; and backwards a finite pair of them
+    gives finite samples, an infinite one infinities of its signs."""
+    inf, nan = float("inf"), float("nan")
+    d = dev()
+    x = torch.zeros(5, N)
+    x[0, 0], x[0, 1] = 2e38, -1e38
+    x[1, 3], x[2, 4], x[3, 2] = inf, -inf, nan
+    x[4, N // 2], x[4, N // 2 + 1] = -3e38, 3e38
+    spec = torch.full((5, N // 2 + 1, 2), 7.0, device=d)
+    assert F.fbfft1D(x.to(d), spec) == F.Success
+    back = torch.zeros(5, N // 2 + 1, 2)
+    back[0, 0, 0], back[0, -1, 0] = inf, 1.0
+    back[1, 0, 0], back[1, -1, 0] = 1.0, inf
+    back[2, 0, 0], back[2, -1, 0] = 1.5e38, 1e38
+    back[3, 0, 0], back[3, -1, 0] = -2e38, -1e38
+    back[4, 0, 0], back[4, -1, 0] = 2.0, -inf
+    y = torch.full((5, N), 7.0, device=d)
+    assert F.fbifft1D(y, back.to(d)) == F.Success
+    torch.cuda.synchronize()
+    ends = spec[:, [0, N // 2]].cpu()
+    assert bool((ends[..., 1] == 0.0).all())
+    want = torch.tensor([x[0, :2].tolist(), x[4, N // 2:N // 2 + 2].tolist()])
+    assert torch.equal(ends[[0, 4], 0, 0], want.sum(1)) and bool(torch.isinf(ends[4, 1, 0]))
+    assert torch.equal(ends[0, 1, 0], want[0, 0] - want[0, 1])
+    even = 1.0 - 2.0 * (torch.arange(N) % 2)
+    assert torch.equal(y.cpu(), torch.stack([torch.full((N,), inf), inf * even, 1.5e38 + 1e38 * even, -2e38 - 1e38 * even,
+                                             -inf * even]))
