@@ -72,6 +72,18 @@ __device__ __forceinline__ Lane128 lane128(int t) {
   return a;
 }
 
+// four floats that start at any float
+typedef float AnyFour __attribute__((ext_vector_type(4), aligned(4)));
+
+// Planes whose samples lie between those of their neighbours share cache lines: an XCD, every eighth
+// workgroup, takes consecutive ones.
+__host__ __device__ __forceinline__ bool interleaved(const RealView& r) { return r.sb > -32 && r.sb < 32 && r.B > 1; }
+__device__ __forceinline__ int planeOf(const RealView& r) {
+  const int b = blockIdx.x;
+  return interleaved(r) ? b % 8 * ((r.B + 7) / 8) + b / 8 : b;
+}
+dim3 planeGrid(const RealView& r) { return dim3(interleaved(r) ? (r.B + 7) / 8 * 8 : r.B); }
+
 // what the wave wrote to LDS is there for all of its lanes
 __device__ __forceinline__ void waveExchange() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -479,7 +491,8 @@ __device__ __forceinline__ constexpr int rowClass64(int base, int k, int e) {
 }
 // value l of class k of a column is y = 8 k + (l ^ k): from base = 8 at64(column, 9 k) base ^ 8 l, and from 8 at64(column, l)
 __device__ __forceinline__ constexpr int columnClass64(int base, int k) { return (base ^ 8 * (9 * k & 15)) + 8 * (9 * k & 48); }
-// where the inverse leaves the packed value j of row 32 i + 16 wave + r: among the places of the wave's rows
+// where the packed value j of row 32 i + 16 wave + r waits, before the forward transform and behind the inverse: among the
+// places of the wave's rows
 __device__ __forceinline__ constexpr int samplePlace64(int wave, int i, int r, int j) {
   return 8 * (1024 * i + 64 * r + 32 * (j >> 4) + 16 * wave + ((j & 15) ^ (8 * (r & 1))));
 }
@@ -500,7 +513,8 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
   __shared__ __align__(8) c32 roots[kLanes64 / 64][64];  // a wave's own: no barrier
   const Lane64 a = lane64(threadIdx.x);
   c32* const tw = roots[a.wave];
-  const int b = blockIdx.x;
+  const int b = FAST_REAL ? blockIdx.x : planeOf(real);
+  if (!FAST_REAL && b >= real.B) return;
   // whether a wave's rows 32 i + 16 wave ... + 15 hold a row of the window
   auto any = [&](int i) __attribute__((always_inline)) {
     const int y = 32 * i + 16 * a.wave;
@@ -516,21 +530,73 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
       staticFor<4>([&](auto mm) { z[i][decltype(mm)::value] = row[4 * decltype(mm)::value]; });
     });
   } else {
-    // implicit zero padding, any strides: loads at places clamped into the window, no branch
-    // between them, and what lies outside counts as zero; whole words where the window has only such
-    const bool words = real.sx == 1 && ((real.sy | real.sb | padL | real.w) & 3) == 0 &&
-                       (reinterpret_cast<uintptr_t>(real.data) & 15) == 0;
-    staticFor<2>([&](auto ii) {
-      constexpr int i = decltype(ii)::value;
-      const int y = 32 * i + 16 * a.wave + a.r - padU;
-      const bool yIn = (unsigned)y < (unsigned)real.h;
-      const float* row = src + (size_t)min(max(y, 0), real.h - 1) * real.sy;
-      if (any(i) && words) {
+    // implicit zero padding, any strides: loads at places clamped into the window, no branch between them, and
+    // what lies outside counts as zero.  Samples side by side move four at a time, from any float on; the words that the
+    // window's ends cut (at places that are the same for every row) are shifted into place.  Others move one by
+    // one, and where neighbours of a row share cache lines a wave takes row after row and turns them in LDS.  us, four
+    // lanes to a row one by one / so: 1763 whole planes 4 bytes off 16 20.2 / 12.6, 2594 windows of 61 x 61 in rows of 64
+    // 27.4 / 17.6; 2000 planes of every second float 22.6 / 17.7, every third 22.8 / 21.9, every sixth 35.3 / 35.6, 300 of
+    // every fourth 10.2 / 8.5, of every eighth 11.6 / 12.0.
+    const bool words = real.sx == 1 && real.w >= 4;
+    const int sx = abs(real.sx);
+    const bool byRow = !words && real.w >= 4 && sx > 0 && sx <= 6 && sx <= abs(real.sy);
+    auto rowAt = [&](int y) __attribute__((always_inline)) {
+      return src + (size_t)min(max(y - padU, 0), real.h - 1) * real.sy;
+    };
+    if (byRow) {
+      const int x = min(max(a.lane - padL, 0), real.w - 1);
+      staticFor<2>([&](auto ii) {
+        constexpr int i = decltype(ii)::value;
+        if (!any(i)) return;
+        float in[16];
+        staticFor<16>([&](auto rr) {
+          constexpr int r = decltype(rr)::value;
+          in[r] = rowAt(32 * i + 16 * a.wave + r)[(size_t)x * real.sx];
+        });
+        staticFor<16>([&](auto rr) {
+          constexpr int r = decltype(rr)::value;
+          reinterpret_cast<float*>(&placed64(cb, samplePlace64(a.wave, i, r, a.lane / 2)))[a.lane % 2] = in[r];
+        });
+      });
+      waveExchange();
+      staticFor<8>([&](auto mm) {
+        constexpr int i = decltype(mm)::value / 4, m = decltype(mm)::value % 4;
+        z[i][m] = *reinterpret_cast<const float4*>(&placed64(cb, samplePlace64(a.wave, i, a.r, 2 * a.l + 8 * m)));
+      });
+    } else if (words) {
+      staticFor<2>([&](auto ii) {
+        constexpr int i = decltype(ii)::value;
+        if (!any(i)) return;
+        const float* const row = rowAt(32 * i + 16 * a.wave + a.r);
         staticFor<4>([&](auto mm) {
           constexpr int m = decltype(mm)::value;
-          z[i][m] = *reinterpret_cast<const float4*>(row + min(max(4 * a.l + 16 * m - padL, 0), real.w - 4));
+          const AnyFour f = *reinterpret_cast<const AnyFour*>(row + min(max(4 * a.l + 16 * m - padL, 0), real.w - 4));
+          z[i][m] = float4{f[0], f[1], f[2], f[3]};
         });
-      } else if (any(i)) {
+      });
+      const int cutLeft = padL & 3, cutRight = -(padL + real.w) & 3;
+      if ((cutLeft | cutRight) != 0) {
+        staticFor<8>([&](auto mm) {
+          constexpr int i = decltype(mm)::value / 4, m = decltype(mm)::value % 4;
+          const int x = 4 * a.l + 16 * m - padL;
+          const float4 f = z[i][m];
+          if (x > real.w - 4 && x < real.w) {  // from float cutRight on
+            z[i][m].x = cutRight == 1 ? f.y : cutRight == 2 ? f.z : f.w;
+            z[i][m].y = cutRight == 1 ? f.z : f.w;
+            z[i][m].z = f.w;
+          }
+          if (x < 0 && x > -4) {  // the first float goes to cutLeft
+            z[i][m].y = f.x;
+            z[i][m].z = cutLeft == 1 ? f.y : f.x;
+            z[i][m].w = cutLeft == 1 ? f.z : cutLeft == 2 ? f.y : f.x;
+          }
+        });
+      }
+    } else {
+      staticFor<2>([&](auto ii) {
+        constexpr int i = decltype(ii)::value;
+        if (!any(i)) return;
+        const float* const row = rowAt(32 * i + 16 * a.wave + a.r);
         staticFor<4>([&](auto mm) {
           constexpr int m = decltype(mm)::value;
           const int x = 4 * a.l + 16 * m - padL;
@@ -539,15 +605,16 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
           z[i][m].z = row[(size_t)min(max(x + 2, 0), real.w - 1) * real.sx];
           z[i][m].w = row[(size_t)min(max(x + 3, 0), real.w - 1) * real.sx];
         });
-      }
-      staticFor<4>([&](auto mm) {
-        constexpr int m = decltype(mm)::value;
-        const int x = 4 * a.l + 16 * m - padL;
-        z[i][m].x = yIn && (unsigned)x < (unsigned)real.w ? z[i][m].x : 0.0f;
-        z[i][m].y = yIn && (unsigned)(x + 1) < (unsigned)real.w ? z[i][m].y : 0.0f;
-        z[i][m].z = yIn && (unsigned)(x + 2) < (unsigned)real.w ? z[i][m].z : 0.0f;
-        z[i][m].w = yIn && (unsigned)(x + 3) < (unsigned)real.w ? z[i][m].w : 0.0f;
       });
+    }
+    staticFor<8>([&](auto mm) {
+      constexpr int i = decltype(mm)::value / 4, m = decltype(mm)::value % 4;
+      const bool yIn = (unsigned)(32 * i + 16 * a.wave + a.r - padU) < (unsigned)real.h;
+      const int x = 4 * a.l + 16 * m - padL;
+      z[i][m].x = yIn && (unsigned)x < (unsigned)real.w ? z[i][m].x : 0.0f;
+      z[i][m].y = yIn && (unsigned)(x + 1) < (unsigned)real.w ? z[i][m].y : 0.0f;
+      z[i][m].z = yIn && (unsigned)(x + 2) < (unsigned)real.w ? z[i][m].z : 0.0f;
+      z[i][m].w = yIn && (unsigned)(x + 3) < (unsigned)real.w ? z[i][m].w : 0.0f;
     });
   }
   fillRoots64<true>(tw, a.lane);
@@ -683,7 +750,8 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
   __shared__ __align__(8) c32 roots[kLanes64 / 64][64];  // a wave's own: no barrier
   const Lane64 a = lane64(threadIdx.x);
   c32* const tw = roots[a.wave];
-  const int b = blockIdx.x;
+  const int b = FAST_REAL ? blockIdx.x : planeOf(real);
+  if (!FAST_REAL && b >= real.B) return;
   auto any = [&](int i) __attribute__((always_inline)) {
     const int y = 32 * i + 16 * a.wave;
     return FAST_REAL || (real.w > 0 && real.h > 0 && y < padU + real.h && y + 16 > padU);
@@ -858,8 +926,8 @@ bool fastCplx(int N, const CplxView& c) {
 }
 
 int launchForward64(const RealView& real, const CplxView& cplx, int padL, int padU, hipStream_t s) {
-  dim3 grid(real.B), block(kLanes64);
   const bool fr = fastReal(64, real, padL, padU), fc = fastCplx(64, cplx);
+  const dim3 grid = fr ? dim3(real.B) : planeGrid(real), block(kLanes64);
   if (fr && fc)
     fft2d64Forward<true, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
   else if (fc)
@@ -872,8 +940,8 @@ int launchForward64(const RealView& real, const CplxView& cplx, int padL, int pa
 }
 
 int launchInverse64(const CplxView& cplx, const RealView& real, int padL, int padU, hipStream_t s) {
-  dim3 grid(real.B), block(kLanes64);
   const bool fr = fastReal(64, real, padL, padU), fc = fastCplx(64, cplx);
+  const dim3 grid = fr ? dim3(real.B) : planeGrid(real), block(kLanes64);
   if (fr && fc)
     fft2d64Inverse<true, true><<<grid, block, 0, s>>>(cplx, real, padL, padU);
   else if (fc)

@@ -418,3 +418,32 @@ def test_inverse_windows_past_the_transform(oracle, N, packed, dh, dw, padL, pad
         at = np.r_[0:8, B - 8:B]
         rc, ref = oracle.fbifft2d(oracle.fbfft2d(x.cpu().numpy()[at], N)[1], N, N)
         assert rc == 0 and rel(got.cpu().numpy()[at], ref[:, padU:padU + ch, padL:padL + cw]) < TOL_FFT
+
+
+# how the 64-point forward transform reads: four samples at a time from any float on, windows whose ends cut such words
+# on either side at each place, windows narrower than one, samples that lie 2 and 7 apart, turned planes, and batches whose
+# planes lie between each other
+@pytest.mark.parametrize("h,w,padL,padU", [(64, 64, 0, 0), (61, 61, 2, 1), (50, 62, 1, 9), (33, 59, 4, 31), (7, 4, 59, 50),
+                                           (64, 5, 3, 0), (20, 6, 58, 44), (40, 7, 30, 10), (9, 3, 61, 3), (12, 1, 17, 0),
+                                           (64, 63, 7, 5), (30, 64, 62, 40)])
+@pytest.mark.parametrize("layout", ["off1", "off3", "gap", "apart2", "apart7", "turned", "between"])
+def test_forward_64_reads_any_layout(oracle, layout, h, w, padL, padU):
+    B, d = 37, dev()
+    x = synth.normal((B, h, w), seed=h + w)
+    at = {"off1": lambda: torch.empty(B * h * w + 1, device=d)[1:].view(B, h, w),
+          "off3": lambda: torch.empty(B * h * w + 3, device=d)[3:].view(B, h, w),
+          "gap": lambda: torch.full((B, h + 1, 64 + 4), float("nan"), device=d)[:, 1:, 2:2 + w],
+          "apart2": lambda: torch.full((B, h, w, 2), float("nan"), device=d)[..., 1],
+          "apart7": lambda: torch.full((B, h, w, 7), float("nan"), device=d)[..., 3],
+          "turned": lambda: torch.empty((B, w, h), device=d).transpose(1, 2),
+          "between": lambda: torch.empty((h, w, B), device=d).permute(2, 0, 1)}[layout]()
+    at.copy_(x)
+    spec = torch.full((B + 1, 33, 64, 2), 7.0, device=d)
+    assert F.fbfft2D(at, spec[:B], padL, padU) == F.Success
+    torch.cuda.synchronize()
+    assert bool((spec[B] == 7.0).all())
+    plane = np.zeros((B, 64, 64), np.float32)
+    ch, cw = min(h, 64 - padU), min(w, 64 - padL)
+    plane[:, padU:padU + ch, padL:padL + cw] = x.numpy()[:, :ch, :cw]
+    rc, want = oracle.fbfft2d(plane, 64)
+    assert rc == 0 and per_plane_rel(spec[:B].cpu().numpy(), want) < TOL_FFT
