@@ -25,8 +25,7 @@
 // -> this: 4096 planes of 128 x 128 101.5 / 96.5 -> 87.4 / 91.0, 19 planes 8.4 / 8.0 -> 6.2 / 6.2, 3773 windows of
 // 73 x 91 87.0 / 85.9 -> 64.7 / 75.2; 16384 of 64 x 64 95.2 / 85.7 -> 84.4 / 84.1, 53 6.6 / 5.7 -> 4.2 / 4.6, 3247 of 36
 // x 58 22.0 / 22.8 -> 18.9 / 22.2; buffers from HBM, 5000 of 64 x 64 33.7 / 33.0 -> 29.9 / 31.5, 3000 of 60 x 60 23.8
-// / 25.5 -> 23.4 / 26.4, of 50 x 50 21.7 / 23.5 -> 17.8 / 25.6 (little over one round of workgroups, whose inverse
-// lost; fewer workgroups per CU or nontemporal loads make it worse).  At 128 points LDS was the limit while its accesses collided
+// / 26.5 -> 23.4 / 23.5, of 50 x 50 21.7 / 23.8 -> 17.8 / 21.7.  At 128 points LDS was the limit while its accesses collided
 // (places from column to column 136 apart: 22.4 of 38.3 million active cycles, 94 / 105 us; 130: 3.6 of 19.4).
 #include "common.h"
 #include "fft_lds.h"
@@ -900,6 +899,45 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
       });
     } else {
       if (!any(i)) return;
+      const int w = min(real.w, 64 - padL);
+      if (real.sx == 1 && w >= 4) {
+        // words of four to any float; a row's last one may cover some of the one before, of the same values.  us, a row
+        // float by float / so: 463 windows of 56 x 56 8.5 / 6.9, 3000 of 50 x 50 to HBM 25.4 / 21.7 (plain stores 23.4), of 60 x
+        // 60 27.5 / 23.5, 16384 of 60 x 60 98.7 / 93.5 (99.4), 2669 whole planes 4 bytes off 26.4 / 22.0.  Rows with gaps between
+        // them leave cache lines partly written: 3137 of 64 x 64 in rows of 67 25.4 / 22.3, nontemporal 27.5.
+        const int x = min(4 * (a.lane % 16), w - 4), from = padL + x, cut = from & 3;
+        const int first = 32 * i + 16 * a.wave + a.lane / 16 - padU;
+        auto word = [&](int j, int k) __attribute__((always_inline)) {
+          return *reinterpret_cast<const float4*>(&placed64(cb, samplePlace64(a.wave, i, 4 * j + a.lane / 16, 2 * k)));
+        };
+        float4 o[4];
+        staticFor<4>([&](auto jj) { o[decltype(jj)::value] = word(decltype(jj)::value, from / 4); });
+        if (((padL | w) & 3) != 0) {
+          staticFor<4>([&](auto jj) {
+            constexpr int j = decltype(jj)::value;
+            const float4 f = o[j], g = word(j, min(from / 4 + 1, 15));
+            const bool odd = cut & 1, two = cut & 2;
+            const float p0 = odd ? f.y : f.x, p1 = odd ? f.z : f.y, p2 = odd ? f.w : f.z, p3 = odd ? g.x : f.w,
+                        p4 = odd ? g.y : g.x, p5 = odd ? g.z : g.y;
+            o[j] = float4{two ? p2 : p0, two ? p3 : p1, two ? p4 : p2, two ? p5 : p3};
+          });
+        }
+        if (4 * (a.lane % 16) >= w) return;
+        auto rows = [&](auto write) __attribute__((always_inline)) {
+          staticFor<4>([&](auto jj) {
+            constexpr int j = decltype(jj)::value;
+            if ((unsigned)(first + 4 * j) < (unsigned)real.h)
+              write(reinterpret_cast<AnyFour*>(dst + (size_t)(first + 4 * j) * real.sy + x), AnyFour{o[j].x, o[j].y, o[j].z, o[j].w});
+          });
+        };
+        if (real.sy == real.w) {
+          rows([](AnyFour* to, AnyFour f) { __builtin_nontemporal_store(f, to); });
+        } else {
+          asm volatile("");  // (or both become plain stores)
+          rows([](AnyFour* to, AnyFour f) { *to = f; });
+        }
+        return;
+      }
       float o[16];
       staticFor<16>([&](auto rr) {
         constexpr int r = decltype(rr)::value;

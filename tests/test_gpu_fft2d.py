@@ -447,3 +447,33 @@ def test_forward_64_reads_any_layout(oracle, layout, h, w, padL, padU):
     plane[:, padU:padU + ch, padL:padL + cw] = x.numpy()[:, :ch, :cw]
     rc, want = oracle.fbfft2d(plane, 64)
     assert rc == 0 and per_plane_rel(spec[:B].cpu().numpy(), want) < TOL_FFT
+
+
+# how the 64-point inverse writes: four samples at a time to any float, row ends within a word at each place, windows that hang over
+# the transform's right edge or its bottom (what is not covered keeps what it held), narrower ones, and other layouts
+@pytest.mark.parametrize("h,w,padL,padU", [(64, 64, 0, 0), (61, 61, 2, 1), (50, 62, 1, 9), (33, 59, 4, 31), (7, 9, 59, 50),
+                                           (64, 5, 3, 0), (20, 6, 58, 44), (40, 7, 30, 10), (9, 3, 61, 3), (12, 1, 17, 0),
+                                           (64, 63, 7, 5), (30, 64, 62, 40), (70, 81, 0, 3), (8, 8, 64, 0)])
+@pytest.mark.parametrize("layout", ["off1", "off3", "gap", "apart2", "turned", "between"])
+def test_inverse_64_writes_any_layout(oracle, layout, h, w, padL, padU):
+    B, d = 37, dev()
+    spec = oracle.fbfft2d(synth.normal((B, 64, 64), seed=h + w).numpy(), 64)[1]
+    n = B * h * w
+    flat = torch.full((2 * n + 100 * B * (h + 1) + 8,), 7.0, device=d)
+    view = {"off1": flat[1:1 + n].view(B, h, w), "off3": flat[3:3 + n].view(B, h, w),
+            "gap": flat[:B * (h + 1) * 100].view(B, h + 1, 100)[:, 1:, 2:2 + w],
+            "apart2": flat[:2 * n].view(B, h, w, 2)[..., 1], "turned": flat[:n].view(B, w, h).transpose(1, 2),
+            "between": flat[:n].view(h, w, B).permute(2, 0, 1)}[layout]
+    assert F.fbifft2D(torch.from_numpy(spec).to(d), view, padL, padU) == F.Success
+    torch.cuda.synchronize()
+    got = view.cpu().numpy().copy()
+    view.fill_(7.0)
+    assert bool((flat == 7.0).all())
+    ch, cw = max(0, min(h, 64 - padU)), max(0, min(w, 64 - padL))
+    assert (got[:, ch:] == 7.0).all() and (got[:, :, cw:] == 7.0).all()
+    if ch and cw:
+        rc, full = oracle.fbifft2d(spec, 64, 64)
+        want = full[:, padU:padU + ch, padL:padL + cw]
+        # (of a few samples the largest may be small beside the others' roundings: the bar is on the plane's scale)
+        err = np.abs(got[:, :ch, :cw].astype(np.float64) - want).max() / np.sqrt((full.astype(np.float64) ** 2).mean())
+        assert rc == 0 and err < TOL_FFT
