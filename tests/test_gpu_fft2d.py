@@ -477,3 +477,23 @@ def test_inverse_64_writes_any_layout(oracle, layout, h, w, padL, padU):
         # (of a few samples the largest may be small beside the others' roundings: the bar is on the plane's scale)
         err = np.abs(got[:, :ch, :cw].astype(np.float64) - want).max() / np.sqrt((full.astype(np.float64) ** 2).mean())
         assert rc == 0 and err < TOL_FFT
+
+
+# spectra that lie in memory the other way round, [ky][kx], and so with gaps between rows and values
+@pytest.mark.parametrize("N,B,h,w,padL,padU", [(64, 1, 64, 64, 0, 0), (64, 9, 40, 51, 3, 20), (128, 1, 128, 128, 0, 0),
+                                               (128, 7, 128, 128, 0, 0), (128, 5, 77, 101, 9, 30), (128, 300, 31, 128, 0, 97)])
+@pytest.mark.parametrize("gaps", [False, True])
+def test_turned_spectra(oracle, N, B, h, w, padL, padU, gaps):
+    d = dev()
+    x = synth.normal((B, h, w), seed=N + B)
+    hold = torch.full((B + 1, N + gaps, N // 2 + 1 + 2 * gaps, 2), 7.0, device=d)
+    view = hold[:B, gaps:, gaps:gaps + N // 2 + 1].transpose(1, 2)
+    assert F.fbfft2D(x.to(d), view, padL, padU) == F.Success
+    back = torch.full((B, h, w), float("nan"), device=d)
+    assert F.fbifft2D(view, back, padL, padU) == F.Success
+    torch.cuda.synchronize()
+    rc, want = oracle.fbfft2d(x.numpy(), N, padL, padU)
+    assert rc == 0 and per_plane_rel(view.cpu().numpy(), want) < TOL_FFT
+    assert per_plane_rel(back.cpu().numpy(), N * N * x.numpy().astype(np.float64)) < TOL_FFT * np.sqrt(N * N / (h * w))
+    view.fill_(7.0)
+    assert bool((hold == 7.0).all())
