@@ -497,3 +497,23 @@ def test_turned_spectra(oracle, N, B, h, w, padL, padU, gaps):
     assert per_plane_rel(back.cpu().numpy(), N * N * x.numpy().astype(np.float64)) < TOL_FFT * np.sqrt(N * N / (h * w))
     view.fill_(7.0)
     assert bool((hold == 7.0).all())
+
+
+# batches whose planes lie between each other: consecutive planes share an XCD, and the grid ends on a multiple of eight
+@pytest.mark.parametrize("N,h,w", [(64, 64, 64), (64, 37, 50), (128, 128, 128), (128, 75, 110)])
+@pytest.mark.parametrize("B", [1, 2, 7, 8, 9, 45])
+def test_planes_between_each_other(oracle, N, h, w, B):
+    d = dev()
+    x = synth.normal((B, h, w), seed=N + B + h)
+    hold = torch.full((h, w, B + 2), 7.0, device=d)
+    view = hold[..., 1:1 + B].permute(2, 0, 1)
+    view.copy_(x)
+    spec = torch.full((B + 1, N // 2 + 1, N, 2), 7.0, device=d)
+    assert F.fbfft2D(view, spec[:B], N - w, 0) == F.Success
+    view.fill_(float("nan"))
+    assert F.fbifft2D(spec[:B], view, N - w, 0) == F.Success
+    torch.cuda.synchronize()
+    rc, want = oracle.fbfft2d(x.numpy(), N, N - w, 0)
+    assert rc == 0 and per_plane_rel(spec[:B].cpu().numpy(), want) < TOL_FFT
+    assert per_plane_rel(view.cpu().numpy(), N * N * x.numpy().astype(np.float64)) < TOL_FFT * np.sqrt(N * N / (h * w))
+    assert bool((spec[B] == 7.0).all()) and bool((hold[..., 0] == 7.0).all()) and bool((hold[..., B + 1] == 7.0).all())
