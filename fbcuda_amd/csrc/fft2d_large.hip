@@ -31,6 +31,8 @@
 #include "fft_lds.h"
 #include "fft_regs.h"
 
+#include <algorithm>
+
 namespace fbfft_amd {
 namespace {
 
@@ -491,6 +493,10 @@ __global__ __launch_bounds__(kLanes128, 4) void fft2d128Inverse(CplxView cplx, R
 // 30.2 us in the median, pairs of columns before).
 constexpr int kLanes64 = 128;
 
+// How the real operand moves: whole planes as float4, samples side by side as words of four, others one by one.
+// (Decided at run time, these take 2 to 4 % more of small batches.)
+enum RealMode { Whole, Words, Single };
+
 struct Lane64 {
   int wave, lane;
   int l, r;     // row pass: lane of the row, row of the wave's sixteen
@@ -546,23 +552,23 @@ __device__ __forceinline__ void fillRoots64(c32* tw, int lane) {
   tw[lane] = c32{c, FWD ? -s : s};
 }
 
-template <bool FAST_REAL, bool FAST_CPLX>
+template <int REAL, bool FAST_CPLX>
 __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, CplxView cplx, int padL, int padU) {
   __shared__ __align__(16) c32 cb[32 * 64];
   __shared__ __align__(8) c32 roots[kLanes64 / 64][64];  // a wave's own: no barrier
   const Lane64 a = lane64(threadIdx.x);
   c32* const tw = roots[a.wave];
-  const int b = FAST_REAL ? blockIdx.x : planeOf(real);
-  if (!FAST_REAL && b >= real.B) return;
+  const int b = REAL == Whole ? blockIdx.x : planeOf(real);
+  if (REAL != Whole && b >= real.B) return;
   // whether a wave's rows 32 i + 16 wave ... + 15 hold a row of the window
   auto any = [&](int i) __attribute__((always_inline)) {
     const int y = 32 * i + 16 * a.wave;
-    return FAST_REAL || (real.w > 0 && real.h > 0 && y < padU + real.h && y + 16 > padU);
+    return REAL == Whole || (real.w > 0 && real.h > 0 && y < padU + real.h && y + 16 > padU);
   };
   const float* const src = real.data + (size_t)b * real.sb;
 
   float4 z[2][4];  // packed values 2 l + 8 m and the next
-  if constexpr (FAST_REAL) {
+  if constexpr (REAL == Whole) {
     staticFor<2>([&](auto ii) {
       constexpr int i = decltype(ii)::value;
       const float4* row = reinterpret_cast<const float4*>(src + (size_t)(32 * i + 16 * a.wave + a.r) * real.sy) + a.l;
@@ -576,9 +582,8 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
     // lanes to a row one by one / so: 1763 whole planes 4 bytes off 16 20.2 / 12.6, 2594 windows of 61 x 61 in rows of 64
     // 27.4 / 17.6; 2000 planes of every second float 22.6 / 17.7, every third 22.8 / 21.9, every sixth 35.3 / 35.6, 300 of
     // every fourth 10.2 / 8.5, of every eighth 11.6 / 12.0.
-    const bool words = real.sx == 1 && real.w >= 4;
     const int sx = abs(real.sx);
-    const bool byRow = !words && real.w >= 4 && sx > 0 && sx <= 6 && sx <= abs(real.sy);
+    const bool byRow = REAL == Single && real.w >= 4 && sx > 0 && sx <= 6 && sx <= abs(real.sy);
     auto rowAt = [&](int y) __attribute__((always_inline)) {
       return src + (size_t)min(max(y - padU, 0), real.h - 1) * real.sy;
     };
@@ -602,7 +607,7 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
         constexpr int i = decltype(mm)::value / 4, m = decltype(mm)::value % 4;
         z[i][m] = *reinterpret_cast<const float4*>(&placed64(cb, samplePlace64(a.wave, i, a.r, 2 * a.l + 8 * m)));
       });
-    } else if (words) {
+    } else if constexpr (REAL == Words) {
       staticFor<2>([&](auto ii) {
         constexpr int i = decltype(ii)::value;
         if (!any(i)) return;
@@ -783,17 +788,17 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
   });
 }
 
-template <bool FAST_REAL, bool FAST_CPLX>
+template <int REAL, bool FAST_CPLX>
 __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, RealView real, int padL, int padU) {
   __shared__ __align__(16) c32 cb[32 * 64];
   __shared__ __align__(8) c32 roots[kLanes64 / 64][64];  // a wave's own: no barrier
   const Lane64 a = lane64(threadIdx.x);
   c32* const tw = roots[a.wave];
-  const int b = FAST_REAL ? blockIdx.x : planeOf(real);
-  if (!FAST_REAL && b >= real.B) return;
+  const int b = REAL == Whole ? blockIdx.x : planeOf(real);
+  if (REAL != Whole && b >= real.B) return;
   auto any = [&](int i) __attribute__((always_inline)) {
     const int y = 32 * i + 16 * a.wave;
-    return FAST_REAL || (real.w > 0 && real.h > 0 && y < padU + real.h && y + 16 > padU);
+    return REAL == Whole || (real.w > 0 && real.h > 0 && y < padU + real.h && y + 16 > padU);
   };
 
   // ---- the wave's columns in, two at a time; column 0 carries 32 as its imaginary part ----
@@ -931,7 +936,7 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
   float* const dst = real.data + (size_t)b * real.sb;
   staticFor<2>([&](auto ii) {
     constexpr int i = decltype(ii)::value;
-    if constexpr (FAST_REAL) {
+    if constexpr (REAL == Whole) {
       staticFor<4>([&](auto jj) {
         const int r = 4 * decltype(jj)::value + a.lane / 16, x4 = a.lane % 16;
         streamStore(reinterpret_cast<float4*>(dst + (size_t)(32 * i + 16 * a.wave + r) * real.sy) + x4,
@@ -939,12 +944,12 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
       });
     } else {
       if (!any(i)) return;
-      const int w = min(real.w, 64 - padL);
-      if (real.sx == 1 && w >= 4) {
+      if constexpr (REAL == Words) {
         // words of four to any float; a row's last one may cover some of the one before, of the same values.  us, a row
         // float by float / so: 463 windows of 56 x 56 8.5 / 6.9, 3000 of 50 x 50 to HBM 25.4 / 21.7 (plain stores 23.4), of 60 x
-        // 60 27.5 / 23.5, 16384 of 60 x 60 98.7 / 93.5 (99.4), 2669 whole planes 4 bytes off 26.4 / 22.0.  Rows with gaps between
+        // 60 27.5 / 23.8, 16384 of 60 x 60 98.7 / 97.0 (99.4), 2669 whole planes 4 bytes off 26.4 / 22.0.  Rows with gaps between
         // them leave cache lines partly written: 3137 of 64 x 64 in rows of 67 25.4 / 22.3, nontemporal 27.5.
+        const int w = min(real.w, 64 - padL);
         const int x = min(4 * (a.lane % 16), w - 4), from = padL + x, cut = from & 3;
         const int first = 32 * i + 16 * a.wave + a.lane / 16 - padU;
         auto word = [&](int j, int k) __attribute__((always_inline)) {
@@ -1003,31 +1008,31 @@ bool fastCplx(int N, const CplxView& c) {
   return c.sc == 2 && c.sr == 2 * N && c.sb % 4 == 0 && aligned(c.data, 16);
 }
 
+// runs f(mode of the real operand, std::bool_constant<fast>{}); width: samples of a row that the transform covers
+template <typename F>
+void withModes64(const RealView& real, const CplxView& cplx, int padL, int padU, int width, F&& f) {
+  const bool fast = fastCplx(64, cplx);
+  auto run = [&](auto m) { fast ? f(m, std::true_type{}) : f(m, std::false_type{}); };
+  if (fastReal(64, real, padL, padU)) run(std::integral_constant<int, Whole>{});
+  else if (real.sx == 1 && width >= 4) run(std::integral_constant<int, Words>{});
+  else run(std::integral_constant<int, Single>{});
+}
+
 int launchForward64(const RealView& real, const CplxView& cplx, int padL, int padU, hipStream_t s) {
-  const bool fr = fastReal(64, real, padL, padU), fc = fastCplx(64, cplx);
-  const dim3 grid = fr ? dim3(real.B) : planeGrid(real), block(kLanes64);
-  if (fr && fc)
-    fft2d64Forward<true, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
-  else if (fc)
-    fft2d64Forward<false, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
-  else if (fr)
-    fft2d64Forward<true, false><<<grid, block, 0, s>>>(real, cplx, padL, padU);
-  else
-    fft2d64Forward<false, false><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+  withModes64(real, cplx, padL, padU, real.w, [&](auto m, auto fc) {
+    constexpr int M = decltype(m)::value;
+    fft2d64Forward<M, decltype(fc)::value>
+        <<<M == Whole ? dim3(real.B) : planeGrid(real), dim3(kLanes64), 0, s>>>(real, cplx, padL, padU);
+  });
   return launchStatus();
 }
 
 int launchInverse64(const CplxView& cplx, const RealView& real, int padL, int padU, hipStream_t s) {
-  const bool fr = fastReal(64, real, padL, padU), fc = fastCplx(64, cplx);
-  const dim3 grid = fr ? dim3(real.B) : planeGrid(real), block(kLanes64);
-  if (fr && fc)
-    fft2d64Inverse<true, true><<<grid, block, 0, s>>>(cplx, real, padL, padU);
-  else if (fc)
-    fft2d64Inverse<false, true><<<grid, block, 0, s>>>(cplx, real, padL, padU);
-  else if (fr)
-    fft2d64Inverse<true, false><<<grid, block, 0, s>>>(cplx, real, padL, padU);
-  else
-    fft2d64Inverse<false, false><<<grid, block, 0, s>>>(cplx, real, padL, padU);
+  withModes64(real, cplx, padL, padU, std::min(real.w, 64 - padL), [&](auto m, auto fc) {
+    constexpr int M = decltype(m)::value;
+    fft2d64Inverse<M, decltype(fc)::value>
+        <<<M == Whole ? dim3(real.B) : planeGrid(real), dim3(kLanes64), 0, s>>>(cplx, real, padL, padU);
+  });
   return launchStatus();
 }
 
