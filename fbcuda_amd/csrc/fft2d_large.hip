@@ -76,15 +76,18 @@ __device__ __forceinline__ Lane128 lane128(int t) {
 // four floats that start at any float
 typedef float AnyFour __attribute__((ext_vector_type(4), aligned(4)));
 
-// Planes whose samples lie between those of their neighbours share cache lines: an XCD, every eighth workgroup, takes
+// Planes whose samples, or bins, lie between those of their neighbours share cache lines: an XCD, every eighth workgroup, takes
 // consecutive ones.  us, forward / inverse, neighbours on eight XCDs -> on one: 6436 windows of 55 x 40 in 64 points 164 / 172 -> 80 /
-// 82, 1652 of 110 x 97 in 128 164 / 232 -> 102 / 111, 100 of 128 x 128 from HBM 23.7 / 22.1 -> 24.8 / 20.4.
-__host__ __device__ __forceinline__ bool interleaved(const RealView& r) { return r.sb > -32 && r.sb < 32 && r.B > 1; }
-__device__ __forceinline__ int planeOf(const RealView& r) {
-  const int b = blockIdx.x;
-  return interleaved(r) ? b % 8 * ((r.B + 7) / 8) + b / 8 : b;
+// 82, 1652 of 110 x 97 in 128 164 / 232 -> 102 / 111, 100 of 128 x 128 from HBM 23.7 / 22.1 -> 24.8 / 20.4; spectra that do, 5000
+// planes of 64 x 64 146 / 154 -> 62 / 52 (one wave a plane, before, 152 / 139), 1300 of 128 x 128 156 / 140 -> 69 / 61 (160 / 128).
+__host__ __device__ __forceinline__ bool interleaved(const RealView& r, const CplxView& c) {
+  return (abs(r.sb) < 32 || abs(c.sb) < 32) && r.B > 1;
 }
-dim3 planeGrid(const RealView& r) { return dim3(interleaved(r) ? (r.B + 7) / 8 * 8 : r.B); }
+__device__ __forceinline__ int planeOf(const RealView& r, const CplxView& c) {
+  const int b = blockIdx.x;
+  return interleaved(r, c) ? b % 8 * ((r.B + 7) / 8) + b / 8 : b;
+}
+dim3 planeGrid(const RealView& r, const CplxView& c) { return dim3(interleaved(r, c) ? (r.B + 7) / 8 * 8 : r.B); }
 
 // Whether a spectrum's values of one ky lie closer together than those of one kx: a turned view, [ky][kx] in memory.
 // At 128 points these move a ky at a time, 64 columns to an instruction.  us, forward / inverse, a column at a time
@@ -113,8 +116,9 @@ __global__ __launch_bounds__(kLanes128, 4) void fft2d128Forward(RealView real, C
   __shared__ __align__(16) c32 cb[64 * kStride128];
   __shared__ __align__(8) c32 tw[256];
   const Lane128 a = lane128(threadIdx.x);
-  const int b = FAST_REAL ? blockIdx.x : planeOf(real);
-  if (!FAST_REAL && b >= real.B) return;
+  constexpr bool ANY = !FAST_REAL || !FAST_CPLX;
+  const int b = ANY ? planeOf(real, cplx) : blockIdx.x;
+  if (ANY && b >= real.B) return;
   // whether a wave's rows 64 i + 8 wave ... + 7 hold a row of the window
   auto any = [&](int i) __attribute__((always_inline)) {
     const int y = 64 * i + 8 * a.wave;
@@ -300,8 +304,9 @@ __global__ __launch_bounds__(kLanes128, 4) void fft2d128Inverse(CplxView cplx, R
   __shared__ __align__(16) c32 cb[64 * kStride128];
   __shared__ __align__(8) c32 tw[256];
   const Lane128 a = lane128(threadIdx.x);
-  const int b = FAST_REAL ? blockIdx.x : planeOf(real);
-  if (!FAST_REAL && b >= real.B) return;
+  constexpr bool ANY = !FAST_REAL || !FAST_CPLX;
+  const int b = ANY ? planeOf(real, cplx) : blockIdx.x;
+  if (ANY && b >= real.B) return;
   // whether a wave's rows 64 i + 8 wave ... + 7 hold a row of the window
   auto any = [&](int i) __attribute__((always_inline)) {
     const int y = 64 * i + 8 * a.wave;
@@ -558,8 +563,9 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Forward(RealView real, Cpl
   __shared__ __align__(8) c32 roots[kLanes64 / 64][64];  // a wave's own: no barrier
   const Lane64 a = lane64(threadIdx.x);
   c32* const tw = roots[a.wave];
-  const int b = REAL == Whole ? blockIdx.x : planeOf(real);
-  if (REAL != Whole && b >= real.B) return;
+  constexpr bool ANY = REAL != Whole || !FAST_CPLX;
+  const int b = ANY ? planeOf(real, cplx) : blockIdx.x;
+  if (ANY && b >= real.B) return;
   // whether a wave's rows 32 i + 16 wave ... + 15 hold a row of the window
   auto any = [&](int i) __attribute__((always_inline)) {
     const int y = 32 * i + 16 * a.wave;
@@ -794,8 +800,9 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
   __shared__ __align__(8) c32 roots[kLanes64 / 64][64];  // a wave's own: no barrier
   const Lane64 a = lane64(threadIdx.x);
   c32* const tw = roots[a.wave];
-  const int b = REAL == Whole ? blockIdx.x : planeOf(real);
-  if (REAL != Whole && b >= real.B) return;
+  constexpr bool ANY = REAL != Whole || !FAST_CPLX;
+  const int b = ANY ? planeOf(real, cplx) : blockIdx.x;
+  if (ANY && b >= real.B) return;
   auto any = [&](int i) __attribute__((always_inline)) {
     const int y = 32 * i + 16 * a.wave;
     return REAL == Whole || (real.w > 0 && real.h > 0 && y < padU + real.h && y + 16 > padU);
@@ -1021,8 +1028,8 @@ void withModes64(const RealView& real, const CplxView& cplx, int padL, int padU,
 int launchForward64(const RealView& real, const CplxView& cplx, int padL, int padU, hipStream_t s) {
   withModes64(real, cplx, padL, padU, real.w, [&](auto m, auto fc) {
     constexpr int M = decltype(m)::value;
-    fft2d64Forward<M, decltype(fc)::value>
-        <<<M == Whole ? dim3(real.B) : planeGrid(real), dim3(kLanes64), 0, s>>>(real, cplx, padL, padU);
+    constexpr bool FC = decltype(fc)::value;
+    fft2d64Forward<M, FC><<<M == Whole && FC ? dim3(real.B) : planeGrid(real, cplx), dim3(kLanes64), 0, s>>>(real, cplx, padL, padU);
   });
   return launchStatus();
 }
@@ -1030,15 +1037,15 @@ int launchForward64(const RealView& real, const CplxView& cplx, int padL, int pa
 int launchInverse64(const CplxView& cplx, const RealView& real, int padL, int padU, hipStream_t s) {
   withModes64(real, cplx, padL, padU, std::min(real.w, 64 - padL), [&](auto m, auto fc) {
     constexpr int M = decltype(m)::value;
-    fft2d64Inverse<M, decltype(fc)::value>
-        <<<M == Whole ? dim3(real.B) : planeGrid(real), dim3(kLanes64), 0, s>>>(cplx, real, padL, padU);
+    constexpr bool FC = decltype(fc)::value;
+    fft2d64Inverse<M, FC><<<M == Whole && FC ? dim3(real.B) : planeGrid(real, cplx), dim3(kLanes64), 0, s>>>(cplx, real, padL, padU);
   });
   return launchStatus();
 }
 
 int launchForward128(const RealView& real, const CplxView& cplx, int padL, int padU, hipStream_t s) {
   const bool fr = fastReal(128, real, padL, padU), fc = fastCplx(128, cplx);
-  const dim3 grid = fr ? dim3(real.B) : planeGrid(real), block(kLanes128);
+  const dim3 grid = fr && fc ? dim3(real.B) : planeGrid(real, cplx), block(kLanes128);
   if (fr && fc)
     fft2d128Forward<true, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
   else if (fc)
@@ -1052,7 +1059,7 @@ int launchForward128(const RealView& real, const CplxView& cplx, int padL, int p
 
 int launchInverse128(const CplxView& cplx, const RealView& real, int padL, int padU, hipStream_t s) {
   const bool fr = fastReal(128, real, padL, padU), fc = fastCplx(128, cplx);
-  const dim3 grid = fr ? dim3(real.B) : planeGrid(real), block(kLanes128);
+  const dim3 grid = fr && fc ? dim3(real.B) : planeGrid(real, cplx), block(kLanes128);
   if (fr && fc)
     fft2d128Inverse<true, true><<<grid, block, 0, s>>>(cplx, real, padL, padU);
   else if (fc)

@@ -517,3 +517,24 @@ def test_planes_between_each_other(oracle, N, h, w, B):
     assert rc == 0 and per_plane_rel(spec[:B].cpu().numpy(), want) < TOL_FFT
     assert per_plane_rel(view.cpu().numpy(), N * N * x.numpy().astype(np.float64)) < TOL_FFT * np.sqrt(N * N / (h * w))
     assert bool((spec[B] == 7.0).all()) and bool((hold[..., 0] == 7.0).all()) and bool((hold[..., B + 1] == 7.0).all())
+
+
+# and the same of spectra: one value of every plane, then the next (real planes whole, cut, and between each other as well)
+@pytest.mark.parametrize("N,h,w", [(64, 64, 64), (64, 37, 50), (128, 128, 128), (128, 75, 110)])
+@pytest.mark.parametrize("B,both", [(2, False), (7, True), (9, False), (45, True)])
+def test_spectra_between_each_other(oracle, N, h, w, B, both):
+    d = dev()
+    x = synth.normal((B, h, w), seed=N + B + w).to(d)
+    real = torch.empty((h, w, B), device=d).permute(2, 0, 1) if both else torch.empty((B, h, w), device=d)
+    real.copy_(x)
+    hold = torch.full((N // 2 + 1, N, B + 2, 2), 7.0, device=d)
+    view = hold[:, :, 1:1 + B].permute(2, 0, 1, 3)
+    assert F.fbfft2D(real, view, 0, N - h) == F.Success
+    real.fill_(float("nan"))
+    assert F.fbifft2D(view, real, 0, N - h) == F.Success
+    torch.cuda.synchronize()
+    rc, want = oracle.fbfft2d(x.cpu().numpy(), N, 0, N - h)
+    assert rc == 0 and per_plane_rel(view.cpu().numpy(), want) < TOL_FFT
+    assert per_plane_rel(real.cpu().numpy(), N * N * x.cpu().numpy().astype(np.float64)) < TOL_FFT * np.sqrt(N * N / (h * w))
+    view.fill_(7.0)
+    assert bool((hold == 7.0).all())
