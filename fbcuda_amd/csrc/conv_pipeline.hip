@@ -1691,6 +1691,8 @@ static bool runsPoint(int N, bool named, int H, int W, int kH, int kW) {
   return kH == 1 && kW == 1 && H * W >= 4 && (!named || N > 32);
 }
 
+static_assert(ConvRoute::Windows + GemmPlan::Split + 1 == ConvRoute::Point, "each kind of contraction has a route");
+
 ConvRoute convRoute(int pass, int N, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
   const bool named = N != 0;
   if (!named) N = fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW);

@@ -49,8 +49,8 @@ class ConvRoute(ctypes.Structure):
     _fields_ = [("kind", ctypes.c_int), ("N", ctypes.c_int), ("splits", ctypes.c_int)]
 
 
-# what a layer pass runs on: convSmall, plane-major spectra, or windows with binGemm<name>
-SMALL, PLANE_MAJOR, REGS_SPLIT_K, REGS_WIDE, REGS_NARROW, DIRECT64, DIRECT128, SPLIT = range(8)
+# what a layer pass runs on: convSmall, plane-major spectra, windows with binGemm<name>, or the products of filters of 1 x 1
+SMALL, PLANE_MAJOR, REGS_SPLIT_K, REGS_WIDE, REGS_NARROW, DIRECT64, DIRECT128, SPLIT, POINT = range(9)
 
 
 def conv_route(pass_, N, B, cin, cout, H, W, kH, kW=None):
@@ -59,7 +59,7 @@ def conv_route(pass_, N, B, cin, cout, H, W, kH, kW=None):
     fn = F.lib()._ZN9fbfft_amd9convRouteEiiiiiiiii
     fn.argtypes, fn.restype = [ctypes.c_int] * 9, ConvRoute
     kW = kH if kW is None else kW
-    r = fn(pass_, N or F.conv_choose_fft_size(pass_, B, cin, cout, H, W, kH, kW), B, cin, cout, H, W, kH, kW)
+    r = fn(pass_, N, B, cin, cout, H, W, kH, kW)
     return r.kind, r.N, r.splits
 
 

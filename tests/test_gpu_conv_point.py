@@ -1,24 +1,14 @@
 """Layers with filters of 1 x 1, whose passes are products of matrices without transforms (conv_point.hip),
 against fp64 products; which calls those are, and what the others still give."""
-import ctypes
-
 import numpy as np
 import pytest
 import torch
 
 import fbcuda_amd as F
 from fbcuda_amd import synth
-from gpu_util import ConvRoute, dev, rel
+from gpu_util import POINT, conv_route, dev, rel
 
 pytestmark = pytest.mark.gpu
-POINT = 8
-
-
-def route(pass_, N, B, cin, cout, H, W):
-    """The library's own host function; N = 0: the size is left to the library."""
-    fn = F.lib()._ZN9fbfft_amd9convRouteEiiiiiiiii
-    fn.argtypes, fn.restype = [ctypes.c_int] * 9, ConvRoute
-    return fn(pass_, N, B, cin, cout, H, W, 1, 1).kind
 
 
 def bar(terms):
@@ -41,7 +31,7 @@ def run(x, w, g, N, accumulate=False, scale=1.0, before=None, point=(True, True,
     d = dev()
     for p in (0, 1, 2):
         if point[p] is not None:
-            assert (route(p, N, B, cin, cout, H, W) == POINT) == point[p]
+            assert (conv_route(p, N, B, cin, cout, H, W, 1)[0] == POINT) == point[p]
     size = max(F.conv_workspace_image(p, B, cin, cout, H, W, 1, 1, N) for p in (0, 1, 2))
     ws = torch.full((size + 256,), 77, dtype=torch.uint8, device=d)
     large = [torch.full((t.shape[0], t.shape[1] + 2) + tuple(t.shape[2:]), 7.0, device=d) for t in (g, x)]
@@ -93,7 +83,7 @@ def test_which_calls():
     compare(x, w, g, run(x, w, g, 64))
     compare(x, w, g, run(x, w, g, 32, point=(False,) * 3))
     compare(x, w, g, run(x, w, g, 16, point=(False,) * 3))
-    assert route(2, 0, 4, 5, 6, 1, 3) != POINT and route(2, 0, 4, 5, 6, 1, 4) == POINT
+    assert conv_route(2, 0, 4, 5, 6, 1, 3, 1)[0] != POINT and conv_route(2, 0, 4, 5, 6, 1, 4, 1)[0] == POINT
 
 
 def test_filters_in_another_order_scale_and_accumulate():
