@@ -248,7 +248,6 @@ int checkConvShapes(int pass, const fbfft_tensor* input, const fbfft_tensor* wei
                     const fbfft_tensor* output, int N) {
   if (!okTensor(input, 4) || !okTensor(weight, 4) || !okTensor(output, 4))
     return FBFFT_UNSUPPORTED_DIMENSION;
-  const bool named = N != 0;
   N = resolveFftSize(N, pass, input, weight);
   if (!convSizeOk(N)) return FBFFT_UNSUPPORTED_SIZE;
   const int B = input->size[0], Cin = input->size[1], H = input->size[2], W = input->size[3];
