@@ -1687,8 +1687,20 @@ static bool smallMayRun(const float* x, const int* xStride, const int* xSize, co
 // product then (conv_point.hip).  us, transforms / product, forward, input gradient, weight gradient: 45 x 79 x 118 x 118,
 // 50 filters 283, 306, 326 / 93, 100, 124; 175 x 21 x 186 x 187, 21 723, 723, 852 / 210, 211, 218; 16 x 27 x 120 x 120, 100 91,
 // 85, 123 / 31, 27, 39; 11 x 13 x 37 x 37, 298 28, (sums 14), 33 / 9, -, 16.  Of 40 random layers none took longer.
-static bool runsPoint(int N, bool named, int H, int W, int kH, int kW) {
-  return kH == 1 && kW == 1 && H * W >= 4 && (!named || N > 32);
+//
+// But where results are few, up to a workgroup of 16 rows x 64 groups of pixels per CU, the product is one chain of loads over all
+// contracted planes, 0.045 to 0.061 us each, while the windows' contraction is cut into ranges: there transforms that
+// are expected to be faster keep the pass (the estimate is 10 to 50 % high in that range).  us, transforms / product, forward: 1 x 4000 x 4
+// x 4, 64 filters 52 / 192; 64 x 1400 x 8 x 8, 256 69 / 83; but 64 x 1000 x 8 x 8, 256 55 / 51, 1 x 4100 x 28 x 28, 400 295 /
+// 237; input gradient 64 x 64 x 8 x 8, 1000 28 / 47.
+static bool runsPoint(int pass, int N, bool named, PassSize size, int B, int Cin, int Cout, int H, int W, int kH, int kW) {
+  if (kH != 1 || kW != 1 || H * W < 4 || (named && N <= 32)) return false;
+  if (pass == 2) return true;
+  const int planes = pass == 0 ? Cin : Cout, rows = pass == 0 ? Cout : Cin;
+  if (std::ceil((double)B * ceilDiv(H * W, 4) / 64) * ceilDiv(rows, 16) > computeUnits()) return true;
+  const double transforms = size.N > 32 ? planeMajorMicroseconds(pass, size.N, B, Cin, Cout)
+                                        : windowsPass(pass, size.N, B, Cin, Cout, H, W, 1, 1, size.maxSplits).us;
+  return 3 + 0.055 * planes <= transforms / 1.2;
 }
 
 static_assert(ConvRoute::Windows + GemmPlan::Split + 1 == ConvRoute::Point, "each kind of contraction has a route");
@@ -1698,7 +1710,7 @@ ConvRoute convRoute(int pass, int N, int B, int Cin, int Cout, int H, int W, int
   if (!named) N = fbfft_conv_choose_fft_size(pass, B, Cin, Cout, H, W, kH, kW);
   const PassSize size = passSize(pass, N, B, Cin, Cout, H, W, kH, kW);
   if (runsSmall(pass, size.N, B, Cin, Cout, H, W, kH, kW)) return {ConvRoute::Small, size.N, 1};
-  if (runsPoint(N, named, H, W, kH, kW)) return {ConvRoute::Point, size.N, 1};
+  if (runsPoint(pass, N, named, size, B, Cin, Cout, H, W, kH, kW)) return {ConvRoute::Point, size.N, 1};
   if (size.N > 32) return {ConvRoute::PlaneMajor, size.N, 1};
   const GemmPlan plan = windowsPass(pass, size.N, B, Cin, Cout, H, W, kH, kW, size.maxSplits).plan;
   return {ConvRoute::Windows + plan.kind, size.N, plan.splits};
@@ -1723,7 +1735,7 @@ int launchConvPass(int pass, int N, bool named, float* x, const int* xStride, co
   if (runsSmall(pass, N, in[0], wt[1], wt[0], H, W, kH, kW) &&
       smallMayRun(x, xStride, xSize, y, yStride, ySize, out, outStride, outSize))
     return launchConvSmall(pass, x, xStride, xSize, y, yStride, ySize, out, outStride, outSize, s);
-  if (runsPoint(given, named, H, W, kH, kW) &&
+  if (runsPoint(pass, given, named, size, in[0], wt[1], wt[0], H, W, kH, kW) &&
       pointMayRun(pass, x, xStride, xSize, y, yStride, ySize, out, outStride, outSize))
     return launchConvPoint(pass, x, xStride, xSize, y, yStride, ySize, out, outStride, outSize, scale, accumulate,
                            workspace, pass == 2 ? convWorkspaceBytes(2, given, in[0], wt[1], wt[0], H, W, 1, 1) : 0, s);

@@ -271,7 +271,8 @@ size_t fbfft_make_tiles_for_pass(int pass, const fbfft_tensor* input, const fbff
  * of those calls; a result that overlaps an operand keeps the transforms).  Filters of 1 x 1
  * are one product of matrices per pass, without transforms, with size 0, 64 or 128 (8, 16 and 32 name the
  * transforms that they run on) where the planes of both image-sized tensors have no gaps and at least four
- * elements; the weight gradient is reproducible there, too. */
+ * elements; the weight gradient is reproducible there, too.  (Forward passes and input gradients of few results
+ * over very many planes keep the transforms where these are expected to be faster.) */
 int fbfft_conv_choose_fft_size(int pass, int batch, int cin, int cout, int H, int W, int kH,
                                int kW);
 

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 import fbcuda_amd as F
-from gpu_util import (DIRECT, LANES, REGISTERS, REGS_NARROW, REGS_SPLIT_K, REGS_WIDE, conv_route, pass_size,
+from gpu_util import (DIRECT, LANES, POINT, REGISTERS, REGS_NARROW, REGS_SPLIT_K, REGS_WIDE, conv_route, pass_size,
                       product_route)
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -445,3 +445,15 @@ def test_calls_without_the_native_module_go_the_general_way(monkeypatch, tmp_pat
         assert F.fbfft1D(x, y) == F.UnsupportedSize
     assert calls == ["on_gpu"] * 2
     assert [w.category for w in seen] == ([RuntimeWarning] if built else [])
+
+
+# filters of 1 x 1 whose results are too few for a workgroup per CU: a long chain over the contracted planes keeps the
+# transforms, which cut it into ranges (us, transforms / product: 52 / 192, 73 / 236, 69 / 83, 28 / 47, 45 / 108); not where the
+# transforms take longer (295 / 237, 446 / 197, 55 / 51), nor where results are many
+@pytest.mark.parametrize("pass_,N,B,cin,cout,H,W,product", [
+    (0, 0, 1, 4000, 64, 4, 4, False), (0, 64, 64, 4100, 64, 8, 8, False), (0, 0, 64, 1400, 256, 8, 8, False),
+    (1, 0, 64, 64, 1000, 8, 8, False), (1, 0, 1, 64, 2000, 56, 56, False),
+    (0, 0, 1, 4100, 400, 28, 28, True), (0, 64, 1, 4096, 1000, 2, 2, True),
+    (0, 0, 64, 4100, 256, 14, 14, True), (1, 0, 64, 600, 4100, 14, 14, True), (2, 0, 1, 4000, 64, 4, 4, True)])
+def test_long_chains_of_1x1_filters_keep_the_transforms(pass_, N, B, cin, cout, H, W, product):
+    assert (conv_route(pass_, N, B, cin, cout, H, W, 1)[0] == POINT) == product
