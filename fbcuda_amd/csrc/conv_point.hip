@@ -137,8 +137,8 @@ struct PointGradArgs {
   const float* x;
   float* part;
   long gB, gM, xB, xC;
-  int C, M, pixels, images;
-  int mTiles, cTiles, ranges, chunks, chunksPerImage;  // chunks of kGradPixels pixels
+  int C, M, pixels, words, groups;  // words: groups of four pixels of an image; groups: of all images
+  int mTiles, cTiles, ranges, chunks;  // chunks of kGradPixels pixels
   int total;
 };
 
@@ -146,7 +146,10 @@ constexpr int kGradPixels = 64;
 
 // The weight gradient: a workgroup takes 32 WM x 32 WC filters over a range of the pixels of all images, 64 at
 // a time through LDS, four waves of 32 x 32; waves that share such a tile take every other (every fourth) eight
-// pixels and add up in wave order.  Its partial sums go to part[range][m][c].
+// pixels and add up in wave order.  Its partial sums go to part[range][m][c].  The 64 pixels are 16 groups of four
+// neighbours of any images, so that small planes, and the ends of others, are not filled up with zeros (us, windows of 8
+// points / 64 pixels of one image / so: 3005 x 3412 x 2 x 2, 195 3904 / 5031 / 296; 493 x 828 x 3 x 5, 199 179 / 215 / 68; 128 x 1203 x 6
+// x 6, 218 84 / 101 / 57).
 template <int WM, int WC>
 __global__ __launch_bounds__(256, 3) void pointGradient(PointGradArgs a) {
   constexpr int ROW = kGradPixels + 4, WK = 4 / (WM * WC), LM = 2 * WM, LC = 2 * WC;
@@ -166,16 +169,16 @@ __global__ __launch_bounds__(256, 3) void pointGradient(PointGradArgs a) {
   const int px = 4 * (t % 16), row = t / 16;
   floatx4 vm[LM], vc[LC];
   auto request = [&](int chunk) __attribute__((always_inline)) {
-    const int b = chunk / a.chunksPerImage, p = (chunk - b * a.chunksPerImage) * kGradPixels + px;
-    const int from = min(p, a.pixels - 4);
+    const int group = chunk * (kGradPixels / 4) + t % 16, known = min(group, a.groups - 1);
+    const int b = (unsigned)known / (unsigned)a.words, p = 4 * (known - b * a.words), from = min(p, a.pixels - 4);
 #pragma unroll
     for (int i = 0; i < LM; ++i) vm[i] = *(GlobalFour)(a.g + b * a.gB + min(m0 + row + 16 * i, a.M - 1) * a.gM + from);
 #pragma unroll
     for (int i = 0; i < LC; ++i) vc[i] = *(GlobalFour)(a.x + b * a.xB + min(c0 + row + 16 * i, a.C - 1) * a.xC + from);
-    return p - from;
+    return group < a.groups ? p - from : 4;
   };
   int d = 0;
-  // the last pixels of an image: those that are there, shifted into place, then zeros
+  // the last pixels of an image: those that are there, shifted into place, then zeros (behind the last image zeros only)
   auto park = [&](float* to, floatx4 f) __attribute__((always_inline)) {
     floatx4 u = f;
     if (d != 0) {
@@ -323,11 +326,11 @@ int launchConvPoint(int pass, const float* x, const int* xStride, const int* xSi
   PointGradArgs a{};
   a.x = x; a.g = y; a.part = static_cast<float*>(workspace);
   a.xB = xStride[0]; a.xC = xStride[1]; a.gB = yStride[0]; a.gM = yStride[1];
-  a.C = xSize[1]; a.M = ySize[1]; a.images = xSize[0]; a.pixels = xSize[2] * xSize[3];
+  a.C = xSize[1]; a.M = ySize[1]; a.pixels = xSize[2] * xSize[3];
+  a.words = ceilDiv(a.pixels, 4); a.groups = xSize[0] * a.words;
   const int wm = a.M <= 32 ? 1 : 2, wc = a.C <= 32 ? 1 : 2;
   a.mTiles = ceilDiv(a.M, 32 * wm); a.cTiles = ceilDiv(a.C, 32 * wc);
-  a.chunksPerImage = ceilDiv(a.pixels, kGradPixels);
-  a.chunks = a.images * a.chunksPerImage;
+  a.chunks = ceilDiv(a.groups, kGradPixels / 4);
   a.ranges = pointRanges(a, wm, wc, room);
   a.total = a.mTiles * a.cTiles * a.ranges;
   const dim3 grid = padded(a.total), block(256);

@@ -69,7 +69,10 @@ def compare(x, w, g, got, scale=1.0, before=0.0):
 @pytest.mark.parametrize("B,cin,cout,H,W", [
     (40, 33, 65, 23, 23), (300, 16, 17, 2, 2), (77, 130, 64, 5, 3), (9, 300, 129, 31, 30), (16, 3, 200, 57, 61),
     (3, 128, 250, 64, 63), (5, 127, 96, 100, 31), (1, 257, 300, 41, 45), (20, 65, 33, 37, 29), (260, 40, 140, 7, 1),
-    (64, 5, 31, 90, 91), (130, 32, 32, 64, 64), (128, 20, 48, 66, 65)])
+    (64, 5, 31, 90, 91), (130, 32, 32, 64, 64), (128, 20, 48, 66, 65),
+    # 64 pixels of a weight gradient's turn out of many images, the last turn partly filled; one to three turns in a range
+    (1, 40, 50, 2, 2), (17, 33, 40, 3, 3), (3, 47, 46, 7, 7), (40, 20, 50, 7, 7), (138, 47, 46, 7, 7), (33, 110, 346, 8, 8),
+    (500, 9, 70, 5, 1), (129, 65, 20, 3, 5), (64, 31, 33, 6, 11)])
 def test_products_vs_fp64(B, cin, cout, H, W):
     x, w, g = operands(B, cin, cout, H, W, extra=1)
     # (small passes are summed in one launch by conv_small.hip)
