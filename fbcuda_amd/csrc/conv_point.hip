@@ -286,12 +286,14 @@ bool pointMayRun(int pass, const float* x, const int* xStride, const int* xSize,
 // every CU a few times over (us, 45 x 79 x 118 x 118, 50 filters: 128 ranges of one tile 134, 256 124, 512 127; 175
 // x 21 x 186 x 187, 21, whose workgroups are smaller: 256 336, 512 229, 1024 218; 69 x 3 x 94 x 94, 45: 256 51, 512 57,
 // 1024 75, to add up), of at least four turns each once there are sixteen (3 x 5 x 11 x 11, 249, six turns: one range
-// 13.3, six 7.5).
+// 13.3, six 7.5); and of two, or one up to 32 ranges, while there are no more workgroups than CUs (at least four / so: 138 x 47 x 7 x 7,
+// 46 18.1 / 13.2, windows of 8 points 14.8; 12 x 20 x 16 x 16, 50 8.1 / 7.2).
 static int pointRanges(const PointGradArgs& a, int wm, int wc, size_t room) {
   const int tiles = a.mTiles * a.cTiles, target = wm * wc == 1 ? 1024 : wm * wc == 2 ? 320 : 640;
   const size_t bytes = sizeof(float) * 1024 * wm * wc * tiles;
   const long fit = (long)std::min<size_t>(room / bytes, 1 << 20);
-  return (int)std::max<long>(1, std::min<long>({ceilDiv(target, tiles), fit, std::max(a.chunks / 4, std::min(a.chunks, 16))}));
+  const int few = std::min(std::max(a.chunks / 2, std::min(a.chunks, 32)), computeUnits() / tiles);
+  return (int)std::max<long>(1, std::min<long>({ceilDiv(target, tiles), fit, std::max({a.chunks / 4, std::min(a.chunks, 16), few})}));
 }
 
 // room: bytes of workspace (weight gradients; at least one range fits any pass's workspace, which holds spectra
