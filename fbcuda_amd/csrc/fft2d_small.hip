@@ -427,9 +427,12 @@ bool dense(const RealView& r, int groups) {
 }
 
 // Inverse, the stream writes every float of a window from LDS, so the transform has to cover the window whole: one that
-// hangs over its edge, or is larger, keeps what it held there (and P of them need not fit in LDS).
-bool covered(int N, const RealView& r, int padL, int padU) {
-  return (long)padL + r.w <= N && (long)padU + r.h <= N;
+// hangs over its edge, or is larger, keeps what it held there (and P of them need not fit in LDS).  And the turn through LDS pays
+// where windows are a good part of the planes: four ninths, at 8 points a quarter.  Window -> Dense, us, 1250 groups of 3 x 5 in 32
+// points 6.1 -> 6.7, of 14 x 5 6.6 -> 7.0, 1500 of 22 x 16 8.1 -> 7.6, of 22 x 30 9.9 -> 8.0; 1250 of 7 x 15 in 16 4.3 -> 4.7, of 15 x
+// 8 4.8 -> 4.7; 6000 of 4 x 1 in 8 5.1 -> 5.3, 3500 of 4 x 4 4.6 -> 4.0.
+bool streams(int N, const RealView& r, int padL, int padU) {
+  return (long)padL + r.w <= N && (long)padU + r.h <= N && (N == 8 ? 16 : 9) * r.h * r.w >= 4 * N * N;
 }
 
 // Forward, the loads of every other column meet in the L1, and the turn through LDS pays where waves would
@@ -481,7 +484,7 @@ int launchInverse(const CplxView& cplx, const RealView& real, int padL, int padU
   using C = SmallCfg<N, PACKED>;
   const int groups = ceilDiv(real.B, C::P);
   const int mode = fastReal(N, real, padL, padU)                               ? Whole
-                   : covered(N, real, padL, padU) && dense(real, groups) ? Dense
+                   : streams(N, real, padL, padU) && dense(real, groups) ? Dense
                                                                                : Window;
   dim3 block(64);
   withModes(mode, fastCplx(N, cplx), [&](auto m, auto fc) {
