@@ -439,12 +439,17 @@ bool streams(int N, const RealView& r, int padL, int padU) {
 // otherwise take two groups, or, at 16 points, rows do not move as pairs, up to there (us, Window -> Dense):
 // 100000 windows of 7 x 7 in 8 points 11.4 -> 8.2, of 5 x 6 11.1 -> 8.0, 36000 of 13 x 13 in 16 15.0 -> 13.0, 20000
 // 8.4 -> 7.2; but 400000 of 7 x 7 31.7 -> 33.1, 160000 of 15 x 15 50.4 -> 51.2, 40000 of 14 x 14 12.8 -> 14.9, 16400
-// of 6 x 6 3.9 -> 4.2, 24576 of 23 x 23 in 32 points 28.8 -> 33.4.
+// of 6 x 6 3.9 -> 4.2, 24576 of 23 x 23 in 32 points 28.8 -> 33.4.  Nor, at 16 points, for windows of less than half a plane
+// below one and a half rounds of waves: 32000 of 7 x 15 10.4 -> 11.9, of 11 x 15 13.5 -> 12.7, 48000 of 7 x 15 15.4 -> 14.0; nor, at
+// 8, for half a plane in pairs and more than four rows: 160000 of 6 x 8 12.6 -> 13.0, 112000 of 8 x 4 9.2 -> 9.6; 160000 of 4 x 8
+// 11.8 -> 10.6.
 template <int N>
 bool denseForward(const RealView& r, int padL, int groups) {
-  if (N == 8) return pairGroups<N>(groups);
   const bool pairs = windowMovesAsPairs(r.data, r.sy, r.sx, r.w, padL) && r.sb % 2 == 0;
-  return !pairs && 4L * groups <= 7 * residentWaves<N>();
+  const int area = r.h * r.w;
+  if (N == 8) return pairGroups<N>(groups) && !(pairs && 2 * area >= N * N && 2 * r.h > N);
+  const long slots = residentWaves<N>();
+  return !pairs && 4L * groups <= 7 * slots && (2 * area >= N * N || 4L * groups >= 6 * slots);
 }
 
 // runs f(mode of the real operand, std::bool_constant<fast>{})

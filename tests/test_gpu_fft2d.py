@@ -370,7 +370,9 @@ def test_windows_beside_the_rows_of_a_wave(oracle, N, h, w, padL, padU):
     (16, 31003, 13, 13, 0, 0), (8, 16369, 7, 7, 0, 1), (8, 16371, 3, 5, 3, 4), (8, 100003, 7, 5, 1, 1), (8, 100001, 1, 1, 7, 0),
     # inverse windows either side of four ninths of a plane, at 8 points a quarter
     (32, 4101, 15, 31, 0, 0), (32, 4101, 14, 32, 0, 1), (16, 8203, 9, 13, 2, 0), (16, 8203, 8, 14, 0, 0),
-    (8, 16389, 4, 4, 1, 2), (8, 16389, 3, 5, 0, 0)])
+    (8, 16389, 4, 4, 1, 2), (8, 16389, 3, 5, 0, 0),
+    # forward either side of half a plane and, below it, of one and a half rounds of waves; pairs of 8 points
+    (16, 9001, 9, 15, 1, 0), (16, 9002, 8, 15, 0, 2), (16, 46003, 8, 15, 0, 0), (8, 160001, 6, 8, 0, 1), (8, 160003, 5, 8, 0, 0)])
 def test_windows_that_move_as_streams(oracle, N, B, h, w, padL, padU):
     d = dev()
     x = synth.normal((B, h, w), seed=B).to(d)
