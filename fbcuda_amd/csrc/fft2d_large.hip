@@ -112,7 +112,8 @@ __device__ __forceinline__ int columnPlace(int column, int c, int k, int l) {
 // where the inverse leaves the packed value j of row y: two rows side by side
 __device__ __forceinline__ int sampleAt(int y, int j) { return y * 64 + (j ^ (8 * (y & 1))); }
 
-template <bool FAST_REAL, bool FAST_CPLX>
+// BY_ROW: a wave takes row after row, 64 samples to an instruction, and turns them in LDS (launchForward128)
+template <bool FAST_REAL, bool FAST_CPLX, bool BY_ROW = false>
 __global__ __launch_bounds__(kLanes128, 4) void fft2d128Forward(RealView real, CplxView cplx, int padL, int padU) {
   __shared__ __align__(16) c32 cb[64 * kStride128];
   __shared__ __align__(8) c32 tw[256];
@@ -139,12 +140,38 @@ __global__ __launch_bounds__(kLanes128, 4) void fft2d128Forward(RealView real, C
     // between them, and what lies outside counts as zero; whole pairs where the window has only such
     const bool pairs = real.sx == 1 && ((real.sy | real.sb | padL | real.w) & 1) == 0 &&
                        (reinterpret_cast<uintptr_t>(real.data) & 7) == 0;
+    if constexpr (BY_ROW) {
+      const int left = min(max(a.lane - padL, 0), real.w - 1), right = min(max(a.lane + 64 - padL, 0), real.w - 1);
+      staticFor<2>([&](auto ii) {
+        constexpr int i = decltype(ii)::value;
+        if (!any(i)) return;
+        float in[8][2];
+        staticFor<8>([&](auto rr) {
+          constexpr int r = decltype(rr)::value;
+          const float* const row = src + (size_t)min(max(64 * i + 8 * a.wave + r - padU, 0), real.h - 1) * real.sy;
+          in[r][0] = row[(size_t)left * real.sx];
+          in[r][1] = row[(size_t)right * real.sx];
+        });
+        staticFor<16>([&](auto rr) {
+          constexpr int r = decltype(rr)::value / 2, j = decltype(rr)::value % 2;
+          const int x = a.lane + 64 * j;
+          reinterpret_cast<float*>(cb + sampleAt(64 * i + 8 * a.wave + r, x / 2))[x % 2] = in[r][j];
+        });
+      });
+      waveExchange();
+    }
     staticFor<2>([&](auto ii) {
       constexpr int i = decltype(ii)::value;
       const int y = 64 * i + 8 * a.wave + a.r - padU;
       const bool yIn = (unsigned)y < (unsigned)real.h;
       const float* row = src + (size_t)min(max(y, 0), real.h - 1) * real.sy;
-      if (any(i) && pairs) {
+      if constexpr (BY_ROW) {
+        if (any(i))
+          staticFor<8>([&](auto mm) {
+            constexpr int m = decltype(mm)::value;
+            z[i][m] = cb[sampleAt(64 * i + 8 * a.wave + a.r, a.l + 8 * m)];
+          });
+      } else if (any(i) && pairs) {
         staticFor<8>([&](auto mm) {
           const int x = 2 * (a.l + 8 * decltype(mm)::value) - padL;
           z[i][decltype(mm)::value] = *reinterpret_cast<const c32*>(row + min(max(x, 0), real.w - 2));
@@ -1045,15 +1072,22 @@ int launchInverse64(const CplxView& cplx, const RealView& real, int padL, int pa
   return launchStatus();
 }
 
+// Samples four floats apart, in rows of most of the plane: row after row.  (us, one lane of eight rows loads from each / so, four
+// lanes of 32 points, which walked down columns, before: one plane 12.7 / 10.5, 11.1; 300 23.1 / 21.6, 22.1; but 300 windows of 101
+// x 90 15.4 / 16.6, and 300 planes of every second float 14.5 / 15.7.)
 int launchForward128(const RealView& real, const CplxView& cplx, int padL, int padU, hipStream_t s) {
-  const bool fr = fastReal(128, real, padL, padU), fc = fastCplx(128, cplx);
+  const bool fr = fastReal(128, real, padL, padU), fc = fastCplx(128, cplx), rows = abs(real.sx) == 4 && real.w >= 104;
   const dim3 grid = fr && fc ? dim3(real.B) : planeGrid(real, cplx), block(kLanes128);
   if (fr && fc)
     fft2d128Forward<true, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+  else if (fc && rows)
+    fft2d128Forward<false, true, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
   else if (fc)
     fft2d128Forward<false, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
   else if (fr)
     fft2d128Forward<true, false><<<grid, block, 0, s>>>(real, cplx, padL, padU);
+  else if (rows)
+    fft2d128Forward<false, false, true><<<grid, block, 0, s>>>(real, cplx, padL, padU);
   else
     fft2d128Forward<false, false><<<grid, block, 0, s>>>(real, cplx, padL, padU);
   return launchStatus();

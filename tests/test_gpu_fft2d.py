@@ -543,3 +543,25 @@ def test_spectra_between_each_other(oracle, N, h, w, B, both):
     assert per_plane_rel(real.cpu().numpy(), N * N * x.cpu().numpy().astype(np.float64)) < TOL_FFT * np.sqrt(N * N / (h * w))
     view.fill_(7.0)
     assert bool((hold == 7.0).all())
+
+
+# samples four floats apart: planes and windows of 128 points either side of 104 columns, which are read row by row from there on
+@pytest.mark.parametrize("h,w,padL,padU", [(128, 128, 0, 0), (128, 104, 3, 0), (77, 103, 9, 30), (5, 111, 17, 60), (61, 128, 0, 67),
+                                           (128, 127, 5, 9), (1, 120, 8, 127)])
+@pytest.mark.parametrize("B", [1, 9])
+@pytest.mark.parametrize("turned", [False, True])
+def test_forward_128_of_samples_four_apart(oracle, h, w, padL, padU, B, turned):
+    d = dev()
+    x = synth.normal((B, h, w), seed=h + w + B)
+    hold = torch.full((B, h, w, 4), float("nan"), device=d)
+    hold[..., 2] = x.to(d)
+    spec = torch.full((B + 1, 128, 65, 2) if turned else (B + 1, 65, 128, 2), 7.0, device=d)
+    view = spec[:B].transpose(1, 2) if turned else spec[:B]
+    assert F.fbfft2D(hold[..., 2], view, padL, padU) == F.Success
+    torch.cuda.synchronize()
+    assert bool((spec[B] == 7.0).all())
+    plane = np.zeros((B, 128, 128), np.float32)
+    ch, cw = min(h, 128 - padU), min(w, 128 - padL)
+    plane[:, padU:padU + ch, padL:padL + cw] = x.numpy()[:, :ch, :cw]
+    rc, want = oracle.fbfft2d(plane, 128)
+    assert rc == 0 and per_plane_rel(view.cpu().numpy(), want) < TOL_FFT
