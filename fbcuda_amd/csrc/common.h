@@ -48,6 +48,15 @@ __device__ __forceinline__ void streamStore(float* p, float v) {
   __builtin_nontemporal_store(v, p);
 }
 
+// Orders the LDS accesses of one wave: what its lanes wrote before is what its lanes
+// read after.  A wave's LDS instructions execute in order, so passes whose places one wave owns
+// need no workgroup barrier between them - only the compiler has to keep the accesses in program order.
+__device__ __forceinline__ void waveExchange() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 inline bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 
 // status of the launches just made; the error is consumed, so that one failed

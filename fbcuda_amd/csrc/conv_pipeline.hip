@@ -105,16 +105,6 @@ struct PlaneSet {
   int numTiles;             // tiles per image
 };
 
-// Orders the LDS accesses of one wave: what its lanes wrote before is what its lanes
-// read after.  The lanes that share a plane sit in one wave, and a wave's LDS
-// instructions execute in order, so the passes over a plane need no workgroup barrier
-// between them - only the compiler has to keep the accesses in program order.
-__device__ __forceinline__ void planeSync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 struct PlaneWindow {
   float* p;
   int h, w, padL, padU;
@@ -279,7 +269,7 @@ __device__ __forceinline__ void forwardBinMajorBody(const ForwardJob& job, int w
   c32 za0[H], za1[H];
   load(ra, za0, za1);
   columnPassForward<N, PAIRS == 0>(za0, za1, plane, l);
-  planeSync();  // the lanes of a plane sit in one wave
+  waveExchange();  // the lanes of a plane sit in one wave
   if constexpr (GROUPS == 2) {
     const int rb = ra + SLOTS;
     const bool second = rb < Rp;  // the same for the whole workgroup
@@ -291,7 +281,7 @@ __device__ __forceinline__ void forwardBinMajorBody(const ForwardJob& job, int w
     if (second) {
       __syncthreads();  // every wave has copied the first run out of the plane buffers
       columnPassForward<N, PAIRS == 0>(zb0, zb1, plane, l);
-      planeSync();
+      waveExchange();
       rowPassInPlace<N, true>(plane, l);
       __syncthreads();
       copyOut(rb);
@@ -368,9 +358,9 @@ __global__ __launch_bounds__(kTF) void inverseBinMajor(const float2* Cs, int I, 
       plane[l] = q;
       plane[l == 0 ? H : N - l] = qm;
     }
-    planeSync();
+    waveExchange();
     rowPassInPlace<N, false>(plane, l);
-    planeSync();
+    waveExchange();
     c32 z0[H], z1[H];
     // PAIRS = 0, no 8-byte stores: a lane takes columns l and l + N/2, so that each store
     // instruction writes a contiguous run per plane (the 27 x 27 layer: 102.4 -> 101.5 us).

@@ -443,13 +443,6 @@ __device__ __forceinline__ int exchangeAt(const Rows256& c, int k, int l) {
   return k * 64 + c.row * 8 + (l ^ (k & 7));
 }
 
-// what the wave wrote to LDS is there for all of its lanes
-__device__ __forceinline__ void waveExchange() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ c32 choose(bool first, c32 a, c32 b) {
   return c32{first ? a.x : b.x, first ? a.y : b.y};
 }

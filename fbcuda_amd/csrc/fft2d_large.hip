@@ -96,13 +96,6 @@ dim3 planeGrid(const RealView& r, const CplxView& c) { return dim3(interleaved(r
 // (At 64 points a column at a time takes 0.80 and 0.86 of what it took then.)
 __device__ __forceinline__ bool nearAcross(const CplxView& c) { return abs(c.sr) < abs(c.sc); }
 
-// what the wave wrote to LDS is there for all of its lanes
-__device__ __forceinline__ void waveExchange() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // where a row keeps value l of class k between its two steps, and column c of a pair value l of class k
 // (of either parity for the two columns): sixteen lanes meet different places on both sides
 __device__ __forceinline__ int rowPlace(int k, int l, int y) { return (k * 8 + (l ^ k)) * kStride128 + y; }

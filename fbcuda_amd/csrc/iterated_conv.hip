@@ -138,14 +138,6 @@ __device__ __forceinline__ void ldsBarrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The lanes of a plane sit in one wave, whose LDS instructions execute in order: only the
-// compiler has to keep them in program order.
-__device__ __forceinline__ void planeSync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // How the planes of one wave are fetched.  Their windows usually lie in one tensor: then a
 // row's address is a scalar base (step and row) plus a lane's 32-bit offset that never
 // changes, and a load costs no vector arithmetic.
@@ -443,12 +435,12 @@ __global__ __launch_bounds__(kThreads) void iteratedConvKernel(ConvArgs a) {
         ldsBarrier();  // the spectra of the previous iteration are consumed by everybody
         storeColumns<N>(p0, p1, plane, l);
       }
-      planeSync();
+      waveExchange();
       rowPassInPlace<N, true>(plane, l);
-      planeSync();
+      waveExchange();
       {  // packed row 0, P[x] = F0[x] + i FH[x], to its virtual bins
         const c32 p = plane[l], m = plane[l == 0 ? H : N - l];
-        planeSync();
+        waveExchange();
         plane[l] = l == 0 ? c32{p.x, m.x} : c32{0.5f * (p.x + m.x), 0.5f * (p.y - m.y)};
         plane[H + l] = l == 0 ? c32{p.y, m.y} : c32{0.5f * (p.y + m.y), 0.5f * (m.x - p.x)};
       }
@@ -556,13 +548,13 @@ __global__ __launch_bounds__(kThreads) void iteratedConvKernel(ConvArgs a) {
         q = c32{c0.x, cH.x};
         qm = c32{c0.y, cH.y};
       }
-      planeSync();
+      waveExchange();
       planeE[le] = q;
       planeE[le == 0 ? H : N - le] = qm;
     }
-    planeSync();
+    waveExchange();
     rowPassInPlace<N, false>(planeE, le);
-    planeSync();
+    waveExchange();
     {
       columnPassInverse<N>(planeE, le, z0, z1);
       const int ai = a0 + RA * rd + se / FO;
