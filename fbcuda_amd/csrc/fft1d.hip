@@ -663,7 +663,16 @@ int launchFft1d(bool forward, int N, float* real, int sb, int sx, float* cplx, i
       case 8: mid(std::integral_constant<int, 8>{}, oneWave); break;
       case 16: mid(std::integral_constant<int, 16>{}, oneWave); break;
       case 32: mid(std::integral_constant<int, 32>{}, oneWave); break;
-      case 64: mid(std::integral_constant<int, 64>{}, oneWave); break;
+      case 64: {
+        // (9 waves per CU; forward, a round of them, 147456 rows, to 1.8, 256 lanes / 64: 160000 14.6 / 15.3, 200000 15.9 / 17.2, 262000 20.2 /
+        // 20.8, but 140000 13.5 / 10.3, 275000 22.7 / 21.5)
+        const long waves = ceilDiv(B, 64), round = 9L * computeUnits();
+        if (forward && waves > round && 5 * waves <= 9 * round)
+          mid(std::integral_constant<int, 64>{}, std::integral_constant<int, 256>{});
+        else
+          mid(std::integral_constant<int, 64>{}, oneWave);
+        break;
+      }
       case 128:
         if (ceilDiv(B, 128) <= computeUnits())
           mid(std::integral_constant<int, 128>{}, std::integral_constant<int, 128>{});

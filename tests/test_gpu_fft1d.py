@@ -191,9 +191,11 @@ def test_inverse_of_256_ignores_imaginary_ends(oracle):
     assert rc == rc2 == F.Success and np.array_equal(got, clean)
 
 
-# ends of the workgroups of 64 rows (up to 64 points) and of 64 and 128 (128 points, either side of the switch)
+# ends of the workgroups of 64 rows (up to 64 points; 256 forward between one and 1.8 rounds of waves) and of 64 and 128
+# (128 points, either side of the switch)
 @pytest.mark.parametrize("N,B", [(8, 63), (8, 65), (16, 64), (16, 129), (32, 127), (32, 4097), (64, 1), (64, 191),
-                                 (128, 63), (128, 65), (128, 32768), (128, 32769), (128, 32897)])
+                                 (128, 63), (128, 65), (128, 32768), (128, 32769), (128, 32897),
+                                 (64, 147456), (64, 147457), (64, 200003), (64, 265408), (64, 265409)])
 def test_ends_of_workgroups(oracle, N, B):
     x = synth.normal((B, N), seed=N + B)
     d = dev()
