@@ -1676,7 +1676,7 @@ static bool smallMayRun(const float* x, const int* xStride, const int* xSize, co
 // way to it (64 and 128; 8 to 32 points name the transforms that they run on).  Each pass is one
 // product then (conv_point.hip).  us, transforms / product, forward, input gradient, weight gradient: 45 x 79 x 118 x 118,
 // 50 filters 283, 306, 326 / 93, 100, 124; 175 x 21 x 186 x 187, 21 723, 723, 852 / 210, 211, 218; 16 x 27 x 120 x 120, 100 91,
-// 85, 123 / 31, 27, 39; 11 x 13 x 37 x 37, 298 28, (sums 14), 33 / 9, -, 16.  Of 40 random layers none took longer.
+// 85, 123 / 31, 27, 39; 11 x 13 x 37 x 37, 298 28, (sums 14), 33 / 9, -, 16.
 //
 // But where results are few, up to a workgroup of 16 rows x 64 groups of pixels per CU, the product is one chain of loads over all
 // contracted planes, 0.045 to 0.061 us each, while the windows' contraction is cut into ranges: there transforms that

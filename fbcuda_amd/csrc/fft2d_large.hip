@@ -24,8 +24,8 @@
 // (fewer lanes with 32 points each, which formed the first butterflies from LDS, every stage between barriers)
 // -> this: 4096 planes of 128 x 128 101.5 / 96.5 -> 87.4 / 91.0, 19 planes 8.4 / 8.0 -> 6.2 / 6.2, 3773 windows of
 // 73 x 91 87.0 / 85.9 -> 64.7 / 75.2; 16384 of 64 x 64 95.2 / 85.7 -> 84.4 / 84.1, 53 6.6 / 5.7 -> 4.2 / 4.6, 3247 of 36
-// x 58 22.0 / 22.8 -> 18.9 / 22.2; buffers from HBM, 5000 of 64 x 64 33.7 / 33.0 -> 29.9 / 31.5, 3000 of 60 x 60 23.8
-// / 26.5 -> 23.4 / 23.5, of 50 x 50 21.7 / 23.8 -> 17.8 / 21.7.  At 128 points LDS was the limit while its accesses collided
+// x 58 22.0 / 22.8 -> 18.9 / 22.2; buffers from HBM, 5000 of 64 x 64 33.7 / 33.0 -> 29.9 / 31.5, 3000 of 60 x 60 22.5
+// / 25.6 -> 21.1 / 23.0, of 50 x 50 21.7 / 23.6 -> 18.5 / 21.6.  At 128 points LDS was the limit while its accesses collided
 // (places from column to column 136 apart: 22.4 of 38.3 million active cycles, 94 / 105 us; 130: 3.6 of 19.4).
 #include "common.h"
 #include "fft_lds.h"

@@ -50,8 +50,8 @@ struct SmallCfg {
 //            Dense: windows one after the other in memory, 16-byte aligned base.  A group's P
 //            windows are a whole number of 16-byte words, which move as one stream; rows of any width are
 //            taken apart and put end to end in LDS.  In place of 4-byte accesses to every other column
-//            (us, before -> this): inverse of 8192 windows of 27 x 27 in 32 points 14.5 -> 11.9, 60000 of
-//            28 x 28 95 -> 70, 160000 of 15 x 15 in 16 87 -> 50, 100000 of 7 x 7 in 8 14.4 -> 7.4.
+//            (us, before -> this): inverse of 8192 windows of 27 x 27 in 32 points 13.8 -> 11.0, from HBM 16.7 ->
+//            12.1, 60000 of 28 x 28 95 -> 69, 160000 of 15 x 15 in 16 87 -> 50, 100000 of 7 x 7 in 8 13.8 -> 7.3.
 //            Window: anything else.
 // FAST_CPLX: each spectrum plane is contiguous and 16-byte aligned.
 // GPW:       groups of P planes a wave processes (1 or 2).  With 2, the loads of
