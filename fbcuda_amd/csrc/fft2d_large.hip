@@ -23,7 +23,7 @@
 // What bounds them is HBM: 6.2 and 5.9 TB/s (128 points), 6.5 and 6.4 (64).  us, forward / inverse, before
 // (fewer lanes with 32 points each, which formed the first butterflies from LDS, every stage between barriers)
 // -> this: 4096 planes of 128 x 128 101.5 / 96.5 -> 87.4 / 91.0, 19 planes 8.4 / 8.0 -> 6.2 / 6.2, 3773 windows of
-// 73 x 91 87.0 / 85.9 -> 64.7 / 75.2; 16384 of 64 x 64 95.2 / 85.7 -> 84.4 / 84.1, 53 6.6 / 5.7 -> 4.2 / 4.6, 3247 of 36
+// 73 x 91 87.0 / 85.9 -> 64.7 / 75.2; 16384 of 64 x 64 95.2 / 85.7 -> 84.4 / 84.1, 53 6.6 / 5.7 -> 4.2 / 4.7, 3247 of 36
 // x 58 22.0 / 22.8 -> 18.9 / 22.2; buffers from HBM, 5000 of 64 x 64 33.7 / 33.0 -> 29.9 / 31.5, 3000 of 60 x 60 22.5
 // / 25.6 -> 21.1 / 23.0, of 50 x 50 21.7 / 23.6 -> 18.5 / 21.6.  At 128 points LDS was the limit while its accesses collided
 // (places from column to column 136 apart: 22.4 of 38.3 million active cycles, 94 / 105 us; 130: 3.6 of 19.4).
@@ -95,6 +95,10 @@ dim3 planeGrid(const RealView& r, const CplxView& c) { return dim3(interleaved(r
 // The inverse's last row, read by a lane value after value / by sixteen lanes: 40 windows of 101 x 90 9.9 / 9.1, 1300 planes 35.2 / 32.9.
 // (At 64 points a column at a time takes 0.80 and 0.86 of what it took then.)
 __device__ __forceinline__ bool nearAcross(const CplxView& c) { return abs(c.sr) < abs(c.sc); }
+
+// The inverse's value of kx = 0 holds even samples in one part and odd ones in the other: multiplied with 1 + 0 i as a complex
+// number, even samples beyond the largest float would make NaN of the odd ones.  (64 points, one plane 4.2 -> 4.3 us.)
+__device__ __forceinline__ c32 choose(bool first, c32 a, c32 b) { return c32{first ? a.x : b.x, first ? a.y : b.y}; }
 
 // where a row keeps value l of class k between its two steps, and column c of a pair value l of class k
 // (of either parity for the two columns): sixteen lanes meet different places on both sides
@@ -449,7 +453,7 @@ __global__ __launch_bounds__(kLanes128, 4) void fft2d128Inverse(CplxView cplx, R
     staticFor<8>([&](auto ll) {
       constexpr int l = decltype(ll)::value;
       c32 v = z[i][slot<8>(l)];
-      if constexpr (l > 0) v = cmul(v, tw[4 * l * a.l]);
+      if constexpr (l > 0) v = choose(a.l == 0, v, cmul(v, tw[4 * l * a.l]));  // (see choose)
       cb[rowPlace(a.l, l, 64 * i + 8 * a.wave + a.r)] = v;
     });
   });
@@ -927,7 +931,7 @@ __global__ __launch_bounds__(kLanes64, 4) void fft2d64Inverse(CplxView cplx, Rea
     staticFor<8>([&](auto jj) {
       constexpr int j = decltype(jj)::value;
       c32 f = v[i][slot<8>(j)];
-      if constexpr (j > 0) f = cmul(f, tw[2 * j * a.l]);
+      if constexpr (j > 0) f = choose(a.l == 0, f, cmul(f, tw[2 * j * a.l]));  // (see choose)
       placed64(cb, rowValue64(classes, j) + 256 * i) = f;
     });
   });

@@ -565,3 +565,22 @@ def test_forward_128_of_samples_four_apart(oracle, h, w, padL, padU, B, turned):
     plane[:, padU:padU + ch, padL:padL + cw] = x.numpy()[:, :ch, :cw]
     rc, want = oracle.fbfft2d(plane, 128)
     assert rc == 0 and per_plane_rel(view.cpu().numpy(), want) < TOL_FFT
+
+
+@pytest.mark.parametrize("N", [64, 128])  # (up to 32 points pairs of columns travel together instead)
+def test_inverse_rows_whose_even_samples_overflow_keep_the_odd_ones(N):
+    """Of the two ends of a spectrum's rows even samples are the sums, odd ones the differences."""
+    d = dev()
+    spec = torch.zeros(3, N // 2 + 1, N, 2)
+    spec[0, 0, 0, 0], spec[0, N // 2, 0, 0] = 2e38, 1.5e38
+    spec[1, 0, 0, 0], spec[1, N // 2, 0, 0] = -2e38, 1.5e38
+    back = torch.full((3, N, N), 7.0, device=d)
+    wide = torch.full((3, N, N + 1), 7.0, device=d)
+    for to in (back, wide[:, :, :N]):
+        assert F.fbifft2D(spec.to(d), to) == F.Success
+        torch.cuda.synchronize()
+        got = to.cpu()
+        assert bool((got[0, :, ::2] == float("inf")).all()) and bool((got[1, :, 1::2] == float("-inf")).all())
+        assert float((got[0, :, 1::2].double() / 0.5e38 - 1).abs().max()) < 1e-6
+        assert float((got[1, :, ::2].double() / -0.5e38 - 1).abs().max()) < 1e-6
+        assert bool((got[2] == 0.0).all())
